@@ -76,6 +76,7 @@ int right_fpt(int D, int P, int Ff, int idr, int relRot, int i) {
 void destroy_ctx(fhip::Ctx& c) {
   if (c.device >= 0) (void)hipSetDevice(c.device);
   fhip::fused_release(c);
+  fhip::staged_release(c);
   for (auto& plane : c.graph)
     for (auto& row : plane)
       for (auto& g : row)
@@ -192,6 +193,7 @@ int fhip_create(const fhip_desc* d, fhip_ctx** out) {
       c.efn = dcopy(d->opp_extrapolate_fn, (size_t)D * F * S, c.stream);
       c.corr = dcopy(d->opp_correction, (size_t)S * F, c.stream);
       if (p.viscous) c.corru = dcopy(d->opp_correct_u, (size_t)D * S * F, c.stream);
+      fhip::staged_setup(c, d);
       c.ws = dcopy(d->w_spts, S, c.stream);
       c.wf = dcopy(d->w_face, Ff, c.stream);
       c.jginv = dcopy(d->jginv_spts, (size_t)D * S * E * D, c.stream);

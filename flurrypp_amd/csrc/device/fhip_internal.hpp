@@ -55,6 +55,15 @@ inline void poison_fill(void* p, size_t bytes) {
   (void)hipDeviceSynchronize();
 }
 
+// A dense operator kept as its non-zero entries, row by row: q entries (padded
+// with zero weights) in each of `groups` partial sums, idx the row of the
+// operand.  q == 0: too many non-zeros per row, applied dense.
+struct RowOp {
+  int m = 0, groups = 1, q = 0;
+  int* idx = nullptr;     // [m][groups][q]
+  double* w = nullptr;    // [m][groups][q]
+};
+
 struct Ctx {
   Sizes z;
   fhip_params prm;
@@ -65,6 +74,10 @@ struct Ctx {
   // operators
   double *sf = nullptr, *grad = nullptr, *efn = nullptr, *corr = nullptr, *corru = nullptr, *ws = nullptr,
          *wf = nullptr;
+  // the same operators by their non-zeros: extrapolation, gradient of all
+  // directions, gradient correction, normal-flux extrapolation and divergence
+  // over the stacked directions, divergence correction (staged path)
+  RowOp r_sf, r_grad, r_corru, r_efn, r_div, r_corr;
   // 1-D tensor-product factors for the fused path (see fhip_fused.hip)
   double* tp = nullptr;
   // metrics
@@ -140,6 +153,8 @@ struct Launch {
 };
 
 // staged path (fhip_staged.hip)
+void staged_setup(Ctx& c, const fhip_desc* d);  // the operators' non-zeros
+void staged_release(Ctx& c);
 void staged_extrapolate_u(Ctx& c);
 void staged_wave_speed(Ctx& c);
 void staged_residual(Ctx& c, int step);
