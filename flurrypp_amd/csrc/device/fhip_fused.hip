@@ -220,6 +220,9 @@ __host__ __device__ constexpr int spt_lds(int D, int P1, int s) {
 template <class R>
 struct Work {
   R *divFe = nullptr, *Ufe = nullptr, *Fne = nullptr, *disFne = nullptr, *dUce = nullptr;
+  // inviscid runs: U at the flux points of every second stage (a stage reads
+  // one of Ufe, Ufe2 and writes the other; a step starts and ends in Ufe)
+  R* Ufe2 = nullptr;
   // viscous runs: each flux point's side of the LDG flux [ele][N][F] (disFne
   // then holds that side's part of the flux jump, +-B dA - disFn), and the
   // gradient at the boundary flux points [D*N][nBnd]
@@ -235,7 +238,7 @@ struct Work {
   void* geo_mem = nullptr;
   bool ready = false;
   void release() {
-    void* ps[] = {divFe, Ufe, Fne, disFne, dUce, Bve, gBnd, Rst, Us, geo_mem};
+    void* ps[] = {divFe, Ufe, Fne, disFne, dUce, Bve, gBnd, Rst, Us, geo_mem, Ufe2};
     for (void* p : ps)
       if (p) (void)hipFree(p);
     *this = Work<R>();
@@ -250,9 +253,9 @@ struct FusedState {
          *iJe = nullptr, *norme = nullptr, *dAe = nullptr, *waveSpe = nullptr;
   int *pL = nullptr, *pR = nullptr, *bc = nullptr;
   // per element flux point, 4 * (partner flux point e*F + f) + side (0 left,
-  // 1 right) or 4 * boundary slot + 2; viscous runs: the face's normal (the
-  // left element's) at every element flux point, boundary face points by slot
-  int *fpart = nullptr, *bndT = nullptr;
+  // 1 right) or 4 * boundary slot + 2; the face's normal (the left element's)
+  // at every element flux point; boundary face points and their codes by slot
+  int *fpart = nullptr, *bndT = nullptr, *bndBc = nullptr;
   double* nfe = nullptr;
   int nBnd = 0;
   // batching: boundary-state table, element -> mesh map, per-mesh dt and activity
@@ -269,6 +272,8 @@ struct FusedState {
   // stages after the first of an RK step); otherwise from the state itself.
   // FP32 kernels always read the FP32 copy.
   bool read_stage = false;
+  // inviscid runs: the stage being formed reads U at the flux points from Ufe2
+  bool odd_stage = false;
   // stream once-touched arrays past the caches: set when U alone (FP64,
   // element-major) exceeds kStreamBytes, i.e. a stage's arrays are many times
   // the 256 MiB infinity cache
@@ -282,7 +287,7 @@ struct FusedState {
     w32.release();
     void* ps[] = {tab_mem, Ue,  U0e,     Uacc,    divF0e,    JGe,    detJe,  iJe,   norme, dAe, waveSpe, pL,
                   pR,      bc,  fpart,   bndT,    nfe,       bst,    meshDt, meshRes, eleMesh, meshStart, active, srce,
-                  dtTicket, vole};
+                  dtTicket, vole, bndBc};
     for (void* p : ps)
       if (p) (void)hipFree(p);
   }
@@ -531,7 +536,7 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
                                           const double* __restrict__ meshDt, const int* __restrict__ active,
                                           const double* __restrict__ srce, R* __restrict__ Rst, int stage,
                                           const RkB& bs, R* __restrict__ Us, int fin, R* __restrict__ Ufe,
-                                          const Tabs& tb) {
+                                          const Tabs& tb, bool hasDt, double dtIn) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1, NC = Sh::NC;
   const int EB = blockDim.x / S;
@@ -564,7 +569,7 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
   }
   if (b < nb) {
     const long long e = e0 + b;
-    const double dt = (local == 1) ? eleDt[e] : (local == 2 ? meshDt[eleMesh[e]] : *dtp);
+    const double dt = hasDt ? dtIn : ((local == 1) ? eleDt[e] : (local == 2 ? meshDt[eleMesh[e]] : *dtp));
     const bool frozen = active && !active[eleMesh[e]];
     const double dj = ld_s<NT>(&detJe[e * S + s]);
     // the stage's state inputs for every field first (uniform branches on the
@@ -655,10 +660,11 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
 }
 
 template <int D, int P, class R, bool NT>
-__device__ __forceinline__ void rk_tail(int E, const R* dv, R* sU, const R* sD, const RkArgs<R>& ra, const Tabs& tb) {
+__device__ __forceinline__ void rk_tail(int E, const R* dv, R* sU, const R* sD, const RkArgs<R>& ra, const Tabs& tb,
+                                        bool hasDt = false, double dtIn = 0) {
   rk_tail_p<D, P, R, NT>(E, dv, sU, sD, ra.mode, ra.a, ra.bcoef, ra.detJe, ra.dtp, ra.eleDt, ra.local, ra.Ue, ra.U0e,
                          ra.Uacc, ra.divF0e, ra.eleMesh, ra.meshDt, ra.active, ra.srce, ra.Rst, ra.stage, ra.bs, ra.Us,
-                         ra.fin, ra.Ufe, tb);
+                         ra.fin, ra.Ufe, tb, hasDt, dtIn);
 }
 
 // Viscous runs, FP32: the volume kernel also folds its own side's LDG part
@@ -688,33 +694,278 @@ struct VFace {
   int nBnd;
 };
 
+// calcDivF_spts of field k at point s of the block's element b, from the
+// transformed flux in sF: the sum over directions in order (matrix cores: y on
+// the vector unit, then z and x added).
+template <int D, int P, class R, int np>
+__device__ __forceinline__ R divergence(const R* sF, int b, int s, int k, int sw, int swx, R opv, bf16x8 abf,
+                                        const Tabs& tb) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
+  constexpr bool mf = kMfma<D, P, R>;
+  R tot = 0;
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    if (mf && d != 1) continue;
+    if constexpr (np != 0) {
+      if (d == 2) {
+        tot = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sF + ((b * D + 2) * N + k) * S), s, abf, tot, np);
+        continue;
+      }
+    }
+    const int* gi = tb.grd_idx + (d * S + s) * P1;
+    const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
+    R a = 0;
+#pragma unroll
+    for (int m = 0; m < P1; m++) a += gw[m] * sF[((b * D + d) * N + k) * S + gi[m]];
+    tot = (d == 0 || mf) ? a : a + tot;
+  }
+  if (mf) {
+    tot = mfma444(opv, sF[((b * D + 2) * N + k) * S + sw], tot);
+    tot = mfma444(sF[((b * D + 0) * N + k) * S + swx], opv, tot);
+  }
+  return tot;
+}
+
 // ---------------------------------------------------------------------------
-// Volume kernel: [corrected gradient], flux, divergence, normal flux at faces
-// [and gradient at faces].  One thread per solution point, EB elements per
-// block, element data staged in LDS.
-template <int D, int P, bool VISC, class R, bool NT, int BF = 0>
+// Stage kernel of inviscid runs: one launch per RK stage.  Each element forms
+// the common flux at its own flux points from U there and across (the left
+// element's order of arguments and normal on both sides, so that both form the
+// same bits), the flux and its divergence, the correction and the RK update,
+// and writes U at its flux points for the next stage into a second array
+// (neighbours still read the first).
+//
+// What it replaces: a face kernel that wrote the common flux once per point
+// pair and a volume kernel that read it back.  A stage is then one dependent
+// launch instead of two, which is what bounds small meshes (about 4.6 us per
+// launch in a captured graph), and on large ones the flux array's write and
+// two reads go (5.8 kB per P3 hex and stage) for one more read of U at the
+// flux points.  The common flux is evaluated on both sides of a pair; the
+// boundary states' code is compiled into the BND instances only, which meshes
+// without boundary faces do not take.
+//
+// Measured, two kernels -> one: 2-D vortex 32x32 P3, 20 RK44 steps 842 -> 683 us;
+// 3-D vortex 17^3 P2, 10 steps 1351 -> 1132 us; 23^3 P4 mixed, 4 steps 2140 ->
+// 1841 us; P4 channel 67x29, update and multigrid cycle 1142 -> 1005 us.
+//
+// Steady runs (local time steps, 2-D) also form the element's time step here,
+// in the step's first stage: it needs only the element's own wave speeds.
+template <class R>
+struct StageFace {
+  const int* fpart;    // [E*F] 4 * partner flux point + side, or 4 * boundary slot + 2
+  const R* Ufe;        // [E][N][F] U at the flux points, this stage's
+  const R* nfe;        // [E][D][F] the face's normal (its left element's)
+  const R* dA;         // [E][F] face area factor
+  double* wave;        // wave speeds of the left and boundary points, or null: not read before they change again
+  const int* bndBc;    // [nBnd] boundary code (number and state row) by slot
+  const double* bst;   // boundary-state table
+  // local time step formed here, or wf null
+  const double *wf, *wavein, *dAd, *vole;
+  double cflfac;
+  double* eleDt;
+};
+
+template <int D, int P, class R, bool NT, bool BND, int BF>
+__device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
+                                           const R* __restrict__ JGe, const StageFace<R>& fc, const Tabs& tb,
+                                           const Phys& ph, const RkArgs<R>& ra) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
+  const int EB = blockDim.x / S;
+  // U, the transformed flux and the flux jump of the block's elements:
+  // [EB*N*S] [EB*D*N*S] [EB*N*F]
+  R* const sU = reinterpret_cast<R*>(fhip_lds);
+  R* const sF = sU + EB * N * S;
+  R* const sD = sF + EB * D * N * S;
+  const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
+  const int b = threadIdx.x / S, s = threadIdx.x - b * S;
+  const int sw = spt_lds(D, P1, s);
+  const bool act = b < nb;
+  const long long e = e0 + b;
+  constexpr bool mf = kMfma<D, P, R>;
+  constexpr int np = kBf16<D, P, R> ? BF : 0;
+  bf16x8 abf = {};
+  if constexpr (np != 0) abf = bf16_opnd_a(tw<float>(tb.d1, tb.d1f), s, np);
+  const int swx = mf ? spt_lds(D, P1, s / 16 + 4 * ((s / 4) % 4) + 16 * (s % 4)) : 0;
+  const R opv = mf ? tw<R>(tb.d1, tb.d1f)[(s % 4) * P1 + s / 16] : R(0);
+  // a thread finishes at most KF flux points; their side codes are loaded
+  // first, since the partners' addresses come from them
+  constexpr int KF = (F + S - 1) / S;
+  const int nP = nb * F;
+  int cd[KF];
+#pragma unroll
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    cd[u] = i < nP ? fc.fpart[(long long)e0 * F + i] : -1;
+  }
+  R vu[N];
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nb * N * S)
+      vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
+  }
+  R G[D][D] = {};
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < D; r++)
+#pragma unroll
+      for (int x = 0; x < D; x++) G[r][x] = JGe[((e * D + r) * D + x) * S + s];
+  }
+  const bool fold = D == 2 && fc.wf;
+  R fo[KF][N];
+#pragma unroll
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+#pragma unroll
+    for (int k = 0; k < N; k++) fo[u][k] = 0;
+    if (i < nP) {
+      const int bb = i / F, f = i - bb * F, side = cd[u] & 3;
+      const long long ob = (long long)(e0 + bb) * N * F + f;
+      R own[N], oth[N], n[D], fn[N];
+#pragma unroll
+      for (int k = 0; k < N; k++) own[k] = fc.Ufe[ob + k * F];
+      long long pb = ob;
+      if (!BND || side != 2) {
+        const int p = cd[u] >> 2, ep = p / F;
+        pb = (long long)ep * N * F + (p - ep * F);
+      }
+#pragma unroll
+      for (int k = 0; k < N; k++) oth[k] = fc.Ufe[pb + k * F];
+#pragma unroll
+      for (int x = 0; x < D; x++) n[x] = ld_s<NT>(&fc.nfe[((long long)(e0 + bb) * D + x) * F + f]);
+      const R dA = ld_s<NT>(&fc.dA[(long long)e0 * F + i]);
+      if (fold) {
+        const int Ff = Sh::Ff;
+        reinterpret_cast<double*>(sD)[i] =
+            fc.wavein[(long long)e0 * F + i] * fc.wf[f % Ff] * fc.dAd[(long long)e0 * F + i];
+      }
+      if constexpr (BND) {
+        if (side == 2) bc_state<D, R>(fc.bndBc[cd[u] >> 2], own, n, oth, ph, fc.bst);
+      }
+      const bool right = side == 1;
+      R UL[N], UR[N];
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        UL[k] = right ? oth[k] : own[k];
+        UR[k] = right ? own[k] : oth[k];
+      }
+      bool roe = false;
+      if constexpr (D == 2) roe = ph.riemann_type != 0 && (!BND || side != 2);
+      if (!roe) {
+        const double lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
+        if (fc.wave && !right) st_s<NT>(lam, &fc.wave[(long long)e0 * F + i]);
+      } else if constexpr (D == 2) {
+        roe2d<R>(UL, UR, n, fn, R(ph.gamma));
+      }
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const R v = mul_rn(fn[k], dA);
+        fo[u][k] = right ? -v : v;
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nb * N * S) {
+      const int r = i / S, q = i - r * S;
+      sU[r * S + spt_lds(D, P1, q)] = vu[u];
+    }
+  }
+  __syncthreads();
+  double dtl = 0;
+  if (fold && act) {
+    double iw = 0;
+    for (int f = 0; f < F; f++) iw += reinterpret_cast<const double*>(sD)[b * F + f];
+    dtl = fc.cflfac * 2 * fc.vole[e] / iw;
+    if (s == 0) fc.eleDt[e] = dtl;
+  }
+  // flux at the point, transformed to the reference element
+  if (act) {
+    R u[N], Fl[D][N];
+#pragma unroll
+    for (int k = 0; k < N; k++) u[k] = sU[(b * N + k) * S + sw];
+    inviscid_flux<D, R, true>(u, Fl, R(ph.gamma));
+#pragma unroll
+    for (int d1 = 0; d1 < D; d1++)
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        R acc = 0;
+#pragma unroll
+        for (int d2 = 0; d2 < D; d2++) acc += G[d1][d2] * Fl[d2][k];
+        sF[((b * D + d1) * N + k) * S + sw] = acc;
+      }
+  }
+  __syncthreads();
+  R dv[N] = {};
+  if (act) {
+#pragma unroll
+    for (int k = 0; k < N; k++) dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, tb);
+  }
+  // the flux jump: the common flux times this side's dA, negated on the right
+  // side, less the extrapolated normal flux (of the sum over directions only
+  // the face's own normal direction is non-zero)
+#pragma unroll
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nP) {
+      const int bb = i / F, f = i - bb * F;
+      const int* xi = tb.ext_idx + f * P1;
+      const int dn = tb.efn_dir[f];
+      const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        R a = 0;
+#pragma unroll
+        for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
+        sD[(bb * N + k) * F + f] = fo[u][k] - a;
+      }
+    }
+  }
+  __syncthreads();
+  rk_tail<D, P, R, NT>(E, dv, sU, sD, ra, tb, fold, dtl);
+}
+
+// Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
+// for FP64 hexes.
+template <int D, int P, class R, bool NT, bool BND>
+__global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_w3(
+    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
+    Phys ph, RkArgs<R> ra) {
+  stage_body<D, P, R, NT, BND, 0>(E, Ue, Us, JGe, fc, tb, ph, ra);
+}
+template <int D, int P, class R, bool NT, bool BND, int BF = 0>
+__global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
+    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
+    Phys ph, RkArgs<R> ra) {
+  stage_body<D, P, R, NT, BND, BF>(E, Ue, Us, JGe, fc, tb, ph, ra);
+}
+
+// ---------------------------------------------------------------------------
+// Volume kernel of viscous runs: corrected gradient, flux, divergence, normal
+// flux and each side's part of the LDG flux at the faces.  One thread per
+// solution point, EB elements per block, element data staged in LDS.
+template <int D, int P, class R, bool NT, int BF = 0>
 __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
                                             const R* __restrict__ dUce,
                                             const R* __restrict__ JGe, const R* __restrict__ iJe,
                                             R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf,
-                                            Tabs tb, Phys ph, const R* __restrict__ Fne, const RkArgs<R>& ra) {
+                                            Tabs tb, Phys ph) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
   const int EB = blockDim.x / S;
-  // sF holds, in turn (viscous runs): dUc at the flux points, the physical
-  // gradient until it has been extrapolated to the faces, then the transformed
-  // flux at the same indices as the gradient.  [EB*N*S] + [EB*N*SF]; viscous
-  // runs also stage the faces' normals for the face loop, [EB*D*F], inviscid
-  // runs keep the flux jump of the RK update there, [EB*N*F]; then the
-  // points' side codes [EB*F] ints
-  constexpr int SF = (VISC && F > D * S) ? F : D * S;
+  // sF holds, in turn: dUc at the flux points, the physical gradient until it
+  // has been extrapolated to the faces, then the transformed flux at the same
+  // indices as the gradient.  [EB*N*S] + [EB*N*SF]; the faces' normals for the
+  // face loop, [EB*D*F], and the points' side codes [EB*F] ints
+  constexpr int SF = F > D * S ? F : D * S;
   R* const sU = reinterpret_cast<R*>(fhip_lds);
   R* const sF = sU + EB * N * S;
   R* const sG = sF;
   R* const sN = sF + EB * N * SF;
-  R* const sD = sN;
-  int* const sP = reinterpret_cast<int*>(VISC ? sN + EB * D * F : sD + EB * N * F);
-  // viscous runs with kJumpInVolume: this side's LDG part at the block's
+  int* const sP = reinterpret_cast<int*>(sN + EB * D * F);
+  // with kJumpInVolume: this side's LDG part at the block's
   // flux points, kept from the first face loop for the last one [EB*N*F]
   R* const sB = reinterpret_cast<R*>(sP + EB * F);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
@@ -733,7 +984,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   const int swx = mf ? spt_lds(D, P1, s / 16 + 4 * ((s / 4) % 4) + 16 * (s % 4)) : 0;
   const R opv = mf ? tw<R>(tb.d1, tb.d1f)[(s % 4) * P1 + s / 16] : R(0);
   // the point's metric terms, loaded first so that their latency overlaps the
-  // staging of the slab (and the gradient of viscous runs)
+  // staging of the slab and the gradient
   R G[D][D] = {};
   auto load_G = [&] {
 #pragma unroll
@@ -744,14 +995,13 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   R inv = 0;
   if (act) {
     load_G();
-    if constexpr (VISC) inv = iJe[e * S + s];
+    inv = iJe[e * S + s];
   }
   {
     // every load of the slabs is issued before the first LDS store, so that
     // their latencies overlap: a thread stages at most N values of U (the
     // block holds at most blockDim / S elements) and KC of dUc
-    constexpr int KC = VISC ? (N * F + S - 1) / S : 1, KN = VISC ? (D * F + S - 1) / S : 1,
-                  KP = (F + S - 1) / S;
+    constexpr int KC = (N * F + S - 1) / S, KN = (D * F + S - 1) / S, KP = (F + S - 1) / S;
     const int nU = nb * N * S, nC = nb * N * F, nN = nb * D * F, nP = nb * F;
     R vu[N], vc[KC], vn[KN];
     int vp[KP];
@@ -760,18 +1010,16 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       const int i = threadIdx.x + u * blockDim.x;
       if (i < nU) vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
     }
-    if constexpr (VISC) {
-      // dUc at the block's flux points (sF serves as sC until the gradient is written)
+    // dUc at the block's flux points (sF serves as sC until the gradient is written)
 #pragma unroll
-      for (int u = 0; u < KC; u++) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < nC) vc[u] = ld_s<NT>(&dUce[(long long)e0 * N * F + i]);
-      }
+    for (int u = 0; u < KC; u++) {
+      const int i = threadIdx.x + u * blockDim.x;
+      if (i < nC) vc[u] = ld_s<NT>(&dUce[(long long)e0 * N * F + i]);
+    }
 #pragma unroll
-      for (int u = 0; u < KN; u++) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < nN) vn[u] = ld_s<NT>(&vf.nfe[(long long)e0 * D * F + i]);
-      }
+    for (int u = 0; u < KN; u++) {
+      const int i = threadIdx.x + u * blockDim.x;
+      if (i < nN) vn[u] = ld_s<NT>(&vf.nfe[(long long)e0 * D * F + i]);
     }
 #pragma unroll
     for (int u = 0; u < KP; u++) {
@@ -786,17 +1034,15 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
         sU[r * S + spt_lds(D, P1, q)] = vu[u];
       }
     }
-    if constexpr (VISC) {
 #pragma unroll
-      for (int u = 0; u < KC; u++) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < nC) sF[i] = vc[u];
-      }
+    for (int u = 0; u < KC; u++) {
+      const int i = threadIdx.x + u * blockDim.x;
+      if (i < nC) sF[i] = vc[u];
+    }
 #pragma unroll
-      for (int u = 0; u < KN; u++) {
-        const int i = threadIdx.x + u * blockDim.x;
-        if (i < nN) sN[i] = vn[u];
-      }
+    for (int u = 0; u < KN; u++) {
+      const int i = threadIdx.x + u * blockDim.x;
+      if (i < nN) sN[i] = vn[u];
     }
 #pragma unroll
     for (int u = 0; u < KP; u++) {
@@ -805,174 +1051,139 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     }
   }
   __syncthreads();
-  // inviscid runs: the common flux at the points this thread finishes in the
-  // last face loop (the pair's left point, the partner's on the right side)
-  // and their dA, loaded now so that the loads are in flight during the flux
-  // and divergence phases
-  constexpr int KFP = VISC ? 1 : (F + S - 1) / S;
-  R pf[KFP][N], pdA[KFP];
-  int psd[KFP];
-  if constexpr (!VISC) {
+  // phase 1: reference-space gradient (opp_grad_spts) plus correction
+  // (opp_correctU), then the physical gradient (correctGradU transform,
+  // src/solver.cpp:1105-1136), kept in LDS for phase 2 and the faces
+  R* const sC = sF;
+  R gr[D][N];
+  if (act) {
 #pragma unroll
-    for (int u = 0; u < KFP; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      psd[u] = 2;
-      pdA[u] = 0;
-#pragma unroll
-      for (int k = 0; k < N; k++) pf[u][k] = 0;
-      if (i < nb * F) {
-        const int code = sP[i], bb = i / F;
-        psd[u] = code & 3;
-        long long pb = (long long)(e0 + bb) * N * F + (i - bb * F);
-        if (psd[u] == 1) {
-          const long long p = code >> 2, ep = p / F;
-          pb = ep * N * F + (p - ep * F);
-        }
-#pragma unroll
-        for (int k = 0; k < N; k++) pf[u][k] = Fne[pb + k * F];
-        pdA[u] = vf.dA[(long long)e0 * F + i];
-      }
-    }
-  }
-  if constexpr (VISC) {
-    // phase 1: reference-space gradient (opp_grad_spts) plus correction
-    // (opp_correctU), then the physical gradient (correctGradU transform,
-    // src/solver.cpp:1105-1136), kept in LDS for phase 2 and the faces
-    R* const sC = sF;
-    R gr[D][N];
-    if (act) {
-#pragma unroll
-      for (int d = 0; d < D; d++) {
-        const int* gi = tb.grd_idx + (d * S + s) * P1;
-        const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
-        const int* ci = tb.cu_idx + (d * S + s) * 2;
-        const R* cw = tw<R>(tb.cu_w, tb.cu_wf) + (d * S + s) * 2;
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-          // the other correction entries of the row are exactly zero
-          R c = 0;
-#pragma unroll
-          for (int j = 0; j < 2; j++) c += cw[j] * sC[(b * N + k) * F + ci[j]];
-          if constexpr (np != 0) {
-            if (d == 2) {
-              gr[d][k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sU + (b * N + k) * S), s, abf, c, np);
-              continue;
-            }
-          }
-          if (mf && d != 1) {  // compile-time: d and mf are constants here
-            gr[d][k] = d == 2 ? mfma444(opv, sU[(b * N + k) * S + sw], c)
-                              : mfma444(sU[(b * N + k) * S + swx], opv, c);
-            continue;
-          }
-          R a = 0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) a += gw[m] * sU[(b * N + k) * S + gi[m]];
-          gr[d][k] = c + a;
-        }
-      }
-      // physical gradient, in place
+    for (int d = 0; d < D; d++) {
+      const int* gi = tb.grd_idx + (d * S + s) * P1;
+      const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
+      const int* ci = tb.cu_idx + (d * S + s) * 2;
+      const R* cw = tw<R>(tb.cu_w, tb.cu_wf) + (d * S + s) * 2;
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        R acc[D];
+        // the other correction entries of the row are exactly zero
+        R c = 0;
 #pragma unroll
-        for (int x = 0; x < D; x++) {
-          acc[x] = gr[0][k] * G[0][x] + gr[1][k] * G[1][x];
-          if constexpr (D == 3) acc[x] += gr[2][k] * G[2][x];
+        for (int j = 0; j < 2; j++) c += cw[j] * sC[(b * N + k) * F + ci[j]];
+        if constexpr (np != 0) {
+          if (d == 2) {
+            gr[d][k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sU + (b * N + k) * S), s, abf, c, np);
+            continue;
+          }
         }
+        if (mf && d != 1) {  // compile-time: d and mf are constants here
+          gr[d][k] = d == 2 ? mfma444(opv, sU[(b * N + k) * S + sw], c)
+                            : mfma444(sU[(b * N + k) * S + swx], opv, c);
+          continue;
+        }
+        R a = 0;
 #pragma unroll
-        for (int x = 0; x < D; x++) gr[x][k] = inv * acc[x];
+        for (int m = 0; m < P1; m++) a += gw[m] * sU[(b * N + k) * S + gi[m]];
+        gr[d][k] = c + a;
       }
     }
-    __syncthreads();  // sC is overwritten by the gradient below
-    if (act) {
+    // physical gradient, in place
 #pragma unroll
-      for (int k = 0; k < N; k++)
+    for (int k = 0; k < N; k++) {
+      R acc[D];
 #pragma unroll
-        for (int x = 0; x < D; x++) sG[((b * D + x) * N + k) * S + sw] = gr[x][k];
+      for (int x = 0; x < D; x++) {
+        acc[x] = gr[0][k] * G[0][x] + gr[1][k] * G[1][x];
+        if constexpr (D == 3) acc[x] += gr[2][k] * G[2][x];
+      }
+#pragma unroll
+      for (int x = 0; x < D; x++) gr[x][k] = inv * acc[x];
     }
-    __syncthreads();
-    // physical gradient at the flux points (extrapolateGradU) and, with U
-    // there (extrapolateU, the same sums as the RK kernel's), this side's
-    // viscous flux folded into its part of the LDG flux
-    // (face::calcViscousFlux, src/face.cpp:216-293); the two sides' parts are
-    // summed where the correction is applied.  Boundary points keep the
-    // gradient for the boundary kernel, which needs the boundary state.
-    for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
-      const int bb = i / F, f = i - bb * F;
-      const long long ee = e0 + bb;
-      const int* xi = tb.ext_idx + f * P1;
-      const R* xw = tw<R>(tb.ext_w, tb.ext_wf) + f * P1;
-      // side code and normal, staged in LDS with the slab
-      const int code = sP[bb * F + f], side = code & 3;
-      R nv[D];
+  }
+  __syncthreads();  // sC is overwritten by the gradient below
+  if (act) {
 #pragma unroll
-      for (int x = 0; x < D; x++) nv[x] = sN[(bb * D + x) * F + f];
-      R g[D][N];
+    for (int k = 0; k < N; k++)
+#pragma unroll
+      for (int x = 0; x < D; x++) sG[((b * D + x) * N + k) * S + sw] = gr[x][k];
+  }
+  __syncthreads();
+  // physical gradient at the flux points (extrapolateGradU) and, with U
+  // there (extrapolateU, the same sums as the RK kernel's), this side's
+  // viscous flux folded into its part of the LDG flux
+  // (face::calcViscousFlux, src/face.cpp:216-293); the two sides' parts are
+  // summed where the correction is applied.  Boundary points keep the
+  // gradient for the boundary kernel, which needs the boundary state.
+  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
+    const int bb = i / F, f = i - bb * F;
+    const long long ee = e0 + bb;
+    const int* xi = tb.ext_idx + f * P1;
+    const R* xw = tw<R>(tb.ext_w, tb.ext_wf) + f * P1;
+    // side code and normal, staged in LDS with the slab
+    const int code = sP[bb * F + f], side = code & 3;
+    R nv[D];
+#pragma unroll
+    for (int x = 0; x < D; x++) nv[x] = sN[(bb * D + x) * F + f];
+    R g[D][N];
+#pragma unroll
+    for (int x = 0; x < D; x++)
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        R a = 0;
+#pragma unroll
+        for (int m = 0; m < P1; m++) a += xw[m] * sG[((bb * D + x) * N + k) * S + xi[m]];
+        g[x][k] = a;
+      }
+    if (side == 2) {
+      const long long slot = code >> 2;
 #pragma unroll
       for (int x = 0; x < D; x++)
 #pragma unroll
-        for (int k = 0; k < N; k++) {
-          R a = 0;
+        for (int k = 0; k < N; k++) vf.gBnd[(x * N + k) * (long long)vf.nBnd + slot] = g[x][k];
+    } else {
+      R u[N], bv[N];
 #pragma unroll
-          for (int m = 0; m < P1; m++) a += xw[m] * sG[((bb * D + x) * N + k) * S + xi[m]];
-          g[x][k] = a;
-        }
-      if (side == 2) {
-        const long long slot = code >> 2;
+      for (int k = 0; k < N; k++) {
+        R a = 0;
 #pragma unroll
-        for (int x = 0; x < D; x++)
+        for (int m = 0; m < P1; m++) a += xw[m] * sU[(bb * N + k) * S + xi[m]];
+        u[k] = a;
+        bv[k] = 0;
+      }
+      ldg_add_side<D, R>(side == 0, u, g, nv, bv, ph);
 #pragma unroll
-          for (int k = 0; k < N; k++) vf.gBnd[(x * N + k) * (long long)vf.nBnd + slot] = g[x][k];
-      } else {
-        R u[N], bv[N];
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-          R a = 0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) a += xw[m] * sU[(bb * N + k) * S + xi[m]];
-          u[k] = a;
-          bv[k] = 0;
-        }
-        ldg_add_side<D, R>(side == 0, u, g, nv, bv, ph);
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-          st_s<NT>(bv[k], &vf.Bve[(ee * N + k) * F + f]);
-          if constexpr (kJumpInVolume<R>) sB[(bb * N + k) * F + f] = bv[k];
-        }
+      for (int k = 0; k < N; k++) {
+        st_s<NT>(bv[k], &vf.Bve[(ee * N + k) * F + f]);
+        if constexpr (kJumpInVolume<R>) sB[(bb * N + k) * F + f] = bv[k];
       }
     }
-    // under the register hold, the metric terms again (from cache): keeping
-    // them live across the face loop above costs more registers than it allows
-    if constexpr (kHold<D, R>) {
-      if (act) load_G();
-    }
+  }
+  // under the register hold, the metric terms again (from cache): keeping
+  // them live across the face loop above costs more registers than it allows
+  if constexpr (kHold<D, R>) {
+    if (act) load_G();
   }
   // phase 2: flux at the point, transformed to the reference element.  It is
-  // formed in registers and stored after a barrier: viscous runs store it over
-  // the gradient slab, which other threads may still be reading in the face
-  // loop, and threads with fewer face points go on here meanwhile.
+  // formed in registers and stored after a barrier, over the gradient slab,
+  // which other threads may still be reading in the face loop; threads with
+  // fewer face points go on here meanwhile.
   R Ft[D][N];
   if (act) {
     R u[N];
 #pragma unroll
     for (int k = 0; k < N; k++) u[k] = sU[(b * N + k) * S + sw];
     R Fl[D][N];
-    if constexpr (VISC) {
-      R g[D][N];
+    R g[D][N];
 #pragma unroll
-      for (int x = 0; x < D; x++)
+    for (int x = 0; x < D; x++)
 #pragma unroll
-        for (int k = 0; k < N; k++) g[x][k] = sG[((b * D + x) * N + k) * S + sw];
-      R Fi[D][N];
-      viscous_flux<D, R>(u, g, Fl, ph);
-      inviscid_flux<D, R>(u, Fi, R(ph.gamma));
+      for (int k = 0; k < N; k++) g[x][k] = sG[((b * D + x) * N + k) * S + sw];
+    R Fi[D][N];
+    viscous_flux<D, R>(u, g, Fl, ph);
+    inviscid_flux<D, R>(u, Fi, R(ph.gamma));
 #pragma unroll
-      for (int d = 0; d < D; d++)
+    for (int d = 0; d < D; d++)
 #pragma unroll
-        for (int k = 0; k < N; k++) Fl[d][k] = Fl[d][k] + Fi[d][k];
-    } else {
-      inviscid_flux<D, R>(u, Fl, R(ph.gamma));
-    }
+      for (int k = 0; k < N; k++) Fl[d][k] = Fl[d][k] + Fi[d][k];
 #pragma unroll
     for (int d1 = 0; d1 < D; d1++)
 #pragma unroll
@@ -983,7 +1194,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
         Ft[d1][k] = acc;
       }
   }
-  if constexpr (VISC) __syncthreads();
+  __syncthreads();
   if (act) {
 #pragma unroll
     for (int d1 = 0; d1 < D; d1++)
@@ -991,119 +1202,61 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       for (int k = 0; k < N; k++) sF[((b * D + d1) * N + k) * S + sw] = Ft[d1][k];
   }
   __syncthreads();
-  R dv[N] = {};  // inviscid runs: divF at the point, for the RK update below
   if (act) {
-    // divergence (calcDivF_spts): sum over directions in order (matrix
-    // cores: y on the vector unit, then z and x added)
+#pragma unroll
+    for (int k = 0; k < N; k++)
+      st_s<NT>(divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, tb), &divFe[(e * N + k) * S + s]);
+  }
+  // faces: discontinuous normal flux.  With kJumpInVolume it stores in its
+  // place this side's part of the correction's flux jump, +-B dA - disFn (B
+  // as written by this thread in the face loop above, - on the right side;
+  // boundary points get - disFn here and + B dA from the boundary kernel).
+  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
+    const int bb = i / F, f = i - bb * F;
+    const long long ee = e0 + bb;
+    const int* xi = tb.ext_idx + f * P1;
+    // extrapolateNormalFlux: of the sum over directions only the face's own
+    // normal direction is non-zero (the other terms are exact zeros)
+    const int dn = tb.efn_dir[f];
+    const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
+    int side = 2;
+    R dA = 0, bv[N];
+    if constexpr (kJumpInVolume<R>) {
+      side = sP[bb * F + f] & 3;
+      dA = vf.dA[ee * F + f];
+      // this thread's own LDG parts from the first face loop (the same
+      // points); read for every point, unused at boundary points
+#pragma unroll
+      for (int k = 0; k < N; k++) bv[k] = sB[(bb * N + k) * F + f];
+    }
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      R tot = 0;
+      R a = 0;
 #pragma unroll
-      for (int d = 0; d < D; d++) {
-        if (mf && d != 1) continue;
-        if constexpr (np != 0) {
-          if (d == 2) {
-            tot = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sF + ((b * D + 2) * N + k) * S), s, abf, tot, np);
-            continue;
-          }
-        }
-        const int* gi = tb.grd_idx + (d * S + s) * P1;
-        const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += gw[m] * sF[((b * D + d) * N + k) * S + gi[m]];
-        tot = (d == 0 || mf) ? a : a + tot;
-      }
-      if (mf) {
-        tot = mfma444(opv, sF[((b * D + 2) * N + k) * S + sw], tot);
-        tot = mfma444(sF[((b * D + 0) * N + k) * S + swx], opv, tot);
-      }
-      if constexpr (VISC) st_s<NT>(tot, &divFe[(e * N + k) * S + s]);
-      else dv[k] = tot;
+      for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
+      if constexpr (kJumpInVolume<R>) a = (side == 2) ? -a : (side == 0 ? bv[k] : -bv[k]) * dA - a;
+      st_s<NT>(a, &disFne[(ee * N + k) * F + f]);
     }
-  }
-  // faces: discontinuous normal flux.  With kJumpInVolume, viscous runs store
-  // in its place this side's part of the correction's flux jump,
-  // +-B dA - disFn (B as written by this thread in the face loop above, - on
-  // the right side; boundary points get - disFn here and + B dA from the
-  // boundary kernel).
-  if constexpr (VISC) {
-    for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
-      const int bb = i / F, f = i - bb * F;
-      const long long ee = e0 + bb;
-      const int* xi = tb.ext_idx + f * P1;
-      // extrapolateNormalFlux: of the sum over directions only the face's own
-      // normal direction is non-zero (the other terms are exact zeros)
-      const int dn = tb.efn_dir[f];
-      const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
-      int side = 2;
-      R dA = 0, bv[N];
-      if constexpr (kJumpInVolume<R>) {
-        side = sP[bb * F + f] & 3;
-        dA = vf.dA[ee * F + f];
-        // this thread's own LDG parts from the first face loop (the same
-        // points); read for every point, unused at boundary points
-#pragma unroll
-        for (int k = 0; k < N; k++) bv[k] = sB[(bb * N + k) * F + f];
-      }
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
-        if constexpr (kJumpInVolume<R>) a = (side == 2) ? -a : (side == 0 ? bv[k] : -bv[k]) * dA - a;
-        st_s<NT>(a, &disFne[(ee * N + k) * F + f]);
-      }
-    }
-  } else {
-    // inviscid runs: the flux jump, the common flux (loaded above) times
-    // this side's dA, negated on the right side, less the extrapolated flux
-#pragma unroll
-    for (int u = 0; u < KFP; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nb * F) {
-        const int bb = i / F, f = i - bb * F;
-        const int* xi = tb.ext_idx + f * P1;
-        const int dn = tb.efn_dir[f];
-        const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-          R a = 0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
-          const R fo = mul_rn(pf[u][k], pdA[u]);
-          sD[(bb * N + k) * F + f] = (psd[u] == 1 ? -fo : fo) - a;
-        }
-      }
-    }
-  }
-  if constexpr (!VISC) {
-    // inviscid runs: the correction, RK update and U at the flux points here
-    // (no partner data is needed past the face kernel's common flux)
-    __syncthreads();
-    rk_tail<D, P, R, NT>(E, dv, sU, sD, ra, tb);
   }
 }
 
 // The volume kernel held to 4 waves per SIMD (at most 128 VGPRs) for quads
 // and the FP32 path, which fit there without spilling (holding the FP32
 // viscous hex kernel to 5 or 6 waves spills 26 or 41 VGPRs and was measured
-// 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes.  Viscous runs
-// reload the metric terms after the face loop; inviscid runs keep them in
-// registers throughout.
-template <int D, int P, bool VISC, class R, bool NT>
+// 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes.
+template <int D, int P, class R, bool NT>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_volume_w3(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
     const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
-    Phys ph, const R* __restrict__ Fne, RkArgs<R> ra) {
-  volume_body<D, P, VISC, R, NT>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph, Fne, ra);
+    Phys ph) {
+  volume_body<D, P, R, NT>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
 }
-template <int D, int P, bool VISC, class R, bool NT, int BF = 0>
+template <int D, int P, class R, bool NT, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_volume_w4(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
     const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
-    Phys ph, const R* __restrict__ Fne, RkArgs<R> ra) {
-  volume_body<D, P, VISC, R, NT, BF>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph, Fne, ra);
+    Phys ph) {
+  volume_body<D, P, R, NT, BF>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
 }
 
 // ---------------------------------------------------------------------------
@@ -1249,7 +1402,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   rk_tail<D, P, R, NT>(E, dv, sU, sD, ra, tb);
 }
 
-__global__ void k_copy_em(long long n, double* __restrict__ dst, const double* __restrict__ src) {
+template <class R>
+__global__ void k_copy_em(long long n, R* __restrict__ dst, const R* __restrict__ src) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
 }
@@ -1700,15 +1854,23 @@ static void set_geometry(Ctx& c, Work<float>& w) {
   }
 }
 
+// A single-stage step with a CFL time step takes its dt from the wave speeds of
+// the residual it is about to apply (solver::update), so they are formed in a
+// launch of their own before it.
+static bool face_first(const Ctx& c) { return !c.prm.viscous && c.z.nRK == 1 && c.prm.dt_type != 0; }
+
 template <class R>
 static void ensure_work(Ctx& c) {
   Work<R>& w = fs(c).work<R>();
   if (w.ready) return;
   const long long E = c.z.E, S = c.z.S, F = c.z.F, N = c.z.N, D = c.z.D;
   w.Ufe = dal<R>(E * N * F);
-  w.Fne = dal<R>(E * N * F);
+  if (!c.prm.viscous) w.Ufe2 = dal<R>(E * N * F);
+  // the face kernel's common flux: inviscid runs take that kernel for its wave
+  // speeds alone, where a single-stage step needs them before its update
+  if (c.prm.viscous || face_first(c)) w.Fne = dal<R>(E * N * F);
   if (c.prm.viscous) {
-    // inviscid runs keep divF and the discontinuous normal flux in the volume kernel
+    // inviscid runs keep divF and the discontinuous normal flux in the stage kernel
     w.divFe = dal<R>(E * N * S);
     w.disFne = dal<R>(E * N * F);
     w.dUce = dal<R>(E * N * F);
@@ -1820,15 +1982,13 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
     FCHK(hipMemcpy(st->bc, bc.data(), bc.size() * 4, hipMemcpyHostToDevice));
     {
       // every element flux point must lie on exactly one face point pair;
-      // its code: 4 * partner flux point + side, or 4 * boundary slot + 2
-      // (viscous runs also keep the face's normal at every point)
-      const bool visc = c.prm.viscous != 0;
+      // its code: 4 * partner flux point + side, or 4 * boundary slot + 2, and
+      // the face's normal
       if (E * F >= (1LL << 29)) throw std::invalid_argument("fused path: more than 2^29 element flux points");
-      std::vector<int> part((size_t)E * F, -1), bt;
-      std::vector<double> nl(visc ? (size_t)E * D * F : 0);
+      std::vector<int> part((size_t)E * F, -1), bt, bb;
+      std::vector<double> nl((size_t)E * D * F);
       // the left element's normal at flux point q (element-major q = e*F + f)
       auto put_normal = [&](int q, int qL) {
-        if (!visc) return;
         const long long e = q / F, f = q - e * F, eL = qL / F, fL = qL - eL * F;
         for (long long x = 0; x < D; x++) nl[(e * D + x) * F + f] = d->norm_fpts[(fL * E + eL) * D + x];
       };
@@ -1840,6 +2000,7 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
         put_normal(pl[t], pl[t]);
         if (pr[t] < 0) {
           bt.push_back(t);
+          bb.push_back(bc[t]);
           part[pl[t]] = 4 * (int)(bt.size() - 1) + 2;
         } else {
           part[pl[t]] = 4 * pr[t];
@@ -1854,12 +2015,14 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
         }
       st->fpart = dal<int>(part.size());
       FCHK(hipMemcpy(st->fpart, part.data(), part.size() * 4, hipMemcpyHostToDevice));
-      if (visc) {
-        st->nBnd = (int)bt.size();
-        st->bndT = dal<int>(bt.size());
-        st->nfe = dal<double>(nl.size());
-        FCHK(hipMemcpy(st->nfe, nl.data(), nl.size() * 8, hipMemcpyHostToDevice));
-        if (!bt.empty()) FCHK(hipMemcpy(st->bndT, bt.data(), bt.size() * 4, hipMemcpyHostToDevice));
+      st->nBnd = (int)bt.size();
+      st->bndT = dal<int>(bt.size());
+      st->bndBc = dal<int>(bb.size());
+      st->nfe = dal<double>(nl.size());
+      FCHK(hipMemcpy(st->nfe, nl.data(), nl.size() * 8, hipMemcpyHostToDevice));
+      if (!bt.empty()) {
+        FCHK(hipMemcpy(st->bndT, bt.data(), bt.size() * 4, hipMemcpyHostToDevice));
+        FCHK(hipMemcpy(st->bndBc, bb.data(), bb.size() * 4, hipMemcpyHostToDevice));
       }
     }
   }
@@ -1911,6 +2074,12 @@ void fused_release(Ctx& c) {
 
 // ---- per-order / per-precision dispatch ------------------------------------
 
+static double cfl_limit_f(int order) {  // getCFLLimit, src/global.cpp:81-105
+  static const double t[6] = {1.393, 0.464, 0.235, 0.1453, 0.100, 0.0736};
+  if (order < 0 || order > 5) throw std::invalid_argument("CFL limit not available for this order!");
+  return t[order];
+}
+
 template <int D, int P, class R>
 struct Runner {
   using Sh = Shape<D, P>;
@@ -1935,7 +2104,7 @@ struct Runner {
     if (k == kVolume)
       return EB * N * (S + SF) * sizeof(R) +
              (visc ? EB * (D * F * sizeof(R) + F * sizeof(int) + (kJumpInVolume<R> ? N * F * sizeof(R) : 0))
-                   : EB * (N * F * sizeof(R) + F * sizeof(int)));
+                   : EB * N * F * sizeof(R));
     if (k == kRk) return EB * N * (S + F) * sizeof(R);
     return 0;
   }
@@ -1966,41 +2135,70 @@ struct Runner {
                          st.bc, w.Ufe, w.nrm, w.Fne, st.waveSpe, w.dUce, c.ph, st.bst);
     FCHK(hipGetLastError());
   }
-  template <bool VISC, bool NT>
-  static void launch_volume_t(Ctx& c, int nt, const RkArgs<R>& ra) {
+  // viscous runs: the volume kernel.  Quads and FP32 are held to 4 waves per
+  // SIMD (128 VGPRs); FP64 hexes, which spill under that hold, to 3 (168 VGPRs:
+  // P3 without spills, where the unheld compiler would take 211 and leave 2
+  // waves)
+  template <bool NT>
+  static void launch_volume_t(Ctx& c, int nt) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     const VFace<R> vf{st.fpart, w.nf, w.Bve, w.gBnd, w.dA, st.nBnd};
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
-    const Tabs& tb = st.tb;
-    // quads and FP32 are held to 4 waves per SIMD (128 VGPRs); FP64 hexes,
-    // which spill under that hold, to 3 (168 VGPRs: P3 without spills, where
-    // the unheld compiler would take 211 and leave 2 waves)
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, true), c.stream, c.z.E, st.Ue, us,
+                         w.dUce, w.JG, w.iJ, w.divFe, w.disFne, vf, st.tb, c.ph);
+    };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2 || c.bf16 == 3) {
-        auto kern = c.bf16 == 2 ? k_volume_w4<D, P, VISC, R, NT, 2> : k_volume_w4<D, P, VISC, R, NT, 3>;
-        hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, VISC), c.stream, c.z.E, st.Ue,
-                           us, w.dUce, w.JG, w.iJ, w.divFe, w.disFne, vf, tb, c.ph, w.Fne, ra);
-        FCHK(hipGetLastError());
-        return;
-      }
+      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, 2>);
+      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, 3>);
+      else go(k_volume_w4<D, P, R, NT>);
+    } else if constexpr (kHold<D, R>) {
+      go(k_volume_w4<D, P, R, NT>);
+    } else {
+      go(k_volume_w3<D, P, R, NT>);
     }
-    if constexpr (kHold<D, R>)
-      hipLaunchKernelGGL((k_volume_w4<D, P, VISC, R, NT>), dim3(nblk(c.z.E, nt / S)), dim3(nt),
-                         lds(kVolume, nt, VISC), c.stream, c.z.E, st.Ue, us, w.dUce, w.JG, w.iJ, w.divFe, w.disFne,
-                         vf, tb, c.ph, w.Fne, ra);
-    else
-      hipLaunchKernelGGL((k_volume_w3<D, P, VISC, R, NT>), dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, VISC),
-                         c.stream, c.z.E, st.Ue, us, w.dUce, w.JG, w.iJ, w.divFe, w.disFne, vf, tb, c.ph, w.Fne, ra);
     FCHK(hipGetLastError());
   }
-  // viscous runs: the volume kernel (ra unused); inviscid runs: the volume
-  // kernel with the RK update of stage ra
-  static void launch_volume(Ctx& c, int nt, const RkArgs<R>& ra) {
-    const bool sm = fs(c).stream && kEleRowsWhole;
-    if (c.prm.viscous) sm ? launch_volume_t<true, true>(c, nt, ra) : launch_volume_t<true, false>(c, nt, ra);
-    else sm ? launch_volume_t<false, true>(c, nt, ra) : launch_volume_t<false, false>(c, nt, ra);
+  // inviscid runs: the stage kernel with the RK update ra
+  template <bool NT, bool BND>
+  static void launch_stage_t(Ctx& c, int nt, RkArgs<R> ra, bool fold) {
+    FusedState& st = fs(c);
+    Work<R>& w = st.work<R>();
+    // wave speeds are read by the next step's dt and after the call: stages
+    // that another stage follows leave them
+    const bool wave = ra.fin || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
+    const StageFace<R> fc{st.fpart, st.odd_stage ? w.Ufe2 : w.Ufe, w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
+                          st.bst, fold ? c.wf : nullptr, st.waveSpe, st.dAe, st.vole,
+                          fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
+    ra.Ufe = st.odd_stage ? w.Ufe : w.Ufe2;
+    const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, false), c.stream, c.z.E, st.Ue, us,
+                         w.JG, fc, st.tb, c.ph, ra);
+    };
+    if constexpr (kBf16<D, P, R>) {
+      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, 2>);
+      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, 3>);
+      else go(k_stage_w4<D, P, R, NT, BND>);
+    } else if constexpr (kHold<D, R>) {
+      go(k_stage_w4<D, P, R, NT, BND>);
+    } else {
+      go(k_stage_w3<D, P, R, NT, BND>);
+    }
+    FCHK(hipGetLastError());
   }
+  static void launch_volume(Ctx& c, int nt) {
+    if (fs(c).stream && kEleRowsWhole) launch_volume_t<true>(c, nt);
+    else launch_volume_t<false>(c, nt);
+  }
+  static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
+    const bool sm = fs(c).stream && kEleRowsWhole, bnd = fs(c).nBnd > 0;
+    if (sm) bnd ? launch_stage_t<true, true>(c, nt, ra, fold) : launch_stage_t<true, false>(c, nt, ra, fold);
+    else bnd ? launch_stage_t<false, true>(c, nt, ra, fold) : launch_stage_t<false, false>(c, nt, ra, fold);
+  }
+  // whether a step's first stage forms the elements' time steps itself
+  static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
   static void launch_face_bnd(Ctx& c, int nt) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2025,13 +2223,22 @@ struct Runner {
                      (mode == 2 || mode == 3 || (mode == 4 && stage == c.z.nRK - 1)) ? 1 : 0, w.Ufe};
   }
   // the RK kernel of viscous runs; inviscid runs do its work at the end of
-  // their volume kernel
+  // their stage kernel
   static void launch_rk(Ctx& c, int nt, int mode, double a, double b, bool write0, int stage = 0) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     auto* kern = (st.stream && kEleRowsWhole) ? k_rk<D, P, R, true> : k_rk<D, P, R, false>;
     hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kRk, nt, false), c.stream, c.z.E, w.divFe, w.Fne,
                        w.disFne, rk_args(c, mode, a, b, write0, stage), st.tb, st.fpart, w.dA, w.Bve);
+    FCHK(hipGetLastError());
+  }
+  // after a step with an odd number of stages: U at the flux points back
+  // where every step starts
+  static void copy_ufe(Ctx& c) {
+    Work<R>& w = fs(c).work<R>();
+    const long long n = (long long)c.z.E * N * F;
+    Launch L(c, nm("fused_copy", "mixed_copy"));
+    hipLaunchKernelGGL(k_copy_em<R>, dim3(nblk(n, 256)), dim3(256), 0, c.stream, n, w.Ufe, w.Ufe2);
     FCHK(hipGetLastError());
   }
   static void extrap(Ctx& c) {
@@ -2065,19 +2272,19 @@ struct Runner {
       FCHK(hipGetLastError());
     }
   }
-  // calcResidual up to what the RK update needs: viscous runs the face,
-  // volume and boundary kernels; inviscid runs the face kernel only (their
-  // volume kernel runs with the update, in rk below)
+  static void face(Ctx& c) {
+    Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
+    launch_face_inv(c, blk(c, kFaceInv));
+  }
+  // calcResidual up to what the RK update needs: the face, volume and boundary
+  // kernels of viscous runs; nothing on inviscid ones, whose stage kernel runs
+  // in rk below
   static void residual(Ctx& c) {
-    const bool visc = c.prm.viscous != 0;
-    {
-      Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
-      launch_face_inv(c, blk(c, kFaceInv));
-    }
-    if (!visc) return;
+    if (!c.prm.viscous) return;
+    face(c);
     {
       Launch L(c, nm("fused_volume_viscous", "mixed_volume_viscous"));
-      launch_volume(c, blk(c, kVolume), RkArgs<R>{});
+      launch_volume(c, blk(c, kVolume));
     }
     if (fs(c).nBnd > 0) {
       Launch L(c, nm("fused_face_boundary", "mixed_face_boundary"));
@@ -2086,15 +2293,16 @@ struct Runner {
   }
   static void rk(Ctx& c, int mode, double a, double b, bool write0, int stage) {
     if (!c.prm.viscous) {
-      Launch L(c, nm("fused_volume_rk", "mixed_volume_rk"));
-      launch_volume(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage));
+      Launch L(c, nm("fused_stage", "mixed_stage"));
+      launch_stage(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage),
+                   folds_dt(c) && (mode == 0 || mode == 6));
       return;
     }
     Launch L(c, nm("fused_rk_update", "mixed_rk_update"));
     launch_rk(c, blk(c, kRk), mode, a, b, write0, stage);
   }
   // Time every valid block size of every kernel on this context's data and
-  // keep the fastest.  The RK kernel (and the volume kernel of inviscid runs,
+  // keep the fastest.  The RK kernel (and the stage kernel of inviscid runs,
   // which includes the update) runs in its middle-stage mode, which rewrites
   // U and the RK accumulator: both are saved and restored, as are the wave
   // speeds the face kernel writes; block shapes never change results.
@@ -2116,12 +2324,15 @@ struct Runner {
     // elements, so sizes between the powers of two pay off where S divides them
     const int cand[7] = {64, 128, 192, 256, 320, 384, 512};
     for (int k = kExtrap; k <= kRk; k++) {
-      if ((k == kFaceBnd && (!visc || st.nBnd == 0)) || (k == kRk && !visc)) continue;
+      if ((k == kFaceBnd && (!visc || st.nBnd == 0)) || ((k == kRk || k == kFaceInv) && !visc)) continue;
       auto run = [&](int nt) {
         switch (k) {
           case kExtrap: launch_extrap(c, nt); break;
           case kFaceInv: launch_face_inv(c, nt); break;
-          case kVolume: launch_volume(c, nt, visc ? RkArgs<R>{} : rk_args(c, 1, 0.5, 1. / 3., false, 0)); break;
+          case kVolume:
+            if (visc) launch_volume(c, nt);
+            else launch_stage(c, nt, rk_args(c, 1, 0.5, 1. / 3., false, 0));
+            break;
           case kFaceBnd: launch_face_bnd(c, nt); break;
           default: launch_rk(c, nt, 1, 0.5, 1. / 3., false);
         }
@@ -2184,7 +2395,10 @@ struct Ops {
   void (*extrap)(Ctx&);
   void (*wave)(Ctx&);
   void (*dt)(Ctx&, double);
+  void (*face)(Ctx&);
   void (*residual)(Ctx&);
+  void (*copy_ufe)(Ctx&);
+  bool (*folds_dt)(const Ctx&);
   void (*rk)(Ctx&, int, double, double, bool, int);
   void (*ensure)(Ctx&);
   void (*tune)(Ctx&);
@@ -2195,7 +2409,7 @@ struct Ops {
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit};
+  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::folds_dt, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit};
 }
 
 template <class R>
@@ -2270,14 +2484,9 @@ void fused_get_blocks(Ctx& c, bool mixed, int* out) {
   std::copy(nt, nt + 5, out);
 }
 
-static double cfl_limit_f(int order) {  // getCFLLimit, src/global.cpp:81-105
-  static const double t[6] = {1.393, 0.464, 0.235, 0.1453, 0.100, 0.0736};
-  if (order < 0 || order > 5) throw std::invalid_argument("CFL limit not available for this order!");
-  return t[order];
-}
-
 void fused_begin(Ctx& c, bool mixed, bool src) {
   FusedState& st = fs(c);
+  st.read_stage = st.odd_stage = false;
   const Sizes& z = c.z;
   Ops o = get_ops(c, mixed);
   o.ensure(c);
@@ -2306,6 +2515,7 @@ constexpr size_t kTransferLds = 64 * 1024;
 
 void fused_em_prepare(Ctx& c, bool mixed) {
   FusedState& st = fs(c);
+  st.read_stage = st.odd_stage = false;
   get_ops(c, mixed).ensure(c);
   if (!st.srce) {
     c.drop_graphs();
@@ -2413,21 +2623,25 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
   const bool cfl = c.prm.dt_type != 0;
   const double cflfac = cfl ? c.prm.cfl * cfl_limit_f(c.z.P) : 0.;
   const bool jameson = c.prm.time_type >= 5;
+  st.odd_stage = false;
   if (nRK == 1) {
-    o.residual(c);
+    if (c.prm.viscous) o.residual(c);
+    else if (cfl) o.face(c);
     if (cfl) {
       if (refresh) o.wave(c);
       o.dt(c, cflfac);
     }
     o.rk(c, jameson ? 4 : 3, A[1], B[0], keep, 0);
+    if (!c.prm.viscous) o.copy_ufe(c);
     return;
   }
   if (cfl) {
     if (refresh) o.wave(c);
-    o.dt(c, cflfac);
+    if (!o.folds_dt(c)) o.dt(c, cflfac);
   }
   for (int step = 0; step < nRK; step++) {
     st.read_stage = step > 0;
+    st.odd_stage = !c.prm.viscous && (step & 1);
     o.residual(c);
     // the Jameson form's first stage reads the state itself (the step's U0)
     int mode;
@@ -2435,7 +2649,8 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
     else mode = (step == 0) ? 0 : (step == nRK - 1 ? 2 : 1);
     o.rk(c, mode, A[step + 1], B[step], keep && step == 0, step);
   }
-  st.read_stage = false;
+  st.read_stage = st.odd_stage = false;
+  if (!c.prm.viscous && (nRK & 1)) o.copy_ufe(c);
 }
 
 }  // namespace fhip

@@ -26,24 +26,33 @@ __device__ __forceinline__ T fmax_(T a, T b) { return a > b ? a : (b != b ? b : 
 template <class T>
 __device__ __forceinline__ T smax(T a, T b) { return (a < b) ? b : a; }
 
-// inviscidFlux, src/flux.cpp:37-76.  F[d][k].
-template <int D, class T>
+// a * b + c rounded once.  Which product of a sum the compiler contracts depends
+// on the code around it, and in FP32 that is a difference of the last bit: where
+// a flux is formed in more than one kernel the choice is written out.
+__device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// inviscidFlux, src/flux.cpp:37-76.  F[d][k].  FUSE: E + p contracted with the
+// product in p (the inviscid kernels; otherwise as the compiler decides).
+template <int D, class T, bool FUSE = false>
 __device__ __forceinline__ void inviscid_flux(const T* U, T F[D][D + 2], T gamma) {
   if constexpr (D == 2) {
     T rho = U[0], ri = T(1) / rho, u = U[1] * ri, v = U[2] * ri, E = U[3];
-    T p = (gamma - T(1)) * (E - T(0.5) * rho * (u * u + v * v));
+    T x = E - T(0.5) * rho * (u * u + v * v), p = (gamma - T(1)) * x;
+    T Ep = FUSE ? fma_(gamma - T(1), x, E) : E + p;
     F[0][0] = rho * u;         F[1][0] = rho * v;
     F[0][1] = rho * u * u + p; F[1][1] = rho * u * v;
     F[0][2] = rho * v * u;     F[1][2] = rho * v * v + p;
-    F[0][3] = (E + p) * u;     F[1][3] = (E + p) * v;
+    F[0][3] = Ep * u;          F[1][3] = Ep * v;
   } else {
     T rho = U[0], ri = T(1) / rho, u = U[1] * ri, v = U[2] * ri, w = U[3] * ri, E = U[4];
-    T p = (gamma - T(1)) * (E - T(0.5) * rho * (u * u + v * v + w * w));
+    T x = E - T(0.5) * rho * (u * u + v * v + w * w), p = (gamma - T(1)) * x;
+    T Ep = FUSE ? fma_(gamma - T(1), x, E) : E + p;
     F[0][0] = rho * u;         F[1][0] = rho * v;         F[2][0] = rho * w;
     F[0][1] = rho * u * u + p; F[1][1] = rho * u * v;     F[2][1] = rho * u * w;
     F[0][2] = rho * v * u;     F[1][2] = rho * v * v + p; F[2][2] = rho * v * w;
     F[0][3] = rho * w * u;     F[1][3] = rho * w * v;     F[2][3] = rho * w * w + p;
-    F[0][4] = (E + p) * u;     F[1][4] = (E + p) * v;     F[2][4] = (E + p) * w;
+    F[0][4] = Ep * u;          F[1][4] = Ep * v;          F[2][4] = Ep * w;
   }
 }
 
@@ -150,8 +159,8 @@ template <int D, class T>
 __device__ __forceinline__ T rusanov(const T* UL, const T* UR, const T* n, T* Fn, T gamma) {
   constexpr int N = D + 2;
   T FL[D][N], FR[D][N];
-  inviscid_flux<D, T>(UL, FL, gamma);
-  inviscid_flux<D, T>(UR, FR, gamma);
+  inviscid_flux<D, T, true>(UL, FL, gamma);
+  inviscid_flux<D, T, true>(UR, FR, gamma);
   T rhoL = UL[0], rhoR = UR[0], riL = T(1) / rhoL, riR = T(1) / rhoR;
   T uL = UL[1] * riL, uR = UR[1] * riR, vL = UL[2] * riL, vR = UR[2] * riR;
   T pL, pR;
@@ -209,9 +218,9 @@ __device__ __forceinline__ void roe2d(const T* UL, const T* UR, const T* n, T* F
   T rhoUnL = UL[1] * n[0] + UL[2] * n[1];
   T rhoUnR = UR[1] * n[0] + UR[2] * n[1];
   Fn[0] = rhoUnL + rhoUnR;
-  Fn[1] = rhoUnL * vL[0] + rhoUnR * vR[0] + (pL + pR) * n[0];
-  Fn[2] = rhoUnL * vL[1] + rhoUnR * vR[1] + (pL + pR) * n[1];
-  Fn[3] = rhoUnL * hL + rhoUnR * hR;
+  Fn[1] = fma_(rhoUnL, vL[0], rhoUnR * vR[0]) + (pL + pR) * n[0];
+  Fn[2] = fma_(rhoUnL, vL[1], rhoUnR * vR[1]) + (pL + pR) * n[1];
+  Fn[3] = fma_(rhoUnL, hL, rhoUnR * hR);
   for (int i = 0; i < 4; i++) du[i] = UR[i] - UL[i];
   T l0 = fabs(unm), lP = fabs(unm + am), lM = fabs(unm - am);
   T eps = T(0.5) * (fabs(rhoUnL / UL[0] - rhoUnR / UR[0]) + fabs(sqrt(g * pL / UL[0]) - sqrt(g * pR / UR[0])));

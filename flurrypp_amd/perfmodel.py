@@ -34,7 +34,7 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     wr = nFF * (N + 1)
     if viscous:
         wr += nFF * N + nFFi * N
-    out["fused_face_inviscid"] = Work((rd + wr) * B8, 0.0)
+        out["fused_face_inviscid"] = Work((rd + wr) * B8, 0.0)
     # volume
     rd = E * (N * S + D * D * S)
     wr = E * (N * S + N * F)
@@ -46,11 +46,12 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
         fl += E * N * (D * S * 2 * P1 + D * S * 2 * 2 * D + (D + 1) * F * 2 * P1)
         out["fused_volume_viscous"] = Work((rd + wr) * B8, fl)
     else:
-        # inviscid runs: the volume kernel also applies the RK update (below);
-        # divF and the discontinuous normal flux stay on chip, the common flux
-        # Fn is read instead (with dA and the side code)
-        vol_rd = rd + E * N * F + E * F * (1 + B4 / B8)
-        vol_wr = wr - E * (N * S + N * F)
+        # inviscid runs: one stage kernel, which also forms the common flux and
+        # applies the RK update (below); divF, the common and the discontinuous
+        # normal flux stay on chip, U at the element's flux points and across
+        # is read instead (with the normal, dA and the side code)
+        vol_rd = rd + E * 2 * N * F + E * F * (D + 1 + B4 / B8)
+        vol_wr = wr - E * (N * S + N * F) + nFF / nRK  # the wave speeds of the last stage
     if viscous and nFFb:
         # boundary LDG flux: U, normal, gradient in; the point's flux part out
         rd = nFFb * (N + D + D * N + 3 * B4 / B8)
@@ -83,7 +84,7 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
         out["fused_rk_update"] = rk
     else:
         # the RK part without its reads of divF, Fn and disFn
-        out["fused_volume_rk"] = Work((vol_rd + vol_wr) * B8 + rk.bytes - E * (N * S + 2 * N * F) * B8, fl + rk.flops)
+        out["fused_stage"] = Work((vol_rd + vol_wr) * B8 + rk.bytes - E * (N * S + 2 * N * F) * B8, fl + rk.flops)
     return out
 
 
@@ -105,10 +106,13 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     wr = nFF * (f4 * N + d8)
     if viscous:
         wr += (nFF + nFFi) * f4 * N
-    out["mixed_face_inviscid"] = Work(rd + wr, 0.0)
-    # volume: U (stage copy), metric terms (inviscid runs: with dA and the
-    # side codes for the common flux)
-    rd = E * f4 * (N * S + D * D * S) + (0 if viscous else E * F * (f4 + i4))
+        out["mixed_face_inviscid"] = Work(rd + wr, 0.0)
+    # volume: U (stage copy), metric terms (inviscid runs, the stage kernel:
+    # with U at the flux points and across, normal, dA and side code, and the
+    # last stage's wave speeds)
+    rd = E * f4 * (N * S + D * D * S)
+    if not viscous:
+        rd += E * F * (f4 * (2 * N + D + 1) + i4) + nFF * d8 / nRK
     if viscous:
         # 1/detJ, dUc, face normal, dA, side code; divF, this side's flux jump
         # (with its LDG part), the LDG part, boundary gradient out
@@ -126,8 +130,6 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
         rd_ = E * (f4 * N * S + d8 * S)                # divF, detJ
         if viscous:
             rd_ += E * (f4 * 3 * N * F + f4 * F + i4 * F)  # Fn, flux jump, partner's LDG part, dA, code
-        else:
-            rd_ += E * f4 * N * F                      # Fn (the volume kernel forms the jump on chip)
         wr_ = E * (f4 * N * F + f4 * N * S)            # U at the faces, stage copy of U
         if time_type >= 5:
             rd_ += E * d8 * N * S                      # U0
@@ -150,7 +152,7 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     if viscous:
         out["mixed_rk_update"] = Work(rk, fp["fused_rk_update"].flops)
     else:
-        out["mixed_volume_rk"] = Work(rd + rk - E * f4 * N * S, fp["fused_volume_rk"].flops)
+        out["mixed_stage"] = Work(rd + rk - E * f4 * N * S, fp["fused_stage"].flops)
     return out
 
 

@@ -84,14 +84,15 @@ def footprint_bytes(nDims: int, order: int, nEles: int, viscous: bool = False, n
     # fused FP64: U, its stage copy, RK accumulator, divF0; wave speeds, metrics (+1/detJ), face
     # tables, the points' side codes, element volumes
     d += 4 * SN + F * (2 + D) + D * D * S + 2 * S + 1.5 * F + 0.5 * F + 1
-    # FP64 work: divF, U/Fn/disFn at the flux points
+    # the faces' normals at every flux point
+    d += D * F
+    # FP64 work: divF, U (two copies on inviscid runs)/Fn/disFn at the flux points
     d += SN + 3 * FN
     # FP32 work (half a double each): the same, stage residuals, FP32 U, FP32 geometry
-    d += 0.5 * (SN + 3 * FN + (nRK - 1) * SN + SN + D * D * S + S + D * F + F)
+    d += 0.5 * (SN + 3 * FN + (nRK - 1) * SN + SN + D * D * S + S + 2 * D * F + F)
     if viscous:
         d += D * SN + D * FN + FN            # staged gradients and dUc
-        d += D * F                           # fused face normals
-        d += 2 * FN + 0.5 * (2 * FN + D * F)  # dUc and LDG side parts, FP64 and FP32
+        d += 2 * FN + 0.5 * 2 * FN           # dUc and LDG side parts, FP64 and FP32
     if pmg_source:
         d += SN                              # P-multigrid source, element-major
     return int(8 * d * nEles * 1.25) + (16 << 20)
