@@ -38,6 +38,7 @@
 #include <cstdio>
 #include <cstring>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "fhip_internal.hpp"
@@ -92,6 +93,10 @@ struct Tabs {
   // P3 hexes, whose FP64 volume kernel contracts with it on the matrix cores)
   const double* d1;
   const float* d1f;
+  // operators of full tensor-product form (Ten below): their 1-D factors
+  // [Ten::NW], FP64 and FP32, or null
+  const double* w1;
+  const float* w1f;
 };
 
 // The 1-D contractions of FP64 P3 hexes along x and z run on the matrix
@@ -214,6 +219,155 @@ __host__ __device__ constexpr int spt_lds(int D, int P1, int s) {
   if (D == 2 || P1 % 2 == 1) return s;
   const int i = s % P1, j = (s / P1) % P1, k = s / (P1 * P1);
   return (k * P1 + (j + k) % P1) * P1 + (i + k) % P1;
+}
+
+// The operators of a quad or hex by their 1-D factors: entry (point, m) sits on
+// a line of the element, at a position that follows from the point's
+// coordinates, and its weight is one of P1*P1 + 4*P1 numbers: the derivative
+// matrix d1[i][m], the extrapolation to the low and high end l[side][m], the
+// correction from the low and high end c[side][i].  A kernel keeps those in LDS
+// and computes the positions.  Read from per-point tables instead (PtTab, FpTab:
+// operators whose non-zeros have this pattern but other values) every use
+// waits for two loads, the position and the weight, a chain through the caches
+// in each phase; entries and their order are the same, so are the sums.
+// Measured, tables -> factors: P4 channel 67x29, update and multigrid cycle 1005
+// -> 941 us; 3-D vortex 23^3 P4 mixed, 4 steps 1841 -> 1711 us; Navier-Stokes
+// Taylor-Green 37^3 P2, 4 steps 7.12 -> 6.91 ms, 48^3 P3 20.36 -> 20.15 ms.
+template <int D, int P>
+struct Ten {
+  static constexpr int P1 = P + 1, NW = P1 * P1 + 4 * P1;
+  static constexpr int L = P1 * P1, C = L + 2 * P1;  // offsets of l and c
+  // slab position of the point at coordinates (i, j, k)
+  __host__ __device__ static constexpr int pos(int i, int j, int k) {
+    if (D == 2) return i + P1 * j;
+    if (P1 % 2 == 1) return i + P1 * (j + P1 * k);
+    int jk = j + k, ik = i + k;
+    jk -= jk >= P1 ? P1 : 0;
+    ik -= ik >= P1 ? P1 : 0;
+    return (k * P1 + jk) * P1 + ik;
+  }
+  // Flux point f: the direction dn of its normal, whether it lies on the high
+  // end, its coordinates in the other directions (getLocFpts,
+  // src/points.cpp:67-162)
+  struct Face {
+    int dn, hi, c[3];
+    __host__ __device__ explicit Face(int f) {
+      c[0] = c[1] = c[2] = 0;
+      if (D == 2) {
+        const int face = f / P1, i = f - face * P1, a = face < 2 ? i : P - i;
+        dn = (face & 1) ? 0 : 1;
+        hi = face == 1 || face == 2;
+        c[0] = dn == 0 ? 0 : a;
+        c[1] = dn == 0 ? a : 0;
+      } else {
+        const int face = f / (P1 * P1), r = f - face * (P1 * P1), j = r / P1, i = r - j * P1;
+        dn = face < 2 ? 2 : (face < 4 ? 0 : 1);
+        hi = face & 1;
+        const int a = (face == 1 || face == 3 || face == 4) ? P - i : i;
+        c[0] = dn == 0 ? 0 : a;
+        c[1] = dn == 0 ? a : (dn == 2 ? j : 0);
+        c[2] = dn == 2 ? 0 : j;
+      }
+    }
+    // the point of the flux point's line at depth m
+    __host__ __device__ int at(int m) const {
+      return pos(dn == 0 ? m : c[0], dn == 1 ? m : c[1], dn == 2 ? m : c[2]);
+    }
+  };
+  struct Point {
+    int c[3];
+    __host__ __device__ explicit Point(int s) {
+      c[0] = s % P1;
+      c[1] = D == 2 ? s / P1 : (s / P1) % P1;
+      c[2] = D == 2 ? 0 : s / (P1 * P1);
+    }
+    __host__ __device__ int line(int d, int m) const {
+      return pos(d == 0 ? m : c[0], d == 1 ? m : c[1], d == 2 ? m : c[2]);
+    }
+  };
+  // Face j's direction and end, and the flux point on it opposite a point
+  __host__ __device__ static constexpr int face_dir(int j) { return D == 2 ? (j & 1 ? 0 : 1) : (j < 2 ? 2 : (j < 4 ? 0 : 1)); }
+  __host__ __device__ static constexpr int face_hi(int j) { return D == 2 ? (j == 1 || j == 2) : (j & 1); }
+  __host__ __device__ static int face_fpt(int j, const int* c) {
+    if (D == 2) {
+      const int a = j & 1 ? c[1] : c[0];
+      return j * P1 + (j < 2 ? a : P - a);
+    }
+    const int a = j == 2 || j == 3 ? c[1] : c[0], b = j < 2 ? c[1] : c[2];
+    return j * P1 * P1 + (j == 1 || j == 3 || j == 4 ? P - a : a) + P1 * b;
+  }
+  // the two faces normal to direction d, ascending
+  __host__ __device__ static constexpr int dir_face(int d, int j) {
+    return D == 2 ? (d == 0 ? 1 + 2 * j : 2 * j) : (d == 2 ? j : 2 * (d + 1) + j);
+  }
+};
+
+// A solution point's operator entries.
+template <int D, int P, class R>
+struct PtTen {
+  using T = Ten<D, P>;
+  const R* w;
+  typename T::Point p;
+  __device__ PtTen(const struct Tabs&, const R* sW, int s) : w(sW), p(s) {}
+  __device__ int grd_idx(int d, int m) const { return p.line(d, m); }
+  __device__ R grd_w(int d, int m) const { return w[p.c[d] * T::P1 + m]; }
+  __device__ int cor_idx(int j) const { return T::face_fpt(j, p.c); }
+  __device__ R cor_w(int j) const { return w[T::C + T::face_hi(j) * T::P1 + p.c[T::face_dir(j)]]; }
+  __device__ int cu_idx(int d, int j) const { return cor_idx(T::dir_face(d, j)); }
+  __device__ R cu_w(int d, int j) const {
+    const R c = cor_w(T::dir_face(d, j));
+    return T::face_hi(T::dir_face(d, j)) ? c : -c;
+  }
+};
+template <int D, int P, class R>
+struct PtTab {
+  static constexpr int P1 = P + 1, S = Shape<D, P>::S, NC = 2 * D;
+  const Tabs& tb;
+  int s;
+  __device__ PtTab(const Tabs& t, const R*, int s_) : tb(t), s(s_) {}
+  __device__ int grd_idx(int d, int m) const { return tb.grd_idx[(d * S + s) * P1 + m]; }
+  __device__ R grd_w(int d, int m) const { return tw<R>(tb.grd_w, tb.grd_wf)[(d * S + s) * P1 + m]; }
+  __device__ int cor_idx(int j) const { return tb.cor_idx[s * NC + j]; }
+  __device__ R cor_w(int j) const { return tw<R>(tb.cor_w, tb.cor_wf)[s * NC + j]; }
+  __device__ int cu_idx(int d, int j) const { return tb.cu_idx[(d * S + s) * 2 + j]; }
+  __device__ R cu_w(int d, int j) const { return tw<R>(tb.cu_w, tb.cu_wf)[(d * S + s) * 2 + j]; }
+};
+// A flux point's operator entries: extrapolation (positions and weights; the
+// sum over them, negated on a low end, is the normal flux's), normal direction.
+template <int D, int P, class R>
+struct FpTen {
+  using T = Ten<D, P>;
+  const R* w;
+  typename T::Face f;
+  __device__ FpTen(const Tabs&, const R* sW, int fpt) : w(sW), f(fpt) {}
+  __device__ int idx(int m) const { return f.at(m); }
+  __device__ R ext_w(int m) const { return w[T::L + f.hi * T::P1 + m]; }
+  __device__ R efn_w(int m) const { return ext_w(m); }
+  __device__ R efn_sign(R a) const { return f.hi ? a : -a; }
+  __device__ int dir() const { return f.dn; }
+};
+template <int D, int P, class R>
+struct FpTab {
+  static constexpr int P1 = P + 1;
+  const Tabs& tb;
+  int f;
+  __device__ FpTab(const Tabs& t, const R*, int fpt) : tb(t), f(fpt) {}
+  __device__ int idx(int m) const { return tb.ext_idx[f * P1 + m]; }
+  __device__ R ext_w(int m) const { return tw<R>(tb.ext_w, tb.ext_wf)[f * P1 + m]; }
+  __device__ R efn_w(int m) const { return tw<R>(tb.efn_w, tb.efn_wf)[f * P1 + m]; }
+  __device__ R efn_sign(R a) const { return a; }
+  __device__ int dir() const { return tb.efn_dir[f]; }
+};
+template <int D, int P, class R, bool TEN>
+using PtOp = std::conditional_t<TEN, PtTen<D, P, R>, PtTab<D, P, R>>;
+template <int D, int P, class R, bool TEN>
+using FpOp = std::conditional_t<TEN, FpTen<D, P, R>, FpTab<D, P, R>>;
+// The 1-D factors into the block's LDS (a barrier follows before their use).
+template <int D, int P, class R, bool TEN>
+__device__ __forceinline__ void stage_factors(R* sW, const Tabs& tb) {
+  if constexpr (TEN) {
+    if (threadIdx.x < Ten<D, P>::NW) sW[threadIdx.x] = tw<R>(tb.w1, tb.w1f)[threadIdx.x];
+  }
 }
 
 // Face and volume intermediates of one precision.
@@ -341,11 +495,13 @@ static void from_em(hipStream_t st, int P, long long E, int K, const double* in,
 
 // ---------------------------------------------------------------------------
 // U at the flux points from U at the solution points (opp_spts_to_fpts rows).
-template <int D, int P, class R>
+template <int D, int P, class R, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) void k_extrap(int E, const double* __restrict__ Ue, R* __restrict__ Ufe,
                                                        R* __restrict__ Us, Tabs tb) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
   const int EB = blockDim.x / S;
   R* const sU = reinterpret_cast<R*>(fhip_lds);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
@@ -369,11 +525,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_extrap(int E, const double* __res
   __syncthreads();
   for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
     int b = i / F, f = i - b * F;
+    const FpOp<D, P, R, TEN> fp(tb, sW, f);
 #pragma unroll
     for (int k = 0; k < N; k++) {
       R acc = 0;
 #pragma unroll
-      for (int m = 0; m < P1; m++) acc += tw<R>(tb.ext_w, tb.ext_wf)[f * P1 + m] * sU[(b * N + k) * S + tb.ext_idx[f * P1 + m]];
+      for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(b * N + k) * S + fp.idx(m)];
       Ufe[((long long)(e0 + b) * N + k) * F + f] = acc;
     }
   }
@@ -527,8 +684,8 @@ struct RkArgs {
 // once for the whole block.
 // The arrays come in as __restrict__ parameters (from RkArgs at the call
 // below), so that the compiler may keep their loads ahead of the stores.
-template <int D, int P, class R, bool NT>
-__device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD, int mode, double a, double bcoef,
+template <int D, int P, class R, bool NT, bool TEN>
+__device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD, const R* sW, int mode, double a, double bcoef,
                                           const double* __restrict__ detJe, const double* __restrict__ dtp,
                                           const double* __restrict__ eleDt, int local, double* __restrict__ Ue,
                                           double* __restrict__ U0e, double* __restrict__ Uacc,
@@ -543,6 +700,7 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
   const long long nS = (long long)E * N * S;
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
   const int b = threadIdx.x / S, s = threadIdx.x - b * S;
+  const PtOp<D, P, R, TEN> po(tb, sW, s);
   if (mode == 5 || mode == 7 || mode == 8) {
     // residual only (calcResidual(0) + correctDivFlux), no update: 5 into
     // divF_spts[0]; 7 subtracted in place from the array divF0e points to
@@ -553,7 +711,7 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
       for (int k = 0; k < N; k++) {
         R c = 0;
 #pragma unroll
-        for (int j = 0; j < NC; j++) c += tw<R>(tb.cor_w, tb.cor_wf)[s * NC + j] * sD[(b * N + k) * F + tb.cor_idx[s * NC + j]];
+        for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
         const double r0 = double(c + dv[k]);
         const long long iu = (e * N + k) * S + s;
         if (mode == 7) {
@@ -602,7 +760,7 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
       const long long iu = (e * N + k) * S + s;
       R c = 0;
 #pragma unroll
-      for (int j = 0; j < NC; j++) c += tw<R>(tb.cor_w, tb.cor_wf)[s * NC + j] * sD[(b * N + k) * F + tb.cor_idx[s * NC + j]];
+      for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
       const double r0 = double(c + dv[k]);
       if (divF0e) st_s<NT>(r0, &divF0e[iu]);
       // P-multigrid source: divF_spts[step] + src_spts (src/solver.cpp:480,514)
@@ -649,20 +807,21 @@ __device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD
   __syncthreads();
   for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
     int bb = i / F, f = i - bb * F;
+    const FpOp<D, P, R, TEN> fp(tb, sW, f);
 #pragma unroll
     for (int k = 0; k < N; k++) {
       R acc = 0;
 #pragma unroll
-      for (int m = 0; m < P1; m++) acc += tw<R>(tb.ext_w, tb.ext_wf)[f * P1 + m] * sU[(bb * N + k) * S + tb.ext_idx[f * P1 + m]];
+      for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
       st_s<NT>(acc, &Ufe[((long long)(e0 + bb) * N + k) * F + f]);
     }
   }
 }
 
-template <int D, int P, class R, bool NT>
-__device__ __forceinline__ void rk_tail(int E, const R* dv, R* sU, const R* sD, const RkArgs<R>& ra, const Tabs& tb,
-                                        bool hasDt = false, double dtIn = 0) {
-  rk_tail_p<D, P, R, NT>(E, dv, sU, sD, ra.mode, ra.a, ra.bcoef, ra.detJe, ra.dtp, ra.eleDt, ra.local, ra.Ue, ra.U0e,
+template <int D, int P, class R, bool NT, bool TEN>
+__device__ __forceinline__ void rk_tail(int E, const R* dv, R* sU, const R* sD, const R* sW, const RkArgs<R>& ra,
+                                        const Tabs& tb, bool hasDt = false, double dtIn = 0) {
+  rk_tail_p<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra.mode, ra.a, ra.bcoef, ra.detJe, ra.dtp, ra.eleDt, ra.local, ra.Ue, ra.U0e,
                          ra.Uacc, ra.divF0e, ra.eleMesh, ra.meshDt, ra.active, ra.srce, ra.Rst, ra.stage, ra.bs, ra.Us,
                          ra.fin, ra.Ufe, tb, hasDt, dtIn);
 }
@@ -697,9 +856,9 @@ struct VFace {
 // calcDivF_spts of field k at point s of the block's element b, from the
 // transformed flux in sF: the sum over directions in order (matrix cores: y on
 // the vector unit, then z and x added).
-template <int D, int P, class R, int np>
+template <int D, int P, class R, int np, class Op>
 __device__ __forceinline__ R divergence(const R* sF, int b, int s, int k, int sw, int swx, R opv, bf16x8 abf,
-                                        const Tabs& tb) {
+                                        const Op& po) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
   constexpr bool mf = kMfma<D, P, R>;
@@ -713,11 +872,9 @@ __device__ __forceinline__ R divergence(const R* sF, int b, int s, int k, int sw
         continue;
       }
     }
-    const int* gi = tb.grd_idx + (d * S + s) * P1;
-    const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
     R a = 0;
 #pragma unroll
-    for (int m = 0; m < P1; m++) a += gw[m] * sF[((b * D + d) * N + k) * S + gi[m]];
+    for (int m = 0; m < P1; m++) a += po.grd_w(d, m) * sF[((b * D + d) * N + k) * S + po.grd_idx(d, m)];
     tot = (d == 0 || mf) ? a : a + tot;
   }
   if (mf) {
@@ -765,7 +922,7 @@ struct StageFace {
   double* eleDt;
 };
 
-template <int D, int P, class R, bool NT, bool BND, int BF>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF>
 __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
                                            const R* __restrict__ JGe, const StageFace<R>& fc, const Tabs& tb,
                                            const Phys& ph, const RkArgs<R>& ra) {
@@ -777,6 +934,8 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
   R* const sU = reinterpret_cast<R*>(fhip_lds);
   R* const sF = sU + EB * N * S;
   R* const sD = sF + EB * D * N * S;
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
   const int b = threadIdx.x / S, s = threadIdx.x - b * S;
   const int sw = spt_lds(D, P1, s);
@@ -900,8 +1059,9 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
   __syncthreads();
   R dv[N] = {};
   if (act) {
+    const PtOp<D, P, R, TEN> po(tb, sW, s);
 #pragma unroll
-    for (int k = 0; k < N; k++) dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, tb);
+    for (int k = 0; k < N; k++) dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po);
   }
   // the flux jump: the common flux times this side's dA, negated on the right
   // side, less the extrapolated normal flux (of the sum over directions only
@@ -911,42 +1071,41 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
     const int i = threadIdx.x + u * blockDim.x;
     if (i < nP) {
       const int bb = i / F, f = i - bb * F;
-      const int* xi = tb.ext_idx + f * P1;
-      const int dn = tb.efn_dir[f];
-      const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
+      const FpOp<D, P, R, TEN> fp(tb, sW, f);
+      const int dn = fp.dir();
 #pragma unroll
       for (int k = 0; k < N; k++) {
         R a = 0;
 #pragma unroll
-        for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
-        sD[(bb * N + k) * F + f] = fo[u][k] - a;
+        for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
+        sD[(bb * N + k) * F + f] = fo[u][k] - fp.efn_sign(a);
       }
     }
   }
   __syncthreads();
-  rk_tail<D, P, R, NT>(E, dv, sU, sD, ra, tb, fold, dtl);
+  rk_tail<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra, tb, fold, dtl);
 }
 
 // Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
 // for FP64 hexes.
-template <int D, int P, class R, bool NT, bool BND>
+template <int D, int P, class R, bool NT, bool BND, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_w3(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, 0>(E, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, 0>(E, Ue, Us, JGe, fc, tb, ph, ra);
 }
-template <int D, int P, class R, bool NT, bool BND, int BF = 0>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, BF>(E, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, BF>(E, Ue, Us, JGe, fc, tb, ph, ra);
 }
 
 // ---------------------------------------------------------------------------
 // Volume kernel of viscous runs: corrected gradient, flux, divergence, normal
 // flux and each side's part of the LDG flux at the faces.  One thread per
 // solution point, EB elements per block, element data staged in LDS.
-template <int D, int P, class R, bool NT, int BF = 0>
+template <int D, int P, class R, bool NT, bool TEN, int BF = 0>
 __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
                                             const R* __restrict__ dUce,
                                             const R* __restrict__ JGe, const R* __restrict__ iJe,
@@ -968,6 +1127,8 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   // with kJumpInVolume: this side's LDG part at the block's
   // flux points, kept from the first face loop for the last one [EB*N*F]
   R* const sB = reinterpret_cast<R*>(sP + EB * F);
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
   const int b = threadIdx.x / S, s = threadIdx.x - b * S;
   const int sw = spt_lds(D, P1, s);
@@ -1056,19 +1217,16 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   // src/solver.cpp:1105-1136), kept in LDS for phase 2 and the faces
   R* const sC = sF;
   R gr[D][N];
+  const PtOp<D, P, R, TEN> po(tb, sW, s);
   if (act) {
 #pragma unroll
     for (int d = 0; d < D; d++) {
-      const int* gi = tb.grd_idx + (d * S + s) * P1;
-      const R* gw = tw<R>(tb.grd_w, tb.grd_wf) + (d * S + s) * P1;
-      const int* ci = tb.cu_idx + (d * S + s) * 2;
-      const R* cw = tw<R>(tb.cu_w, tb.cu_wf) + (d * S + s) * 2;
 #pragma unroll
       for (int k = 0; k < N; k++) {
         // the other correction entries of the row are exactly zero
         R c = 0;
 #pragma unroll
-        for (int j = 0; j < 2; j++) c += cw[j] * sC[(b * N + k) * F + ci[j]];
+        for (int j = 0; j < 2; j++) c += po.cu_w(d, j) * sC[(b * N + k) * F + po.cu_idx(d, j)];
         if constexpr (np != 0) {
           if (d == 2) {
             gr[d][k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sU + (b * N + k) * S), s, abf, c, np);
@@ -1082,7 +1240,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
         }
         R a = 0;
 #pragma unroll
-        for (int m = 0; m < P1; m++) a += gw[m] * sU[(b * N + k) * S + gi[m]];
+        for (int m = 0; m < P1; m++) a += po.grd_w(d, m) * sU[(b * N + k) * S + po.grd_idx(d, m)];
         gr[d][k] = c + a;
       }
     }
@@ -1116,8 +1274,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
     const int bb = i / F, f = i - bb * F;
     const long long ee = e0 + bb;
-    const int* xi = tb.ext_idx + f * P1;
-    const R* xw = tw<R>(tb.ext_w, tb.ext_wf) + f * P1;
+    const FpOp<D, P, R, TEN> fp(tb, sW, f);
     // side code and normal, staged in LDS with the slab
     const int code = sP[bb * F + f], side = code & 3;
     R nv[D];
@@ -1130,7 +1287,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       for (int k = 0; k < N; k++) {
         R a = 0;
 #pragma unroll
-        for (int m = 0; m < P1; m++) a += xw[m] * sG[((bb * D + x) * N + k) * S + xi[m]];
+        for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sG[((bb * D + x) * N + k) * S + fp.idx(m)];
         g[x][k] = a;
       }
     if (side == 2) {
@@ -1145,7 +1302,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       for (int k = 0; k < N; k++) {
         R a = 0;
 #pragma unroll
-        for (int m = 0; m < P1; m++) a += xw[m] * sU[(bb * N + k) * S + xi[m]];
+        for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
         u[k] = a;
         bv[k] = 0;
       }
@@ -1205,7 +1362,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   if (act) {
 #pragma unroll
     for (int k = 0; k < N; k++)
-      st_s<NT>(divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, tb), &divFe[(e * N + k) * S + s]);
+      st_s<NT>(divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po), &divFe[(e * N + k) * S + s]);
   }
   // faces: discontinuous normal flux.  With kJumpInVolume it stores in its
   // place this side's part of the correction's flux jump, +-B dA - disFn (B
@@ -1214,11 +1371,10 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
     const int bb = i / F, f = i - bb * F;
     const long long ee = e0 + bb;
-    const int* xi = tb.ext_idx + f * P1;
+    const FpOp<D, P, R, TEN> fp(tb, sW, f);
     // extrapolateNormalFlux: of the sum over directions only the face's own
     // normal direction is non-zero (the other terms are exact zeros)
-    const int dn = tb.efn_dir[f];
-    const R* ew = tw<R>(tb.efn_w, tb.efn_wf) + f * P1;
+    const int dn = fp.dir();
     int side = 2;
     R dA = 0, bv[N];
     if constexpr (kJumpInVolume<R>) {
@@ -1233,7 +1389,8 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     for (int k = 0; k < N; k++) {
       R a = 0;
 #pragma unroll
-      for (int m = 0; m < P1; m++) a += ew[m] * sF[((bb * D + dn) * N + k) * S + xi[m]];
+      for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
+      a = fp.efn_sign(a);
       if constexpr (kJumpInVolume<R>) a = (side == 2) ? -a : (side == 0 ? bv[k] : -bv[k]) * dA - a;
       st_s<NT>(a, &disFne[(ee * N + k) * F + f]);
     }
@@ -1244,19 +1401,19 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
 // and the FP32 path, which fit there without spilling (holding the FP32
 // viscous hex kernel to 5 or 6 waves spills 26 or 41 VGPRs and was measured
 // 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes.
-template <int D, int P, class R, bool NT>
+template <int D, int P, class R, bool NT, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_volume_w3(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
     const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
     Phys ph) {
-  volume_body<D, P, R, NT>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
+  volume_body<D, P, R, NT, TEN>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
 }
-template <int D, int P, class R, bool NT, int BF = 0>
+template <int D, int P, class R, bool NT, bool TEN, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_volume_w4(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
     const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
     Phys ph) {
-  volume_body<D, P, R, NT, BF>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
+  volume_body<D, P, R, NT, TEN, BF>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
 }
 
 // ---------------------------------------------------------------------------
@@ -1311,7 +1468,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_face_bnd(int nB, const int* __res
 // exactly once per launch go through nontemporal loads and stores (they
 // stream past the caches); arrays read twice (the LDG side parts and the
 // inviscid common flux, read by both sides of a face) stay cached.
-template <int D, int P, class R, bool NT>
+template <int D, int P, class R, bool NT, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ divFe, const R* __restrict__ Fne,
                                              const R* __restrict__ disFne, RkArgs<R> ra, Tabs tb,
                                              const int* __restrict__ fpart, const R* __restrict__ dAe,
@@ -1321,6 +1478,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   const int EB = blockDim.x / S;
   R* const sU = reinterpret_cast<R*>(fhip_lds);  // [EB*N*S]
   R* const sD = sU + EB * N * S;                  // [EB*N*F] Fn - disFn at the block's flux points
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
   const int b = threadIdx.x / S, s = threadIdx.x - b * S;
   // The flux points' loads are unconditional (a boundary point reads its own
@@ -1399,7 +1558,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
 #pragma unroll
     for (int k = 0; k < N; k++) dv[k] = ld_s<NT>(&divFe[((e0 + b) * (long long)N + k) * S + s]);
   }
-  rk_tail<D, P, R, NT>(E, dv, sU, sD, ra, tb);
+  rk_tail<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra, tb);
 }
 
 template <class R>
@@ -1718,7 +1877,66 @@ static bool build_d1(const Ctx& c, const fhip_desc* dsc, std::vector<double>& d1
   return true;
 }
 
-static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& blob, size_t off[17]) {
+// The 1-D factors (Ten) of the dense operators, or false where an entry of one
+// of them is not what the factors give.
+template <int D, int P>
+static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w) {
+  using T = Ten<D, P>;
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, F = Sh::F, P1 = Sh::P1;
+  w.assign(T::NW, 0.);
+  std::copy(d1.begin(), d1.end(), w.begin());
+  // l and c from the first point of a face on each end of direction 0
+  for (int j = 0; j < 2 * D; j++) {
+    if (T::face_dir(j) != 0) continue;
+    const int f = j * Sh::Ff, hi = T::face_hi(j);
+    const typename T::Face face(f);
+    for (int m = 0; m < P1; m++) {
+      int cc[3] = {m, face.c[1], face.c[2]};
+      const int q = cc[0] + P1 * (cc[1] + P1 * cc[2]);
+      w[T::L + hi * P1 + m] = d->opp_spts_to_fpts[(size_t)f * S + q];
+      w[T::C + hi * P1 + m] = d->opp_correction[(size_t)q * F + T::face_fpt(j, cc)];
+    }
+  }
+  for (int f = 0; f < F; f++) {
+    const typename T::Face face(f);
+    const int j = f / Sh::Ff;
+    if (face.dn != T::face_dir(j) || face.hi != T::face_hi(j)) return false;
+    for (int q = 0; q < S; q++) {
+      const typename T::Point p(q);
+      bool on = true;
+      for (int x = 0; x < D; x++) on = on && (x == face.dn || p.c[x] == face.c[x]);
+      if (on != (T::face_fpt(j, p.c) == f)) return false;
+      const double l = on ? w[T::L + face.hi * P1 + p.c[face.dn]] : 0., cr = on ? w[T::C + face.hi * P1 + p.c[face.dn]] : 0.;
+      if (!(d->opp_spts_to_fpts[(size_t)f * S + q] == l && d->opp_correction[(size_t)q * F + f] == cr)) return false;
+      for (int x = 0; x < D; x++) {
+        const double sg = x == face.dn ? (face.hi ? 1. : -1.) : 0.;
+        if (!(d->opp_extrapolate_fn[((size_t)x * F + f) * S + q] == l * sg)) return false;
+        if (c.prm.viscous && !(d->opp_correct_u[((size_t)x * S + q) * F + f] == cr * sg)) return false;
+      }
+    }
+  }
+  return true;
+}
+
+static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w) {
+  switch (c.z.D * 10 + c.z.P) {
+    case 20: return build_ten<2, 0>(c, d, d1, w);
+    case 21: return build_ten<2, 1>(c, d, d1, w);
+    case 22: return build_ten<2, 2>(c, d, d1, w);
+    case 23: return build_ten<2, 3>(c, d, d1, w);
+    case 24: return build_ten<2, 4>(c, d, d1, w);
+    case 25: return build_ten<2, 5>(c, d, d1, w);
+    case 30: return build_ten<3, 0>(c, d, d1, w);
+    case 31: return build_ten<3, 1>(c, d, d1, w);
+    case 32: return build_ten<3, 2>(c, d, d1, w);
+    case 33: return build_ten<3, 3>(c, d, d1, w);
+    case 34: return build_ten<3, 4>(c, d, d1, w);
+    default: return build_ten<3, 5>(c, d, d1, w);
+  }
+}
+
+static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& blob, size_t off[19]) {
   const int D = c.z.D, S = c.z.S, F = c.z.F, P1 = c.z.P + 1, NC = 2 * D;
   std::vector<int> ext_idx((size_t)F * P1, 0), efn_dir(F, 0), grd_idx((size_t)D * S * P1, 0),
       cor_idx((size_t)S * NC, 0), cu_idx((size_t)D * S * 2, 0);
@@ -1810,10 +2028,15 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
   putf(cu_w, off[14]);
   // the matrix-core path of FP64 P3 hexes needs the 1-D derivative matrix
   std::vector<double> d1;
-  off[15] = off[16] = 0;
+  off[15] = off[16] = off[17] = off[18] = 0;
   if (build_d1(c, d, d1)) {
     put(d1.data(), d1.size() * 8, off[15]);
     putf(d1, off[16]);
+    std::vector<double> w;
+    if (build_ten(c, d, d1, w)) {
+      put(w.data(), w.size() * 8, off[17]);
+      putf(w, off[18]);
+    }
   } else if (D == 3 && P1 == 4) {
     return false;
   }
@@ -1887,7 +2110,7 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
   const Sizes& z = c.z;
   if (z.P < 0 || z.P > 5) return false;
   std::vector<char> blob;
-  size_t off[17];
+  size_t off[19];
   if (!build_tables(c, d, blob, off)) return false;
   auto* st = new FusedState();
   c.fused = st;
@@ -1899,7 +2122,8 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
                 (const int*)(base + off[6]),    (const double*)(base + off[7]), (const int*)(base + off[8]),
                 (const double*)(base + off[9]), (const float*)(base + off[10]), (const float*)(base + off[11]),
                 (const float*)(base + off[12]), (const float*)(base + off[13]), (const float*)(base + off[14]),
-                off[15] ? (const double*)(base + off[15]) : nullptr, off[16] ? (const float*)(base + off[16]) : nullptr};
+                off[15] ? (const double*)(base + off[15]) : nullptr, off[16] ? (const float*)(base + off[16]) : nullptr,
+                off[17] ? (const double*)(base + off[17]) : nullptr, off[18] ? (const float*)(base + off[18]) : nullptr};
   const long long E = z.E, S = z.S, F = z.F, N = z.N, D = z.D;
   st->stream = E * N * S * (long long)sizeof(double) > kStreamBytes;
   st->Ue = dal<double>(E * N * S);
@@ -2118,8 +2342,8 @@ struct Runner {
     Work<R>& w = st.work<R>();
     // the FP32 stage copy starts from the state; the FP64 one is first
     // written by a step's first stage (which reads the state itself)
-    hipLaunchKernelGGL((k_extrap<D, P, R>), dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kExtrap, nt, false), c.stream,
-                       c.z.E, st.Ue, w.Ufe, sizeof(R) == 4 ? w.Us : nullptr, st.tb);
+    auto* kern = st.tb.w1 ? k_extrap<D, P, R, true> : k_extrap<D, P, R, false>;
+    hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kExtrap, nt, false), c.stream, c.z.E, st.Ue, w.Ufe, sizeof(R) == 4 ? w.Us : nullptr, st.tb);
     FCHK(hipGetLastError());
   }
   static void launch_face_inv(Ctx& c, int nt) {
@@ -2139,7 +2363,7 @@ struct Runner {
   // SIMD (128 VGPRs); FP64 hexes, which spill under that hold, to 3 (168 VGPRs:
   // P3 without spills, where the unheld compiler would take 211 and leave 2
   // waves)
-  template <bool NT>
+  template <bool NT, bool TEN>
   static void launch_volume_t(Ctx& c, int nt) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2150,18 +2374,18 @@ struct Runner {
                          w.dUce, w.JG, w.iJ, w.divFe, w.disFne, vf, st.tb, c.ph);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, 2>);
-      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, 3>);
-      else go(k_volume_w4<D, P, R, NT>);
+      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, TEN, 2>);
+      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, TEN, 3>);
+      else go(k_volume_w4<D, P, R, NT, TEN>);
     } else if constexpr (kHold<D, R>) {
-      go(k_volume_w4<D, P, R, NT>);
+      go(k_volume_w4<D, P, R, NT, TEN>);
     } else {
-      go(k_volume_w3<D, P, R, NT>);
+      go(k_volume_w3<D, P, R, NT, TEN>);
     }
     FCHK(hipGetLastError());
   }
   // inviscid runs: the stage kernel with the RK update ra
-  template <bool NT, bool BND>
+  template <bool NT, bool BND, bool TEN>
   static void launch_stage_t(Ctx& c, int nt, RkArgs<R> ra, bool fold) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2178,24 +2402,29 @@ struct Runner {
                          w.JG, fc, st.tb, c.ph, ra);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, 2>);
-      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, 3>);
-      else go(k_stage_w4<D, P, R, NT, BND>);
+      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, 2>);
+      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, 3>);
+      else go(k_stage_w4<D, P, R, NT, BND, TEN>);
     } else if constexpr (kHold<D, R>) {
-      go(k_stage_w4<D, P, R, NT, BND>);
+      go(k_stage_w4<D, P, R, NT, BND, TEN>);
     } else {
-      go(k_stage_w3<D, P, R, NT, BND>);
+      go(k_stage_w3<D, P, R, NT, BND, TEN>);
     }
     FCHK(hipGetLastError());
   }
   static void launch_volume(Ctx& c, int nt) {
-    if (fs(c).stream && kEleRowsWhole) launch_volume_t<true>(c, nt);
-    else launch_volume_t<false>(c, nt);
+    if (!fs(c).tb.w1) launch_volume_t<false, false>(c, nt);
+    else if (fs(c).stream && kEleRowsWhole) launch_volume_t<true, true>(c, nt);
+    else launch_volume_t<false, true>(c, nt);
   }
   static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
     const bool sm = fs(c).stream && kEleRowsWhole, bnd = fs(c).nBnd > 0;
-    if (sm) bnd ? launch_stage_t<true, true>(c, nt, ra, fold) : launch_stage_t<true, false>(c, nt, ra, fold);
-    else bnd ? launch_stage_t<false, true>(c, nt, ra, fold) : launch_stage_t<false, false>(c, nt, ra, fold);
+    // operators read from their tables: one instance for every mesh
+    if (!fs(c).tb.w1) launch_stage_t<false, true, false>(c, nt, ra, fold);
+    else if (sm && bnd) launch_stage_t<true, true, true>(c, nt, ra, fold);
+    else if (sm) launch_stage_t<true, false, true>(c, nt, ra, fold);
+    else if (bnd) launch_stage_t<false, true, true>(c, nt, ra, fold);
+    else launch_stage_t<false, false, true>(c, nt, ra, fold);
   }
   // whether a step's first stage forms the elements' time steps itself
   static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
@@ -2227,7 +2456,8 @@ struct Runner {
   static void launch_rk(Ctx& c, int nt, int mode, double a, double b, bool write0, int stage = 0) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
-    auto* kern = (st.stream && kEleRowsWhole) ? k_rk<D, P, R, true> : k_rk<D, P, R, false>;
+    auto* kern = !st.tb.w1 ? k_rk<D, P, R, false, false>
+                           : ((st.stream && kEleRowsWhole) ? k_rk<D, P, R, true, true> : k_rk<D, P, R, false, true>);
     hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kRk, nt, false), c.stream, c.z.E, w.divFe, w.Fne,
                        w.disFne, rk_args(c, mode, a, b, write0, stage), st.tb, st.fpart, w.dA, w.Bve);
     FCHK(hipGetLastError());
