@@ -403,7 +403,7 @@ struct FusedState {
   Tabs tb{};
   void* tab_mem = nullptr;
   // FP64 element-major state, metrics and wave speeds (both paths)
-  double *Ue = nullptr, *U0e = nullptr, *Uacc = nullptr, *divF0e = nullptr, *JGe = nullptr, *detJe = nullptr,
+  double *Ue = nullptr, *Uacc = nullptr, *divF0e = nullptr, *JGe = nullptr, *detJe = nullptr,
          *iJe = nullptr, *norme = nullptr, *dAe = nullptr, *waveSpe = nullptr;
   int *pL = nullptr, *pR = nullptr, *bc = nullptr;
   // per element flux point, 4 * (partner flux point e*F + f) + side (0 left,
@@ -439,7 +439,7 @@ struct FusedState {
   ~FusedState() {
     w64.release();
     w32.release();
-    void* ps[] = {tab_mem, Ue,  U0e,     Uacc,    divF0e,    JGe,    detJe,  iJe,   norme, dAe, waveSpe, pL,
+    void* ps[] = {tab_mem, Ue,           Uacc,    divF0e,    JGe,    detJe,  iJe,   norme, dAe, waveSpe, pL,
                   pR,      bc,  fpart,   bndT,    nfe,       bst,    meshDt, meshRes, eleMesh, meshStart, active, srce,
                   dtTicket, vole, bndBc};
     for (void* p : ps)
@@ -640,9 +640,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_face_inv(int nFF, const int* __re
 // folded into one pass per stage, FP64) and U at the flux points for the
 // next stage.  mode: 0 first classical stage, 1 middle classical stage,
 // 2 last classical stage, 3 single-stage forward Euler, 4 Jameson-form stage,
-// 6 first Jameson-form stage (which also keeps U as the step's U0 where a
-// separate U0 is kept); 5, 7 and 8 the residual alone (see rk_tail_p).
-// Classical stages combine into U0 - sum_j b_j r_j / detJ dt in timeStepB's
+// 6 first Jameson-form stage; 5, 7 and 8 the residual alone (see rk_point).
+// Classical stages combine into U0 - sum_j b_j r_j (dt / detJ) in timeStepB's
 // order (src/solver.cpp:504-536): either through the FP64 accumulator Uacc, or
 // (mixed path, Rst given) from the stored stage residuals, which FP32 holds
 // exactly there since they are sums of FP32 values; both give the same bits.
@@ -661,7 +660,6 @@ struct RkArgs {
   const double* eleDt;
   int local;
   double* Ue;
-  double* U0e;
   double* Uacc;
   double* divF0e;
   const int* eleMesh;
@@ -676,154 +674,153 @@ struct RkArgs {
   R* Ufe;
 };
 
-// correctDivFlux, timeStepA/B and U at the flux points for the next stage, for
-// the block's elements: dv holds this thread's divF (one value per field),
-// sD the flux jump at the block's flux points, and sU receives the new state
-// (its previous contents are no longer read).  Ends with every thread of the
-// block past a barrier unless mode is 5 (residual only), which returns at
-// once for the whole block.
-// The arrays come in as __restrict__ parameters (from RkArgs at the call
-// below), so that the compiler may keep their loads ahead of the stores.
+// What the update of one solution point reads besides its flux jump and divF,
+// loaded ahead of the phases that form those (rk_load), so that the loads are in
+// flight meanwhile: a launch on a small mesh is a chain of such waits.
+template <int D, class R>
+struct RkIn {
+  static constexpr int N = D + 2;
+  double dj, dt;
+  double u[N];    // U at the step's start (its U0; U itself in the first stage)
+  double acc[N];  // RK accumulator; mode 7: the source that the residual is taken from
+  double src[N];  // P-multigrid source
+  R rs[3][N];     // mixed path, last stage: the residuals of the first three stages
+  bool frozen;
+};
+
+template <int D, int P, class R, bool NT>
+__device__ __forceinline__ RkIn<D, R> rk_load(int E, long long e, int s, const RkArgs<R>& ra) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, N = Sh::N;
+  RkIn<D, R> in{};
+  const int mode = ra.mode;
+  const long long at = e * N * S + s;
+  if (mode == 5 || mode == 7 || mode == 8) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      if (mode == 7) in.acc[k] = ra.divF0e[at + k * S];
+      if (mode == 8) in.src[k] = ra.srce[at + k * S];
+    }
+    return in;
+  }
+  in.dj = ld_s<NT>(&ra.detJe[e * S + s]);
+  // (the state itself is the step's U0 until the last stage writes it)
+#pragma unroll
+  for (int k = 0; k < N; k++) in.u[k] = ld_s<NT>(&ra.Ue[at + k * S]);
+  if (!ra.Rst && (mode == 1 || mode == 2)) {
+#pragma unroll
+    for (int k = 0; k < N; k++) in.acc[k] = ld_s<NT>(&ra.Uacc[at + k * S]);
+  }
+  if (ra.srce) {
+#pragma unroll
+    for (int k = 0; k < N; k++) in.src[k] = ra.srce[at + k * S];
+  }
+  if (sizeof(R) == 4 && ra.Rst && mode == 2) {
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      if (j < ra.stage) {
+#pragma unroll
+        for (int k = 0; k < N; k++) in.rs[j][k] = ld_s<NT>(&ra.Rst[j * ((long long)E * N * S) + at + k * S]);
+      }
+  }
+  in.dt = ra.local == 1 ? ra.eleDt[e] : (ra.local == 2 ? ra.meshDt[ra.eleMesh[e]] : *ra.dtp);
+  in.frozen = ra.active && !ra.active[ra.eleMesh[e]];
+  return in;
+}
+
+// correctDivFlux and timeStepA/B at point s of the block's element b: dv holds
+// its divF (one value per field), sD the flux jump at the block's flux points,
+// and sU receives the new state (its previous contents are no longer read).
+// The increment is coefficient * residual * (dt / detJ), one division per point.
 template <int D, int P, class R, bool NT, bool TEN>
-__device__ __forceinline__ void rk_tail_p(int E, const R* dv, R* sU, const R* sD, const R* sW, int mode, double a, double bcoef,
-                                          const double* __restrict__ detJe, const double* __restrict__ dtp,
-                                          const double* __restrict__ eleDt, int local, double* __restrict__ Ue,
-                                          double* __restrict__ U0e, double* __restrict__ Uacc,
-                                          double* __restrict__ divF0e, const int* __restrict__ eleMesh,
-                                          const double* __restrict__ meshDt, const int* __restrict__ active,
-                                          const double* __restrict__ srce, R* __restrict__ Rst, int stage,
-                                          const RkB& bs, R* __restrict__ Us, int fin, R* __restrict__ Ufe,
-                                          const Tabs& tb, bool hasDt, double dtIn) {
+__device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const R* dv, R* sU, const R* sD, const R* sW,
+                                         const RkIn<D, R>& in, const RkArgs<R>& ra, const Tabs& tb) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1, NC = Sh::NC;
-  const int EB = blockDim.x / S;
-  const long long nS = (long long)E * N * S;
-  const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
-  const int b = threadIdx.x / S, s = threadIdx.x - b * S;
+  const int mode = ra.mode;
   const PtOp<D, P, R, TEN> po(tb, sW, s);
+  R res[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    R c = 0;
+#pragma unroll
+    for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
+    res[k] = c + dv[k];
+  }
+  const long long at = e * N * S + s;
   if (mode == 5 || mode == 7 || mode == 8) {
     // residual only (calcResidual(0) + correctDivFlux), no update: 5 into
     // divF_spts[0]; 7 subtracted in place from the array divF0e points to
     // (the P-multigrid source); 8 plus the source into divF_spts[0]
-    if (b < nb) {
-      const long long e = e0 + b;
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        R c = 0;
-#pragma unroll
-        for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
-        const double r0 = double(c + dv[k]);
-        const long long iu = (e * N + k) * S + s;
-        if (mode == 7) {
-          double v = divF0e[iu];
-          v -= r0;
-          divF0e[iu] = v;
-        } else {
-          st_s<NT>(mode == 8 ? r0 + srce[iu] : r0, &divF0e[iu]);
-        }
-      }
-    }
-    return;  // uniform over the block: no barrier follows for anyone
-  }
-  if (b < nb) {
-    const long long e = e0 + b;
-    const double dt = hasDt ? dtIn : ((local == 1) ? eleDt[e] : (local == 2 ? meshDt[eleMesh[e]] : *dtp));
-    const bool frozen = active && !active[eleMesh[e]];
-    const double dj = ld_s<NT>(&detJe[e * S + s]);
-    // the stage's state inputs for every field first (uniform branches on the
-    // mode), so that their loads are in flight together: U itself is an input
-    // of the first and the single stage only (and of frozen batch members,
-    // which keep it)
-    double uin[N], u0in[N], accin[N];
-    const bool needU = mode == 0 || mode == 3 || mode == 6 || frozen;
-    const bool needU0 = mode == 1 || mode == 4 || (mode == 2 && Rst);
-    const bool needAcc = !Rst && (mode == 1 || mode == 2);
-#pragma unroll
-    for (int k = 0; k < N; k++) uin[k] = u0in[k] = accin[k] = 0.0;
-    if (needU) {
-#pragma unroll
-      for (int k = 0; k < N; k++) uin[k] = ld_s<NT>(&Ue[(e * N + k) * S + s]);
-    }
-    if (needU0) {
-      // with a stage copy the state stays the step's U0 until the last stage
-      // writes it, and no separate U0 is kept (U0e null)
-      const double* u0 = U0e ? U0e : Ue;
-#pragma unroll
-      for (int k = 0; k < N; k++) u0in[k] = ld_s<NT>(&u0[(e * N + k) * S + s]);
-    }
-    if (needAcc) {
-#pragma unroll
-      for (int k = 0; k < N; k++) accin[k] = ld_s<NT>(&Uacc[(e * N + k) * S + s]);
-    }
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      const long long iu = (e * N + k) * S + s;
-      R c = 0;
-#pragma unroll
-      for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
-      const double r0 = double(c + dv[k]);
-      if (divF0e) st_s<NT>(r0, &divF0e[iu]);
-      // P-multigrid source: divF_spts[step] + src_spts (src/solver.cpp:480,514)
-      const double r = srce ? r0 + srce[iu] : r0;
-      const double u = uin[k];
-      double un;
-      if (mode == 0) {
-        if (U0e) st_s<NT>(u, &U0e[iu]);
-        if (Rst) st_s<NT>(R(r), &Rst[iu]);
-        else st_s<NT>(u - bcoef * r / dj * dt, &Uacc[iu]);
-        un = u - a * r / dj * dt;
-      } else if (mode == 1) {
-        if (Rst) st_s<NT>(R(r), &Rst[stage * nS + iu]);
-        else st_s<NT>(accin[k] - bcoef * r / dj * dt, &Uacc[iu]);
-        un = u0in[k] - a * r / dj * dt;
-      } else if (mode == 2) {
-        double acc;
-        if (Rst) {
-          acc = u0in[k];
-          for (int j = 0; j < stage; j++) acc = acc - bs.b[j] * double(ld_s<NT>(&Rst[j * nS + iu])) / dj * dt;
-        } else {
-          acc = accin[k];
-        }
-        un = acc - bcoef * r / dj * dt;
-      } else if (mode == 3) {
-        un = u - bcoef * r / dj * dt;
-      } else if (mode == 6) {
-        if (U0e) st_s<NT>(u, &U0e[iu]);
-        un = u - a * r / dj * dt;
-      } else {
-        un = u0in[k] - a * r / dj * dt;
-      }
-      if (frozen) un = u;
-      // with a stage copy the state is written at the step's last stage
-      // only (earlier stages leave it at the step's start, its U0, and write
-      // the copy); the FP32 copy is written at the last stage too (the flux
-      // kernels read U only through it), the FP64 one is not (the next
-      // step's first stage reads the state itself)
-      if (!Us || fin) st_s<NT>(un, &Ue[iu]);
-      if (Us && (sizeof(R) == 4 || !fin)) st_s<NT>(R(un), &Us[iu]);
-      sU[(b * N + k) * S + spt_lds(D, P1, s)] = R(un);
+      const double r0 = double(res[k]);
+      if (mode == 7) ra.divF0e[at + k * S] = in.acc[k] - r0;
+      else st_s<NT>(mode == 8 ? r0 + in.src[k] : r0, &ra.divF0e[at + k * S]);
     }
+    return;
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
-    int bb = i / F, f = i - bb * F;
-    const FpOp<D, P, R, TEN> fp(tb, sW, f);
+  const double q = in.dt / in.dj;
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      R acc = 0;
+  for (int k = 0; k < N; k++) {
+    const long long iu = at + k * S;
+    const double r0 = double(res[k]);
+    if (ra.divF0e) st_s<NT>(r0, &ra.divF0e[iu]);
+    // P-multigrid source: divF_spts[step] + src_spts (src/solver.cpp:480,514)
+    const double r = ra.srce ? r0 + in.src[k] : r0;
+    const double u = in.u[k];
+    double un;
+    if (mode == 0) {
+      if (ra.Rst) st_s<NT>(R(r), &ra.Rst[iu]);
+      else st_s<NT>(u - ra.bcoef * r * q, &ra.Uacc[iu]);
+      un = u - ra.a * r * q;
+    } else if (mode == 1) {
+      if (ra.Rst) st_s<NT>(R(r), &ra.Rst[ra.stage * ((long long)E * N * S) + iu]);
+      else st_s<NT>(in.acc[k] - ra.bcoef * r * q, &ra.Uacc[iu]);
+      un = u - ra.a * r * q;
+    } else if (mode == 2) {
+      double acc = in.acc[k];
+      if (ra.Rst) {
+        acc = u;
 #pragma unroll
-      for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
-      st_s<NT>(acc, &Ufe[((long long)(e0 + bb) * N + k) * F + f]);
+        for (int j = 0; j < 3; j++)
+          if (j < ra.stage) acc = acc - ra.bs.b[j] * double(in.rs[j][k]) * q;
+#pragma unroll
+        for (int j = 3; j < 7; j++)  // constant indices: the arguments stay out of scratch
+          if (j < ra.stage) acc = acc - ra.bs.b[j] * double(ld_s<NT>(&ra.Rst[j * ((long long)E * N * S) + iu])) * q;
+      }
+      un = acc - ra.bcoef * r * q;
+    } else if (mode == 3) {
+      un = u - ra.bcoef * r * q;
+    } else {
+      un = u - ra.a * r * q;
     }
+    if (in.frozen) un = u;
+    // the state is written at the step's last stage only (earlier stages
+    // leave it at the step's start, its U0, and write the stage copy); the
+    // FP32 copy is written at the last stage too (the flux kernels read U
+    // only through it), the FP64 one is not (the next step's first stage
+    // reads the state itself)
+    if (ra.fin) st_s<NT>(un, &ra.Ue[iu]);
+    if (sizeof(R) == 4 || !ra.fin) st_s<NT>(R(un), &ra.Us[iu]);
+    sU[(b * N + k) * S + spt_lds(D, P1, s)] = R(un);
   }
 }
 
+// extrapolateU at flux point i of the block, from the states in sU.
 template <int D, int P, class R, bool NT, bool TEN>
-__device__ __forceinline__ void rk_tail(int E, const R* dv, R* sU, const R* sD, const R* sW, const RkArgs<R>& ra,
-                                        const Tabs& tb, bool hasDt = false, double dtIn = 0) {
-  rk_tail_p<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra.mode, ra.a, ra.bcoef, ra.detJe, ra.dtp, ra.eleDt, ra.local, ra.Ue, ra.U0e,
-                         ra.Uacc, ra.divF0e, ra.eleMesh, ra.meshDt, ra.active, ra.srce, ra.Rst, ra.stage, ra.bs, ra.Us,
-                         ra.fin, ra.Ufe, tb, hasDt, dtIn);
+__device__ __forceinline__ void face_point(int i, int e0, const R* sU, const R* sW, R* Ufe, const Tabs& tb) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
+  const int bb = i / F, f = i - bb * F;
+  const FpOp<D, P, R, TEN> fp(tb, sW, f);
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    R acc = 0;
+#pragma unroll
+    for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
+    st_s<NT>(acc, &Ufe[((long long)(e0 + bb) * N + k) * F + f]);
+  }
 }
 
 // Viscous runs, FP32: the volume kernel also folds its own side's LDG part
@@ -903,7 +900,9 @@ __device__ __forceinline__ R divergence(const R* sF, int b, int s, int k, int sw
 //
 // Measured, two kernels -> one: 2-D vortex 32x32 P3, 20 RK44 steps 842 -> 683 us;
 // 3-D vortex 17^3 P2, 10 steps 1351 -> 1132 us; 23^3 P4 mixed, 4 steps 2140 ->
-// 1841 us; P4 channel 67x29, update and multigrid cycle 1142 -> 1005 us.
+// 1841 us; P4 channel 67x29, update and multigrid cycle 1142 -> 1005 us.  With
+// the points apart, the update's inputs loaded early and one division per point
+// (below): vortex 663 -> 587 us, channel 941 -> 678 us, 17^3 P2 1109 -> 903 us.
 //
 // Steady runs (local time steps, 2-D) also form the element's time step here,
 // in the step's first stage: it needs only the element's own wave speeds.
@@ -922,13 +921,23 @@ struct StageFace {
   double* eleDt;
 };
 
-template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF>
-__device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
+// Two forms.  Apart: a block's threads are the solution points' waves and then
+// the flux points' (stage_threads), so that the two kinds of work of a phase run
+// side by side: the common flux beside the flux at the points, the flux jump
+// beside the divergence; the update's inputs (2-D) are loaded with the slab.  On
+// a small mesh, where a CU holds a few waves, a launch takes as long as the
+// instructions and waits of one wave, and this shortens them.  Together: a
+// thread does a solution point and then ceil(F/S) flux points; more elements are
+// in flight per register, which is what counts once the mesh fills the chip
+// (kApartWaves below).
+__host__ __device__ constexpr int up64(int n) { return (n + 63) / 64 * 64; }
+
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF>
+__device__ __forceinline__ void stage_body(int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us,
                                            const R* __restrict__ JGe, const StageFace<R>& fc, const Tabs& tb,
                                            const Phys& ph, const RkArgs<R>& ra) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
-  const int EB = blockDim.x / S;
   // U, the transformed flux and the flux jump of the block's elements:
   // [EB*N*S] [EB*D*N*S] [EB*N*F]
   R* const sU = reinterpret_cast<R*>(fhip_lds);
@@ -939,24 +948,24 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
   const int b = threadIdx.x / S, s = threadIdx.x - b * S;
   const int sw = spt_lds(D, P1, s);
-  const bool act = b < nb;
+  const bool act = (int)threadIdx.x < nb * S;  // a solution point's thread
   const long long e = e0 + b;
+  // the thread's flux points: fi(u) < nP (negative: none)
+  constexpr int KF = APART ? 1 : (F + S - 1) / S;
+  const int fb = APART ? up64(EB * S) : 0, nP = nb * F;
+  auto fi = [&](int u) { return (int)threadIdx.x - fb + u * (int)blockDim.x; };
+  auto flx = [&](int u) { return (!APART || fi(u) >= 0) && fi(u) < nP; };
   constexpr bool mf = kMfma<D, P, R>;
   constexpr int np = kBf16<D, P, R> ? BF : 0;
   bf16x8 abf = {};
-  if constexpr (np != 0) abf = bf16_opnd_a(tw<float>(tb.d1, tb.d1f), s, np);
+  if constexpr (np != 0) abf = bf16_opnd_a(tw<float>(tb.d1, tb.d1f), s % 64, np);
   const int swx = mf ? spt_lds(D, P1, s / 16 + 4 * ((s / 4) % 4) + 16 * (s % 4)) : 0;
   const R opv = mf ? tw<R>(tb.d1, tb.d1f)[(s % 4) * P1 + s / 16] : R(0);
-  // a thread finishes at most KF flux points; their side codes are loaded
-  // first, since the partners' addresses come from them
-  constexpr int KF = (F + S - 1) / S;
-  const int nP = nb * F;
+  const bool fold = D == 2 && fc.wf;
+  // the flux points' side codes first: the partners' addresses come from them
   int cd[KF];
 #pragma unroll
-  for (int u = 0; u < KF; u++) {
-    const int i = threadIdx.x + u * blockDim.x;
-    cd[u] = i < nP ? fc.fpart[(long long)e0 * F + i] : -1;
-  }
+  for (int u = 0; u < KF; u++) cd[u] = flx(u) ? fc.fpart[(long long)e0 * F + fi(u)] : 0;
   R vu[N];
 #pragma unroll
   for (int u = 0; u < N; u++) {
@@ -965,65 +974,68 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
       vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
   }
   R G[D][D] = {};
+  RkIn<D, R> in{};
   if (act) {
 #pragma unroll
     for (int r = 0; r < D; r++)
 #pragma unroll
       for (int x = 0; x < D; x++) G[r][x] = JGe[((e * D + r) * D + x) * S + s];
+    if constexpr (APART && D == 2) in = rk_load<D, P, R, NT>(E, e, s, ra);
   }
-  const bool fold = D == 2 && fc.wf;
-  R fo[KF][N];
+  R own[N], oth[N], n[D], dA = 0, fo[KF][N];
+  // U at flux point u and across, its normal and dA
+  auto load_face = [&](int u) {
+    const int i = fi(u), bb = i / F, f = i - bb * F;
+    const long long ob = (long long)(e0 + bb) * N * F + f;
 #pragma unroll
-  for (int u = 0; u < KF; u++) {
-    const int i = threadIdx.x + u * blockDim.x;
+    for (int k = 0; k < N; k++) own[k] = fc.Ufe[ob + k * F];
 #pragma unroll
-    for (int k = 0; k < N; k++) fo[u][k] = 0;
-    if (i < nP) {
-      const int bb = i / F, f = i - bb * F, side = cd[u] & 3;
-      const long long ob = (long long)(e0 + bb) * N * F + f;
-      R own[N], oth[N], n[D], fn[N];
-#pragma unroll
-      for (int k = 0; k < N; k++) own[k] = fc.Ufe[ob + k * F];
-      long long pb = ob;
-      if (!BND || side != 2) {
-        const int p = cd[u] >> 2, ep = p / F;
-        pb = (long long)ep * N * F + (p - ep * F);
-      }
-#pragma unroll
-      for (int k = 0; k < N; k++) oth[k] = fc.Ufe[pb + k * F];
-#pragma unroll
-      for (int x = 0; x < D; x++) n[x] = ld_s<NT>(&fc.nfe[((long long)(e0 + bb) * D + x) * F + f]);
-      const R dA = ld_s<NT>(&fc.dA[(long long)e0 * F + i]);
-      if (fold) {
-        const int Ff = Sh::Ff;
-        reinterpret_cast<double*>(sD)[i] =
-            fc.wavein[(long long)e0 * F + i] * fc.wf[f % Ff] * fc.dAd[(long long)e0 * F + i];
-      }
-      if constexpr (BND) {
-        if (side == 2) bc_state<D, R>(fc.bndBc[cd[u] >> 2], own, n, oth, ph, fc.bst);
-      }
-      const bool right = side == 1;
-      R UL[N], UR[N];
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        UL[k] = right ? oth[k] : own[k];
-        UR[k] = right ? own[k] : oth[k];
-      }
-      bool roe = false;
-      if constexpr (D == 2) roe = ph.riemann_type != 0 && (!BND || side != 2);
-      if (!roe) {
-        const double lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
-        if (fc.wave && !right) st_s<NT>(lam, &fc.wave[(long long)e0 * F + i]);
-      } else if constexpr (D == 2) {
-        roe2d<R>(UL, UR, n, fn, R(ph.gamma));
-      }
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        const R v = mul_rn(fn[k], dA);
-        fo[u][k] = right ? -v : v;
-      }
+    for (int x = 0; x < D; x++) n[x] = ld_s<NT>(&fc.nfe[((long long)(e0 + bb) * D + x) * F + f]);
+    dA = ld_s<NT>(&fc.dA[(long long)e0 * F + i]);
+    long long pb = ob;
+    if (!BND || (cd[u] & 3) != 2) {
+      const int p = cd[u] >> 2, ep = p / F;
+      pb = (long long)ep * N * F + (p - ep * F);
     }
-  }
+#pragma unroll
+    for (int k = 0; k < N; k++) oth[k] = fc.Ufe[pb + k * F];
+    if (fold)
+      reinterpret_cast<double*>(sD)[i] =
+          fc.wavein[(long long)e0 * F + i] * fc.wf[f % Sh::Ff] * fc.dAd[(long long)e0 * F + i];
+  };
+  // the common flux times this side's dA, negated on the right side
+  auto common = [&](int u) {
+    const int side = cd[u] & 3;
+    if constexpr (BND) {
+      if (side == 2) bc_state<D, R>(fc.bndBc[cd[u] >> 2], own, n, oth, ph, fc.bst);
+    }
+    const bool right = side == 1;
+    R UL[N], UR[N], fn[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      UL[k] = right ? oth[k] : own[k];
+      UR[k] = right ? own[k] : oth[k];
+    }
+    bool roe = false;
+    if constexpr (D == 2) roe = ph.riemann_type != 0 && (!BND || side != 2);
+    if (!roe) {
+      const double lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
+      if (fc.wave && !right) st_s<NT>(lam, &fc.wave[(long long)e0 * F + fi(u)]);
+    } else if constexpr (D == 2) {
+      roe2d<R>(UL, UR, n, fn, R(ph.gamma));
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const R v = mul_rn(fn[k], dA);
+      fo[u][k] = right ? -v : v;
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < KF; u++)
+    if (flx(u)) {
+      load_face(u);
+      if constexpr (!APART) common(u);
+    }
 #pragma unroll
   for (int u = 0; u < N; u++) {
     const int i = threadIdx.x + u * blockDim.x;
@@ -1034,14 +1046,14 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
   }
   __syncthreads();
   double dtl = 0;
-  if (fold && act) {
-    double iw = 0;
-    for (int f = 0; f < F; f++) iw += reinterpret_cast<const double*>(sD)[b * F + f];
-    dtl = fc.cflfac * 2 * fc.vole[e] / iw;
-    if (s == 0) fc.eleDt[e] = dtl;
-  }
-  // flux at the point, transformed to the reference element
   if (act) {
+    if (fold) {
+      double iw = 0;
+      for (int g = 0; g < F; g++) iw += reinterpret_cast<const double*>(sD)[b * F + g];
+      dtl = fc.cflfac * 2 * fc.vole[e] / iw;
+      if (s == 0) fc.eleDt[e] = dtl;
+    }
+    // flux at the point, transformed to the reference element
     R u[N], Fl[D][N];
 #pragma unroll
     for (int k = 0; k < N; k++) u[k] = sU[(b * N + k) * S + sw];
@@ -1056,21 +1068,26 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
         sF[((b * D + d1) * N + k) * S + sw] = acc;
       }
   }
+  if constexpr (APART) {
+    if (flx(0)) common(0);
+  }
   __syncthreads();
-  R dv[N] = {};
+  R dv[N];
   if (act) {
+    // (without the registers for the update's inputs earlier)
+    if constexpr (!(APART && D == 2)) in = rk_load<D, P, R, NT>(E, e, s, ra);
+    if (fold) in.dt = dtl;
     const PtOp<D, P, R, TEN> po(tb, sW, s);
 #pragma unroll
     for (int k = 0; k < N; k++) dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po);
   }
-  // the flux jump: the common flux times this side's dA, negated on the right
-  // side, less the extrapolated normal flux (of the sum over directions only
-  // the face's own normal direction is non-zero)
 #pragma unroll
-  for (int u = 0; u < KF; u++) {
-    const int i = threadIdx.x + u * blockDim.x;
-    if (i < nP) {
-      const int bb = i / F, f = i - bb * F;
+  for (int u = 0; u < KF; u++)
+    if (flx(u)) {
+      // the flux jump: the common flux less the extrapolated normal flux (of
+      // the sum over directions only the face's own normal direction is
+      // non-zero)
+      const int bb = fi(u) / F, f = fi(u) - bb * F;
       const FpOp<D, P, R, TEN> fp(tb, sW, f);
       const int dn = fp.dir();
 #pragma unroll
@@ -1081,24 +1098,28 @@ __device__ __forceinline__ void stage_body(int E, const double* __restrict__ Ue,
         sD[(bb * N + k) * F + f] = fo[u][k] - fp.efn_sign(a);
       }
     }
-  }
   __syncthreads();
-  rk_tail<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra, tb, fold, dtl);
+  if (act) rk_point<D, P, R, NT, TEN>(E, e, b, s, dv, sU, sD, sW, in, ra, tb);
+  if (ra.mode == 5 || ra.mode == 7 || ra.mode == 8) return;  // uniform over the launch
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < KF; u++)
+    if (flx(u)) face_point<D, P, R, NT, TEN>(fi(u), e0, sU, sW, ra.Ufe, tb);
 }
 
 // Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
 // for FP64 hexes.
-template <int D, int P, class R, bool NT, bool BND, bool TEN>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_w3(
-    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
+    int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, 0>(E, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, 0>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
-template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
-    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
+    int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, BF>(E, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, BF>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
 
 // ---------------------------------------------------------------------------
@@ -1553,12 +1574,16 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
     }
   }
   __syncthreads();
-  R dv[N];
   if (b < nb) {
+    R dv[N];
 #pragma unroll
     for (int k = 0; k < N; k++) dv[k] = ld_s<NT>(&divFe[((e0 + b) * (long long)N + k) * S + s]);
+    const RkIn<D, R> in = rk_load<D, P, R, NT>(E, e0 + b, s, ra);
+    rk_point<D, P, R, NT, TEN>(E, e0 + b, b, s, dv, sU, sD, sW, in, ra, tb);
   }
-  rk_tail<D, P, R, NT, TEN>(E, dv, sU, sD, sW, ra, tb);
+  if (ra.mode == 5 || ra.mode == 7 || ra.mode == 8) return;  // uniform over the launch
+  __syncthreads();
+  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) face_point<D, P, R, NT, TEN>(i, e0, sU, sW, ra.Ufe, tb);
 }
 
 template <class R>
@@ -2320,6 +2345,28 @@ struct Runner {
   // streamed store covers whole blocks only when those rows are whole blocks.
   static constexpr bool kEleRowsWhole = (S * sizeof(R)) % 64 == 0 && (F * sizeof(R)) % 64 == 0;
   static int& blk(Ctx& c, int k) { return fs(c).nt[sizeof(R) == 4 ? 1 : 0][k]; }
+  // Elements of a block of the stage kernel's form with solution and flux points
+  // apart, within nt threads (one at least), and its threads: whole waves of
+  // solution points, then whole waves of flux points
+  static constexpr int stage_threads(int EB) { return up64(EB * S) + up64(EB * Sh::F); }
+  static_assert(stage_threads(1) <= kMaxBlock);
+  static int stage_eles(int nt) {
+    int EB = 1;
+    while (stage_threads(EB + 1) <= nt) EB++;
+    return EB;
+  }
+  static constexpr size_t stage_lds(size_t EB) { return EB * N * (S + D * S + Sh::F) * sizeof(R); }
+  // Which form of the stage kernel: apart while every wave of the launch can be
+  // resident at once (256 CUs x 16 waves), together beyond.  Measured per stage,
+  // apart / together, tuned sizes: quads P3 32^2 (512 waves) 5.9 / 6.6 us, 64^2
+  // (2048) 7.2 / 7.6, 96^2 (4608) 12.5 / 11.5; P4 hexes 8^3 (2200) 10.4 / 10.6,
+  // 12^3 (7425) 28.4 / 23.9; FP32 P3 hexes 8^3 (1280) 7.3 / 9.9, 12^3 (4320) 13.9 /
+  // 13.3, 16^3 (10240) 23.2 / 19.5.  FP64 hexes of orders 1 to 3, whose
+  // registers hold the other form to 3 waves per SIMD and whose blocks fill
+  // their waves, gain further up: P2 20^3 (10125) 27.7 / 30.3, P3 16^3 (10240)
+  // 26.4 / 28.9, P2 28^3 (27783) 64.2 / 62.2.
+  static constexpr long long kApartWaves = D == 3 && P >= 1 && P <= 3 && sizeof(R) == 8 ? 12288 : 4096;
+  static bool apart(const Ctx& c) { return (long long)c.z.E * (S + F) <= kApartWaves * 64; }
   // LDS bytes of an element kernel at block size nt (0 for the face kernels)
   static size_t lds(int k, int nt, bool visc) {
     const size_t EB = nt / S;
@@ -2385,7 +2432,7 @@ struct Runner {
     FCHK(hipGetLastError());
   }
   // inviscid runs: the stage kernel with the RK update ra
-  template <bool NT, bool BND, bool TEN>
+  template <bool NT, bool BND, bool TEN, bool APART>
   static void launch_stage_t(Ctx& c, int nt, RkArgs<R> ra, bool fold) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2397,18 +2444,19 @@ struct Runner {
                           fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
     ra.Ufe = st.odd_stage ? w.Ufe : w.Ufe2;
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
+    const int EB = APART ? stage_eles(nt) : nt / S, threads = APART ? stage_threads(EB) : nt;
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, false), c.stream, c.z.E, st.Ue, us,
+      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(threads), stage_lds(EB), c.stream, c.z.E, EB, st.Ue, us,
                          w.JG, fc, st.tb, c.ph, ra);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, 2>);
-      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, 3>);
-      else go(k_stage_w4<D, P, R, NT, BND, TEN>);
+      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 2>);
+      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 3>);
+      else go(k_stage_w4<D, P, R, NT, BND, TEN, APART>);
     } else if constexpr (kHold<D, R>) {
-      go(k_stage_w4<D, P, R, NT, BND, TEN>);
+      go(k_stage_w4<D, P, R, NT, BND, TEN, APART>);
     } else {
-      go(k_stage_w3<D, P, R, NT, BND, TEN>);
+      go(k_stage_w3<D, P, R, NT, BND, TEN, APART>);
     }
     FCHK(hipGetLastError());
   }
@@ -2420,11 +2468,13 @@ struct Runner {
   static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
     const bool sm = fs(c).stream && kEleRowsWhole, bnd = fs(c).nBnd > 0;
     // operators read from their tables: one instance for every mesh
-    if (!fs(c).tb.w1) launch_stage_t<false, true, false>(c, nt, ra, fold);
-    else if (sm && bnd) launch_stage_t<true, true, true>(c, nt, ra, fold);
-    else if (sm) launch_stage_t<true, false, true>(c, nt, ra, fold);
-    else if (bnd) launch_stage_t<false, true, true>(c, nt, ra, fold);
-    else launch_stage_t<false, false, true>(c, nt, ra, fold);
+    if (!fs(c).tb.w1) launch_stage_t<false, true, false, false>(c, nt, ra, fold);
+    else if (sm && bnd) launch_stage_t<true, true, true, false>(c, nt, ra, fold);
+    else if (sm) launch_stage_t<true, false, true, false>(c, nt, ra, fold);
+    else if (apart(c) && bnd) launch_stage_t<false, true, true, true>(c, nt, ra, fold);
+    else if (apart(c)) launch_stage_t<false, false, true, true>(c, nt, ra, fold);
+    else if (bnd) launch_stage_t<false, true, true, false>(c, nt, ra, fold);
+    else launch_stage_t<false, false, true, false>(c, nt, ra, fold);
   }
   // whether a step's first stage forms the elements' time steps itself
   static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
@@ -2446,7 +2496,7 @@ struct Runner {
     const double* src = mode == 8 ? st.srce : (st.use_src && mode != 7 ? st.srce : nullptr);
     return RkArgs<R>{mode, a, b, st.detJe, c.d_dt, c.eleDt,
                      c.prm.dt_type == 2 ? 1 : (c.prm.dt_type == 1 && st.nMesh > 1 ? 2 : 0), st.Ue,
-                     w.Us ? nullptr : st.U0e, st.Uacc,
+                     st.Uacc,
                      d0, st.eleMesh, st.meshDt, st.active, src,
                      (w.Rst && !st.use_src) ? w.Rst : nullptr, stage, bs, w.Us,
                      (mode == 2 || mode == 3 || (mode == 4 && stage == c.z.nRK - 1)) ? 1 : 0, w.Ufe};

@@ -70,6 +70,23 @@ def test_blocks_of_every_order(order, nt):
     s.close()
 
 
+@pytest.mark.parametrize("n,order", [(33, 0), (67, 3), (112, 1)])
+def test_both_forms_agree(n, order):
+    """Solution and flux points in threads of their own (small meshes) and in the
+    same threads: the same state, on either side of the size where one takes
+    over."""
+    states = []
+    for m in (1, 3):  # copies of one mesh merged into a context: beyond the limit with three
+        from flurrypp_amd.batch import BatchedSolver, Member
+        setup, U = cases.bump2d(nx=n, ny=n // 2, order=order, cfl=0.3)
+        b = BatchedSolver([Member(setup, U) for _ in range(m)], path=PATH_FUSED)
+        b.step(3)
+        states += b.states()
+        b.close()
+    for st in states[1:]:
+        np.testing.assert_allclose(st, states[0], rtol=1e-13, atol=1e-14)
+
+
 @pytest.mark.parametrize("order", [0, 1, 3])
 def test_hexes(order):
     setup, U = cases.tgv3d(n=3, order=order, viscous=0, jitter=0.1)
