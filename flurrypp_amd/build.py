@@ -77,11 +77,14 @@ def build_hip() -> Path:
     dev = CSRC / "device"
     obj = LIB / "obj"
     obj.mkdir(exist_ok=True)
-    names = ("fhip_api", "fhip_staged", "fhip_fused")
+    # the fused kernels' file is compiled per family of shapes, too
+    units = [(n, n, []) for n in ("fhip_api", "fhip_staged", "fhip_fused")]
+    units += [(f"fhip_fused_{k}", "fhip_fused", [f"-DFHIP_FAMILY={k}"]) for k in range(6)]
+    names = [u[0] for u in units]
     digest = source_hash("hip")
     procs = []
-    for n in names:
-        cmd = [HIPCC, *HIP_FLAGS, f"-I{INC}", f"-I{dev}", "-c", str(dev / f"{n}.hip"), "-o", str(obj / f"{n}.o")]
+    for n, src, defs in units:
+        cmd = [HIPCC, *HIP_FLAGS, *defs, f"-I{INC}", f"-I{dev}", "-c", str(dev / f"{src}.hip"), "-o", str(obj / f"{n}.o")]
         print("+", " ".join(cmd), flush=True)
         procs.append(subprocess.Popen(cmd))
     bad = [n for n, p in zip(names, procs) if p.wait() != 0]

@@ -11,17 +11,15 @@
 //
 // Data live element-major on the device ([ele][field][point]) so that a block
 // of elements is one contiguous slab.  Per RK stage:
-//   face_inv   common inviscid flux times dA on both sides of every face
-//              flux point (+ LDG common U, dUc)
-//   volume     [gradient + correction + physical transform], inviscid (and
-//              viscous) flux, transformed flux, divergence, discontinuous
-//              normal flux at the faces [and each side's part of the LDG
-//              viscous flux at its flux points]
-//   face_bnd   LDG viscous flux at boundary flux points (viscous runs with
-//              boundaries only)
-//   rk         correction of the divergence (common flux = inviscid part +
-//              both sides' LDG parts), RK update, U at the faces of the next
-//              stage
+//   inviscid   stage      common flux of the element's own flux points, flux,
+//                         divergence, correction, RK update, U at the faces
+//   viscous    volume     common inviscid flux and LDG common U at the element's
+//                         own flux points, corrected gradient, inviscid and
+//                         viscous flux, divergence, this side's part of the LDG
+//                         viscous flux, correction with all but the other
+//                         side's part
+//              rk         correction with the other sides' LDG parts, RK update,
+//                         U at the faces of the next stage
 //
 // Every kernel is templated on R, the type of the face and volume
 // intermediates and of the flux arithmetic: double for the FP64 path, float
@@ -373,14 +371,14 @@ __device__ __forceinline__ void stage_factors(R* sW, const Tabs& tb) {
 // Face and volume intermediates of one precision.
 template <class R>
 struct Work {
-  R *divFe = nullptr, *Ufe = nullptr, *Fne = nullptr, *disFne = nullptr, *dUce = nullptr;
+  R *divFe = nullptr, *Ufe = nullptr;
   // inviscid runs: U at the flux points of every second stage (a stage reads
   // one of Ufe, Ufe2 and writes the other; a step starts and ends in Ufe)
   R* Ufe2 = nullptr;
-  // viscous runs: each flux point's side of the LDG flux [ele][N][F] (disFne
-  // then holds that side's part of the flux jump, +-B dA - disFn), and the
-  // gradient at the boundary flux points [D*N][nBnd]
-  R *Bve = nullptr, *gBnd = nullptr;
+  // viscous runs: each flux point's side of the LDG flux [ele][N][F] (divFe then
+  // holds the divergence corrected with all but the other sides' parts)
+  R* Bve = nullptr;
+  R* Jne = nullptr;  // mixed path: the flux jump less the other side's part (divFe is then uncorrected)
   R* Rst = nullptr;  // mixed path: residual of each classical RK stage but the last
   // mixed path: U at the solution points rounded to FP32, the only form in
   // which the flux kernels read it; the RK stages inside a step keep their
@@ -392,7 +390,7 @@ struct Work {
   void* geo_mem = nullptr;
   bool ready = false;
   void release() {
-    void* ps[] = {divFe, Ufe, Fne, disFne, dUce, Bve, gBnd, Rst, Us, geo_mem, Ufe2};
+    void* ps[] = {divFe, Ufe, Bve, Jne, Rst, Us, geo_mem, Ufe2};
     for (void* p : ps)
       if (p) (void)hipFree(p);
     *this = Work<R>();
@@ -408,8 +406,8 @@ struct FusedState {
   int *pL = nullptr, *pR = nullptr, *bc = nullptr;
   // per element flux point, 4 * (partner flux point e*F + f) + side (0 left,
   // 1 right) or 4 * boundary slot + 2; the face's normal (the left element's)
-  // at every element flux point; boundary face points and their codes by slot
-  int *fpart = nullptr, *bndT = nullptr, *bndBc = nullptr;
+  // at every element flux point; boundary codes by slot
+  int *fpart = nullptr, *bndBc = nullptr;
   double* nfe = nullptr;
   int nBnd = 0;
   // batching: boundary-state table, element -> mesh map, per-mesh dt and activity
@@ -440,7 +438,7 @@ struct FusedState {
     w64.release();
     w32.release();
     void* ps[] = {tab_mem, Ue,           Uacc,    divF0e,    JGe,    detJe,  iJe,   norme, dAe, waveSpe, pL,
-                  pR,      bc,  fpart,   bndT,    nfe,       bst,    meshDt, meshRes, eleMesh, meshStart, active, srce,
+                  pR,      bc,  fpart,   nfe,       bst,    meshDt, meshRes, eleMesh, meshStart, active, srce,
                   dtTicket, vole, bndBc};
     for (void* p : ps)
       if (p) (void)hipFree(p);
@@ -449,9 +447,9 @@ struct FusedState {
   Work<R>& work();
 };
 template <>
-Work<double>& FusedState::work<double>() { return w64; }
+inline Work<double>& FusedState::work<double>() { return w64; }
 template <>
-Work<float>& FusedState::work<float>() { return w32; }
+inline Work<float>& FusedState::work<float>() { return w32; }
 
 // ---------------------------------------------------------------------------
 // Layout conversions between FlurryPP's [pt][ele][k] and element-major
@@ -459,7 +457,7 @@ Work<float>& FusedState::work<float>() { return w32; }
 // [P][E*K] <-> [E*K][P].  32x32 tiles through LDS so that reads and writes
 // are both coalesced; tiles are numbered on a 1-D grid.
 constexpr int kTile = 32;
-__global__ __launch_bounds__(256) void k_transpose(long long R, long long C, const double* __restrict__ in,
+static __global__ __launch_bounds__(256) void k_transpose(long long R, long long C, const double* __restrict__ in,
                                                    double* __restrict__ out) {
   __shared__ double t[kTile][kTile + 1];
   const long long tilesC = (C + kTile - 1) / kTile;
@@ -541,7 +539,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_extrap(int E, const double* __res
 // (nontemporal); on smaller ones they stay plain, since there the next kernel
 // of the stage finds them in L2 or the infinity cache (measured both ways).
 // A kernel streams only where the rows it stores are whole 64-byte blocks
-// (Runner::kFaceRowsWhole, kEleRowsWhole).
+// (Runner::kEleRowsWhole).
 template <bool NT, class T>
 __device__ __forceinline__ T ld_s(const T* p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
@@ -551,13 +549,6 @@ template <bool NT, class T>
 __device__ __forceinline__ void st_s(T v, T* p) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
   else *p = v;
-}
-// U at a face flux point, read once per face kernel launch: streamed in FP64
-// only; FP32 loads stay cached, since a 128-byte line then spans more face
-// points that other waves read (measured slower when streamed).
-template <bool NT, class R>
-__device__ __forceinline__ R ld_face(const R* p) {
-  return ld_s<NT && sizeof(R) == 8>(p);
 }
 // A product rounded on its own (never contracted into a following add).
 __device__ __forceinline__ double mul_rn(double a, double b) { return __dmul_rn(a, b); }
@@ -584,55 +575,49 @@ __device__ __forceinline__ void bc_state(int code, const R* UL, const R* n, R* U
   }
 }
 
-template <int D, int P, class R, bool NT>
+// The common inviscid flux fn of a point pair (left and right state, the left
+// element's normal); true where the flux has a wave speed lam (Roe has none).
+template <int D, class R>
+__device__ __forceinline__ bool pair_flux(bool bnd, const R* UL, const R* UR, const R* n, R* fn, const Phys& ph,
+                                          double& lam) {
+  if constexpr (D == 2) {
+    if (ph.riemann_type != 0 && !bnd) {
+      roe2d<R>(UL, UR, n, fn, R(ph.gamma));
+      return false;
+    }
+  }
+  lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
+  return true;
+}
+
+// The wave speeds of the common inviscid flux, one thread per point pair, for
+// the inviscid runs that need them ahead of their stage kernel (face_first).
+template <int D, int P, class R>
 __global__ __launch_bounds__(kMaxBlock) void k_face_inv(int nFF, const int* __restrict__ pLa, const int* __restrict__ pRa,
                                                    const int* __restrict__ bca, const R* __restrict__ Ufe,
-                                                   const R* __restrict__ norme,
-                                                   R* __restrict__ Fne, double* __restrict__ waveSpe,
-                                                   R* __restrict__ dUce, Phys ph,
+                                                   const R* __restrict__ norme, double* __restrict__ waveSpe, Phys ph,
                                                    const double* __restrict__ bst) {
   using Sh = Shape<D, P>;
   constexpr int F = Sh::F, N = Sh::N;
   int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nFF) return;
-  const int pl = ld_s<NT>(&pLa[t]), pr = ld_s<NT>(&pRa[t]),
-            bc = ld_s<NT>(&bca[t]);
+  const int pl = pLa[t], pr = pRa[t], bc = bca[t];
   const long long eL = pl / F, fL = pl - eL * F;
   const long long bL = eL * N * F + fL;
   R UL[N], UR[N], n[D], fn[N];
 #pragma unroll
-  for (int k = 0; k < N; k++) UL[k] = ld_face<NT>(&Ufe[bL + k * F]);
+  for (int k = 0; k < N; k++) UL[k] = Ufe[bL + k * F];
 #pragma unroll
-  for (int d = 0; d < D; d++) n[d] = ld_s<NT>(&norme[(eL * D + d) * F + fL]);
-  long long bR = 0;
+  for (int d = 0; d < D; d++) n[d] = norme[(eL * D + d) * F + fL];
   if (pr < 0) {
     bc_state<D, R>(bc, UL, n, UR, ph, bst);
   } else {
-    const long long eR = pr / F, fR = pr - eR * F;
-    bR = eR * N * F + fR;
+    const long long eR = pr / F, fR = pr - eR * F, bR = eR * N * F + fR;
 #pragma unroll
-    for (int k = 0; k < N; k++) UR[k] = ld_face<NT>(&Ufe[bR + k * F]);
+    for (int k = 0; k < N; k++) UR[k] = Ufe[bR + k * F];
   }
-  if (pr < 0 || ph.riemann_type == 0)
-    st_s<NT>(double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma))), &waveSpe[pl]);
-  else {
-    if constexpr (D == 2) roe2d<R>(UL, UR, n, fn, R(ph.gamma));
-  }
-  // the common inviscid flux once per point pair, at its left point; the
-  // kernel that applies the correction scales it by each side's dA (negated
-  // on the right), and viscous runs add the LDG flux there, where both
-  // sides' parts meet
-#pragma unroll
-  for (int k = 0; k < N; k++) st_s<NT>(fn[k], &Fne[bL + k * F]);
-  if (ph.viscous) {
-    R pf = (pr < 0) ? R(0) : ldg_pen<D, R>(n, R(ph.pen_fact));
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      R uc = (pr < 0) ? R(0.5) * (UL[k] + UR[k]) : R(0.5) * (UL[k] + UR[k]) - pf * (UL[k] - UR[k]);
-      st_s<NT>(uc - UL[k], &dUce[bL + k * F]);
-      if (pr >= 0) st_s<NT>(uc - UR[k], &dUce[bR + k * F]);
-    }
-  }
+  double lam;
+  if (pair_flux<D, R>(pr < 0, UL, UR, n, fn, ph, lam)) waveSpe[pl] = lam;
 }
 
 // ---------------------------------------------------------------------------
@@ -728,6 +713,17 @@ __device__ __forceinline__ RkIn<D, R> rk_load(int E, long long e, int s, const R
   return in;
 }
 
+// correctDivFlux of field k at a point of the block's element b, from the flux
+// jump in sD.
+template <int D, int P, class R, class Op>
+__device__ __forceinline__ R correction(const R* sD, int b, int k, const Op& po) {
+  using Sh = Shape<D, P>;
+  R c = 0;
+#pragma unroll
+  for (int j = 0; j < Sh::NC; j++) c += po.cor_w(j) * sD[(b * Sh::N + k) * Sh::F + po.cor_idx(j)];
+  return c;
+}
+
 // correctDivFlux and timeStepA/B at point s of the block's element b: dv holds
 // its divF (one value per field), sD the flux jump at the block's flux points,
 // and sU receives the new state (its previous contents are no longer read).
@@ -736,17 +732,12 @@ template <int D, int P, class R, bool NT, bool TEN>
 __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const R* dv, R* sU, const R* sD, const R* sW,
                                          const RkIn<D, R>& in, const RkArgs<R>& ra, const Tabs& tb) {
   using Sh = Shape<D, P>;
-  constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1, NC = Sh::NC;
+  constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
   const int mode = ra.mode;
   const PtOp<D, P, R, TEN> po(tb, sW, s);
   R res[N];
 #pragma unroll
-  for (int k = 0; k < N; k++) {
-    R c = 0;
-#pragma unroll
-    for (int j = 0; j < NC; j++) c += po.cor_w(j) * sD[(b * N + k) * F + po.cor_idx(j)];
-    res[k] = c + dv[k];
-  }
+  for (int k = 0; k < N; k++) res[k] = correction<D, P, R>(sD, b, k, po) + dv[k];
   const long long at = e * N * S + s;
   if (mode == 5 || mode == 7 || mode == 8) {
     // residual only (calcResidual(0) + correctDivFlux), no update: 5 into
@@ -823,31 +814,23 @@ __device__ __forceinline__ void face_point(int i, int e0, const R* sU, const R* 
   }
 }
 
-// Viscous runs, FP32: the volume kernel also folds its own side's LDG part
-// into the flux jump (disFne := +-B dA - disFn), so the RK kernel reads one
-// array less.  FP64 keeps disFn and B apart: its volume kernel is short of
-// registers, and reading B back at the end of the element costs it more than
-// the RK kernel saves (measured).
-template <class R>
-constexpr bool kJumpInVolume = sizeof(R) == 4;
-
 // Shapes whose volume kernel is held to 4 waves per SIMD (128 VGPRs): quads
 // and the FP32 path.  FP64 hexes need more registers and are held to 3.
 template <int D, class R>
 constexpr bool kHold = D == 2 || sizeof(R) == 4;
 
-// The volume kernel's flux-point inputs and outputs besides the slabs: the
-// side codes and dA (every run), and for viscous runs what it leaves at the
-// flux points in place of the gradient there (see the face loop of
-// volume_body).
+// The volume kernel's flux-point inputs and outputs.
 template <class R>
 struct VFace {
   const int* fpart;    // [E*F] 4 * partner flux point + side, or 4 * boundary slot + 2
+  const R* Ufe;        // [E][N][F] U at the flux points
   const R* nfe;        // [E][D][F] the face's normal (its left element's)
-  R* Bve;              // [E][N][F] this side's part of the LDG flux . n
-  R* gBnd;             // [D*N][nBnd] gradient at the boundary flux points
   const R* dA;         // [E][F] face area factor
-  int nBnd;
+  R* Bve;              // [E][N][F] this side's part of the LDG flux . n (interior points)
+  R* Jne;              // [E][N][F] kJumpOut: the flux jump, less the other side's part
+  double* wave;        // wave speeds of the left and boundary points, or null: not read before they change again
+  const int* bndBc;    // [nBnd] boundary code (number and state row) by slot
+  const double* bst;   // boundary-state table
 };
 
 // calcDivF_spts of field k at point s of the block's element b, from the
@@ -1016,14 +999,9 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
       UL[k] = right ? oth[k] : own[k];
       UR[k] = right ? own[k] : oth[k];
     }
-    bool roe = false;
-    if constexpr (D == 2) roe = ph.riemann_type != 0 && (!BND || side != 2);
-    if (!roe) {
-      const double lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
-      if (fc.wave && !right) st_s<NT>(lam, &fc.wave[(long long)e0 * F + fi(u)]);
-    } else if constexpr (D == 2) {
-      roe2d<R>(UL, UR, n, fn, R(ph.gamma));
-    }
+    double lam;
+    if (pair_flux<D, R>(BND && side == 2, UL, UR, n, fn, ph, lam) && fc.wave && !right)
+      st_s<NT>(lam, &fc.wave[(long long)e0 * F + fi(u)]);
 #pragma unroll
     for (int k = 0; k < N; k++) {
       const R v = mul_rn(fn[k], dA);
@@ -1123,31 +1101,65 @@ __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) 
 }
 
 // ---------------------------------------------------------------------------
-// Volume kernel of viscous runs: corrected gradient, flux, divergence, normal
-// flux and each side's part of the LDG flux at the faces.  One thread per
-// solution point, EB elements per block, element data staged in LDS.
-template <int D, int P, class R, bool NT, bool TEN, int BF = 0>
+// The same value, as far as the compiler can tell another one: what is computed
+// from it is not kept in registers from an earlier phase.
+__device__ __forceinline__ int fresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// A value that is complete here: what is computed from it is not moved up among
+// the sums that form it, which costs the registers of both.
+template <class T>
+__device__ __forceinline__ void pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// Where the correction with this side's part of the flux jump is applied.  FP64:
+// here, so that the jump stays on chip.  FP32: by the RK kernel, together with
+// the other side's part; split in two, the correction's roundings would differ
+// by some 1e-8 of the state after a step, for 6% of the stage's traffic.
+template <class R>
+constexpr bool kJumpOut = sizeof(R) == 4;
+
+// Whether the flux jump takes U's place in LDS (which has to be that large), not
+// the transformed flux's, which would cost a barrier; P0 blocks, of many
+// elements, would not fit the LDS limit.
+template <int D, int P>
+constexpr bool jump_over_u = P > 0;
+
+// Volume kernel of viscous runs: all of a stage's residual but the other sides'
+// parts of the LDG flux.  Solution points and then flux points in the same
+// threads, EB elements per block, element data staged in LDS.
+//
+// What a stage costs is its traffic, and most of that was intermediates: the
+// common inviscid flux and the common U, written by a face kernel and read here
+// and by the RK kernel, and the flux jump, written here and read there.  Both
+// sides of a pair now form the common flux from U there and across (one read of
+// U at the flux points; the own side is extrapolated again from the slab), and
+// FP64 corrects the divergence with this side's part of the jump before it is
+// written: 7.3 -> 4.6 GB per stage at 48^3 P3.  Sums that form a value are pinned before what uses them: otherwise
+// both are live at once and the FP64 P3 kernel spills 136 registers.
+// Measured, three kernels -> two: Navier-Stokes Taylor-Green 4 steps, 48^3 P3
+// 20.07 -> 16.8 ms; 37^3 P2 6.89 -> 4.30 ms; 40^3 P3 mixed 7.93 -> 6.86 ms; 21^3
+// P4 with monitor 1.43 -> 1.22 ms.
+template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
 __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue, const R* __restrict__ Us,
-                                            const R* __restrict__ dUce,
                                             const R* __restrict__ JGe, const R* __restrict__ iJe,
-                                            R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf,
-                                            Tabs tb, Phys ph) {
+                                            R* __restrict__ divFe, const VFace<R>& vf, const Tabs& tb, const Phys& ph) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
   const int EB = blockDim.x / S;
-  // sF holds, in turn: dUc at the flux points, the physical gradient until it
-  // has been extrapolated to the faces, then the transformed flux at the same
-  // indices as the gradient.  [EB*N*S] + [EB*N*SF]; the faces' normals for the
-  // face loop, [EB*D*F], and the points' side codes [EB*F] ints
-  constexpr int SF = F > D * S ? F : D * S;
+  // sU holds U until the flux has been formed, then the flux jump; sF holds, in
+  // turn: dUc at the flux points, the physical gradient until it has been
+  // extrapolated to the faces, then the transformed flux at the same indices as
+  // the gradient.  [EB*N*SU] + [EB*N*max(F,D*S)]
+  constexpr int SU = !kJumpOut<R> && jump_over_u<D, P> && F > S ? F : S;
   R* const sU = reinterpret_cast<R*>(fhip_lds);
-  R* const sF = sU + EB * N * S;
+  R* const sF = sU + EB * N * SU;
+  R* const sD = jump_over_u<D, P> ? sU : sF;
   R* const sG = sF;
-  R* const sN = sF + EB * N * SF;
-  int* const sP = reinterpret_cast<int*>(sN + EB * D * F);
-  // with kJumpInVolume: this side's LDG part at the block's
-  // flux points, kept from the first face loop for the last one [EB*N*F]
-  R* const sB = reinterpret_cast<R*>(sP + EB * F);
+  R* const sC = sF;
   __shared__ R sW[Ten<D, P>::NW];
   stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
@@ -1155,6 +1167,10 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   const int sw = spt_lds(D, P1, s);
   const bool act = b < nb;
   const long long e = e0 + b;
+  // the thread's flux points: fi(u) < nP
+  constexpr int KF = (F + S - 1) / S;
+  const int nP = nb * F;
+  auto fi = [&](int u) { return (int)threadIdx.x + u * (int)blockDim.x; };
   // matrix-core contractions: this lane's operator entry d1[s % 4][s / 16]
   // and the slab position of the point whose x and z are this lane's z and x
   constexpr bool mf = kMfma<D, P, R>;
@@ -1165,8 +1181,35 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   if constexpr (np != 0) abf = bf16_opnd_a(tw<float>(tb.d1, tb.d1f), s, np);
   const int swx = mf ? spt_lds(D, P1, s / 16 + 4 * ((s / 4) % 4) + 16 * (s % 4)) : 0;
   const R opv = mf ? tw<R>(tb.d1, tb.d1f)[(s % 4) * P1 + s / 16] : R(0);
-  // the point's metric terms, loaded first so that their latency overlaps the
-  // staging of the slab and the gradient
+  // every load is issued before the first LDS store, so that their latencies
+  // overlap; the flux points' side codes first: the partners' addresses come
+  // from them
+  int cd[KF];
+#pragma unroll
+  for (int u = 0; u < KF; u++) cd[u] = fi(u) < nP ? vf.fpart[(long long)e0 * F + fi(u)] : 0;
+  const int nU = nb * N * S;
+  R vu[N];
+#pragma unroll
+  for (int u = 0; u < N; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nU) vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
+  }
+  // U across and the normal
+  R fn[KF][N], nv[KF][D];
+#pragma unroll
+  for (int u = 0; u < KF; u++)
+    if (fi(u) < nP) {
+      const int i = fi(u), bb = i / F, f = i - bb * F;
+#pragma unroll
+      for (int x = 0; x < D; x++) nv[u][x] = ld_s<NT>(&vf.nfe[((long long)(e0 + bb) * D + x) * F + f]);
+      if (!BND || (cd[u] & 3) != 2) {
+        const int p = cd[u] >> 2, ep = p / F;
+        const long long pb = (long long)ep * N * F + (p - ep * F);
+#pragma unroll
+        for (int k = 0; k < N; k++) fn[u][k] = vf.Ufe[pb + k * F];
+      }
+    }
+  // the point's metric terms
   R G[D][D] = {};
   auto load_G = [&] {
 #pragma unroll
@@ -1179,67 +1222,63 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     load_G();
     inv = iJe[e * S + s];
   }
-  {
-    // every load of the slabs is issued before the first LDS store, so that
-    // their latencies overlap: a thread stages at most N values of U (the
-    // block holds at most blockDim / S elements) and KC of dUc
-    constexpr int KC = (N * F + S - 1) / S, KN = (D * F + S - 1) / S, KP = (F + S - 1) / S;
-    const int nU = nb * N * S, nC = nb * N * F, nN = nb * D * F, nP = nb * F;
-    R vu[N], vc[KC], vn[KN];
-    int vp[KP];
 #pragma unroll
-    for (int u = 0; u < N; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nU) vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
-    }
-    // dUc at the block's flux points (sF serves as sC until the gradient is written)
-#pragma unroll
-    for (int u = 0; u < KC; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nC) vc[u] = ld_s<NT>(&dUce[(long long)e0 * N * F + i]);
-    }
-#pragma unroll
-    for (int u = 0; u < KN; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nN) vn[u] = ld_s<NT>(&vf.nfe[(long long)e0 * D * F + i]);
-    }
-#pragma unroll
-    for (int u = 0; u < KP; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nP) vp[u] = vf.fpart[(long long)e0 * F + i];
-    }
-#pragma unroll
-    for (int u = 0; u < N; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nU) {
-        const int r = i / S, q = i - r * S;
-        sU[r * S + spt_lds(D, P1, q)] = vu[u];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < KC; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nC) sF[i] = vc[u];
-    }
-#pragma unroll
-    for (int u = 0; u < KN; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nN) sN[i] = vn[u];
-    }
-#pragma unroll
-    for (int u = 0; u < KP; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i < nP) sP[i] = vp[u];
+  for (int u = 0; u < N; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nU) {
+      const int r = i / S, q = i - r * S;
+      sU[r * S + spt_lds(D, P1, q)] = vu[u];
     }
   }
+  __syncthreads();
+  // U at flux point f of the block's element bb (the RK kernel's sums and bits)
+  auto u_face = [&](int bb, const FpOp<D, P, R, TEN>& fp, R* own) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      R a = 0;
+#pragma unroll
+      for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
+      own[k] = a;
+      pin(own[k]);
+    }
+  };
+  // the common inviscid flux (FP64: with the LDG penalty on the states, which
+  // FP32 leaves in the two sides' parts), and the common U less U, from U on both sides (in the left side's order on either)
+#pragma unroll
+  for (int u = 0; u < KF; u++)
+    if (fi(u) < nP) {
+      const int i = fresh(fi(u)), bb = i / F, f = i - bb * F, side = cd[u] & 3;
+      const FpOp<D, P, R, TEN> fp(tb, sW, f);
+      const bool right = side == 1, bnd = BND && side == 2;
+      R own[N], UL[N], UR[N];
+      u_face(bb, fp, own);
+      if constexpr (BND) {
+        if (bnd) bc_state<D, R>(vf.bndBc[cd[u] >> 2], own, nv[u], fn[u], ph, vf.bst);
+      }
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        UL[k] = right ? fn[u][k] : own[k];
+        UR[k] = right ? own[k] : fn[u][k];
+      }
+      double lam;
+      if (pair_flux<D, R>(bnd, UL, UR, nv[u], fn[u], ph, lam) && vf.wave && !right)
+        st_s<NT>(lam, &vf.wave[(long long)e0 * F + i]);
+      const R pf = bnd ? R(0) : ldg_pen<D, R>(nv[u], R(ph.pen_fact));
+      const R tn = bnd || kJumpOut<R> ? R(0) : ldg_tau<D, R>(nv[u], R(ph.tau));
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const R uc = bnd ? R(0.5) * (UL[k] + UR[k]) : R(0.5) * (UL[k] + UR[k]) - pf * (UL[k] - UR[k]);
+        sC[(bb * N + k) * F + f] = uc - own[k];
+        if constexpr (!kJumpOut<R>) fn[u][k] += tn * (UL[k] - UR[k]);
+      }
+    }
   __syncthreads();
   // phase 1: reference-space gradient (opp_grad_spts) plus correction
   // (opp_correctU), then the physical gradient (correctGradU transform,
   // src/solver.cpp:1105-1136), kept in LDS for phase 2 and the faces
-  R* const sC = sF;
   R gr[D][N];
-  const PtOp<D, P, R, TEN> po(tb, sW, s);
   if (act) {
+    const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
 #pragma unroll
     for (int d = 0; d < D; d++) {
 #pragma unroll
@@ -1286,55 +1325,61 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       for (int x = 0; x < D; x++) sG[((b * D + x) * N + k) * S + sw] = gr[x][k];
   }
   __syncthreads();
-  // physical gradient at the flux points (extrapolateGradU) and, with U
-  // there (extrapolateU, the same sums as the RK kernel's), this side's
-  // viscous flux folded into its part of the LDG flux
-  // (face::calcViscousFlux, src/face.cpp:216-293); the two sides' parts are
-  // summed where the correction is applied.  Boundary points keep the
-  // gradient for the boundary kernel, which needs the boundary state.
-  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
-    const int bb = i / F, f = i - bb * F;
-    const long long ee = e0 + bb;
-    const FpOp<D, P, R, TEN> fp(tb, sW, f);
-    // side code and normal, staged in LDS with the slab
-    const int code = sP[bb * F + f], side = code & 3;
-    R nv[D];
+  // physical gradient at the flux points (extrapolateGradU) and, with U there,
+  // this side's viscous flux folded into its part of the LDG flux
+  // (face::calcViscousFlux, src/face.cpp:216-293).  fn becomes the common flux,
+  // as far as it is known on this side, times dA, outward: the other side's
+  // part is added by the RK kernel.  Boundary points take the boundary state's
+  // flux (boundFace::applyViscousBCs, src/boundFace.cpp:316-352).
+  R bo[kJumpOut<R> ? KF : 1][N], dA = 0;
 #pragma unroll
-    for (int x = 0; x < D; x++) nv[x] = sN[(bb * D + x) * F + f];
-    R g[D][N];
+  for (int u = 0; u < KF; u++)
+    if (fi(u) < nP) {
+      const int i = fresh(fi(u)), bb = i / F, f = i - bb * F, side = cd[u] & 3;
+      const FpOp<D, P, R, TEN> fp(tb, sW, f);
+      dA = ld_s<NT>(&vf.dA[(long long)e0 * F + i]);
+      R g[D][N];
 #pragma unroll
-    for (int x = 0; x < D; x++)
+      for (int x = 0; x < D; x++) {
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        R a = 0;
+        for (int k = 0; k < N; k++) {
+          R a = 0;
 #pragma unroll
-        for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sG[((bb * D + x) * N + k) * S + fp.idx(m)];
-        g[x][k] = a;
+          for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sG[((bb * D + x) * N + k) * S + fp.idx(m)];
+          g[x][k] = a;
+          pin(g[x][k]);
+        }
       }
-    if (side == 2) {
-      const long long slot = code >> 2;
+      R own[N], bv[N];
+      u_face(bb, fp, own);
+      if (BND && side == 2) {
+        R UR[N], nF[N], d12[N];
+        const int bc = vf.bndBc[cd[u] >> 2];
+        bc_state<D, R>(bc, own, nv[u], UR, ph, vf.bst);
+        const bool adiabatic = (bc & 15) == 10;
+        if (adiabatic) adiabatic_grad<D, R>(own, UR, g, R(ph.gamma));
+        ldg_side<D, R>(adiabatic ? UR : own, g, nv[u], nF, d12, ph);
 #pragma unroll
-      for (int x = 0; x < D; x++)
+        for (int k = 0; k < N; k++) bv[k] = 0;
+        ldg_boundary<D, R>(own, UR, nF, nv[u], bv, ph);
+      } else {
+        if constexpr (kJumpOut<R>) {
 #pragma unroll
-        for (int k = 0; k < N; k++) vf.gBnd[(x * N + k) * (long long)vf.nBnd + slot] = g[x][k];
-    } else {
-      R u[N], bv[N];
+          for (int k = 0; k < N; k++) bv[k] = 0;
+          ldg_add_side<D, R>(side == 0, own, g, nv[u], bv, ph);
+        } else {
+          ldg_part<D, R>(side == 0, own, g, nv[u], bv, ph);
+        }
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
-        u[k] = a;
-        bv[k] = 0;
+        for (int k = 0; k < N; k++) st_s<NT>(bv[k], &vf.Bve[((long long)(e0 + bb) * N + k) * F + f]);
       }
-      ldg_add_side<D, R>(side == 0, u, g, nv, bv, ph);
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        st_s<NT>(bv[k], &vf.Bve[(ee * N + k) * F + f]);
-        if constexpr (kJumpInVolume<R>) sB[(bb * N + k) * F + f] = bv[k];
+        const R v = kJumpOut<R> ? mul_rn(fn[u][k], dA) : (fn[u][k] + bv[k]) * dA;
+        fn[u][k] = side == 1 ? -v : v;
+        if constexpr (kJumpOut<R>) bo[u][k] = side == 1 ? -bv[k] : bv[k];
       }
     }
-  }
   // under the register hold, the metric terms again (from cache): keeping
   // them live across the face loop above costs more registers than it allows
   if constexpr (kHold<D, R>) {
@@ -1380,41 +1425,56 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       for (int k = 0; k < N; k++) sF[((b * D + d1) * N + k) * S + sw] = Ft[d1][k];
   }
   __syncthreads();
+  R dv[N];
   if (act) {
-#pragma unroll
-    for (int k = 0; k < N; k++)
-      st_s<NT>(divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po), &divFe[(e * N + k) * S + s]);
-  }
-  // faces: discontinuous normal flux.  With kJumpInVolume it stores in its
-  // place this side's part of the correction's flux jump, +-B dA - disFn (B
-  // as written by this thread in the face loop above, - on the right side;
-  // boundary points get - disFn here and + B dA from the boundary kernel).
-  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
-    const int bb = i / F, f = i - bb * F;
-    const long long ee = e0 + bb;
-    const FpOp<D, P, R, TEN> fp(tb, sW, f);
-    // extrapolateNormalFlux: of the sum over directions only the face's own
-    // normal direction is non-zero (the other terms are exact zeros)
-    const int dn = fp.dir();
-    int side = 2;
-    R dA = 0, bv[N];
-    if constexpr (kJumpInVolume<R>) {
-      side = sP[bb * F + f] & 3;
-      dA = vf.dA[ee * F + f];
-      // this thread's own LDG parts from the first face loop (the same
-      // points); read for every point, unused at boundary points
-#pragma unroll
-      for (int k = 0; k < N; k++) bv[k] = sB[(bb * N + k) * F + f];
-    }
+    const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      R a = 0;
-#pragma unroll
-      for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
-      a = fp.efn_sign(a);
-      if constexpr (kJumpInVolume<R>) a = (side == 2) ? -a : (side == 0 ? bv[k] : -bv[k]) * dA - a;
-      st_s<NT>(a, &disFne[(ee * N + k) * F + f]);
+      dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po);
+      if constexpr (kJumpOut<R>) st_s<NT>(dv[k], &divFe[(e * N + k) * S + s]);
     }
+  }
+  // faces: the flux jump, less the other side's part (extrapolateNormalFlux: of
+  // the sum over directions only the face's own normal direction is non-zero)
+#pragma unroll
+  for (int u = 0; u < KF; u++)
+    if (fi(u) < nP) {
+      const int i = fresh(fi(u)), bb = i / F, f = i - bb * F;
+      const FpOp<D, P, R, TEN> fp(tb, sW, f);
+      const int dn = fp.dir();
+      const R dJ = kJumpOut<R> ? (KF == 1 ? dA : vf.dA[(long long)e0 * F + i]) : R(0);
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        R a = 0;
+#pragma unroll
+        for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
+        a = fp.efn_sign(a);
+        if constexpr (kJumpOut<R>) {
+          const R j = bo[u][k] * dJ - a;
+          st_s<NT>(fn[u][k] + j, &vf.Jne[((long long)(e0 + bb) * N + k) * F + f]);
+          continue;
+        }
+        fn[u][k] -= a;
+        if constexpr (jump_over_u<D, P>) sD[(bb * N + k) * F + f] = fn[u][k];
+      }
+    }
+  if constexpr (kJumpOut<R>) return;
+  if constexpr (!jump_over_u<D, P>) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < KF; u++)
+      if (fi(u) < nP) {
+        const int i = fresh(fi(u)), bb = i / F, f = i - bb * F;
+#pragma unroll
+        for (int k = 0; k < N; k++) sD[(bb * N + k) * F + f] = fn[u][k];
+      }
+  }
+  __syncthreads();
+  if (act) {
+    const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
+#pragma unroll
+    for (int k = 0; k < N; k++)
+      st_s<NT>(correction<D, P, R>(sD, b, k, po) + dv[k], &divFe[(e * N + k) * S + s]);
   }
 }
 
@@ -1422,83 +1482,32 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
 // and the FP32 path, which fit there without spilling (holding the FP32
 // viscous hex kernel to 5 or 6 waves spills 26 or 41 VGPRs and was measured
 // 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes.
-template <int D, int P, class R, bool NT, bool TEN>
+template <int D, int P, class R, bool NT, bool BND, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_volume_w3(
-    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
-    const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
-    Phys ph) {
-  volume_body<D, P, R, NT, TEN>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
+    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, const R* __restrict__ iJe,
+    R* __restrict__ divFe, VFace<R> vf, Tabs tb, Phys ph) {
+  volume_body<D, P, R, NT, BND, TEN>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
 }
-template <int D, int P, class R, bool NT, bool TEN, int BF = 0>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_volume_w4(
-    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ dUce, const R* __restrict__ JGe,
-    const R* __restrict__ iJe, R* __restrict__ divFe, R* __restrict__ disFne, VFace<R> vf, Tabs tb,
-    Phys ph) {
-  volume_body<D, P, R, NT, TEN, BF>(E, Ue, Us, dUce, JGe, iJe, divFe, disFne, vf, tb, ph);
+    int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, const R* __restrict__ iJe,
+    R* __restrict__ divFe, VFace<R> vf, Tabs tb, Phys ph) {
+  volume_body<D, P, R, NT, BND, TEN, BF>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
 }
 
-// ---------------------------------------------------------------------------
-// LDG flux at the boundary flux points (face::calcViscousFlux with the
-// boundary state of boundFace::applyViscousBCs, src/face.cpp:216-293,
-// src/boundFace.cpp:316-352): one thread per boundary point, from the
-// gradient the volume kernel left there.  The result goes where the volume
-// kernel puts an interior point's side of the flux, or (kJumpInVolume) times
-// dA into the point's flux jump, which the volume kernel set to -disFn.
-template <int D, int P, class R>
-__global__ __launch_bounds__(kMaxBlock) void k_face_bnd(int nB, const int* __restrict__ bndT,
-                                                   const int* __restrict__ pLa, const int* __restrict__ bca,
-                                                   const R* __restrict__ Ufe, const R* __restrict__ gBnd,
-                                                   const R* __restrict__ norme, const R* __restrict__ dAe,
-                                                   R* __restrict__ Bve, R* __restrict__ Cne, Phys ph,
-                                                   const double* __restrict__ bst) {
-  using Sh = Shape<D, P>;
-  constexpr int F = Sh::F, N = Sh::N;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nB) return;
-  const int t = bndT[i], pl = pLa[t], bc = bca[t];
-  const long long eL = pl / F, fL = pl - eL * F;
-  const long long bL = eL * N * F + fL;
-  R UL[N], UR[N], n[D], g[D][N], nF[N], d12[N], bv[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) UL[k] = Ufe[bL + k * F];
-#pragma unroll
-  for (int d = 0; d < D; d++) n[d] = norme[(eL * D + d) * F + fL];
-#pragma unroll
-  for (int d = 0; d < D; d++)
-#pragma unroll
-    for (int k = 0; k < N; k++) g[d][k] = gBnd[(d * N + k) * (long long)nB + i];
-  bc_state<D, R>(bc, UL, n, UR, ph, bst);
-  const bool adiabatic = (bc & 15) == 10;
-  if (adiabatic) adiabatic_grad<D, R>(UL, UR, g, R(ph.gamma));
-  ldg_side<D, R>(adiabatic ? UR : UL, g, n, nF, d12, ph);
-#pragma unroll
-  for (int k = 0; k < N; k++) bv[k] = 0;
-  ldg_boundary<D, R>(UL, UR, nF, n, bv, ph);
-  if constexpr (kJumpInVolume<R>) {
-    const R dA = dAe[pl];
-#pragma unroll
-    for (int k = 0; k < N; k++) Cne[bL + k * F] = bv[k] * dA + Cne[bL + k * F];
-  } else {
-#pragma unroll
-    for (int k = 0; k < N; k++) Bve[bL + k * F] = bv[k];
-  }
-}
-
-// Correction of the divergence, RK update and U at the flux points, after the
-// viscous volume kernel.  With NT, the arrays this kernel reads or writes
-// exactly once per launch go through nontemporal loads and stores (they
-// stream past the caches); arrays read twice (the LDG side parts and the
-// inviscid common flux, read by both sides of a face) stay cached.
+// After the viscous volume kernel: correction of the divergence with the other
+// sides' LDG parts (FP32: with the whole flux jump), RK update and U at the flux points.  With NT, the arrays
+// this kernel reads or writes exactly once per launch go through nontemporal
+// loads and stores (they stream past the caches).
 template <int D, int P, class R, bool NT, bool TEN>
-__global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ divFe, const R* __restrict__ Fne,
-                                             const R* __restrict__ disFne, RkArgs<R> ra, Tabs tb,
+__global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ divFe, RkArgs<R> ra, Tabs tb,
                                              const int* __restrict__ fpart, const R* __restrict__ dAe,
-                                             const R* __restrict__ Bve) {
+                                             const R* __restrict__ Bve, const R* __restrict__ Jne) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N;
   const int EB = blockDim.x / S;
   R* const sU = reinterpret_cast<R*>(fhip_lds);  // [EB*N*S]
-  R* const sD = sU + EB * N * S;                  // [EB*N*F] Fn - disFn at the block's flux points
+  R* const sD = sU + EB * N * S;                  // [EB*N*F] the flux jump (FP64: the other side's part of it)
   __shared__ R sW[Ten<D, P>::NW];
   stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
@@ -1508,69 +1517,30 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   // the points a thread stages, issued before their LDS stores, so that their
   // latencies overlap.  A thread stages at most KF = ceil(F / S) points.
   constexpr int KF = (F + S - 1) / S;
-  if constexpr (kJumpInVolume<R>) {
-    // viscous: disFne holds this side's jump part +-B dA - disFn; add the
-    // inviscid part (Fne at the pair's left point, times dA) and the partner
-    // side's B times dA, negated on the right side
-    int cd[KF];
+  int cd[KF];
 #pragma unroll
-    for (int u = 0; u < KF; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      cd[u] = (i < nb * F) ? fpart[(long long)e0 * F + i] : 2;
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    cd[u] = (i < nb * F) ? fpart[(long long)e0 * F + i] : 2;
+  }
+#pragma unroll
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i >= nb * F) break;
+    const int bb = i / F, f = i - bb * F;
+    const int code = cd[u], side = code & 3;
+    const R dA = dAe[(long long)e0 * F + i];
+    const long long ob = (long long)(e0 + bb) * N * F + f;
+    long long pb = ob;
+    if (side != 2) {
+      const long long p = code >> 2, ep = p / F;
+      pb = ep * N * F + (p - ep * F);
     }
 #pragma unroll
-    for (int u = 0; u < KF; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i >= nb * F) break;
-      const int bb = i / F, f = i - bb * F;
-      const long long ef = (long long)(e0 + bb) * F + f, ob = (long long)(e0 + bb) * N * F + f;
-      const int code = cd[u], side = code & 3;
-      const R dA = dAe[ef];
-      long long pb = ob;
-      if (side != 2) {
-        const long long p = code >> 2, ep = p / F;
-        pb = ep * N * F + (p - ep * F);
-      }
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        const R bp = Bve[pb + k * F];
-        // the pair's inviscid flux (at its left point) times this side's dA
-        const R fo = mul_rn(Fne[(side == 1 ? pb : ob) + k * F], dA);
-        const R base = (side == 1 ? -fo : fo) + ld_s<NT>(&disFne[ob + k * F]);
-        sD[(bb * N + k) * F + f] = (side == 2) ? base : base + (side == 0 ? bp : -bp) * dA;
-      }
-    }
-  } else {
-    // viscous: common flux = inviscid part (Fne at the pair's left point)
-    // plus both sides' LDG parts, times dA, negated on the right side
-    int cd[KF];
-#pragma unroll
-    for (int u = 0; u < KF; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      cd[u] = (i < nb * F) ? fpart[(long long)e0 * F + i] : 2;
-    }
-#pragma unroll
-    for (int u = 0; u < KF; u++) {
-      const int i = threadIdx.x + u * blockDim.x;
-      if (i >= nb * F) break;
-      const int bb = i / F, f = i - bb * F;
-      const long long ef = (long long)(e0 + bb) * F + f, ob = (long long)(e0 + bb) * N * F + f;
-      const int code = cd[u], side = code & 3;
-      const R dA = dAe[ef];
-      long long pb = ob;
-      if (side != 2) {
-        const long long p = code >> 2, ep = p / F;
-        pb = ep * N * F + (p - ep * F);
-      }
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        const R bo = Bve[ob + k * F], bp = Bve[pb + k * F];
-        R bv = (side != 2) ? bo + bp : bo;
-        if (side == 1) bv = -bv;
-        // the pair's inviscid flux (at its left point) times this side's dA
-        const R fo = mul_rn(Fne[(side == 1 ? pb : ob) + k * F], dA);
-        sD[(bb * N + k) * F + f] = ((side == 1 ? -fo : fo) + bv * dA) - ld_s<NT>(&disFne[ob + k * F]);
-      }
+    for (int k = 0; k < N; k++) {
+      const R bp = ld_s<NT>(&Bve[pb + k * F]);
+      const R base = kJumpOut<R> ? ld_s<NT>(&Jne[ob + k * F]) : R(0);
+      sD[(bb * N + k) * F + f] = side == 2 ? base : base + (side == 0 ? bp : -bp) * dA;
     }
   }
   __syncthreads();
@@ -1598,7 +1568,7 @@ __global__ void k_copy_em(long long n, R* __restrict__ dst, const R* __restrict_
 // multiGrid::restrict_pmg (src/multigrid.cpp:315-345) and the start of
 // compute_source_term (:381-398): the coarse level's U = R U_fine, its FAS
 // source = R divF_fine (the residual of U is subtracted later) and sol = U.
-__global__ void k_restrict_em(long long rows, int Sc, int Sf, int kc, const double* __restrict__ R,
+static __global__ void k_restrict_em(long long rows, int Sc, int Sf, int kc, const double* __restrict__ R,
                               const double* __restrict__ Uf, const double* __restrict__ divFf,
                               double* __restrict__ Uc, double* __restrict__ srcc, double* __restrict__ solc) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1626,7 +1596,7 @@ __global__ void k_restrict_em(long long rows, int Sc, int Sf, int kc, const doub
 
 // prolong_err (src/multigrid.cpp:347-364): U_up += P (U - sol) of the level
 // below.
-__global__ void k_prolong_em(long long rows, int Su, int Sc, int kc, const double* __restrict__ Pm,
+static __global__ void k_prolong_em(long long rows, int Su, int Sc, int kc, const double* __restrict__ Pm,
                              const double* __restrict__ Uc, const double* __restrict__ solc, double* __restrict__ Uu) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= rows * Su) return;
@@ -1653,7 +1623,7 @@ __global__ void k_prolong_em(long long rows, int Su, int Sc, int kc, const doubl
 // wave read consecutive entries) and the block's rows staged in LDS: nr rows
 // per block, one output per thread, the sums in the same order as above.
 // Used where the operator and the rows fit in 64 KiB.
-__global__ void k_restrict_em_lds(long long rows, int Sc, int Sf, int kc, int nr, const double* __restrict__ R,
+static __global__ void k_restrict_em_lds(long long rows, int Sc, int Sf, int kc, int nr, const double* __restrict__ R,
                                   const double* __restrict__ Uf, const double* __restrict__ divFf,
                                   double* __restrict__ Uc, double* __restrict__ srcc, double* __restrict__ solc) {
   double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sf][Sc]
@@ -1692,7 +1662,7 @@ __global__ void k_restrict_em_lds(long long rows, int Sc, int Sf, int kc, int nr
   srcc[t] = cd;
 }
 
-__global__ void k_prolong_em_lds(long long rows, int Su, int Sc, int kc, int nr, const double* __restrict__ Pm,
+static __global__ void k_prolong_em_lds(long long rows, int Su, int Sc, int kc, int nr, const double* __restrict__ Pm,
                                  const double* __restrict__ Uc, const double* __restrict__ solc,
                                  double* __restrict__ Uu) {
   double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sc][Su]
@@ -1820,7 +1790,7 @@ __global__ __launch_bounds__(256) void k_ele_dt_em(int E, const double* __restri
 }
 
 // Per-mesh minimum of the element time steps (batched contexts, dt_type 1).
-__global__ void k_mesh_dt_min(const int* __restrict__ start, const double* __restrict__ eleDt,
+static __global__ void k_mesh_dt_min(const int* __restrict__ start, const double* __restrict__ eleDt,
                               double* __restrict__ meshDt) {
   __shared__ double red[256];
   const int m = blockIdx.x;
@@ -1837,7 +1807,7 @@ __global__ void k_mesh_dt_min(const int* __restrict__ start, const double* __res
 
 // Per-mesh residual norm over divF_spts[0] (element-major), as
 // ele::getNormResidual summed over the mesh's elements (src/ele.cpp:1922-1945).
-__global__ void k_mesh_res(int S, int N, int type, const int* __restrict__ start, const double* __restrict__ divF0e,
+static __global__ void k_mesh_res(int S, int N, int type, const int* __restrict__ start, const double* __restrict__ divF0e,
                            const double* __restrict__ detJe, const double* __restrict__ ws, double* __restrict__ out) {
   __shared__ double red[256];
   const int m = blockIdx.x;
@@ -1876,6 +1846,7 @@ static T* dal(size_t n) {
   return (T*)p;
 }
 
+#ifndef FHIP_FAMILY
 // Extract the non-zero structure of the dense operators.  Returns false if an
 // operator row has more non-zeros than the tensor-product structure allows.
 // opp_grad_spts as one 1-D derivative matrix (Tabs::d1): true when every
@@ -2068,7 +2039,9 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
   return true;
 }
 
-__global__ void k_round_f32(long long n, const double* __restrict__ in, float* __restrict__ out) {
+#endif  // FHIP_FAMILY
+
+static __global__ void k_round_f32(long long n, const double* __restrict__ in, float* __restrict__ out) {
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
     out[i] = float(in[i]);
 }
@@ -2111,19 +2084,14 @@ template <class R>
 static void ensure_work(Ctx& c) {
   Work<R>& w = fs(c).work<R>();
   if (w.ready) return;
-  const long long E = c.z.E, S = c.z.S, F = c.z.F, N = c.z.N, D = c.z.D;
+  const long long E = c.z.E, S = c.z.S, F = c.z.F, N = c.z.N;
   w.Ufe = dal<R>(E * N * F);
   if (!c.prm.viscous) w.Ufe2 = dal<R>(E * N * F);
-  // the face kernel's common flux: inviscid runs take that kernel for its wave
-  // speeds alone, where a single-stage step needs them before its update
-  if (c.prm.viscous || face_first(c)) w.Fne = dal<R>(E * N * F);
   if (c.prm.viscous) {
     // inviscid runs keep divF and the discontinuous normal flux in the stage kernel
     w.divFe = dal<R>(E * N * S);
-    w.disFne = dal<R>(E * N * F);
-    w.dUce = dal<R>(E * N * F);
     w.Bve = dal<R>(E * N * F);
-    w.gBnd = dal<R>((long long)D * N * fs(c).nBnd);
+    if (kJumpOut<R>) w.Jne = dal<R>(E * N * F);
   }
   if (sizeof(R) == 4 && c.z.nRK > 1 && c.prm.time_type < 5) w.Rst = dal<R>((long long)(c.z.nRK - 1) * E * N * S);
   w.Us = dal<R>(E * N * S);
@@ -2131,6 +2099,7 @@ static void ensure_work(Ctx& c) {
   w.ready = true;
 }
 
+#ifndef FHIP_FAMILY
 bool fused_setup(Ctx& c, const fhip_desc* d) {
   const Sizes& z = c.z;
   if (z.P < 0 || z.P > 5) return false;
@@ -2265,12 +2234,10 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
       st->fpart = dal<int>(part.size());
       FCHK(hipMemcpy(st->fpart, part.data(), part.size() * 4, hipMemcpyHostToDevice));
       st->nBnd = (int)bt.size();
-      st->bndT = dal<int>(bt.size());
       st->bndBc = dal<int>(bb.size());
       st->nfe = dal<double>(nl.size());
       FCHK(hipMemcpy(st->nfe, nl.data(), nl.size() * 8, hipMemcpyHostToDevice));
       if (!bt.empty()) {
-        FCHK(hipMemcpy(st->bndT, bt.data(), bt.size() * 4, hipMemcpyHostToDevice));
         FCHK(hipMemcpy(st->bndBc, bb.data(), bb.size() * 4, hipMemcpyHostToDevice));
       }
     }
@@ -2321,6 +2288,8 @@ void fused_release(Ctx& c) {
   c.fused = nullptr;
 }
 
+#endif  // FHIP_FAMILY
+
 // ---- per-order / per-precision dispatch ------------------------------------
 
 static double cfl_limit_f(int order) {  // getCFLLimit, src/global.cpp:81-105
@@ -2334,13 +2303,9 @@ struct Runner {
   using Sh = Shape<D, P>;
   static constexpr int S = Sh::S, F = Sh::F, N = Sh::N;
   static const char* nm(const char* f64, const char* f32) { return sizeof(R) == 8 ? f64 : f32; }
-  // The face kernel stores each side's flux into that element's rows of one
-  // face (Ff values per field).  Streamed (nontemporal) stores pay only when
-  // such a row is whole 64-byte blocks, the memory's write granule: a partial
-  // block written past the caches costs a read-modify-write (measured: FP64
-  // P2/P4/P5 face kernels 1.7-1.4x faster without streaming, P3 rows of 128
-  // and 64 bytes faster with it).
-  static constexpr bool kFaceRowsWhole = (Sh::Ff * sizeof(R)) % 64 == 0;
+  // Streamed (nontemporal) stores pay only when the rows that a kernel stores are
+  // whole 64-byte blocks, the memory's write granule: a partial block written
+  // past the caches costs a read-modify-write.
   // The element kernels store rows of S or F values per field; a wave's
   // streamed store covers whole blocks only when those rows are whole blocks.
   static constexpr bool kEleRowsWhole = (S * sizeof(R)) % 64 == 0 && (F * sizeof(R)) % 64 == 0;
@@ -2372,10 +2337,7 @@ struct Runner {
     const size_t EB = nt / S;
     const size_t SF = (visc && F > D * S) ? F : D * S;
     if (k == kExtrap) return EB * N * S * sizeof(R);
-    if (k == kVolume)
-      return EB * N * (S + SF) * sizeof(R) +
-             (visc ? EB * (D * F * sizeof(R) + F * sizeof(int) + (kJumpInVolume<R> ? N * F * sizeof(R) : 0))
-                   : EB * N * F * sizeof(R));
+    if (k == kVolume) return visc ? EB * N * ((!kJumpOut<R> && jump_over_u<D, P> && F > S ? F : S) + SF) * sizeof(R) : EB * N * (S + SF + F) * sizeof(R);
     if (k == kRk) return EB * N * (S + F) * sizeof(R);
     return 0;
   }
@@ -2398,36 +2360,32 @@ struct Runner {
     Work<R>& w = st.work<R>();
     const int nFF = c.z.nFaceFpts;
     if (nFF == 0) return;
-    if (st.stream && kFaceRowsWhole)
-      hipLaunchKernelGGL((k_face_inv<D, P, R, true>), dim3(nblk(nFF, nt)), dim3(nt), 0, c.stream, nFF, st.pL, st.pR,
-                         st.bc, w.Ufe, w.nrm, w.Fne, st.waveSpe, w.dUce, c.ph, st.bst);
-    else
-      hipLaunchKernelGGL((k_face_inv<D, P, R, false>), dim3(nblk(nFF, nt)), dim3(nt), 0, c.stream, nFF, st.pL, st.pR,
-                         st.bc, w.Ufe, w.nrm, w.Fne, st.waveSpe, w.dUce, c.ph, st.bst);
+    hipLaunchKernelGGL((k_face_inv<D, P, R>), dim3(nblk(nFF, nt)), dim3(nt), 0, c.stream, nFF, st.pL, st.pR, st.bc,
+                       w.Ufe, w.nrm, st.waveSpe, c.ph, st.bst);
     FCHK(hipGetLastError());
   }
   // viscous runs: the volume kernel.  Quads and FP32 are held to 4 waves per
   // SIMD (128 VGPRs); FP64 hexes, which spill under that hold, to 3 (168 VGPRs:
   // P3 without spills, where the unheld compiler would take 211 and leave 2
   // waves)
-  template <bool NT, bool TEN>
-  static void launch_volume_t(Ctx& c, int nt) {
+  template <bool NT, bool BND, bool TEN>
+  static void launch_volume_t(Ctx& c, int nt, bool wave) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
-    const VFace<R> vf{st.fpart, w.nf, w.Bve, w.gBnd, w.dA, st.nBnd};
+    const VFace<R> vf{st.fpart, w.Ufe, w.nf, w.dA, w.Bve, w.Jne, wave ? st.waveSpe : nullptr, st.bndBc, st.bst};
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, true), c.stream, c.z.E, st.Ue, us,
-                         w.dUce, w.JG, w.iJ, w.divFe, w.disFne, vf, st.tb, c.ph);
+                         w.JG, w.iJ, w.divFe, vf, st.tb, c.ph);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, TEN, 2>);
-      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, TEN, 3>);
-      else go(k_volume_w4<D, P, R, NT, TEN>);
+      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, BND, TEN, 2>);
+      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, BND, TEN, 3>);
+      else go(k_volume_w4<D, P, R, NT, BND, TEN>);
     } else if constexpr (kHold<D, R>) {
-      go(k_volume_w4<D, P, R, NT, TEN>);
+      go(k_volume_w4<D, P, R, NT, BND, TEN>);
     } else {
-      go(k_volume_w3<D, P, R, NT, TEN>);
+      go(k_volume_w3<D, P, R, NT, BND, TEN>);
     }
     FCHK(hipGetLastError());
   }
@@ -2460,32 +2418,32 @@ struct Runner {
     }
     FCHK(hipGetLastError());
   }
-  static void launch_volume(Ctx& c, int nt) {
-    if (!fs(c).tb.w1) launch_volume_t<false, false>(c, nt);
-    else if (fs(c).stream && kEleRowsWhole) launch_volume_t<true, true>(c, nt);
-    else launch_volume_t<false, true>(c, nt);
+  // (instances that stream exist only for the orders whose rows are whole)
+  static void launch_volume(Ctx& c, int nt, bool wave) {
+    const bool bnd = fs(c).nBnd > 0;
+    if (!fs(c).tb.w1) return launch_volume_t<false, true, false>(c, nt, wave);
+    if constexpr (kEleRowsWhole) {
+      if (fs(c).stream) return bnd ? launch_volume_t<true, true, true>(c, nt, wave) : launch_volume_t<true, false, true>(c, nt, wave);
+    }
+    if (bnd) launch_volume_t<false, true, true>(c, nt, wave);
+    else launch_volume_t<false, false, true>(c, nt, wave);
   }
   static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
-    const bool sm = fs(c).stream && kEleRowsWhole, bnd = fs(c).nBnd > 0;
+    const bool bnd = fs(c).nBnd > 0;
     // operators read from their tables: one instance for every mesh
-    if (!fs(c).tb.w1) launch_stage_t<false, true, false, false>(c, nt, ra, fold);
-    else if (sm && bnd) launch_stage_t<true, true, true, false>(c, nt, ra, fold);
-    else if (sm) launch_stage_t<true, false, true, false>(c, nt, ra, fold);
-    else if (apart(c) && bnd) launch_stage_t<false, true, true, true>(c, nt, ra, fold);
+    if (!fs(c).tb.w1) return launch_stage_t<false, true, false, false>(c, nt, ra, fold);
+    if constexpr (kEleRowsWhole) {
+      if (fs(c).stream)
+        return bnd ? launch_stage_t<true, true, true, false>(c, nt, ra, fold)
+                   : launch_stage_t<true, false, true, false>(c, nt, ra, fold);
+    }
+    if (apart(c) && bnd) launch_stage_t<false, true, true, true>(c, nt, ra, fold);
     else if (apart(c)) launch_stage_t<false, false, true, true>(c, nt, ra, fold);
     else if (bnd) launch_stage_t<false, true, true, false>(c, nt, ra, fold);
     else launch_stage_t<false, false, true, false>(c, nt, ra, fold);
   }
   // whether a step's first stage forms the elements' time steps itself
   static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
-  static void launch_face_bnd(Ctx& c, int nt) {
-    FusedState& st = fs(c);
-    Work<R>& w = st.work<R>();
-    if (st.nBnd == 0) return;
-    hipLaunchKernelGGL((k_face_bnd<D, P, R>), dim3(nblk(st.nBnd, nt)), dim3(nt), 0, c.stream, st.nBnd, st.bndT, st.pL,
-                       st.bc, w.Ufe, w.gBnd, w.nrm, w.dA, w.Bve, w.disFne, c.ph, st.bst);
-    FCHK(hipGetLastError());
-  }
   static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2506,10 +2464,12 @@ struct Runner {
   static void launch_rk(Ctx& c, int nt, int mode, double a, double b, bool write0, int stage = 0) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
-    auto* kern = !st.tb.w1 ? k_rk<D, P, R, false, false>
-                           : ((st.stream && kEleRowsWhole) ? k_rk<D, P, R, true, true> : k_rk<D, P, R, false, true>);
-    hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kRk, nt, false), c.stream, c.z.E, w.divFe, w.Fne,
-                       w.disFne, rk_args(c, mode, a, b, write0, stage), st.tb, st.fpart, w.dA, w.Bve);
+    auto* kern = st.tb.w1 ? k_rk<D, P, R, false, true> : k_rk<D, P, R, false, false>;
+    if constexpr (kEleRowsWhole) {
+      if (st.tb.w1 && st.stream) kern = k_rk<D, P, R, true, true>;
+    }
+    hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kRk, nt, false), c.stream, c.z.E, w.divFe,
+                       rk_args(c, mode, a, b, write0, stage), st.tb, st.fpart, w.dA, w.Bve, w.Jne);
     FCHK(hipGetLastError());
   }
   // after a step with an odd number of stages: U at the flux points back
@@ -2556,20 +2516,13 @@ struct Runner {
     Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
     launch_face_inv(c, blk(c, kFaceInv));
   }
-  // calcResidual up to what the RK update needs: the face, volume and boundary
-  // kernels of viscous runs; nothing on inviscid ones, whose stage kernel runs
-  // in rk below
-  static void residual(Ctx& c) {
+  // calcResidual up to what the RK update needs: the volume kernel of viscous
+  // runs (wave: with the wave speeds, which stages that another stage follows
+  // leave); nothing on inviscid ones, whose stage kernel runs in rk below
+  static void residual(Ctx& c, bool wave) {
     if (!c.prm.viscous) return;
-    face(c);
-    {
-      Launch L(c, nm("fused_volume_viscous", "mixed_volume_viscous"));
-      launch_volume(c, blk(c, kVolume));
-    }
-    if (fs(c).nBnd > 0) {
-      Launch L(c, nm("fused_face_boundary", "mixed_face_boundary"));
-      launch_face_bnd(c, blk(c, kFaceBnd));
-    }
+    Launch L(c, nm("fused_volume_viscous", "mixed_volume_viscous"));
+    launch_volume(c, blk(c, kVolume), wave);
   }
   static void rk(Ctx& c, int mode, double a, double b, bool write0, int stage) {
     if (!c.prm.viscous) {
@@ -2604,16 +2557,14 @@ struct Runner {
     // elements, so sizes between the powers of two pay off where S divides them
     const int cand[7] = {64, 128, 192, 256, 320, 384, 512};
     for (int k = kExtrap; k <= kRk; k++) {
-      if ((k == kFaceBnd && (!visc || st.nBnd == 0)) || ((k == kRk || k == kFaceInv) && !visc)) continue;
+      if (k == kFaceBnd || k == kFaceInv || (k == kRk && !visc)) continue;
       auto run = [&](int nt) {
         switch (k) {
           case kExtrap: launch_extrap(c, nt); break;
-          case kFaceInv: launch_face_inv(c, nt); break;
           case kVolume:
-            if (visc) launch_volume(c, nt);
+            if (visc) launch_volume(c, nt, false);
             else launch_stage(c, nt, rk_args(c, 1, 0.5, 1. / 3., false, 0));
             break;
-          case kFaceBnd: launch_face_bnd(c, nt); break;
           default: launch_rk(c, nt, 1, 0.5, 1. / 3., false);
         }
       };
@@ -2676,7 +2627,7 @@ struct Ops {
   void (*wave)(Ctx&);
   void (*dt)(Ctx&, double);
   void (*face)(Ctx&);
-  void (*residual)(Ctx&);
+  void (*residual)(Ctx&, bool);
   void (*copy_ufe)(Ctx&);
   bool (*folds_dt)(const Ctx&);
   void (*rk)(Ctx&, int, double, double, bool, int);
@@ -2692,30 +2643,40 @@ static Ops ops_for() {
   return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::folds_dt, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit};
 }
 
-template <class R>
-static Ops get_ops_r(const Ctx& c) {
-  const int D = c.z.D, P = c.z.P;
-  if (D == 2) {
-    switch (P) {
-      case 0: return ops_for<2, 0, R>();
-      case 1: return ops_for<2, 1, R>();
-      case 2: return ops_for<2, 2, R>();
-      case 3: return ops_for<2, 3, R>();
-      case 4: return ops_for<2, 4, R>();
-      default: return ops_for<2, 5, R>();
-    }
+// The kernels of one dimension, precision and range of orders.  This file is
+// compiled once for each (FHIP_FAMILY = 0 to 5, side by side: one after the
+// other they take minutes) and once without for everything else.
+Ops ops_2d_f64(int P), ops_2d_f32(int P), ops_3d_f64_low(int P), ops_3d_f64_high(int P), ops_3d_f32_low(int P),
+    ops_3d_f32_high(int P);
+#ifdef FHIP_FAMILY
+template <int D, int P0, int P, class R>
+static Ops ops_range(int p) {
+  if constexpr (P > P0) {
+    if (p < P) return ops_range<D, P0, P - 1, R>(p);
   }
-  switch (P) {
-    case 0: return ops_for<3, 0, R>();
-    case 1: return ops_for<3, 1, R>();
-    case 2: return ops_for<3, 2, R>();
-    case 3: return ops_for<3, 3, R>();
-    case 4: return ops_for<3, 4, R>();
-    default: return ops_for<3, 5, R>();
-  }
+  return ops_for<D, P, R>();
 }
+#if FHIP_FAMILY == 0
+Ops ops_2d_f64(int P) { return ops_range<2, 0, 5, double>(P); }
+#elif FHIP_FAMILY == 1
+Ops ops_2d_f32(int P) { return ops_range<2, 0, 5, float>(P); }
+#elif FHIP_FAMILY == 2
+Ops ops_3d_f64_low(int P) { return ops_range<3, 0, 2, double>(P); }
+#elif FHIP_FAMILY == 3
+Ops ops_3d_f64_high(int P) { return ops_range<3, 3, 5, double>(P); }
+#elif FHIP_FAMILY == 4
+Ops ops_3d_f32_low(int P) { return ops_range<3, 0, 2, float>(P); }
+#else
+Ops ops_3d_f32_high(int P) { return ops_range<3, 3, 5, float>(P); }
+#endif
+#else
 
-static Ops get_ops(const Ctx& c, bool mixed) { return mixed ? get_ops_r<float>(c) : get_ops_r<double>(c); }
+static Ops get_ops(const Ctx& c, bool mixed) {
+  const int P = c.z.P;
+  if (c.z.D == 2) return mixed ? ops_2d_f32(P) : ops_2d_f64(P);
+  if (P < 3) return mixed ? ops_3d_f32_low(P) : ops_3d_f64_low(P);
+  return mixed ? ops_3d_f32_high(P) : ops_3d_f64_high(P);
+}
 
 // Tuned block sizes, shared by the contexts of one process: keyed by
 // (nDims, order, precision, viscous, log2 of the element count).
@@ -2817,7 +2778,7 @@ void fused_em_import_wave(Ctx& c) {
 void fused_em_residual(Ctx& c, bool mixed, int how) {
   Ops o = get_ops(c, mixed);
   fs(c).use_src = false;
-  o.residual(c);
+  o.residual(c, true);
   o.rk(c, how == 1 ? 7 : (how == 2 ? 8 : 5), 0., 0., true, 0);
 }
 
@@ -2886,7 +2847,7 @@ void fused_residual(Ctx& c, bool mixed) {
   const Sizes& z = c.z;
   Ops o = get_ops(c, mixed);
   fused_begin(c, mixed, false);
-  o.residual(c);
+  o.residual(c, true);
   o.rk(c, 5, 0., 0., true, 0);
   from_em(c.stream, z.S, z.E, z.N, st.divF0e, c.divF);
   from_em(c.stream, z.F, z.E, 1, st.waveSpe, c.waveSp);
@@ -2905,7 +2866,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
   const bool jameson = c.prm.time_type >= 5;
   st.odd_stage = false;
   if (nRK == 1) {
-    if (c.prm.viscous) o.residual(c);
+    if (c.prm.viscous) o.residual(c, true);
     else if (cfl) o.face(c);
     if (cfl) {
       if (refresh) o.wave(c);
@@ -2922,7 +2883,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
   for (int step = 0; step < nRK; step++) {
     st.read_stage = step > 0;
     st.odd_stage = !c.prm.viscous && (step & 1);
-    o.residual(c);
+    o.residual(c, step == nRK - 1);
     // the Jameson form's first stage reads the state itself (the step's U0)
     int mode;
     if (jameson) mode = step == 0 ? 6 : 4;
@@ -2932,5 +2893,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
   st.read_stage = st.odd_stage = false;
   if (!c.prm.viscous && (nRK & 1)) o.copy_ufe(c);
 }
+
+#endif  // FHIP_FAMILY
 
 }  // namespace fhip

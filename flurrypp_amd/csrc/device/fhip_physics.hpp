@@ -401,6 +401,33 @@ __device__ __forceinline__ void ldg_side(const T* U, const T g[D][D + 2], const 
 //   sum_d Fc[d] n[d] = [nFL / 2 + pf |n|^2 (nFL + n[2] d12L) + tau |n|^2 UL]
 //                    + [nFR / 2 - pf |n|^2 nFR - tau |n|^2 UR],
 // so each side adds its bracket and only N values carry over between sides.
+// One side's bracket without its tau term, for that side's viscous flux F at the
+// point.
+template <int D, class T>
+__device__ __forceinline__ T ldg_tau(const T* n, T tau) {
+  T nn = n[0] * n[0] + n[1] * n[1];
+  if constexpr (D == 3) nn += n[2] * n[2];
+  return tau * nn;
+}
+
+template <int D, class T>
+__device__ __forceinline__ void ldg_part(bool left, const T* U, const T g[D][D + 2], const T* n, T* part,
+                                         const Phys& ph) {
+  constexpr int N = D + 2;
+  T F[D][N], nF[N], d12[N];
+  viscous_flux<D, T>(U, g, F, ph);
+  ldg_project<D, T>(F, n, nF, d12);
+  T nn = n[0] * n[0] + n[1] * n[1];
+  if constexpr (D == 3) nn += n[2] * n[2];
+  const T pn = ldg_pen<D, T>(n, T(ph.pen_fact)) * nn;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    T s = nF[k];
+    if constexpr (D == 3) s += n[2] * d12[k];
+    part[k] = left ? T(0.5) * nF[k] + pn * s : (T(0.5) - pn) * nF[k];
+  }
+}
+
 // Adds one side's bracket for that side's viscous flux F at the point.
 template <int D, class T>
 __device__ __forceinline__ void ldg_add_flux(bool left, const T* U, const T F[D][D + 2], const T* n, T* Fn,

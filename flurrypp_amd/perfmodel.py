@@ -27,22 +27,15 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     F = 2 * D * P1 ** (D - 1)
     nFFi = nFF - nFFb
     out = {}
-    # face_inviscid: read UL, UR (interior), normal, 3 int32 per face flux
-    # point; write Fn once per pair (at L), the wave speed (+ dUc L (+R) in
-    # viscous runs)
-    rd = nFF * (N + D + 3 * B4 / B8) + nFFi * N
-    wr = nFF * (N + 1)
-    if viscous:
-        wr += nFF * N + nFFi * N
-        out["fused_face_inviscid"] = Work((rd + wr) * B8, 0.0)
-    # volume
+    # volume: U, the metric terms
     rd = E * (N * S + D * D * S)
-    wr = E * (N * S + N * F)
     fl = E * N * (D * S * 2 * P1 + F * D * 2 * P1)   # divergence + normal-flux extrapolation
     if viscous:
-        rd += E * (S + N * F)                        # detJ, dUc
-        rd += E * F * (D + B4 / B8)                  # face normal, side/partner code
-        wr += E * N * F + nFFb * D * N               # side of the LDG flux; boundary gradient
+        # 1/detJ; U across, normal, dA, side/partner code at the flux points;
+        # the corrected divergence, each side's part of the LDG flux and the
+        # last stage's wave speeds out
+        rd += E * S + 2 * nFFi * N + E * F * (D + 1 + B4 / B8)
+        wr = E * N * S + 2 * nFFi * N + nFF / nRK
         fl += E * N * (D * S * 2 * P1 + D * S * 2 * 2 * D + (D + 1) * F * 2 * P1)
         out["fused_volume_viscous"] = Work((rd + wr) * B8, fl)
     else:
@@ -51,18 +44,14 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
         # normal flux stay on chip, U at the element's flux points and across
         # is read instead (with the normal, dA and the side code)
         vol_rd = rd + E * 2 * N * F + E * F * (D + 1 + B4 / B8)
-        vol_wr = wr - E * (N * S + N * F) + nFF / nRK  # the wave speeds of the last stage
-    if viscous and nFFb:
-        # boundary LDG flux: U, normal, gradient in; the point's flux part out
-        rd = nFFb * (N + D + D * N + 3 * B4 / B8)
-        wr = nFFb * N
-        out["fused_face_boundary"] = Work((rd + wr) * B8, 0.0)
+        vol_wr = nFF / nRK                           # the wave speeds of the last stage
     # rk update, averaged over the stages of one step
     per_stage = []
     for st in range(nRK):
-        rd = E * (N * S + 2 * N * F + S)             # divF, Fn, disFn, detJ
+        rd = E * S                                   # detJ
         if viscous:
-            rd += E * F * (2 * N + 1 + B4 / B8)      # both sides' LDG parts, dA, partner code
+            # divF; the partners' LDG parts, dA, partner code
+            rd += E * N * S + 2 * nFFi * N + E * F * (1 + B4 / B8)
         wr = E * (N * S + N * F)                     # U, U at the faces
         if time_type >= 5:
             rd += E * N * S                          # U0
@@ -83,8 +72,7 @@ def fused_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     if viscous:
         out["fused_rk_update"] = rk
     else:
-        # the RK part without its reads of divF, Fn and disFn
-        out["fused_stage"] = Work((vol_rd + vol_wr) * B8 + rk.bytes - E * (N * S + 2 * N * F) * B8, fl + rk.flops)
+        out["fused_stage"] = Work((vol_rd + vol_wr) * B8 + rk.bytes, fl + rk.flops)
     return out
 
 
@@ -100,13 +88,6 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     f4, d8, i4 = 4, 8, 4
     fp = fused_work(D, P, E, nFF, nFFb, viscous, nRK, time_type)
     out = {}
-    # face: 3 ints, UL, UR, normal in; Fn once per pair (at L), wave speed
-    # (FP64) [+ dUc L (+R)] out
-    rd = nFF * (3 * i4 + f4 * (N + D)) + nFFi * f4 * N
-    wr = nFF * (f4 * N + d8)
-    if viscous:
-        wr += (nFF + nFFi) * f4 * N
-        out["mixed_face_inviscid"] = Work(rd + wr, 0.0)
     # volume: U (stage copy), metric terms (inviscid runs, the stage kernel:
     # with U at the flux points and across, normal, dA and side code, and the
     # last stage's wave speeds)
@@ -114,22 +95,19 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     if not viscous:
         rd += E * F * (f4 * (2 * N + D + 1) + i4) + nFF * d8 / nRK
     if viscous:
-        # 1/detJ, dUc, face normal, dA, side code; divF, this side's flux jump
-        # (with its LDG part), the LDG part, boundary gradient out
-        rd += E * (f4 * (S + N * F + D * F + F) + i4 * F)
-        wr = E * f4 * (N * S + 2 * N * F) + nFFb * f4 * D * N
+        # 1/detJ; U across, normal, dA, side code; the corrected divergence, the
+        # LDG side parts and the last stage's wave speeds out
+        rd += E * (f4 * (S + D * F + F) + i4 * F) + f4 * 2 * nFFi * N
+        wr = E * f4 * N * S + f4 * 2 * nFFi * N + nFF * d8 / nRK
         out["mixed_volume_viscous"] = Work(rd + wr, fp["fused_volume_viscous"].flops)
-        if nFFb:
-            # U, normal, gradient, 3 ints, dA in; the point's flux jump updated
-            out["mixed_face_boundary"] = Work(nFFb * (f4 * (N + D + D * N + 1) + 3 * i4 + 2 * f4 * N), 0.0)
     # classical RK stages keep their residuals in FP32 (the form without a
     # multigrid source); the FP64 state, written at the last stage only, is
     # also the step's U0; Jameson-form stages read it and write the state last
     per_stage = []
     for st in range(nRK):
-        rd_ = E * (f4 * N * S + d8 * S)                # divF, detJ
+        rd_ = E * d8 * S                               # detJ
         if viscous:
-            rd_ += E * (f4 * 3 * N * F + f4 * F + i4 * F)  # Fn, flux jump, partner's LDG part, dA, code
+            rd_ += E * (f4 * N * S + f4 * F + i4 * F) + f4 * 2 * nFFi * N  # divF, dA, code; partner's LDG part
         wr_ = E * (f4 * N * F + f4 * N * S)            # U at the faces, stage copy of U
         if time_type >= 5:
             rd_ += E * d8 * N * S                      # U0
@@ -152,7 +130,7 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     if viscous:
         out["mixed_rk_update"] = Work(rk, fp["fused_rk_update"].flops)
     else:
-        out["mixed_stage"] = Work(rd + rk - E * f4 * N * S, fp["fused_stage"].flops)
+        out["mixed_stage"] = Work(rd + rk, fp["fused_stage"].flops)
     return out
 
 

@@ -86,13 +86,13 @@ def footprint_bytes(nDims: int, order: int, nEles: int, viscous: bool = False, n
     d += 4 * SN + F * (2 + D) + D * D * S + 2 * S + 1.5 * F + 0.5 * F + 1
     # the faces' normals at every flux point
     d += D * F
-    # FP64 work: divF, U (two copies on inviscid runs)/Fn/disFn at the flux points
-    d += SN + 3 * FN
+    # FP64 work: stage copy or divF, two arrays at the flux points (U, and its second copy on inviscid
+    # runs or the LDG side parts)
+    d += SN + 2 * FN
     # FP32 work (half a double each): the same, stage residuals, FP32 U, FP32 geometry
-    d += 0.5 * (SN + 3 * FN + (nRK - 1) * SN + SN + D * D * S + S + 2 * D * F + F)
+    d += 0.5 * (SN + 2 * FN + (nRK - 1) * SN + SN + D * D * S + S + 2 * D * F + F)
     if viscous:
         d += D * SN + D * FN + FN            # staged gradients and dUc
-        d += 2 * FN + 0.5 * 2 * FN           # dUc and LDG side parts, FP64 and FP32
     if pmg_source:
         d += SN                              # P-multigrid source, element-major
     return int(8 * d * nEles * 1.25) + (16 << 20)
