@@ -73,8 +73,7 @@ enum { kExtrap = 0, kFaceInv = 1, kVolume = 2, kFaceBnd = 3, kRk = 4 };
 // Sparse operator tables (device pointers into one allocation).  Indices of
 // solution points are positions in the swizzled LDS layout (spt_lds below).
 struct Tabs {
-  const int* ext_idx;   // [F][P1]    solution points feeding flux point f
-  const double* ext_w;  // [F][P1]    opp_spts_to_fpts entries
+  const double* ext_w;  // [F][P1]    opp_spts_to_fpts entries (of the points in line)
   const int* efn_dir;   // [F]        the one direction d with opp_extrapolate_fn[d][f] != 0
   const double* efn_w;  // [F][P1]    opp_extrapolate_fn[efn_dir[f]] entries (same points)
   const int* grd_idx;   // [D][S][P1]
@@ -95,6 +94,8 @@ struct Tabs {
   // [Ten::NW], FP64 and FP32, or null
   const double* w1;
   const float* w1f;
+  // [F][(P1+3)/4] solution points feeding flux point f, one byte each (S <= 216)
+  const unsigned* line;
 };
 
 // The 1-D contractions of FP64 P3 hexes along x and z run on the matrix
@@ -330,19 +331,18 @@ struct PtTab {
   __device__ int cu_idx(int d, int j) const { return tb.cu_idx[(d * S + s) * 2 + j]; }
   __device__ R cu_w(int d, int j) const { return tw<R>(tb.cu_w, tb.cu_wf)[(d * S + s) * 2 + j]; }
 };
-// A flux point's operator entries: extrapolation (positions and weights; the
-// sum over them, negated on a low end, is the normal flux's), normal direction.
+// A flux point's operator entries: extrapolation weights (the sum over them,
+// negated on a low end, is the normal flux's), normal direction.
 template <int D, int P, class R>
 struct FpTen {
   using T = Ten<D, P>;
   const R* w;
-  typename T::Face f;
-  __device__ FpTen(const Tabs&, const R* sW, int fpt) : w(sW), f(fpt) {}
-  __device__ int idx(int m) const { return f.at(m); }
-  __device__ R ext_w(int m) const { return w[T::L + f.hi * T::P1 + m]; }
+  int face;
+  __device__ FpTen(const Tabs&, const R* sW, int fpt) : w(sW), face(fpt / Shape<D, P>::Ff) {}
+  __device__ R ext_w(int m) const { return w[T::L + T::face_hi(face) * T::P1 + m]; }
   __device__ R efn_w(int m) const { return ext_w(m); }
-  __device__ R efn_sign(R a) const { return f.hi ? a : -a; }
-  __device__ int dir() const { return f.dn; }
+  __device__ R efn_sign(R a) const { return T::face_hi(face) ? a : -a; }
+  __device__ int dir() const { return T::face_dir(face); }
 };
 template <int D, int P, class R>
 struct FpTab {
@@ -350,7 +350,6 @@ struct FpTab {
   const Tabs& tb;
   int f;
   __device__ FpTab(const Tabs& t, const R*, int fpt) : tb(t), f(fpt) {}
-  __device__ int idx(int m) const { return tb.ext_idx[f * P1 + m]; }
   __device__ R ext_w(int m) const { return tw<R>(tb.ext_w, tb.ext_wf)[f * P1 + m]; }
   __device__ R efn_w(int m) const { return tw<R>(tb.efn_w, tb.efn_wf)[f * P1 + m]; }
   __device__ R efn_sign(R a) const { return a; }
@@ -367,6 +366,41 @@ __device__ __forceinline__ void stage_factors(R* sW, const Tabs& tb) {
     if (threadIdx.x < Ten<D, P>::NW) sW[threadIdx.x] = tw<R>(tb.w1, tb.w1f)[threadIdx.x];
   }
 }
+
+// The solution points of a flux point's line, by slab position in a byte each: a
+// register or two, loaded with a kernel's first loads and kept for all its phases
+// (computed, with the selects on the face's direction, they are some 100
+// instructions).
+template <int P1>
+struct Packed {
+  static constexpr int W = (P1 + 3) / 4;
+  unsigned v[W];
+  __device__ void load(const Tabs& tb, int f) {
+#pragma unroll
+    for (int j = 0; j < W; j++) v[j] = tb.line[f * W + j];
+  }
+  __device__ int operator[](int m) const { return (v[m / 4] >> (8 * (m % 4))) & 255; }
+};
+// Pointers to those points in an element's slab and their weights.  The fields of
+// the slab are then at constant offsets, which LDS reads take for nothing: an
+// address formed for each read (an add, often a multiply) and the weights read
+// again for each field were a third of the viscous volume kernel's instructions.
+template <int P1, class R>
+struct LineOp {
+  const R* q[P1];
+  R w[P1];
+  template <class At, class W>
+  __device__ LineOp(const R* slab, const At& at, const W& weight) {
+#pragma unroll
+    for (int m = 0; m < P1; m++) q[m] = slab + at(m), w[m] = weight(m);
+  }
+  __device__ R operator()(int off) const {
+    R a = 0;
+#pragma unroll
+    for (int m = 0; m < P1; m++) a += w[m] * q[m][off];
+    return a;
+  }
+};
 
 // Face and volume intermediates of one precision.
 template <class R>
@@ -524,13 +558,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_extrap(int E, const double* __res
   for (int i = threadIdx.x; i < nb * F; i += blockDim.x) {
     int b = i / F, f = i - b * F;
     const FpOp<D, P, R, TEN> fp(tb, sW, f);
+    Packed<P1> lp;
+    lp.load(tb, f);
+    const LineOp<P1, R> line(sU + b * N * S, [&](int m) { return lp[m]; }, [&](int m) { return fp.ext_w(m); });
+    R* const o = Ufe + (long long)(e0 + b) * N * F + f;
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      R acc = 0;
-#pragma unroll
-      for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(b * N + k) * S + fp.idx(m)];
-      Ufe[((long long)(e0 + b) * N + k) * F + f] = acc;
-    }
+    for (int k = 0; k < N; k++) o[k * F] = line(k * S);
   }
 }
 
@@ -713,15 +746,15 @@ __device__ __forceinline__ RkIn<D, R> rk_load(int E, long long e, int s, const R
   return in;
 }
 
-// correctDivFlux of field k at a point of the block's element b, from the flux
-// jump in sD.
+// correctDivFlux at a point of the block's element b, from the flux jump in sD:
+// out[k] is the correction of field k plus dv[k].
 template <int D, int P, class R, class Op>
-__device__ __forceinline__ R correction(const R* sD, int b, int k, const Op& po) {
+__device__ __forceinline__ void correction(const R* sD, int b, const Op& po, const R* dv, R* out) {
   using Sh = Shape<D, P>;
-  R c = 0;
+  const LineOp<Sh::NC, R> line(sD + b * Sh::N * Sh::F, [&](int j) { return po.cor_idx(j); },
+                               [&](int j) { return po.cor_w(j); });
 #pragma unroll
-  for (int j = 0; j < Sh::NC; j++) c += po.cor_w(j) * sD[(b * Sh::N + k) * Sh::F + po.cor_idx(j)];
-  return c;
+  for (int k = 0; k < Sh::N; k++) out[k] = line(k * Sh::F) + dv[k];
 }
 
 // correctDivFlux and timeStepA/B at point s of the block's element b: dv holds
@@ -736,8 +769,7 @@ __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const
   const int mode = ra.mode;
   const PtOp<D, P, R, TEN> po(tb, sW, s);
   R res[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) res[k] = correction<D, P, R>(sD, b, k, po) + dv[k];
+  correction<D, P, R>(sD, b, po, dv, res);
   const long long at = e * N * S + s;
   if (mode == 5 || mode == 7 || mode == 8) {
     // residual only (calcResidual(0) + correctDivFlux), no update: 5 into
@@ -752,6 +784,7 @@ __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const
     return;
   }
   const double q = in.dt / in.dj;
+  R* const qu = sU + b * N * S + spt_lds(D, P1, s);
 #pragma unroll
   for (int k = 0; k < N; k++) {
     const long long iu = at + k * S;
@@ -794,24 +827,22 @@ __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const
     // reads the state itself)
     if (ra.fin) st_s<NT>(un, &ra.Ue[iu]);
     if (sizeof(R) == 4 || !ra.fin) st_s<NT>(R(un), &ra.Us[iu]);
-    sU[(b * N + k) * S + spt_lds(D, P1, s)] = R(un);
+    qu[k * S] = R(un);
   }
 }
 
 // extrapolateU at flux point i of the block, from the states in sU.
 template <int D, int P, class R, bool NT, bool TEN>
-__device__ __forceinline__ void face_point(int i, int e0, const R* sU, const R* sW, R* Ufe, const Tabs& tb) {
+__device__ __forceinline__ void face_point(int i, int e0, const Packed<P + 1>& lp, const R* sU, const R* sW, R* Ufe,
+                                           const Tabs& tb) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
   const int bb = i / F, f = i - bb * F;
   const FpOp<D, P, R, TEN> fp(tb, sW, f);
+  const LineOp<P1, R> line(sU + bb * N * S, [&](int m) { return lp[m]; }, [&](int m) { return fp.ext_w(m); });
+  R* const o = Ufe + (long long)(e0 + bb) * N * F + f;
 #pragma unroll
-  for (int k = 0; k < N; k++) {
-    R acc = 0;
-#pragma unroll
-    for (int m = 0; m < P1; m++) acc += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
-    st_s<NT>(acc, &Ufe[((long long)(e0 + bb) * N + k) * F + f]);
-  }
+  for (int k = 0; k < N; k++) st_s<NT>(line(k * S), &o[k * F]);
 }
 
 // Shapes whose volume kernel is held to 4 waves per SIMD (128 VGPRs): quads
@@ -833,35 +864,43 @@ struct VFace {
   const double* bst;   // boundary-state table
 };
 
-// calcDivF_spts of field k at point s of the block's element b, from the
-// transformed flux in sF: the sum over directions in order (matrix cores: y on
-// the vector unit, then z and x added).
+// calcDivF_spts at point s of the block's element b, from the transformed flux in
+// sF: the sum over directions in order (matrix cores: y on the vector unit, then
+// z and x added).
 template <int D, int P, class R, int np, class Op>
-__device__ __forceinline__ R divergence(const R* sF, int b, int s, int k, int sw, int swx, R opv, bf16x8 abf,
-                                        const Op& po) {
+__device__ __forceinline__ void divergence(const R* sF, int b, int s, int sw, int swx, R opv, bf16x8 abf, const Op& po,
+                                           R* dv) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
   constexpr bool mf = kMfma<D, P, R>;
-  R tot = 0;
+  const R* const f0 = sF + b * D * N * S;
 #pragma unroll
   for (int d = 0; d < D; d++) {
     if (mf && d != 1) continue;
     if constexpr (np != 0) {
       if (d == 2) {
-        tot = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sF + ((b * D + 2) * N + k) * S), s, abf, tot, np);
+#pragma unroll
+        for (int k = 0; k < N; k++)
+          dv[k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(f0 + (2 * N + k) * S), s, abf, dv[k], np);
         continue;
       }
     }
-    R a = 0;
+    const LineOp<P1, R> line(f0 + d * N * S, [&](int m) { return po.grd_idx(d, m); },
+                             [&](int m) { return po.grd_w(d, m); });
 #pragma unroll
-    for (int m = 0; m < P1; m++) a += po.grd_w(d, m) * sF[((b * D + d) * N + k) * S + po.grd_idx(d, m)];
-    tot = (d == 0 || mf) ? a : a + tot;
+    for (int k = 0; k < N; k++) {
+      const R a = line(k * S);
+      dv[k] = (d == 0 || mf) ? a : a + dv[k];
+    }
   }
   if (mf) {
-    tot = mfma444(opv, sF[((b * D + 2) * N + k) * S + sw], tot);
-    tot = mfma444(sF[((b * D + 0) * N + k) * S + swx], opv, tot);
+    const R *const qz = f0 + 2 * N * S + sw, *const qx = f0 + swx;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      dv[k] = mfma444(opv, qz[k * S], dv[k]);
+      dv[k] = mfma444(qx[k * S], opv, dv[k]);
+    }
   }
-  return tot;
 }
 
 // ---------------------------------------------------------------------------
@@ -947,8 +986,12 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   const bool fold = D == 2 && fc.wf;
   // the flux points' side codes first: the partners' addresses come from them
   int cd[KF];
+  Packed<P1> lp[KF];
 #pragma unroll
-  for (int u = 0; u < KF; u++) cd[u] = flx(u) ? fc.fpart[(long long)e0 * F + fi(u)] : 0;
+  for (int u = 0; u < KF; u++) {
+    cd[u] = flx(u) ? fc.fpart[(long long)e0 * F + fi(u)] : 0;
+    lp[u].load(tb, flx(u) ? fi(u) % F : 0);
+  }
   R vu[N];
 #pragma unroll
   for (int u = 0; u < N; u++) {
@@ -1033,9 +1076,11 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
     }
     // flux at the point, transformed to the reference element
     R u[N], Fl[D][N];
+    const R* const qu = sU + b * N * S + sw;
 #pragma unroll
-    for (int k = 0; k < N; k++) u[k] = sU[(b * N + k) * S + sw];
+    for (int k = 0; k < N; k++) u[k] = qu[k * S];
     inviscid_flux<D, R, true>(u, Fl, R(ph.gamma));
+    R* const qf = sF + b * D * N * S + sw;
 #pragma unroll
     for (int d1 = 0; d1 < D; d1++)
 #pragma unroll
@@ -1043,7 +1088,7 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
         R acc = 0;
 #pragma unroll
         for (int d2 = 0; d2 < D; d2++) acc += G[d1][d2] * Fl[d2][k];
-        sF[((b * D + d1) * N + k) * S + sw] = acc;
+        qf[(d1 * N + k) * S] = acc;
       }
   }
   if constexpr (APART) {
@@ -1056,8 +1101,7 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
     if constexpr (!(APART && D == 2)) in = rk_load<D, P, R, NT>(E, e, s, ra);
     if (fold) in.dt = dtl;
     const PtOp<D, P, R, TEN> po(tb, sW, s);
-#pragma unroll
-    for (int k = 0; k < N; k++) dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po);
+    divergence<D, P, R, np>(sF, b, s, sw, swx, opv, abf, po, dv);
   }
 #pragma unroll
   for (int u = 0; u < KF; u++)
@@ -1067,14 +1111,11 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
       // non-zero)
       const int bb = fi(u) / F, f = fi(u) - bb * F;
       const FpOp<D, P, R, TEN> fp(tb, sW, f);
-      const int dn = fp.dir();
+      const LineOp<P1, R> line(sF + (bb * D + fp.dir()) * N * S, [&](int m) { return lp[u][m]; },
+                               [&](int m) { return fp.efn_w(m); });
+      R* const o = sD + bb * N * F + f;
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
-        sD[(bb * N + k) * F + f] = fo[u][k] - fp.efn_sign(a);
-      }
+      for (int k = 0; k < N; k++) o[k * F] = fo[u][k] - fp.efn_sign(line(k * S));
     }
   __syncthreads();
   if (act) rk_point<D, P, R, NT, TEN>(E, e, b, s, dv, sU, sD, sW, in, ra, tb);
@@ -1082,7 +1123,7 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < KF; u++)
-    if (flx(u)) face_point<D, P, R, NT, TEN>(fi(u), e0, sU, sW, ra.Ufe, tb);
+    if (flx(u)) face_point<D, P, R, NT, TEN>(fi(u), e0, lp[u], sU, sW, ra.Ufe, tb);
 }
 
 // Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
@@ -1185,14 +1226,22 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   // overlap; the flux points' side codes first: the partners' addresses come
   // from them
   int cd[KF];
+  Packed<P1> lp[KF];
 #pragma unroll
-  for (int u = 0; u < KF; u++) cd[u] = fi(u) < nP ? vf.fpart[(long long)e0 * F + fi(u)] : 0;
-  const int nU = nb * N * S;
+  for (int u = 0; u < KF; u++) {
+    cd[u] = fi(u) < nP ? vf.fpart[(long long)e0 * F + fi(u)] : 0;
+    lp[u].load(tb, fi(u) < nP ? fi(u) % F : 0);
+  }
   R vu[N];
+  if (act) {
+    const long long at = e * N * S + s;
+    if (Us) {
 #pragma unroll
-  for (int u = 0; u < N; u++) {
-    const int i = threadIdx.x + u * blockDim.x;
-    if (i < nU) vu[u] = Us ? ld_s<NT>(&Us[(long long)e0 * N * S + i]) : R(ld_s<NT>(&Ue[(long long)e0 * N * S + i]));
+      for (int k = 0; k < N; k++) vu[k] = ld_s<NT>(&Us[at + k * S]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; k++) vu[k] = R(ld_s<NT>(&Ue[at + k * S]));
+    }
   }
   // U across and the normal
   R fn[KF][N], nv[KF][D];
@@ -1222,55 +1271,75 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     load_G();
     inv = iJe[e * S + s];
   }
+  if (act) {
+    R* const q = sU + b * N * S + sw;
 #pragma unroll
-  for (int u = 0; u < N; u++) {
-    const int i = threadIdx.x + u * blockDim.x;
-    if (i < nU) {
-      const int r = i / S, q = i - r * S;
-      sU[r * S + spt_lds(D, P1, q)] = vu[u];
-    }
+    for (int k = 0; k < N; k++) q[k * S] = vu[k];
   }
   __syncthreads();
-  // U at flux point f of the block's element bb (the RK kernel's sums and bits)
-  auto u_face = [&](int bb, const FpOp<D, P, R, TEN>& fp, R* own) {
+  // U at flux point u, of the block's element bb (the RK kernel's sums and bits)
+  auto u_face = [&](int u, int bb, const FpOp<D, P, R, TEN>& fp, R* own) {
+    const LineOp<P1, R> line(sU + bb * N * S, [&](int m) { return lp[u][m]; }, [&](int m) { return fp.ext_w(m); });
 #pragma unroll
     for (int k = 0; k < N; k++) {
-      R a = 0;
-#pragma unroll
-      for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sU[(bb * N + k) * S + fp.idx(m)];
-      own[k] = a;
+      own[k] = line(k * S);
       pin(own[k]);
     }
   };
   // the common inviscid flux (FP64: with the LDG penalty on the states, which
-  // FP32 leaves in the two sides' parts), and the common U less U, from U on both sides (in the left side's order on either)
+  // FP32 leaves in the two sides' parts), and the common U less U,
+  // from U on both sides; the flux outward
 #pragma unroll
   for (int u = 0; u < KF; u++)
     if (fi(u) < nP) {
       const int i = fresh(fi(u)), bb = i / F, f = i - bb * F, side = cd[u] & 3;
       const FpOp<D, P, R, TEN> fp(tb, sW, f);
       const bool right = side == 1, bnd = BND && side == 2;
-      R own[N], UL[N], UR[N];
-      u_face(bb, fp, own);
+      R own[N];
+      u_face(u, bb, fp, own);
       if constexpr (BND) {
         if (bnd) bc_state<D, R>(vf.bndBc[cd[u] >> 2], own, nv[u], fn[u], ph, vf.bst);
       }
-#pragma unroll
-      for (int k = 0; k < N; k++) {
-        UL[k] = right ? fn[u][k] : own[k];
-        UR[k] = right ? own[k] : fn[u][k];
-      }
       double lam;
-      if (pair_flux<D, R>(bnd, UL, UR, nv[u], fn[u], ph, lam) && vf.wave && !right)
-        st_s<NT>(lam, &vf.wave[(long long)e0 * F + i]);
-      const R pf = bnd ? R(0) : ldg_pen<D, R>(nv[u], R(ph.pen_fact));
+      bool has_lam;
+      R pf = bnd ? R(0) : ldg_pen<D, R>(nv[u], R(ph.pen_fact));
       const R tn = bnd || kJumpOut<R> ? R(0) : ldg_tau<D, R>(nv[u], R(ph.tau));
+      R* const qc = sC + bb * N * F + f;
+      R fc[N];
+      if constexpr (D == 3) {
+        // from this side: its state first and the normal outward.  Rusanov's flux
+        // from the other side is the same bits with the sign turned
+        R no[D];
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        const R uc = bnd ? R(0.5) * (UL[k] + UR[k]) : R(0.5) * (UL[k] + UR[k]) - pf * (UL[k] - UR[k]);
-        sC[(bb * N + k) * F + f] = uc - own[k];
-        if constexpr (!kJumpOut<R>) fn[u][k] += tn * (UL[k] - UR[k]);
+        for (int x = 0; x < D; x++) no[x] = right ? -nv[u][x] : nv[u][x];
+        if (right) pf = -pf;
+        has_lam = pair_flux<D, R>(bnd, own, fn[u], no, fc, ph, lam);
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          const R du = own[k] - fn[u][k], mid = R(0.5) * (own[k] + fn[u][k]);
+          qc[k * F] = (bnd ? mid : mid - pf * du) - own[k];
+          if constexpr (!kJumpOut<R>) fc[k] += tn * du;
+          fn[u][k] = fc[k];
+        }
+      } else {
+        R UL[N], UR[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          UL[k] = right ? fn[u][k] : own[k];
+          UR[k] = right ? own[k] : fn[u][k];
+        }
+        has_lam = pair_flux<D, R>(bnd, UL, UR, nv[u], fc, ph, lam);
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          const R du = UL[k] - UR[k], mid = R(0.5) * (UL[k] + UR[k]);
+          qc[k * F] = (bnd ? mid : mid - pf * du) - own[k];
+          if constexpr (!kJumpOut<R>) fc[k] += tn * du;
+          fn[u][k] = right ? -fc[k] : fc[k];
+        }
       }
+      if (has_lam && vf.wave && !right) st_s<NT>(lam, &vf.wave[(long long)e0 * F + i]);
+#pragma unroll
+      for (int k = 0; k < N; k++) pin(fn[u][k]);
     }
   __syncthreads();
   // phase 1: reference-space gradient (opp_grad_spts) plus correction
@@ -1279,30 +1348,29 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   R gr[D][N];
   if (act) {
     const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
+    const R *const qu = sU + b * N * S, *const qc = sC + b * N * F;
 #pragma unroll
     for (int d = 0; d < D; d++) {
+      // the other correction entries of the row are exactly zero
+      const LineOp<2, R> cor(qc, [&](int j) { return po.cu_idx(d, j); }, [&](int j) { return po.cu_w(d, j); });
+      if constexpr (np != 0) {
+        if (d == 2) {
 #pragma unroll
-      for (int k = 0; k < N; k++) {
-        // the other correction entries of the row are exactly zero
-        R c = 0;
-#pragma unroll
-        for (int j = 0; j < 2; j++) c += po.cu_w(d, j) * sC[(b * N + k) * F + po.cu_idx(d, j)];
-        if constexpr (np != 0) {
-          if (d == 2) {
-            gr[d][k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(sU + (b * N + k) * S), s, abf, c, np);
-            continue;
-          }
-        }
-        if (mf && d != 1) {  // compile-time: d and mf are constants here
-          gr[d][k] = d == 2 ? mfma444(opv, sU[(b * N + k) * S + sw], c)
-                            : mfma444(sU[(b * N + k) * S + swx], opv, c);
+          for (int k = 0; k < N; k++)
+            gr[d][k] = mfma_z_bf16<D, P1>(reinterpret_cast<const float*>(qu + k * S), s, abf, cor(k * F), np);
           continue;
         }
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += po.grd_w(d, m) * sU[(b * N + k) * S + po.grd_idx(d, m)];
-        gr[d][k] = c + a;
       }
+      if (mf && d != 1) {  // compile-time: d and mf are constants here
+        const R* const q = qu + (d == 2 ? sw : swx);
+#pragma unroll
+        for (int k = 0; k < N; k++)
+          gr[d][k] = d == 2 ? mfma444(opv, q[k * S], cor(k * F)) : mfma444(q[k * S], opv, cor(k * F));
+        continue;
+      }
+      const LineOp<P1, R> line(qu, [&](int m) { return po.grd_idx(d, m); }, [&](int m) { return po.grd_w(d, m); });
+#pragma unroll
+      for (int k = 0; k < N; k++) gr[d][k] = cor(k * F) + line(k * S);
     }
     // physical gradient, in place
 #pragma unroll
@@ -1318,11 +1386,12 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     }
   }
   __syncthreads();  // sC is overwritten by the gradient below
+  R* const qg = sG + b * D * N * S + sw;
   if (act) {
 #pragma unroll
     for (int k = 0; k < N; k++)
 #pragma unroll
-      for (int x = 0; x < D; x++) sG[((b * D + x) * N + k) * S + sw] = gr[x][k];
+      for (int x = 0; x < D; x++) qg[(x * N + k) * S] = gr[x][k];
   }
   __syncthreads();
   // physical gradient at the flux points (extrapolateGradU) and, with U there,
@@ -1339,19 +1408,20 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
       const FpOp<D, P, R, TEN> fp(tb, sW, f);
       dA = ld_s<NT>(&vf.dA[(long long)e0 * F + i]);
       R g[D][N];
+      {
+        const LineOp<P1, R> line(sG + bb * D * N * S, [&](int m) { return lp[u][m]; },
+                                 [&](int m) { return fp.ext_w(m); });
 #pragma unroll
-      for (int x = 0; x < D; x++) {
+        for (int x = 0; x < D; x++) {
 #pragma unroll
-        for (int k = 0; k < N; k++) {
-          R a = 0;
-#pragma unroll
-          for (int m = 0; m < P1; m++) a += fp.ext_w(m) * sG[((bb * D + x) * N + k) * S + fp.idx(m)];
-          g[x][k] = a;
-          pin(g[x][k]);
+          for (int k = 0; k < N; k++) {
+            g[x][k] = line((x * N + k) * S);
+            pin(g[x][k]);
+          }
         }
       }
       R own[N], bv[N];
-      u_face(bb, fp, own);
+      u_face(u, bb, fp, own);
       if (BND && side == 2) {
         R UR[N], nF[N], d12[N];
         const int bc = vf.bndBc[cd[u] >> 2];
@@ -1370,14 +1440,15 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
         } else {
           ldg_part<D, R>(side == 0, own, g, nv[u], bv, ph);
         }
+        R* const o = vf.Bve + (long long)(e0 + bb) * N * F + f;
 #pragma unroll
-        for (int k = 0; k < N; k++) st_s<NT>(bv[k], &vf.Bve[((long long)(e0 + bb) * N + k) * F + f]);
+        for (int k = 0; k < N; k++) st_s<NT>(bv[k], &o[k * F]);
       }
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const R v = kJumpOut<R> ? mul_rn(fn[u][k], dA) : (fn[u][k] + bv[k]) * dA;
-        fn[u][k] = side == 1 ? -v : v;
-        if constexpr (kJumpOut<R>) bo[u][k] = side == 1 ? -bv[k] : bv[k];
+        const R bs = side == 1 ? -bv[k] : bv[k];
+        fn[u][k] = kJumpOut<R> ? mul_rn(fn[u][k], dA) : (fn[u][k] + bs) * dA;
+        if constexpr (kJumpOut<R>) bo[u][k] = bs;
       }
     }
   // under the register hold, the metric terms again (from cache): keeping
@@ -1391,15 +1462,16 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   // fewer face points go on here meanwhile.
   R Ft[D][N];
   if (act) {
+    const R* const qs = sU + b * N * S + sw;
     R u[N];
 #pragma unroll
-    for (int k = 0; k < N; k++) u[k] = sU[(b * N + k) * S + sw];
+    for (int k = 0; k < N; k++) u[k] = qs[k * S];
     R Fl[D][N];
     R g[D][N];
 #pragma unroll
     for (int x = 0; x < D; x++)
 #pragma unroll
-      for (int k = 0; k < N; k++) g[x][k] = sG[((b * D + x) * N + k) * S + sw];
+      for (int k = 0; k < N; k++) g[x][k] = qg[(x * N + k) * S];
     R Fi[D][N];
     viscous_flux<D, R>(u, g, Fl, ph);
     inviscid_flux<D, R>(u, Fi, R(ph.gamma));
@@ -1422,16 +1494,16 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
 #pragma unroll
     for (int d1 = 0; d1 < D; d1++)
 #pragma unroll
-      for (int k = 0; k < N; k++) sF[((b * D + d1) * N + k) * S + sw] = Ft[d1][k];
+      for (int k = 0; k < N; k++) qg[(d1 * N + k) * S] = Ft[d1][k];
   }
   __syncthreads();
   R dv[N];
   if (act) {
     const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
+    divergence<D, P, R, np>(sF, b, s, sw, swx, opv, abf, po, dv);
+    if constexpr (kJumpOut<R>) {
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      dv[k] = divergence<D, P, R, np>(sF, b, s, k, sw, swx, opv, abf, po);
-      if constexpr (kJumpOut<R>) st_s<NT>(dv[k], &divFe[(e * N + k) * S + s]);
+      for (int k = 0; k < N; k++) st_s<NT>(dv[k], &divFe[e * N * S + s + k * S]);
     }
   }
   // faces: the flux jump, less the other side's part (extrapolateNormalFlux: of
@@ -1441,14 +1513,12 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
     if (fi(u) < nP) {
       const int i = fresh(fi(u)), bb = i / F, f = i - bb * F;
       const FpOp<D, P, R, TEN> fp(tb, sW, f);
-      const int dn = fp.dir();
+      const LineOp<P1, R> line(sF + (bb * D + fp.dir()) * N * S, [&](int m) { return lp[u][m]; },
+                               [&](int m) { return fp.efn_w(m); });
       const R dJ = kJumpOut<R> ? (KF == 1 ? dA : vf.dA[(long long)e0 * F + i]) : R(0);
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        R a = 0;
-#pragma unroll
-        for (int m = 0; m < P1; m++) a += fp.efn_w(m) * sF[((bb * D + dn) * N + k) * S + fp.idx(m)];
-        a = fp.efn_sign(a);
+        const R a = fp.efn_sign(line(k * S));
         if constexpr (kJumpOut<R>) {
           const R j = bo[u][k] * dJ - a;
           st_s<NT>(fn[u][k] + j, &vf.Jne[((long long)(e0 + bb) * N + k) * F + f]);
@@ -1472,9 +1542,9 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   __syncthreads();
   if (act) {
     const PtOp<D, P, R, TEN> po(tb, sW, fresh(s));
+    correction<D, P, R>(sD, b, po, dv, dv);
 #pragma unroll
-    for (int k = 0; k < N; k++)
-      st_s<NT>(correction<D, P, R>(sD, b, k, po) + dv[k], &divFe[(e * N + k) * S + s]);
+    for (int k = 0; k < N; k++) st_s<NT>(dv[k], &divFe[e * N * S + s + k * S]);
   }
 }
 
@@ -1518,10 +1588,12 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   // latencies overlap.  A thread stages at most KF = ceil(F / S) points.
   constexpr int KF = (F + S - 1) / S;
   int cd[KF];
+  Packed<P + 1> lp[KF];
 #pragma unroll
   for (int u = 0; u < KF; u++) {
     const int i = threadIdx.x + u * blockDim.x;
     cd[u] = (i < nb * F) ? fpart[(long long)e0 * F + i] : 2;
+    lp[u].load(tb, (i < nb * F) ? i % F : 0);
   }
 #pragma unroll
   for (int u = 0; u < KF; u++) {
@@ -1553,7 +1625,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   }
   if (ra.mode == 5 || ra.mode == 7 || ra.mode == 8) return;  // uniform over the launch
   __syncthreads();
-  for (int i = threadIdx.x; i < nb * F; i += blockDim.x) face_point<D, P, R, NT, TEN>(i, e0, sU, sW, ra.Ufe, tb);
+#pragma unroll
+  for (int u = 0; u < KF; u++) {
+    const int i = threadIdx.x + u * blockDim.x;
+    if (i < nb * F) face_point<D, P, R, NT, TEN>(i, e0, lp[u], sU, sW, ra.Ufe, tb);
+  }
 }
 
 template <class R>
@@ -1876,12 +1952,14 @@ static bool build_d1(const Ctx& c, const fhip_desc* dsc, std::vector<double>& d1
 // The 1-D factors (Ten) of the dense operators, or false where an entry of one
 // of them is not what the factors give.
 template <int D, int P>
-static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w) {
+static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w,
+                      std::vector<int>& line) {
   using T = Ten<D, P>;
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, P1 = Sh::P1;
   w.assign(T::NW, 0.);
   std::copy(d1.begin(), d1.end(), w.begin());
+  std::vector<int> at((size_t)F * P1);
   // l and c from the first point of a face on each end of direction 0
   for (int j = 0; j < 2 * D; j++) {
     if (T::face_dir(j) != 0) continue;
@@ -1898,6 +1976,7 @@ static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double
     const typename T::Face face(f);
     const int j = f / Sh::Ff;
     if (face.dn != T::face_dir(j) || face.hi != T::face_hi(j)) return false;
+    for (int m = 0; m < P1; m++) at[(size_t)f * P1 + m] = face.at(m);
     for (int q = 0; q < S; q++) {
       const typename T::Point p(q);
       bool on = true;
@@ -1912,23 +1991,25 @@ static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double
       }
     }
   }
+  line = at;
   return true;
 }
 
-static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w) {
+static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double>& d1, std::vector<double>& w,
+                      std::vector<int>& line) {
   switch (c.z.D * 10 + c.z.P) {
-    case 20: return build_ten<2, 0>(c, d, d1, w);
-    case 21: return build_ten<2, 1>(c, d, d1, w);
-    case 22: return build_ten<2, 2>(c, d, d1, w);
-    case 23: return build_ten<2, 3>(c, d, d1, w);
-    case 24: return build_ten<2, 4>(c, d, d1, w);
-    case 25: return build_ten<2, 5>(c, d, d1, w);
-    case 30: return build_ten<3, 0>(c, d, d1, w);
-    case 31: return build_ten<3, 1>(c, d, d1, w);
-    case 32: return build_ten<3, 2>(c, d, d1, w);
-    case 33: return build_ten<3, 3>(c, d, d1, w);
-    case 34: return build_ten<3, 4>(c, d, d1, w);
-    default: return build_ten<3, 5>(c, d, d1, w);
+    case 20: return build_ten<2, 0>(c, d, d1, w, line);
+    case 21: return build_ten<2, 1>(c, d, d1, w, line);
+    case 22: return build_ten<2, 2>(c, d, d1, w, line);
+    case 23: return build_ten<2, 3>(c, d, d1, w, line);
+    case 24: return build_ten<2, 4>(c, d, d1, w, line);
+    case 25: return build_ten<2, 5>(c, d, d1, w, line);
+    case 30: return build_ten<3, 0>(c, d, d1, w, line);
+    case 31: return build_ten<3, 1>(c, d, d1, w, line);
+    case 32: return build_ten<3, 2>(c, d, d1, w, line);
+    case 33: return build_ten<3, 3>(c, d, d1, w, line);
+    case 34: return build_ten<3, 4>(c, d, d1, w, line);
+    default: return build_ten<3, 5>(c, d, d1, w, line);
   }
 }
 
@@ -2003,7 +2084,6 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
     std::memcpy(blob.data() + o, p, bytes);
   };
   blob.clear();
-  put(ext_idx.data(), ext_idx.size() * 4, off[0]);
   put(ext_w.data(), ext_w.size() * 8, off[1]);
   put(efn_dir.data(), efn_dir.size() * 4, off[2]);
   put(efn_w.data(), efn_w.size() * 8, off[3]);
@@ -2025,17 +2105,23 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
   // the matrix-core path of FP64 P3 hexes needs the 1-D derivative matrix
   std::vector<double> d1;
   off[15] = off[16] = off[17] = off[18] = 0;
+  std::vector<int> line = ext_idx;  // with the factors: by depth, zero weights included
   if (build_d1(c, d, d1)) {
     put(d1.data(), d1.size() * 8, off[15]);
     putf(d1, off[16]);
     std::vector<double> w;
-    if (build_ten(c, d, d1, w)) {
+    if (build_ten(c, d, d1, w, line)) {
       put(w.data(), w.size() * 8, off[17]);
       putf(w, off[18]);
     }
   } else if (D == 3 && P1 == 4) {
     return false;
   }
+  const int W = (P1 + 3) / 4;
+  std::vector<unsigned> packed((size_t)F * W, 0u);
+  for (int f = 0; f < F; f++)
+    for (int m = 0; m < P1; m++) packed[(size_t)f * W + m / 4] |= (unsigned)line[(size_t)f * P1 + m] << (8 * (m % 4));
+  put(packed.data(), packed.size() * 4, off[0]);
   return true;
 }
 
@@ -2111,13 +2197,14 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
   st->tab_mem = dal<char>(blob.size());
   FCHK(hipMemcpy(st->tab_mem, blob.data(), blob.size(), hipMemcpyHostToDevice));
   char* base = (char*)st->tab_mem;
-  st->tb = Tabs{(const int*)(base + off[0]),    (const double*)(base + off[1]), (const int*)(base + off[2]),
+  st->tb = Tabs{(const double*)(base + off[1]), (const int*)(base + off[2]),
                 (const double*)(base + off[3]), (const int*)(base + off[4]),    (const double*)(base + off[5]),
                 (const int*)(base + off[6]),    (const double*)(base + off[7]), (const int*)(base + off[8]),
                 (const double*)(base + off[9]), (const float*)(base + off[10]), (const float*)(base + off[11]),
                 (const float*)(base + off[12]), (const float*)(base + off[13]), (const float*)(base + off[14]),
                 off[15] ? (const double*)(base + off[15]) : nullptr, off[16] ? (const float*)(base + off[16]) : nullptr,
-                off[17] ? (const double*)(base + off[17]) : nullptr, off[18] ? (const float*)(base + off[18]) : nullptr};
+                off[17] ? (const double*)(base + off[17]) : nullptr, off[18] ? (const float*)(base + off[18]) : nullptr,
+                (const unsigned*)(base + off[0])};
   const long long E = z.E, S = z.S, F = z.F, N = z.N, D = z.D;
   st->stream = E * N * S * (long long)sizeof(double) > kStreamBytes;
   st->Ue = dal<double>(E * N * S);
