@@ -237,9 +237,21 @@ int fhip_create(const fhip_desc* d, fhip_ctx** out) {
           }
         }
       }
-      c.ft.ptL = dcopy(c.h_ptL.data(), c.h_ptL.size(), c.stream);
-      c.ft.ptR = dcopy(c.h_ptR.data(), c.h_ptR.size(), c.stream);
-      c.ft.bc = dcopy(bc.data(), bc.size(), c.stream);
+      // the staged face kernels' order: by left point (fpt*E + ele), so that the
+      // lanes of a wave take one flux point of consecutive elements and their
+      // rows of every array are neighbours.  In the faces' order each lane's 40
+      // bytes lie E rows from the next lane's.
+      std::vector<int> at((size_t)F * E, -1), sl, sr, sb;
+      for (int t = 0; t < z.nFaceFpts; t++) at[c.h_ptL[t]] = t;
+      for (int t : at)
+        if (t >= 0) {
+          sl.push_back(c.h_ptL[t]);
+          sr.push_back(c.h_ptR[t]);
+          sb.push_back(bc[t]);
+        }
+      c.ft.ptL = dcopy(sl.data(), sl.size(), c.stream);
+      c.ft.ptR = dcopy(sr.data(), sr.size(), c.stream);
+      c.ft.bc = dcopy(sb.data(), sb.size(), c.stream);
 
       const size_t nS = z.nS(), nF = z.nF();
       c.U = dcopy<double>(nullptr, nS, c.stream);

@@ -74,13 +74,18 @@ static void opgemm(Ctx& c, const char* name, int m, int k, const double* A, cons
 // mesh of 18^3 P3 hexes launches 114 blocks on 256 CUs.  The row is uniform
 // over the wave, so entries come through scalar loads.  Measured on 18^3 P3
 // hexes (29,160 columns): the products of one Navier-Stokes residual took 5.99
-// ms dense (17 launches) and take 0.148 ms this way (7 launches).
+// ms dense (17 launches) and took 0.148 ms this way (7 launches).  Two further
+// forms save an array's way through memory: the result subtracted from another
+// array (from; the flux jump), and a second operator's product added to it (q2
+// entries per row of idx2, w2 over B2; the divergence's correction).
 constexpr int kRowsPerWave = 8;
 template <int Q>
 __global__ __launch_bounds__(256) void k_oprows(int m, long long n, int groups, const int* __restrict__ idx,
                                                  const double* __restrict__ w, const double* __restrict__ B,
                                                  long long strideB, double* __restrict__ C, long long strideC,
-                                                 int beta) {
+                                                 int beta, const double* __restrict__ from, int q2,
+                                                 const int* __restrict__ idx2, const double* __restrict__ w2,
+                                                 const double* __restrict__ B2) {
   const long long j = (long long)blockIdx.x * 64 + (threadIdx.x & 63);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (j >= n) return;
@@ -100,8 +105,14 @@ __global__ __launch_bounds__(256) void k_oprows(int m, long long n, int groups, 
       for (int q = 0; q < Q; q++) s += wt[q] * B[ix[q] * n];
       tot = g ? s + tot : s;
     }
+    if (q2) {
+      double s = 0.0;
+#pragma unroll 2
+      for (int q = 0; q < q2; q++) s += w2[(long long)i * q2 + q] * B2[idx2[(long long)i * q2 + q] * n + j];
+      tot = s + tot;
+    }
     double* cp = C + i * n;
-    *cp = beta ? tot + *cp : tot;
+    *cp = from ? from[i * n + j] - tot : (beta ? tot + *cp : tot);
   }
 }
 
@@ -170,12 +181,13 @@ void staged_release(Ctx& c) {
 
 // op applied to `count` operands strideB apart, into outputs strideC apart.
 static void oprows(Ctx& c, const char* name, const RowOp& op, const double* B, double* C, bool beta, int count = 1,
-                   long long strideB = 0, long long strideC = 0) {
+                   long long strideB = 0, long long strideC = 0, const double* from = nullptr,
+                   const RowOp* op2 = nullptr, const double* B2 = nullptr) {
   const long long n = (long long)c.z.E * c.z.N;
   const dim3 grid(blocks_for(n, 64), blocks_for(op.m, 4 * kRowsPerWave), count);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(256), 0, c.stream, op.m, n, op.groups, op.idx, op.w, B, strideB, C, strideC,
-                       beta ? 1 : 0);
+                       beta ? 1 : 0, from, op2 ? op2->q : 0, op2 ? op2->idx : nullptr, op2 ? op2->w : nullptr, B2);
   };
   Launch L(c, name);
   switch (op.q) {
@@ -191,11 +203,11 @@ static void oprows(Ctx& c, const char* name, const RowOp& op, const double* B, d
 }
 
 // ---------------------------------------------------------------------------
-// calcInviscidFlux_spts (src/solver.cpp:707-736): one thread per (spt, ele).
+// calcInviscidFlux_spts (src/solver.cpp:707-736): one thread per (spt, ele); the
+// transform follows with the viscous flux.
 template <int D>
 __global__ __launch_bounds__(256) void k_inviscid_spts(long long nPts, long long SE, const double* __restrict__ U,
-                                                        const double* __restrict__ JG, double* __restrict__ Fs,
-                                                        double gamma, int transform) {
+                                                        double* __restrict__ Fs, double gamma) {
   constexpr int N = D + 2;
   long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nPts) return;
@@ -203,27 +215,10 @@ __global__ __launch_bounds__(256) void k_inviscid_spts(long long nPts, long long
 #pragma unroll
   for (int k = 0; k < N; k++) u[k] = U[p * N + k];
   inviscid_flux<D, double>(u, F, gamma);
-  if (!transform) {
 #pragma unroll
-    for (int d = 0; d < D; d++)
+  for (int d = 0; d < D; d++)
 #pragma unroll
-      for (int k = 0; k < N; k++) Fs[(d * SE + p) * N + k] = F[d][k];
-    return;
-  }
-  double G[D][D];
-#pragma unroll
-  for (int d1 = 0; d1 < D; d1++)
-#pragma unroll
-    for (int d2 = 0; d2 < D; d2++) G[d1][d2] = JG[(d1 * SE + p) * D + d2];
-#pragma unroll
-  for (int d1 = 0; d1 < D; d1++)
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-      double acc = 0.;
-#pragma unroll
-      for (int d2 = 0; d2 < D; d2++) acc += G[d1][d2] * F[d2][k];
-      Fs[(d1 * SE + p) * N + k] = acc;
-    }
+    for (int k = 0; k < N; k++) Fs[(d * SE + p) * N + k] = F[d][k];
 }
 
 // ---------------------------------------------------------------------------
@@ -254,13 +249,11 @@ __global__ __launch_bounds__(256) void k_face_inviscid(int nFF, const int* __res
   else {
     if constexpr (D == 2) roe2d<double>(UL, UR, n, fn, ph.gamma);
   }
-  double dAL = dA[pl];
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    faceFn[(long long)t * N + k] = fn[k];
-    Fn[(long long)pl * N + k] = fn[k] * dAL;
-  }
+  // (viscous runs: the viscous face pass, which follows, adds to faceFn and
+  // writes Fn)
   if (ph.viscous) {
+#pragma unroll
+    for (int k = 0; k < N; k++) faceFn[(long long)t * N + k] = fn[k];
     double pf = (pr < 0) ? 0.0 : ldg_pen<D, double>(n, ph.pen_fact);
 #pragma unroll
     for (int k = 0; k < N; k++) {
@@ -268,7 +261,11 @@ __global__ __launch_bounds__(256) void k_face_inviscid(int nFF, const int* __res
       dUc[(long long)pl * N + k] = uc - UL[k];
       if (pr >= 0) dUc[(long long)pr * N + k] = uc - UR[k];
     }
+    return;
   }
+  double dAL = dA[pl];
+#pragma unroll
+  for (int k = 0; k < N; k++) Fn[(long long)pl * N + k] = fn[k] * dAL;
   if (pr >= 0) {
     double dAR = dA[pr];
 #pragma unroll
@@ -331,6 +328,124 @@ __global__ __launch_bounds__(256) void k_viscous_spts(long long nPts, long long 
 #pragma unroll
       for (int d2 = 0; d2 < D; d2++) acc += JG[(d1 * SE + p) * D + d2] * Fv[d2][k];
       Fs[(d1 * SE + p) * N + k] = acc;
+    }
+}
+
+// All pointwise work between the operators in one kernel, for operators of rows
+// with at most 6 entries (2 in the gradient's correction): gradient, its
+// correction (opp_correctU) and physical transform (viscous runs), inviscid and
+// viscous flux, transformed flux; the sums are those of k_oprows, k_grad_transform,
+// k_inviscid_spts and k_viscous_spts, in their order.  Those kernels moved the
+// gradient and the flux of every point through memory seven times.
+//
+// A wave takes one solution point of 64 elements, as 64 * N contiguous columns for
+// the operators and for every load and store of fields, and as 64 points for the
+// physics, with its part of LDS between the two: a thread per point that reads and
+// writes its fields itself touches a 40-byte stride with each access, which took
+// as long as the bytes again.  18^3 P3 hexes: 132 us in five kernels, now 50 us.
+template <int D, int Q, bool VISC>
+__global__ __launch_bounds__(256) void k_point_flux(int S, int E, const int* __restrict__ gi,
+                                                     const double* __restrict__ gw, const int* __restrict__ ci,
+                                                     const double* __restrict__ cw, const double* __restrict__ U,
+                                                     const double* __restrict__ dUc, const double* __restrict__ JG,
+                                                     const double* __restrict__ detj, double* __restrict__ dU,
+                                                     double* __restrict__ Fs, Phys ph) {
+  constexpr int N = D + 2, C = 64 * N;
+  __shared__ double lds[4][(D + 1) * C];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = blockIdx.y * 4 + wave, e0 = blockIdx.x * 64;
+  const int ne = s < S ? min(64, E - e0) : 0, nc = ne * N;  // elements and columns of this wave
+  const long long n = (long long)E * N, j0 = (long long)e0 * N, SE = (long long)S * E;
+  double* const su = lds[wave];      // [64][N] U
+  double* const sv = su + C;         // [D][64][N] gradient, then flux
+#pragma unroll
+  for (int t = 0; t < N; t++) {
+    const int c = t * 64 + lane;
+    if (c < nc) {
+      const double* const u = U + j0 + c;
+      su[c] = u[s * n];
+      if constexpr (VISC) {
+        const double* const uc = dUc + j0 + c;
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          const int i = d * S + s;
+          double g = 0.0, a = 0.0;
+#pragma unroll
+          for (int q = 0; q < Q; q++) g += gw[i * Q + q] * u[gi[i * Q + q] * n];
+#pragma unroll
+          for (int q = 0; q < 2; q++) a += cw[i * 2 + q] * uc[ci[i * 2 + q] * n];
+          sv[d * C + c] = a + g;
+        }
+      }
+    }
+  }
+  const long long p = (long long)s * E + e0 + lane;
+  double G[D][D];
+  if (lane < ne) {
+#pragma unroll
+    for (int r = 0; r < D; r++)
+#pragma unroll
+      for (int x = 0; x < D; x++) G[r][x] = JG[(r * SE + p) * D + x];
+  }
+  __syncthreads();
+  double g[D][N];
+  if constexpr (VISC) {
+    if (lane < ne) {
+      const double inv = 1. / detj[p];
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        double r[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) r[d] = sv[d * C + lane * N + k];
+#pragma unroll
+        for (int x = 0; x < D; x++) {
+          double acc = r[0] * G[0][x] + r[1] * G[1][x];
+          if constexpr (D == 3) acc += r[2] * G[2][x];
+          g[x][k] = inv * acc;
+          sv[x * C + lane * N + k] = g[x][k];
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < D; d++)
+#pragma unroll
+      for (int t = 0; t < N; t++) {
+        const int c = t * 64 + lane;
+        if (c < nc) dU[((long long)d * S + s) * n + j0 + c] = sv[d * C + c];
+      }
+    __syncthreads();
+  }
+  if (lane < ne) {
+    double u[N], F[D][N];
+#pragma unroll
+    for (int k = 0; k < N; k++) u[k] = su[lane * N + k];
+    inviscid_flux<D, double>(u, F, ph.gamma);
+    if constexpr (VISC) {
+      double Fv[D][N];
+      viscous_flux<D, double>(u, g, Fv, ph);
+#pragma unroll
+      for (int d = 0; d < D; d++)
+#pragma unroll
+        for (int k = 0; k < N; k++) F[d][k] = Fv[d][k] + F[d][k];
+    }
+#pragma unroll
+    for (int d1 = 0; d1 < D; d1++)
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        double acc = 0.;
+#pragma unroll
+        for (int d2 = 0; d2 < D; d2++) acc += G[d1][d2] * F[d2][k];
+        sv[d1 * C + lane * N + k] = acc;
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < D; d++)
+#pragma unroll
+    for (int t = 0; t < N; t++) {
+      const int c = t * 64 + lane;
+      if (c < nc) Fs[((long long)d * S + s) * n + j0 + c] = sv[d * C + c];
     }
 }
 
@@ -402,22 +517,23 @@ __global__ void k_copy(long long n, double* __restrict__ dst, const double* __re
   if (i < n) dst[i] = src[i];
 }
 
-// timeStepA / timeStepB (src/solver.cpp:470-536); dt from device memory.
-__global__ __launch_bounds__(256) void k_time_step(long long nPts, int N, long long E, int modeB, double rk,
+// timeStepA / timeStepB (src/solver.cpp:470-536); dt from device memory.  A thread
+// per value: one per point, each access at a stride of 40 bytes, took 24 us on
+// 18^3 P3 hexes where this takes 11 us.
+template <int N>
+__global__ __launch_bounds__(256) void k_time_step(long long n, unsigned E, int modeB, double rk,
                                                     double* __restrict__ U, const double* __restrict__ U0,
                                                     const double* __restrict__ divF, const double* __restrict__ src,
                                                     const double* __restrict__ detj, const double* __restrict__ dtp,
                                                     const double* __restrict__ eleDt, int local) {
-  long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nPts) return;
-  double dt = local ? eleDt[p % E] : *dtp;
-  double dj = detj[p];
-  for (int k = 0; k < N; k++) {
-    long long i = p * N + k;
-    double r = src ? (divF[i] + src[i]) : divF[i];
-    if (modeB) U[i] -= rk * r / dj * dt;
-    else U[i] = U0[i] - rk * r / dj * dt;
-  }
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const long long p = i / N;
+  const double dt = local ? eleDt[p % E] : *dtp;
+  const double dj = detj[p];
+  const double r = src ? (divF[i] + src[i]) : divF[i];
+  if (modeB) U[i] -= rk * r / dj * dt;
+  else U[i] = U0[i] - rk * r / dj * dt;
 }
 
 // calcWaveSpFpts for every element (src/ele.cpp:1097-1124).  waveSp is
@@ -608,6 +724,33 @@ void staged_wave_speed(Ctx& c) {
   HIPCHK(hipGetLastError());
 }
 
+template <int D, bool VISC>
+static void launch_point_flux(Ctx& c) {
+  const dim3 grid(blocks_for(c.z.E, 64), blocks_for(c.z.S, 4));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, c.stream, c.z.S, c.z.E, c.r_grad.idx, c.r_grad.w, c.r_corru.idx,
+                       c.r_corru.w, c.U, c.dUc, c.jginv, c.detj, c.dU, c.Fs, c.ph);
+  };
+  Launch L(c, "point_flux");
+  if constexpr (VISC) {
+    switch (c.r_grad.q) {
+      case 1: go(k_point_flux<D, 1, true>); break;
+      case 2: go(k_point_flux<D, 2, true>); break;
+      case 3: go(k_point_flux<D, 3, true>); break;
+      case 4: go(k_point_flux<D, 4, true>); break;
+      case 5: go(k_point_flux<D, 5, true>); break;
+      default: go(k_point_flux<D, 6, true>); break;
+    }
+  } else {
+    go(k_point_flux<D, 1, false>);
+  }
+  HIPCHK(hipGetLastError());
+}
+static void launch_point_flux(Ctx& c) {
+  if (c.z.D == 2) c.prm.viscous ? launch_point_flux<2, true>(c) : launch_point_flux<2, false>(c);
+  else c.prm.viscous ? launch_point_flux<3, true>(c) : launch_point_flux<3, false>(c);
+}
+
 void staged_residual(Ctx& c, int step) {
   const Sizes& z = c.z;
   const long long nS = z.nS(), nF = z.nF(), SE = (long long)z.S * z.E, FE = (long long)z.F * z.E;
@@ -615,14 +758,18 @@ void staged_residual(Ctx& c, int step) {
   double* divF = c.divF + step * nS;
   unsigned gS = blocks_for(SE, 256), gFF = blocks_for(z.nFaceFpts, 256);
 
+  // the pointwise kernels in one
+  const bool points = c.r_grad.q <= 6 && (!visc || (c.r_grad.q > 0 && c.r_corru.q == 2));
+
   staged_extrapolate_u(c);
-  if (visc && c.r_grad.q) oprows(c, "oprows_grad_u", c.r_grad, c.U, c.dU, false);
+  if (points) {
+  } else if (visc && c.r_grad.q) oprows(c, "oprows_grad_u", c.r_grad, c.U, c.dU, false);
   else if (visc)
     for (int d = 0; d < z.D; d++) opgemm(c, "opgemm_grad_u", z.S, z.S, c.grad + (long long)d * z.S * z.S, c.U, c.dU + d * nS, false);
-  {
+  if (!points) {
     Launch L(c, "inviscid_spts");
-    if (z.D == 2) hipLaunchKernelGGL(k_inviscid_spts<2>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.jginv, c.Fs, c.ph.gamma, visc ? 0 : 1);
-    else hipLaunchKernelGGL(k_inviscid_spts<3>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.jginv, c.Fs, c.ph.gamma, visc ? 0 : 1);
+    if (z.D == 2) hipLaunchKernelGGL(k_inviscid_spts<2>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.Fs, c.ph.gamma);
+    else hipLaunchKernelGGL(k_inviscid_spts<3>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.Fs, c.ph.gamma);
     HIPCHK(hipGetLastError());
   }
   if (z.nFaceFpts > 0) {
@@ -631,10 +778,12 @@ void staged_residual(Ctx& c, int step) {
     else hipLaunchKernelGGL(k_face_inviscid<3>, dim3(gFF), dim3(256), 0, c.stream, z.nFaceFpts, c.ft.ptL, c.ft.ptR, c.ft.bc, c.Uf, c.norm, c.da, c.Fn, c.faceFn, c.waveSp, c.dUc, c.ph);
     HIPCHK(hipGetLastError());
   }
+  if (points) launch_point_flux(c);
   if (visc) {
-    if (c.r_corru.q) oprows(c, "oprows_correct_grad_u", c.r_corru, c.dUc, c.dU, true);
+    if (points) {
+    } else if (c.r_corru.q) oprows(c, "oprows_correct_grad_u", c.r_corru, c.dUc, c.dU, true);
     else for (int d = 0; d < z.D; d++) opgemm(c, "opgemm_correct_grad_u", z.S, z.F, c.corru + (long long)d * z.S * z.F, c.dUc, c.dU + d * nS, true);
-    {
+    if (!points) {
       Launch L(c, "grad_transform");
       if (z.D == 2) hipLaunchKernelGGL(k_grad_transform<2>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.dU, c.jginv, c.detj);
       else hipLaunchKernelGGL(k_grad_transform<3>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.dU, c.jginv, c.detj);
@@ -642,7 +791,7 @@ void staged_residual(Ctx& c, int step) {
     }
     if (c.r_sf.q) oprows(c, "oprows_extrapolate_grad_u", c.r_sf, c.dU, c.dUf, false, z.D, nS, nF);
     else for (int d = 0; d < z.D; d++) opgemm(c, "opgemm_extrapolate_grad_u", z.F, z.S, c.sf, c.dU + d * nS, c.dUf + d * nF, false);
-    {
+    if (!points) {
       Launch L(c, "viscous_spts");
       if (z.D == 2) hipLaunchKernelGGL(k_viscous_spts<2>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.dU, c.jginv, c.Fs, c.ph);
       else hipLaunchKernelGGL(k_viscous_spts<3>, dim3(gS), dim3(256), 0, c.stream, SE, SE, c.U, c.dU, c.jginv, c.Fs, c.ph);
@@ -656,35 +805,34 @@ void staged_residual(Ctx& c, int step) {
     }
   }
   // extrapolateNormalFlux (static grid), calcDivF_spts, correctDivFlux
-  if (c.r_efn.q) oprows(c, "oprows_extrapolate_fn", c.r_efn, c.Fs, c.disFn, false);
+  if (c.r_efn.q) oprows(c, "oprows_flux_jump", c.r_efn, c.Fs, c.disFn, false, 1, 0, 0, c.Fn);
   else for (int d = 0; d < z.D; d++) opgemm(c, "opgemm_extrapolate_fn", z.F, z.S, c.efn + (long long)d * z.F * z.S, c.Fs + d * nS, c.disFn, d > 0);
-  if (c.r_div.q) oprows(c, "oprows_div_f", c.r_div, c.Fs, divF, false);
+  const bool both = c.r_efn.q && c.r_div.q && c.r_corr.q;
+  if (both) oprows(c, "oprows_div_f", c.r_div, c.Fs, divF, false, 1, 0, 0, nullptr, &c.r_corr, c.disFn);
+  else if (c.r_div.q) oprows(c, "oprows_div_f", c.r_div, c.Fs, divF, false);
   else for (int d = 0; d < z.D; d++) opgemm(c, "opgemm_div_f", z.S, z.S, c.grad + (long long)d * z.S * z.S, c.Fs + d * nS, divF, d > 0);
-  {
+  if (!c.r_efn.q) {
     Launch L(c, "sub_fn");
     hipLaunchKernelGGL(k_sub, dim3(blocks_for(nF, 256)), dim3(256), 0, c.stream, nF, c.Fn, c.disFn);
     HIPCHK(hipGetLastError());
   }
+  if (both) return;
   if (c.r_corr.q) oprows(c, "oprows_correction", c.r_corr, c.disFn, divF, true);
   else opgemm(c, "opgemm_correction", z.S, z.F, c.corr, c.disFn, divF, true);
 }
 
-void staged_time_step_a(Ctx& c, int step, double rk, bool src) {
-  long long SE = (long long)c.z.S * c.z.E;
-  Launch L(c, "time_step_a");
-  hipLaunchKernelGGL(k_time_step, dim3(blocks_for(SE, 256)), dim3(256), 0, c.stream, SE, c.z.N, (long long)c.z.E, 0, rk, c.U,
-                     c.U0, c.divF + step * c.z.nS(), src ? c.src : nullptr, c.detj, c.d_dt, c.eleDt, c.prm.dt_type == 2 ? 1 : 0);
+static void time_step(Ctx& c, const char* name, int modeB, double rk, int step, bool src) {
+  const long long n = c.z.nS();
+  Launch L(c, name);
+  auto* kern = c.z.D == 2 ? k_time_step<4> : k_time_step<5>;
+  hipLaunchKernelGGL(kern, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, (unsigned)c.z.E, modeB, rk, c.U, c.U0,
+                     c.divF + step * n, src ? c.src : nullptr, c.detj, c.d_dt, c.eleDt, c.prm.dt_type == 2 ? 1 : 0);
   HIPCHK(hipGetLastError());
 }
 
-void staged_time_step_b(Ctx& c, int step, bool src) {
-  long long SE = (long long)c.z.S * c.z.E;
-  Launch L(c, "time_step_b");
-  hipLaunchKernelGGL(k_time_step, dim3(blocks_for(SE, 256)), dim3(256), 0, c.stream, SE, c.z.N, (long long)c.z.E, 1,
-                     c.prm.rk_b[step], c.U, c.U0, c.divF + step * c.z.nS(), src ? c.src : nullptr, c.detj, c.d_dt, c.eleDt,
-                     c.prm.dt_type == 2 ? 1 : 0);
-  HIPCHK(hipGetLastError());
-}
+void staged_time_step_a(Ctx& c, int step, double rk, bool src) { time_step(c, "time_step_a", 0, rk, step, src); }
+
+void staged_time_step_b(Ctx& c, int step, bool src) { time_step(c, "time_step_b", 1, c.prm.rk_b[step], step, src); }
 
 static double cfl_limit(int order) {  // getCFLLimit, src/global.cpp:81-105
   static const double t[6] = {1.393, 0.464, 0.235, 0.1453, 0.100, 0.0736};
