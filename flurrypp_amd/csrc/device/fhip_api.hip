@@ -797,11 +797,13 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
   CycleStream one(mg);
   const int n = (int)mg->lv.size();
   fhip::Ctx& fine = mg->lv[n - 1]->c;
+  std::vector<fhip::Ctx*> coarse;
   for (int i = 0; i + 1 < n; i++) {
     fhip::fused_em_prepare(mg->lv[i]->c, mixed);
-    fhip::fused_em_import_wave(mg->lv[i]->c);
+    coarse.push_back(&mg->lv[i]->c);
   }
-  fhip::fused_begin(fine, mixed, false);
+  fhip::Ctx* const top = &fine;
+  fhip::fused_em_begin(coarse.data(), n - 1, &top, 1, mixed);
   fhip::fused_em_residual(fine, mixed);
   auto smooth = [&](fhip::Ctx& g) {
     fhip::fused_em_set_src(g, true);
@@ -826,9 +828,8 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
     smooth(g);
     fhip::pmg_prolong_em(up, g.z.S, mg->Pro[i], fhip::fused_em_array(g, 0), mg->sol[i]);
     if (i + 2 < n) fhip::fused_em_extrap(up, mixed);  // the next level up smooths from here
-    fhip::fused_em_export_u(g);
   }
-  fhip::fused_end(fine);
+  fhip::fused_em_end(coarse.data(), n - 1, &top, 1);
 }
 
 // The batched cycle: every mesh goes through the steps of
@@ -839,14 +840,14 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
 static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
   CycleStream one(mg);
   const int nc = (int)mg->lv.size();
+  std::vector<fhip::Ctx*> coarse, fine;
   for (int j = 0; j < nc; j++) {
     fhip::fused_em_prepare(mg->lv[j]->c, mixed);
-    fhip::fused_em_import_wave(mg->lv[j]->c);
+    coarse.push_back(&mg->lv[j]->c);
   }
-  for (fhip_ctx* h : mg->fine) {
-    fhip::fused_begin(h->c, mixed, false);
-    fhip::fused_em_residual(h->c, mixed);
-  }
+  for (fhip_ctx* h : mg->fine) fine.push_back(&h->c);
+  fhip::fused_em_begin(coarse.data(), nc, fine.data(), (int)fine.size(), mixed);
+  for (fhip::Ctx* f : fine) fhip::fused_em_residual(*f, mixed);
   auto smooth = [&](fhip::Ctx& g) {
     fhip::fused_em_set_src(g, true);
     for (int k = 0; k < mg->smooth; k++) update_step(g, true, mixed, true, false, false);
@@ -881,9 +882,8 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
       fhip::pmg_prolong_em(up, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0) + offA, mg->sol[j] + offA);
       fhip::fused_em_extrap(up, mixed);  // the next level up smooths from here
     }
-    fhip::fused_em_export_u(g);
   }
-  for (fhip_ctx* h : mg->fine) fhip::fused_end(h->c);
+  fhip::fused_em_end(coarse.data(), nc, fine.data(), (int)fine.size());
 }
 
 // The first cycle on a path runs launch by launch (it also allocates what the

@@ -486,16 +486,35 @@ template <>
 inline Work<float>& FusedState::work<float>() { return w32; }
 
 // ---------------------------------------------------------------------------
+#ifndef FHIP_FAMILY
 // Layout conversions between FlurryPP's [pt][ele][k] and element-major
 // [ele][k][pt]: both are the transpose of a matrix with one row per point,
 // [P][E*K] <-> [E*K][P].  32x32 tiles through LDS so that reads and writes
-// are both coalesced; tiles are numbered on a 1-D grid.
-constexpr int kTile = 32;
-static __global__ __launch_bounds__(256) void k_transpose(long long R, long long C, const double* __restrict__ in,
-                                                   double* __restrict__ out) {
+// are both coalesced; tiles are numbered on a 1-D grid over all the arrays that
+// a call converts at one place (Layouts): on a small mesh each launch is some 4
+// us.  One each -> together: a step of the 8x8 P3 vortex 55 -> 49 us, update and
+// cycle of the P4 channel 67x29 690 -> 652 us.
+constexpr int kTile = 32, kMaxLayouts = 16;
+struct LayoutJobs {
+  int n = 0;
+  unsigned tiles = 0;
+  struct Job {
+    long long R, C;  // in [R][C] -> out [C][R]
+    const double* in;
+    double* out;
+    unsigned first;  // its first tile
+  } job[kMaxLayouts];
+};
+static __global__ __launch_bounds__(256) void k_transpose(LayoutJobs jobs) {
   __shared__ double t[kTile][kTile + 1];
-  const long long tilesC = (C + kTile - 1) / kTile;
-  const long long r0 = (blockIdx.x / tilesC) * kTile, c0 = (blockIdx.x % tilesC) * kTile;
+  int n = 0;
+  while (n + 1 < jobs.n && blockIdx.x >= jobs.job[n + 1].first) n++;
+  const LayoutJobs::Job& jb = jobs.job[n];
+  const long long R = jb.R, C = jb.C;
+  const double* const __restrict__ in = jb.in;
+  double* const __restrict__ out = jb.out;
+  const unsigned tilesC = (unsigned)((C + kTile - 1) / kTile), tile = blockIdx.x - jb.first;
+  const long long r0 = (long long)(tile / tilesC) * kTile, c0 = (long long)(tile % tilesC) * kTile;
   const int tx = threadIdx.x % kTile, ty = threadIdx.x / kTile;  // ty 0..7
 #pragma unroll
   for (int j = 0; j < kTile; j += 8) {
@@ -510,20 +529,32 @@ static __global__ __launch_bounds__(256) void k_transpose(long long R, long long
   }
 }
 
-// in [P][E][K] -> out [E][K][P]
-static void to_em(hipStream_t st, int P, long long E, int K, const double* in, double* out) {
-  const long long R = P, C = E * K;
-  const long long tiles = ((R + kTile - 1) / kTile) * ((C + kTile - 1) / kTile);
-  hipLaunchKernelGGL(k_transpose, dim3((unsigned)tiles), dim3(256), 0, st, R, C, in, out);
-  FCHK(hipGetLastError());
-}
-// in [E][K][P] -> out [P][E][K]
-static void from_em(hipStream_t st, int P, long long E, int K, const double* in, double* out) {
-  const long long R = E * K, C = P;
-  const long long tiles = ((R + kTile - 1) / kTile) * ((C + kTile - 1) / kTile);
-  hipLaunchKernelGGL(k_transpose, dim3((unsigned)tiles), dim3(256), 0, st, R, C, in, out);
-  FCHK(hipGetLastError());
-}
+// The conversions of one place of a call, launched together (go, or when full).
+// They must not depend on each other.
+struct Layouts {
+  hipStream_t st;
+  LayoutJobs jobs;
+  explicit Layouts(hipStream_t s) : st(s) {}
+  void add(long long R, long long C, const double* in, double* out) {
+    if (R == 0 || C == 0) return;
+    const long long tiles = ((R + kTile - 1) / kTile) * ((C + kTile - 1) / kTile);
+    if (jobs.n == kMaxLayouts || jobs.tiles + tiles > 0x7fffffffll) go();
+    jobs.job[jobs.n++] = LayoutJobs::Job{R, C, in, out, jobs.tiles};
+    jobs.tiles += (unsigned)tiles;
+  }
+  // in [P][E][K] -> out [E][K][P]
+  void to_em(int P, long long E, int K, const double* in, double* out) { add(P, E * K, in, out); }
+  // in [E][K][P] -> out [P][E][K]
+  void from_em(int P, long long E, int K, const double* in, double* out) { add(E * K, P, in, out); }
+  void go() {
+    if (jobs.n) {
+      hipLaunchKernelGGL(k_transpose, dim3(jobs.tiles), dim3(256), 0, st, jobs);
+      FCHK(hipGetLastError());
+    }
+    jobs = LayoutJobs();
+  }
+};
+#endif  // FHIP_FAMILY
 
 // ---------------------------------------------------------------------------
 // U at the flux points from U at the solution points (opp_spts_to_fpts rows).
@@ -2812,14 +2843,14 @@ void fused_get_blocks(Ctx& c, bool mixed, int* out) {
   std::copy(nt, nt + 5, out);
 }
 
-void fused_begin(Ctx& c, bool mixed, bool src) {
+// What a call on the fused paths starts from, element-major.
+static void add_begin(Ctx& c, bool mixed, bool src, Layouts& lay) {
   FusedState& st = fs(c);
   st.read_stage = st.odd_stage = false;
   const Sizes& z = c.z;
-  Ops o = get_ops(c, mixed);
-  o.ensure(c);
+  get_ops(c, mixed).ensure(c);
   long long nS = (long long)z.E * z.N * z.S;
-  to_em(c.stream, z.S, z.E, z.N, c.U, st.Ue);
+  lay.to_em(z.S, z.E, z.N, c.U, st.Ue);
   st.use_src = src;
   if (src) {
     if (!c.src) throw std::invalid_argument("no P-multigrid source term on this context");
@@ -2828,11 +2859,16 @@ void fused_begin(Ctx& c, bool mixed, bool src) {
       FCHK(hipMalloc(&st.srce, nS * sizeof(double)));
       poison_fill(st.srce, nS * sizeof(double));
     }
-    to_em(c.stream, z.S, z.E, z.N, c.src, st.srce);
+    lay.to_em(z.S, z.E, z.N, c.src, st.srce);
   }
-  to_em(c.stream, z.F, z.E, 1, c.waveSp, st.waveSpe);
-  FCHK(hipGetLastError());
-  o.extrap(c);
+  lay.to_em(z.F, z.E, 1, c.waveSp, st.waveSpe);
+}
+
+void fused_begin(Ctx& c, bool mixed, bool src) {
+  Layouts lay(c.stream);
+  add_begin(c, mixed, src, lay);
+  lay.go();
+  get_ops(c, mixed).extrap(c);
 }
 
 // P-multigrid cycle with every level kept element-major (the transfers above;
@@ -2854,12 +2890,19 @@ void fused_em_prepare(Ctx& c, bool mixed) {
 
 void fused_em_extrap(Ctx& c, bool mixed) { get_ops(c, mixed).extrap(c); }
 
-// The wave speeds from FlurryPP's layout: the face kernel rewrites only the
-// entries of left and boundary flux points (the reference's calcWaveSp
-// stores into the left element); the others keep what the level holds.
-void fused_em_import_wave(Ctx& c) {
-  to_em(c.stream, c.z.F, c.z.E, 1, c.waveSp, fs(c).waveSpe);
-  FCHK(hipGetLastError());
+// The start of a cycle: fused_begin of the fine levels, and the coarse levels'
+// wave speeds, of which the stage kernel rewrites only the entries of left and
+// boundary flux points (the reference's calcWaveSp stores into the left element)
+// and the time steps sum all.  All on one stream.
+void fused_em_begin(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool mixed) {
+  Layouts lay(fine[0]->stream);
+  for (int i = 0; i < nc; i++) {
+    const Ctx& c = *coarse[i];
+    lay.to_em(c.z.F, c.z.E, 1, c.waveSp, fs(*coarse[i]).waveSpe);
+  }
+  for (int i = 0; i < nf; i++) add_begin(*fine[i], mixed, false, lay);
+  lay.go();
+  for (int i = 0; i < nf; i++) get_ops(*fine[i], mixed).extrap(*fine[i]);
 }
 
 void fused_em_residual(Ctx& c, bool mixed, int how) {
@@ -2876,11 +2919,26 @@ double* fused_em_array(Ctx& c, int which) {
   return which == 0 ? st.Ue : (which == 1 ? st.divF0e : st.srce);
 }
 
-void fused_em_export_u(Ctx& c) {
+static void add_end(Ctx& c, Layouts& lay) {
   FusedState& st = fs(c);
   st.use_src = false;
-  from_em(c.stream, c.z.S, c.z.E, c.z.N, st.Ue, c.U);
-  FCHK(hipGetLastError());
+  const Sizes& z = c.z;
+  lay.from_em(z.S, z.E, z.N, st.Ue, c.U);
+  lay.from_em(z.S, z.E, z.N, st.divF0e, c.divF);
+  lay.from_em(z.F, z.E, 1, st.waveSpe, c.waveSp);
+}
+
+// The end of a cycle on the element-major levels: U of the coarse levels cs, and
+// what fused_end writes back of the fine ones.
+void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf) {
+  Layouts lay(fine[0]->stream);
+  for (int i = 0; i < nc; i++) {
+    Ctx& c = *coarse[i];
+    fs(c).use_src = false;
+    lay.from_em(c.z.S, c.z.E, c.z.N, fs(c).Ue, c.U);
+  }
+  for (int i = 0; i < nf; i++) add_end(*fine[i], lay);
+  lay.go();
 }
 
 void pmg_restrict_em(Ctx& c, long long e0, long long ne, int Sf, const double* R, const double* Uf,
@@ -2918,13 +2976,9 @@ void pmg_prolong_em(Ctx& up, int Sc, const double* Pm, const double* Uc, const d
 }
 
 void fused_end(Ctx& c) {
-  FusedState& st = fs(c);
-  st.use_src = false;
-  const Sizes& z = c.z;
-  from_em(c.stream, z.S, z.E, z.N, st.Ue, c.U);
-  from_em(c.stream, z.S, z.E, z.N, st.divF0e, c.divF);
-  from_em(c.stream, z.F, z.E, 1, st.waveSpe, c.waveSp);
-  FCHK(hipGetLastError());
+  Layouts lay(c.stream);
+  add_end(c, lay);
+  lay.go();
 }
 
 // calcResidual(0) at the current state (src/solver.cpp:366-445) on a fused
@@ -2936,9 +2990,10 @@ void fused_residual(Ctx& c, bool mixed) {
   fused_begin(c, mixed, false);
   o.residual(c, true);
   o.rk(c, 5, 0., 0., true, 0);
-  from_em(c.stream, z.S, z.E, z.N, st.divF0e, c.divF);
-  from_em(c.stream, z.F, z.E, 1, st.waveSpe, c.waveSp);
-  FCHK(hipGetLastError());
+  Layouts lay(c.stream);
+  lay.from_em(z.S, z.E, z.N, st.divF0e, c.divF);
+  lay.from_em(z.F, z.E, 1, st.waveSpe, c.waveSp);
+  lay.go();
 }
 
 // One iteration of solver::update (src/solver.cpp:319-363) on a fused path.

@@ -196,11 +196,11 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep = true);
 // and into the upper level up (U += P (U_c - sol_c)).
 void fused_em_prepare(Ctx& c, bool mixed);
 void fused_em_extrap(Ctx& c, bool mixed);
-void fused_em_import_wave(Ctx& c);
+void fused_em_begin(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool mixed);
 void fused_em_residual(Ctx& c, bool mixed, int how = 0);
 void fused_em_set_src(Ctx& c, bool on);
 double* fused_em_array(Ctx& c, int which);
-void fused_em_export_u(Ctx& c);
+void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf);
 // (restriction into the coarse elements [e0, e0 + ne) from the fine rows Uf,
 // divFf of those elements)
 void pmg_restrict_em(Ctx& c, long long e0, long long ne, int Sf, const double* R, const double* Uf,
