@@ -814,9 +814,8 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
     fhip::Ctx& g = mg->lv[i]->c;
     fhip::Ctx& f = mg->lv[i + 1]->c;
     // restriction of U and divF_spts[0]; compute_source_term (src/multigrid.cpp:381-398)
-    fhip::pmg_restrict_em(g, 0, g.z.E, f.z.S, mg->R[i], fhip::fused_em_array(f, 0), fhip::fused_em_array(f, 1),
+    fhip::pmg_restrict_em(g, mixed, 0, g.z.E, f.z.S, mg->R[i], fhip::fused_em_array(f, 0), fhip::fused_em_array(f, 1),
                           mg->sol[i]);
-    fhip::fused_em_extrap(g, mixed);
     fhip::fused_em_residual(g, mixed, 1);  // source -= residual
     smooth(g);
     if (i > 0) fhip::fused_em_residual(g, mixed, 2);  // residual + source, restricted below
@@ -826,8 +825,8 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
     fhip::Ctx& g = mg->lv[i]->c;
     fhip::Ctx& up = mg->lv[i + 1]->c;
     smooth(g);
-    fhip::pmg_prolong_em(up, g.z.S, mg->Pro[i], fhip::fused_em_array(g, 0), mg->sol[i]);
-    if (i + 2 < n) fhip::fused_em_extrap(up, mixed);  // the next level up smooths from here
+    // (a coarse level smooths from there)
+    fhip::pmg_prolong_em(up, mixed, g.z.S, mg->Pro[i], fhip::fused_em_array(g, 0), mg->sol[i], i + 2 < n);
   }
   fhip::fused_em_end(coarse.data(), n - 1, &top, 1);
 }
@@ -858,15 +857,14 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
     const long long eA = mg->splitE[j];
     if (mg->fineOf[j] >= 0) {
       fhip::Ctx& f = mg->fine[mg->fineOf[j]]->c;
-      fhip::pmg_restrict_em(g, 0, eA, f.z.S, mg->R[j], fhip::fused_em_array(f, 0), fhip::fused_em_array(f, 1),
+      fhip::pmg_restrict_em(g, mixed, 0, eA, f.z.S, mg->R[j], fhip::fused_em_array(f, 0), fhip::fused_em_array(f, 1),
                             mg->sol[j]);
     }
     if (j + 1 < nc) {
       fhip::Ctx& f = mg->lv[j + 1]->c;
-      fhip::pmg_restrict_em(g, eA, g.z.E - eA, f.z.S, mg->R[j], fhip::fused_em_array(f, 0),
+      fhip::pmg_restrict_em(g, mixed, eA, g.z.E - eA, f.z.S, mg->R[j], fhip::fused_em_array(f, 0),
                             fhip::fused_em_array(f, 1), mg->sol[j]);
     }
-    fhip::fused_em_extrap(g, mixed);
     fhip::fused_em_residual(g, mixed, 1);  // source -= residual
     smooth(g);
     if (j > 0) fhip::fused_em_residual(g, mixed, 2);  // residual + source, restricted below
@@ -876,11 +874,12 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
     const long long offA = mg->splitE[j] * g.z.N * g.z.S;
     smooth(g);
     if (mg->fineOf[j] >= 0)
-      fhip::pmg_prolong_em(mg->fine[mg->fineOf[j]]->c, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0), mg->sol[j]);
+      fhip::pmg_prolong_em(mg->fine[mg->fineOf[j]]->c, mixed, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0),
+                           mg->sol[j], false);
     if (j + 1 < nc) {
       fhip::Ctx& up = mg->lv[j + 1]->c;
-      fhip::pmg_prolong_em(up, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0) + offA, mg->sol[j] + offA);
-      fhip::fused_em_extrap(up, mixed);  // the next level up smooths from here
+      // (which smooths from there)
+      fhip::pmg_prolong_em(up, mixed, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0) + offA, mg->sol[j] + offA, true);
     }
   }
   fhip::fused_em_end(coarse.data(), nc, fine.data(), (int)fine.size());

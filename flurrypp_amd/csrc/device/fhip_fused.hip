@@ -1727,77 +1727,115 @@ static __global__ void k_prolong_em(long long rows, int Su, int Sc, int kc, cons
 }
 
 // The same transfers with the operator (transposed, so that the lanes of a
-// wave read consecutive entries) and the block's rows staged in LDS: nr rows
-// per block, one output per thread, the sums in the same order as above.
-// Used where the operator and the rows fit in 64 KiB.
-static __global__ void k_restrict_em_lds(long long rows, int Sc, int Sf, int kc, int nr, const double* __restrict__ R,
-                                  const double* __restrict__ Uf, const double* __restrict__ divFf,
-                                  double* __restrict__ Uc, double* __restrict__ srcc, double* __restrict__ solc) {
-  double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sf][Sc]
-  double* const sU = sA + Sc * Sf;                          // [nr][Sf]
-  double* const sV = sU + nr * Sf;                          // [nr][Sf]
-  const long long r0 = (long long)blockIdx.x * nr;
-  const int nb = (int)min((long long)nr, rows - r0);
-  for (int j = threadIdx.x; j < Sc * Sf; j += blockDim.x) {
-    const int i = j / Sf;
-    sA[(j - i * Sf) * Sc + i] = R[j];
+// wave read consecutive entries) and the rows of the block's EB elements staged in
+// LDS, one output per thread, the sums in the same order as above; and, where Ufe
+// is given, the level's new U at the flux points (and its FP32 copy), which the
+// level's next residual or smoothing step starts from.  Used where an element's
+// rows fit a block and all of it 64 KiB.
+template <int D, int P, class R, bool TEN>
+__device__ __forceinline__ void transfer_faces(int e0, int nb, const R* sX, const R* sW, R* Ufe, const Tabs& tb) {
+  for (int i = threadIdx.x; i < nb * Shape<D, P>::F; i += blockDim.x) {
+    Packed<P + 1> lp;
+    lp.load(tb, i % Shape<D, P>::F);
+    face_point<D, P, R, false, TEN>(i, e0, lp, sX, sW, Ufe, tb);
   }
-  for (int j = threadIdx.x; j < nb * Sf; j += blockDim.x) {
+}
+template <int D, int P, class R, bool TEN>
+__global__ __launch_bounds__(kMaxBlock) void k_restrict_lds(int ne, int EB, int Sf, int kc, const double* __restrict__ A,
+                                                             const double* __restrict__ Uf,
+                                                             const double* __restrict__ divFf, double* __restrict__ Uc,
+                                                             double* __restrict__ srcc, double* __restrict__ solc,
+                                                             R* __restrict__ Ufe, R* __restrict__ Us, Tabs tb) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
+  const int e0 = blockIdx.x * EB, nb = min(EB, ne - e0), nr = EB * N, rows = nb * N;
+  double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sf][S]
+  double* const sU = sA + S * Sf;                           // [nr][Sf]
+  double* const sV = sU + nr * Sf;                          // [nr][Sf]
+  R* const sX = reinterpret_cast<R*>(sV + nr * Sf);         // [nr][S]
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
+  const long long r0 = (long long)e0 * N;
+  for (int j = threadIdx.x; j < S * Sf; j += blockDim.x) {
+    const int i = j / Sf;
+    sA[(j - i * Sf) * S + i] = A[j];
+  }
+  for (int j = threadIdx.x; j < rows * Sf; j += blockDim.x) {
     sU[j] = Uf[r0 * Sf + j];
     sV[j] = divFf[r0 * Sf + j];
   }
   __syncthreads();
-  const int rr = threadIdx.x / Sc, i = threadIdx.x - rr * Sc;
-  if (rr >= nb) return;
-  const double* u = sU + rr * Sf;
-  const double* d = sV + rr * Sf;
-  double cu = 0, cd = 0;
-  for (int l0 = 0; l0 < Sf; l0 += kc) {
-    const int n = min(kc, Sf - l0);
-    double su = 0, sd = 0;
-    for (int l = 0; l < n; l++) {
-      const double a = sA[(l0 + l) * Sc + i];
-      su += a * u[l0 + l];
-      sd += a * d[l0 + l];
+  const int rr = threadIdx.x / S, i = threadIdx.x - rr * S;
+  if (rr < rows) {
+    const double* u = sU + rr * Sf;
+    const double* d = sV + rr * Sf;
+    double cu = 0, cd = 0;
+    for (int l0 = 0; l0 < Sf; l0 += kc) {
+      const int n = min(kc, Sf - l0);
+      double su = 0, sd = 0;
+      for (int l = 0; l < n; l++) {
+        const double a = sA[(l0 + l) * S + i];
+        su += a * u[l0 + l];
+        sd += a * d[l0 + l];
+      }
+      cu = l0 ? su + cu : su;
+      cd = l0 ? sd + cd : sd;
     }
-    cu = l0 ? su + cu : su;
-    cd = l0 ? sd + cd : sd;
+    const long long t = r0 * S + threadIdx.x;
+    Uc[t] = cu;
+    solc[t] = cu;
+    srcc[t] = cd;
+    sX[rr * S + spt_lds(D, P1, i)] = R(cu);
+    if (Us) Us[t] = R(cu);
   }
-  const long long t = r0 * Sc + threadIdx.x;
-  Uc[t] = cu;
-  solc[t] = cu;
-  srcc[t] = cd;
+  __syncthreads();
+  transfer_faces<D, P, R, TEN>(e0, nb, sX, sW, Ufe, tb);
 }
 
-static __global__ void k_prolong_em_lds(long long rows, int Su, int Sc, int kc, int nr, const double* __restrict__ Pm,
-                                 const double* __restrict__ Uc, const double* __restrict__ solc,
-                                 double* __restrict__ Uu) {
-  double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sc][Su]
-  double* const sV = sA + Su * Sc;                          // [nr][Sc]: U - sol
-  const long long r0 = (long long)blockIdx.x * nr;
-  const int nb = (int)min((long long)nr, rows - r0);
-  for (int j = threadIdx.x; j < Su * Sc; j += blockDim.x) {
+template <int D, int P, class R, bool TEN>
+__global__ __launch_bounds__(kMaxBlock) void k_prolong_lds(int ne, int EB, int Sc, int kc, const double* __restrict__ A,
+                                                            const double* __restrict__ Uc,
+                                                            const double* __restrict__ solc, double* __restrict__ Uu,
+                                                            R* __restrict__ Ufe, R* __restrict__ Us, Tabs tb) {
+  using Sh = Shape<D, P>;
+  constexpr int S = Sh::S, N = Sh::N, P1 = Sh::P1;
+  const int e0 = blockIdx.x * EB, nb = min(EB, ne - e0), nr = EB * N, rows = nb * N;
+  double* const sA = reinterpret_cast<double*>(fhip_lds);  // [Sc][S]
+  double* const sV = sA + S * Sc;                           // [nr][Sc]: U - sol
+  R* const sX = reinterpret_cast<R*>(sV + nr * Sc);         // [nr][S]
+  __shared__ R sW[Ten<D, P>::NW];
+  stage_factors<D, P, R, TEN>(sW, tb);
+  const long long r0 = (long long)e0 * N;
+  for (int j = threadIdx.x; j < S * Sc; j += blockDim.x) {
     const int i = j / Sc;
-    sA[(j - i * Sc) * Su + i] = Pm[j];
+    sA[(j - i * Sc) * S + i] = A[j];
   }
-  for (int j = threadIdx.x; j < nb * Sc; j += blockDim.x) {
+  for (int j = threadIdx.x; j < rows * Sc; j += blockDim.x) {
     double v = Uc[r0 * Sc + j];
     v -= solc[r0 * Sc + j];
     sV[j] = v;
   }
   __syncthreads();
-  const int rr = threadIdx.x / Su, i = threadIdx.x - rr * Su;
-  if (rr >= nb) return;
-  const double* v = sV + rr * Sc;
-  const long long t = r0 * Su + threadIdx.x;
-  double c = Uu[t];
-  for (int l0 = 0; l0 < Sc; l0 += kc) {
-    const int n = min(kc, Sc - l0);
-    double s = 0;
-    for (int l = 0; l < n; l++) s += sA[(l0 + l) * Su + i] * v[l0 + l];
-    c = s + c;
+  const int rr = threadIdx.x / S, i = threadIdx.x - rr * S;
+  if (rr < rows) {
+    const double* v = sV + rr * Sc;
+    const long long t = r0 * S + threadIdx.x;
+    double c = Uu[t];
+    for (int l0 = 0; l0 < Sc; l0 += kc) {
+      const int n = min(kc, Sc - l0);
+      double s = 0;
+      for (int l = 0; l < n; l++) s += sA[(l0 + l) * S + i] * v[l0 + l];
+      c = s + c;
+    }
+    Uu[t] = c;
+    if (Ufe) {
+      sX[rr * S + spt_lds(D, P1, i)] = R(c);
+      if (Us) Us[t] = R(c);
+    }
   }
-  Uu[t] = c;
+  if (!Ufe) return;  // uniform over the launch
+  __syncthreads();
+  transfer_faces<D, P, R, TEN>(e0, nb, sX, sW, Ufe, tb);
 }
 
 // Wave speeds from U at the flux points (ele::calcWaveSpFpts), element-major.
@@ -2603,6 +2641,37 @@ struct Runner {
     Launch L(c, nm("fused_extrapolate", "mixed_extrapolate"));
     launch_extrap(c, blk(c, kExtrap));
   }
+  // The transfers in LDS into this level (restriction: its elements [e0, e0 + ne)),
+  // with U at its flux points (prolongation: if extrap).  False, and nothing
+  // done, where they do not fit.
+  static int transfer_eles() { return N * S <= kMaxBlock ? std::max(1, 256 / (N * S)) : 0; }
+  static bool restrict_lds(Ctx& c, long long e0, long long ne, int Sf, int kc, const double* A, const double* Uf,
+                           const double* divFf, double* solc) {
+    FusedState& st = fs(c);
+    Work<R>& w = st.work<R>();
+    const int EB = transfer_eles(), nr = EB * N;
+    const size_t bytes = ((size_t)S * Sf + 2 * (size_t)nr * Sf) * sizeof(double) + (size_t)nr * S * sizeof(R);
+    if (!EB || bytes > kMaxLds) return false;
+    auto* kern = st.tb.w1 ? k_restrict_lds<D, P, R, true> : k_restrict_lds<D, P, R, false>;
+    const long long off = e0 * N * S;
+    hipLaunchKernelGGL(kern, dim3(nblk(ne, EB)), dim3(nr * S), bytes, c.stream, (int)ne, EB, Sf, kc, A, Uf, divFf,
+                       st.Ue + off, st.srce + off, solc + off, w.Ufe + e0 * N * F,
+                       sizeof(R) == 4 ? w.Us + off : nullptr, st.tb);
+    FCHK(hipGetLastError());
+    return true;
+  }
+  static bool prolong_lds(Ctx& c, int Sc, int kc, const double* A, const double* Uc, const double* solc, bool extrap) {
+    FusedState& st = fs(c);
+    Work<R>& w = st.work<R>();
+    const int EB = transfer_eles(), nr = EB * N;
+    const size_t bytes = ((size_t)S * Sc + (size_t)nr * Sc) * sizeof(double) + (size_t)nr * S * sizeof(R);
+    if (!EB || bytes > kMaxLds) return false;
+    auto* kern = st.tb.w1 ? k_prolong_lds<D, P, R, true> : k_prolong_lds<D, P, R, false>;
+    hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(nr * S), bytes, c.stream, c.z.E, EB, Sc, kc, A, Uc, solc,
+                       st.Ue, extrap ? w.Ufe : nullptr, sizeof(R) == 4 ? w.Us : nullptr, st.tb);
+    FCHK(hipGetLastError());
+    return true;
+  }
   static void wave(Ctx& c) {
     FusedState& st = fs(c);
     long long n = (long long)c.z.E * Sh::F;
@@ -2753,12 +2822,14 @@ struct Ops {
   void (*tune)(Ctx&);
   bool (*check)(Ctx&, const int*);
   void (*fit)(Ctx&);
+  bool (*restrict_lds)(Ctx&, long long, long long, int, int, const double*, const double*, const double*, double*);
+  bool (*prolong_lds)(Ctx&, int, int, const double*, const double*, const double*, bool);
 };
 
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::folds_dt, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit};
+  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::folds_dt, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
 }
 
 // The kernels of one dimension, precision and range of orders.  This file is
@@ -2874,8 +2945,6 @@ void fused_begin(Ctx& c, bool mixed, bool src) {
 // P-multigrid cycle with every level kept element-major (the transfers above;
 // a level's FlurryPP-layout arrays are written back by the caller at the end).
 static int opgemm_chunk(int k) { return k <= 16 ? 16 : (k <= 32 ? 32 : 64); }
-// LDS the staged transfers may take (operator plus the block's rows)
-constexpr size_t kTransferLds = 64 * 1024;
 
 void fused_em_prepare(Ctx& c, bool mixed) {
   FusedState& st = fs(c);
@@ -2887,8 +2956,6 @@ void fused_em_prepare(Ctx& c, bool mixed) {
     poison_fill(st.srce, (size_t)c.z.E * c.z.N * c.z.S * sizeof(double));
   }
 }
-
-void fused_em_extrap(Ctx& c, bool mixed) { get_ops(c, mixed).extrap(c); }
 
 // The start of a cycle: fused_begin of the fine levels, and the coarse levels'
 // wave speeds, of which the stage kernel rewrites only the entries of left and
@@ -2941,38 +3008,39 @@ void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf) {
   lay.go();
 }
 
-void pmg_restrict_em(Ctx& c, long long e0, long long ne, int Sf, const double* R, const double* Uf,
+// Both leave U at the level's flux points current (prolongation: if extrap).
+// Restriction and extrapolation, prolongation and extrapolation in one launch
+// each, and a level's launches with them: update and cycle of the P4 channel
+// 67x29 652 -> 630 us.
+void pmg_restrict_em(Ctx& c, bool mixed, long long e0, long long ne, int Sf, const double* R, const double* Uf,
                      const double* divFf, double* solc) {
   FusedState& st = fs(c);
   if (e0 < 0 || ne < 0 || e0 + ne > c.z.E) throw std::invalid_argument("restriction rows out of range");
   if (ne == 0) return;
-  const long long rows = ne * c.z.N;
-  const int Sc = c.z.S, nr = 256 / Sc;
-  const long long off = e0 * c.z.N * Sc;  // the first coarse element's rows
-  Launch L(c, "pmg_restrict");
-  const size_t lds = ((size_t)Sc * Sf + 2 * (size_t)nr * Sf) * sizeof(double);
-  if (nr >= 1 && lds <= kTransferLds)
-    hipLaunchKernelGGL(k_restrict_em_lds, dim3((unsigned)((rows + nr - 1) / nr)), dim3(nr * Sc), lds, c.stream,
-                       rows, Sc, Sf, opgemm_chunk(Sf), nr, R, Uf, divFf, st.Ue + off, st.srce + off, solc + off);
-  else
-    hipLaunchKernelGGL(k_restrict_em, dim3(nblk(rows * Sc, 256)), dim3(256), 0, c.stream, rows, Sc, Sf,
+  const Ops o = get_ops(c, mixed);
+  {
+    Launch L(c, "pmg_restrict");
+    if (o.restrict_lds(c, e0, ne, Sf, opgemm_chunk(Sf), R, Uf, divFf, solc)) return;
+    const long long rows = ne * c.z.N, off = e0 * c.z.N * c.z.S;  // the first coarse element's rows
+    hipLaunchKernelGGL(k_restrict_em, dim3(nblk(rows * c.z.S, 256)), dim3(256), 0, c.stream, rows, c.z.S, Sf,
                        opgemm_chunk(Sf), R, Uf, divFf, st.Ue + off, st.srce + off, solc + off);
-  FCHK(hipGetLastError());
+    FCHK(hipGetLastError());
+  }
+  o.extrap(c);
 }
 
-void pmg_prolong_em(Ctx& up, int Sc, const double* Pm, const double* Uc, const double* solc) {
+void pmg_prolong_em(Ctx& up, bool mixed, int Sc, const double* Pm, const double* Uc, const double* solc, bool extrap) {
   FusedState& st = fs(up);
-  const long long rows = (long long)up.z.E * up.z.N;
-  Launch L(up, "pmg_prolong");
-  const int Su = up.z.S, nr = 256 / Su;
-  const size_t lds = ((size_t)Su * Sc + (size_t)nr * Sc) * sizeof(double);
-  if (nr >= 1 && lds <= kTransferLds)
-    hipLaunchKernelGGL(k_prolong_em_lds, dim3((unsigned)((rows + nr - 1) / nr)), dim3(nr * Su), lds, up.stream,
-                       rows, Su, Sc, opgemm_chunk(Sc), nr, Pm, Uc, solc, st.Ue);
-  else
-    hipLaunchKernelGGL(k_prolong_em, dim3(nblk(rows * Su, 256)), dim3(256), 0, up.stream, rows, Su, Sc,
+  const Ops o = get_ops(up, mixed);
+  {
+    Launch L(up, "pmg_prolong");
+    if (o.prolong_lds(up, Sc, opgemm_chunk(Sc), Pm, Uc, solc, extrap)) return;
+    const long long rows = (long long)up.z.E * up.z.N;
+    hipLaunchKernelGGL(k_prolong_em, dim3(nblk(rows * up.z.S, 256)), dim3(256), 0, up.stream, rows, up.z.S, Sc,
                        opgemm_chunk(Sc), Pm, Uc, solc, st.Ue);
-  FCHK(hipGetLastError());
+    FCHK(hipGetLastError());
+  }
+  if (extrap) o.extrap(up);
 }
 
 void fused_end(Ctx& c) {

@@ -187,15 +187,15 @@ void fused_end(Ctx& c);                // export U, divF_spts[0] and wave speeds
 // reads skip it)
 void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep = true);
 // P-multigrid cycle on element-major levels: work arrays and the FAS source
-// allocated; U at the flux points of the current U; the residual (no source)
+// allocated; the start of a cycle; the residual (no source)
 // and the wave speeds, the residual written (how) 0: into divF_spts[0],
 // 1: subtracted from the source in place, 2: plus the source into
 // divF_spts[0]; the source on or off for the RK
-// update; U, divF_spts[0] or the source (which 0, 1, 2); U written back to
-// FlurryPP's layout; the transfers into the coarse level c (U, source, sol)
-// and into the upper level up (U += P (U_c - sol_c)).
+// update; U, divF_spts[0] or the source (which 0, 1, 2); a cycle's results
+// written back to FlurryPP's layout; the transfers into the coarse level c (U,
+// source, sol) and into the upper level up (U += P (U_c - sol_c)), with U at the
+// flux points there.
 void fused_em_prepare(Ctx& c, bool mixed);
-void fused_em_extrap(Ctx& c, bool mixed);
 void fused_em_begin(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool mixed);
 void fused_em_residual(Ctx& c, bool mixed, int how = 0);
 void fused_em_set_src(Ctx& c, bool on);
@@ -203,9 +203,9 @@ double* fused_em_array(Ctx& c, int which);
 void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf);
 // (restriction into the coarse elements [e0, e0 + ne) from the fine rows Uf,
 // divFf of those elements)
-void pmg_restrict_em(Ctx& c, long long e0, long long ne, int Sf, const double* R, const double* Uf,
+void pmg_restrict_em(Ctx& c, bool mixed, long long e0, long long ne, int Sf, const double* R, const double* Uf,
                      const double* divFf, double* solc);
-void pmg_prolong_em(Ctx& up, int Sc, const double* Pm, const double* Uc, const double* solc);
+void pmg_prolong_em(Ctx& up, bool mixed, int Sc, const double* Pm, const double* Uc, const double* solc, bool extrap);
 void fused_residual(Ctx& c, bool mixed);  // divF_spts[0] and wave speeds of the current U
 // block sizes of the fused kernels (extrapolate, face_inviscid, volume, face_boundary, rk)
 void fused_autotune(Ctx& c, bool mixed, int* out);
