@@ -784,6 +784,19 @@ static void pmg_cycle_body(fhip_pmg* mg, const std::vector<char>& fused, const s
   }
 }
 
+// The smoothing steps of an element-major level; source: its FAS source is the
+// restricted residual still, from which the level's own is to be taken.
+static void em_smooth(fhip_pmg* mg, fhip::Ctx& g, bool mixed, bool source) {
+  const bool in_step = source && mg->smooth > 0 && fhip::fused_em_source_in_step(g);
+  if (source && !in_step) fhip::fused_em_residual(g, mixed, 1);
+  fhip::fused_em_set_src(g, true);
+  for (int k = 0; k < mg->smooth; k++) {
+    if (k == 0 && in_step) fhip::fused_rk_step(g, false, mixed, false, true);
+    else update_step(g, true, mixed, true, false, false);
+  }
+  fhip::fused_em_set_src(g, false);
+}
+
 // The same cycle when every level runs a fused path of one precision: the
 // levels stay element-major from the fine level's import to the end (no
 // layout conversions around each residual and smoothing pass); the
@@ -805,19 +818,14 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
   fhip::Ctx* const top = &fine;
   fhip::fused_em_begin(coarse.data(), n - 1, &top, 1, mixed);
   fhip::fused_em_residual(fine, mixed);
-  auto smooth = [&](fhip::Ctx& g) {
-    fhip::fused_em_set_src(g, true);
-    for (int k = 0; k < mg->smooth; k++) update_step(g, true, mixed, true, false, false);
-    fhip::fused_em_set_src(g, false);
-  };
+  auto smooth = [&](fhip::Ctx& g) { em_smooth(mg, g, mixed, false); };
   for (int i = n - 2; i >= 0; i--) {
     fhip::Ctx& g = mg->lv[i]->c;
     fhip::Ctx& f = mg->lv[i + 1]->c;
     // restriction of U and divF_spts[0]; compute_source_term (src/multigrid.cpp:381-398)
     fhip::pmg_restrict_em(g, mixed, 0, g.z.E, f.z.S, mg->R[i], fhip::fused_em_array(f, 0), fhip::fused_em_array(f, 1),
                           mg->sol[i]);
-    fhip::fused_em_residual(g, mixed, 1);  // source -= residual
-    smooth(g);
+    em_smooth(mg, g, mixed, true);  // source -= residual
     if (i > 0) fhip::fused_em_residual(g, mixed, 2);  // residual + source, restricted below
   }
   // upward: smooth again, prolong_err (src/multigrid.cpp:347-364)
@@ -847,11 +855,7 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
   for (fhip_ctx* h : mg->fine) fine.push_back(&h->c);
   fhip::fused_em_begin(coarse.data(), nc, fine.data(), (int)fine.size(), mixed);
   for (fhip::Ctx* f : fine) fhip::fused_em_residual(*f, mixed);
-  auto smooth = [&](fhip::Ctx& g) {
-    fhip::fused_em_set_src(g, true);
-    for (int k = 0; k < mg->smooth; k++) update_step(g, true, mixed, true, false, false);
-    fhip::fused_em_set_src(g, false);
-  };
+  auto smooth = [&](fhip::Ctx& g) { em_smooth(mg, g, mixed, false); };
   for (int j = nc - 1; j >= 0; j--) {
     fhip::Ctx& g = mg->lv[j]->c;
     const long long eA = mg->splitE[j];
@@ -865,8 +869,7 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
       fhip::pmg_restrict_em(g, mixed, eA, g.z.E - eA, f.z.S, mg->R[j], fhip::fused_em_array(f, 0),
                             fhip::fused_em_array(f, 1), mg->sol[j]);
     }
-    fhip::fused_em_residual(g, mixed, 1);  // source -= residual
-    smooth(g);
+    em_smooth(mg, g, mixed, true);  // source -= residual
     if (j > 0) fhip::fused_em_residual(g, mixed, 2);  // residual + source, restricted below
   }
   for (int j = 0; j < nc; j++) {

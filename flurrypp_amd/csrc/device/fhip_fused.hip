@@ -721,6 +721,7 @@ struct RkArgs {
   R* Us;
   int fin;
   R* Ufe;
+  double* makeSrc;  // MK instances of the stage kernel: srce, to be written
 };
 
 // What the update of one solution point reads besides its flux jump and divF,
@@ -792,7 +793,9 @@ __device__ __forceinline__ void correction(const R* sD, int b, const Op& po, con
 // its divF (one value per field), sD the flux jump at the block's flux points,
 // and sU receives the new state (its previous contents are no longer read).
 // The increment is coefficient * residual * (dt / detJ), one division per point.
-template <int D, int P, class R, bool NT, bool TEN>
+// MK (a multigrid level's first smoothing stage): the source becomes itself less
+// the residual that the stage forms, before it is used.
+template <int D, int P, class R, bool NT, bool TEN, bool MK = false>
 __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const R* dv, R* sU, const R* sD, const R* sW,
                                          const RkIn<D, R>& in, const RkArgs<R>& ra, const Tabs& tb) {
   using Sh = Shape<D, P>;
@@ -822,7 +825,12 @@ __device__ __forceinline__ void rk_point(int E, long long e, int b, int s, const
     const double r0 = double(res[k]);
     if (ra.divF0e) st_s<NT>(r0, &ra.divF0e[iu]);
     // P-multigrid source: divF_spts[step] + src_spts (src/solver.cpp:480,514)
-    const double r = ra.srce ? r0 + in.src[k] : r0;
+    double src = in.src[k];
+    if constexpr (MK) {
+      src -= r0;
+      ra.makeSrc[iu] = src;
+    }
+    const double r = ra.srce ? r0 + src : r0;
     const double u = in.u[k];
     double un;
     if (mode == 0) {
@@ -968,7 +976,8 @@ struct StageFace {
   double* wave;        // wave speeds of the left and boundary points, or null: not read before they change again
   const int* bndBc;    // [nBnd] boundary code (number and state row) by slot
   const double* bst;   // boundary-state table
-  // local time step formed here, or wf null
+  // local time step formed here, or wf null: from the wave speeds left by the
+  // stage before, or (MK) those of this stage where it forms them
   const double *wf, *wavein, *dAd, *vole;
   double cflfac;
   double* eleDt;
@@ -985,7 +994,7 @@ struct StageFace {
 // (kApartWaves below).
 __host__ __device__ constexpr int up64(int n) { return (n + 63) / 64 * 64; }
 
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, bool MK = false>
 __device__ __forceinline__ void stage_body(int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us,
                                            const R* __restrict__ JGe, const StageFace<R>& fc, const Tabs& tb,
                                            const Phys& ph, const RkArgs<R>& ra) {
@@ -996,6 +1005,9 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   R* const sU = reinterpret_cast<R*>(fhip_lds);
   R* const sF = sU + EB * N * S;
   R* const sD = sF + EB * D * N * S;
+  // [EB*F] each flux point's term of the local time step: in sD, which the flux
+  // jump takes over later, or (MK) behind it
+  double* const sT = reinterpret_cast<double*>(MK ? sD + EB * N * F : sD);
   __shared__ R sW[Ten<D, P>::NW];
   stage_factors<D, P, R, TEN>(sW, tb);
   const int e0 = blockIdx.x * EB, nb = min(EB, E - e0);
@@ -1056,9 +1068,8 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
     }
 #pragma unroll
     for (int k = 0; k < N; k++) oth[k] = fc.Ufe[pb + k * F];
-    if (fold)
-      reinterpret_cast<double*>(sD)[i] =
-          fc.wavein[(long long)e0 * F + i] * fc.wf[f % Sh::Ff] * fc.dAd[(long long)e0 * F + i];
+    if (fold && (!MK || (cd[u] & 3) == 1))
+      sT[i] = fc.wavein[(long long)e0 * F + i] * fc.wf[f % Sh::Ff] * fc.dAd[(long long)e0 * F + i];
   };
   // the common flux times this side's dA, negated on the right side
   auto common = [&](int u) {
@@ -1074,8 +1085,12 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
       UR[k] = right ? own[k] : oth[k];
     }
     double lam;
-    if (pair_flux<D, R>(BND && side == 2, UL, UR, n, fn, ph, lam) && fc.wave && !right)
-      st_s<NT>(lam, &fc.wave[(long long)e0 * F + fi(u)]);
+    const bool has_lam = pair_flux<D, R>(BND && side == 2, UL, UR, n, fn, ph, lam);
+    if (has_lam && fc.wave && !right) st_s<NT>(lam, &fc.wave[(long long)e0 * F + fi(u)]);
+    if (MK && fold && !right) {
+      const long long i = (long long)e0 * F + fi(u);
+      sT[fi(u)] = (has_lam ? lam : fc.wavein[i]) * fc.wf[fi(u) % Sh::Ff] * fc.dAd[i];
+    }
 #pragma unroll
     for (int k = 0; k < N; k++) {
       const R v = mul_rn(fn[k], dA);
@@ -1098,13 +1113,14 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   }
   __syncthreads();
   double dtl = 0;
+  auto local_dt = [&] {
+    double iw = 0;
+    for (int g = 0; g < F; g++) iw += sT[b * F + g];
+    dtl = fc.cflfac * 2 * fc.vole[e] / iw;
+    if (s == 0) fc.eleDt[e] = dtl;
+  };
   if (act) {
-    if (fold) {
-      double iw = 0;
-      for (int g = 0; g < F; g++) iw += reinterpret_cast<const double*>(sD)[b * F + g];
-      dtl = fc.cflfac * 2 * fc.vole[e] / iw;
-      if (s == 0) fc.eleDt[e] = dtl;
-    }
+    if (!MK && fold) local_dt();
     // flux at the point, transformed to the reference element
     R u[N], Fl[D][N];
     const R* const qu = sU + b * N * S + sw;
@@ -1130,6 +1146,7 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   if (act) {
     // (without the registers for the update's inputs earlier)
     if constexpr (!(APART && D == 2)) in = rk_load<D, P, R, NT>(E, e, s, ra);
+    if (MK && fold) local_dt();
     if (fold) in.dt = dtl;
     const PtOp<D, P, R, TEN> po(tb, sW, s);
     divergence<D, P, R, np>(sF, b, s, sw, swx, opv, abf, po, dv);
@@ -1149,7 +1166,7 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
       for (int k = 0; k < N; k++) o[k * F] = fo[u][k] - fp.efn_sign(line(k * S));
     }
   __syncthreads();
-  if (act) rk_point<D, P, R, NT, TEN>(E, e, b, s, dv, sU, sD, sW, in, ra, tb);
+  if (act) rk_point<D, P, R, NT, TEN, MK>(E, e, b, s, dv, sU, sD, sW, in, ra, tb);
   if (ra.mode == 5 || ra.mode == 7 || ra.mode == 8) return;  // uniform over the launch
   __syncthreads();
 #pragma unroll
@@ -1165,11 +1182,11 @@ __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) 
     Phys ph, RkArgs<R> ra) {
   stage_body<D, P, R, NT, BND, TEN, APART, 0>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF = 0>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF = 0, bool MK = false>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
     int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, APART, BF>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, BF, MK>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
 
 // ---------------------------------------------------------------------------
@@ -2546,7 +2563,7 @@ struct Runner {
     FCHK(hipGetLastError());
   }
   // inviscid runs: the stage kernel with the RK update ra
-  template <bool NT, bool BND, bool TEN, bool APART>
+  template <bool NT, bool BND, bool TEN, bool APART, bool MK = false>
   static void launch_stage_t(Ctx& c, int nt, RkArgs<R> ra, bool fold) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2558,9 +2575,12 @@ struct Runner {
                           fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
     ra.Ufe = st.odd_stage ? w.Ufe : w.Ufe2;
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
-    const int EB = APART ? stage_eles(nt) : nt / S, threads = APART ? stage_threads(EB) : nt;
+    int EB = APART ? stage_eles(nt) : nt / S;
+    auto bytes = [&] { return stage_lds(EB) + (MK ? EB * F * sizeof(double) : 0); };
+    while (EB > 1 && bytes() > kMaxLds) EB--;
+    const int threads = APART ? stage_threads(EB) : (EB == nt / S ? nt : EB * S);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(threads), stage_lds(EB), c.stream, c.z.E, EB, st.Ue, us,
+      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(threads), bytes(), c.stream, c.z.E, EB, st.Ue, us,
                          w.JG, fc, st.tb, c.ph, ra);
     };
     if constexpr (kBf16<D, P, R>) {
@@ -2568,7 +2588,7 @@ struct Runner {
       else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 3>);
       else go(k_stage_w4<D, P, R, NT, BND, TEN, APART>);
     } else if constexpr (kHold<D, R>) {
-      go(k_stage_w4<D, P, R, NT, BND, TEN, APART>);
+      go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, MK>);
     } else {
       go(k_stage_w3<D, P, R, NT, BND, TEN, APART>);
     }
@@ -2585,22 +2605,29 @@ struct Runner {
     else launch_volume_t<false, false, true>(c, nt, wave);
   }
   static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
+    if constexpr (D == 2) {
+      if (ra.makeSrc) return launch_stage_i<true>(c, nt, ra, fold);
+    }
+    if constexpr (kEleRowsWhole) {
+      if (fs(c).tb.w1 && fs(c).stream)
+        return fs(c).nBnd > 0 ? launch_stage_t<true, true, true, false>(c, nt, ra, fold)
+                              : launch_stage_t<true, false, true, false>(c, nt, ra, fold);
+    }
+    launch_stage_i<false>(c, nt, ra, fold);
+  }
+  template <bool MK>
+  static void launch_stage_i(Ctx& c, int nt, const RkArgs<R>& ra, bool fold) {
     const bool bnd = fs(c).nBnd > 0;
     // operators read from their tables: one instance for every mesh
-    if (!fs(c).tb.w1) return launch_stage_t<false, true, false, false>(c, nt, ra, fold);
-    if constexpr (kEleRowsWhole) {
-      if (fs(c).stream)
-        return bnd ? launch_stage_t<true, true, true, false>(c, nt, ra, fold)
-                   : launch_stage_t<true, false, true, false>(c, nt, ra, fold);
-    }
-    if (apart(c) && bnd) launch_stage_t<false, true, true, true>(c, nt, ra, fold);
-    else if (apart(c)) launch_stage_t<false, false, true, true>(c, nt, ra, fold);
-    else if (bnd) launch_stage_t<false, true, true, false>(c, nt, ra, fold);
-    else launch_stage_t<false, false, true, false>(c, nt, ra, fold);
+    if (!fs(c).tb.w1) launch_stage_t<false, true, false, false, MK>(c, nt, ra, fold);
+    else if (apart(c) && bnd) launch_stage_t<false, true, true, true, MK>(c, nt, ra, fold);
+    else if (apart(c)) launch_stage_t<false, false, true, true, MK>(c, nt, ra, fold);
+    else if (bnd) launch_stage_t<false, true, true, false, MK>(c, nt, ra, fold);
+    else launch_stage_t<false, false, true, false, MK>(c, nt, ra, fold);
   }
   // whether a step's first stage forms the elements' time steps itself
   static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
-  static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage) {
+  static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src = false) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     RkB bs{};
@@ -2613,7 +2640,8 @@ struct Runner {
                      st.Uacc,
                      d0, st.eleMesh, st.meshDt, st.active, src,
                      (w.Rst && !st.use_src) ? w.Rst : nullptr, stage, bs, w.Us,
-                     (mode == 2 || mode == 3 || (mode == 4 && stage == c.z.nRK - 1)) ? 1 : 0, w.Ufe};
+                     (mode == 2 || mode == 3 || (mode == 4 && stage == c.z.nRK - 1)) ? 1 : 0, w.Ufe,
+                     make_src ? st.srce : nullptr};
   }
   // the RK kernel of viscous runs; inviscid runs do its work at the end of
   // their stage kernel
@@ -2711,10 +2739,10 @@ struct Runner {
     Launch L(c, nm("fused_volume_viscous", "mixed_volume_viscous"));
     launch_volume(c, blk(c, kVolume), wave);
   }
-  static void rk(Ctx& c, int mode, double a, double b, bool write0, int stage) {
+  static void rk(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src) {
     if (!c.prm.viscous) {
       Launch L(c, nm("fused_stage", "mixed_stage"));
-      launch_stage(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage),
+      launch_stage(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage, make_src),
                    folds_dt(c) && (mode == 0 || mode == 6));
       return;
     }
@@ -2817,7 +2845,7 @@ struct Ops {
   void (*residual)(Ctx&, bool);
   void (*copy_ufe)(Ctx&);
   bool (*folds_dt)(const Ctx&);
-  void (*rk)(Ctx&, int, double, double, bool, int);
+  void (*rk)(Ctx&, int, double, double, bool, int, bool);
   void (*ensure)(Ctx&);
   void (*tune)(Ctx&);
   bool (*check)(Ctx&, const int*);
@@ -2976,7 +3004,17 @@ void fused_em_residual(Ctx& c, bool mixed, int how) {
   Ops o = get_ops(c, mixed);
   fs(c).use_src = false;
   o.residual(c, true);
-  o.rk(c, how == 1 ? 7 : (how == 2 ? 8 : 5), 0., 0., true, 0);
+  o.rk(c, how == 1 ? 7 : (how == 2 ? 8 : 5), 0., 0., true, 0, false);
+}
+
+// Whether a level's first smoothing step can take the residual that its source
+// needs from its own first stage, which forms the same one: inviscid 2-D runs of
+// several stages, where a time step that needs the wave speeds of that residual
+// is formed in the stage too.  One launch of 11 per level on the way down:
+// update and cycle of the P4 channel 67x29 630 -> 611 us.  (Instances of their own:
+// as a switch in the stage kernel it cost every stage 0.5 of 7.2 us.)
+bool fused_em_source_in_step(const Ctx& c) {
+  return !c.prm.viscous && c.z.nRK > 1 && c.z.D == 2 && (c.prm.dt_type == 0 || c.prm.dt_type == 2);
 }
 
 void fused_em_set_src(Ctx& c, bool on) { fs(c).use_src = on; }
@@ -3057,7 +3095,7 @@ void fused_residual(Ctx& c, bool mixed) {
   Ops o = get_ops(c, mixed);
   fused_begin(c, mixed, false);
   o.residual(c, true);
-  o.rk(c, 5, 0., 0., true, 0);
+  o.rk(c, 5, 0., 0., true, 0, false);
   Layouts lay(c.stream);
   lay.from_em(z.S, z.E, z.N, st.divF0e, c.divF);
   lay.from_em(z.F, z.E, 1, st.waveSpe, c.waveSp);
@@ -3065,7 +3103,7 @@ void fused_residual(Ctx& c, bool mixed) {
 }
 
 // One iteration of solver::update (src/solver.cpp:319-363) on a fused path.
-void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
+void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   Ops o = get_ops(c, mixed);
   FusedState& st = fs(c);
   const int nRK = c.z.nRK;
@@ -3082,7 +3120,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
       if (refresh) o.wave(c);
       o.dt(c, cflfac);
     }
-    o.rk(c, jameson ? 4 : 3, A[1], B[0], keep, 0);
+    o.rk(c, jameson ? 4 : 3, A[1], B[0], keep, 0, false);
     if (!c.prm.viscous) o.copy_ufe(c);
     return;
   }
@@ -3098,7 +3136,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep) {
     int mode;
     if (jameson) mode = step == 0 ? 6 : 4;
     else mode = (step == 0) ? 0 : (step == nRK - 1 ? 2 : 1);
-    o.rk(c, mode, A[step + 1], B[step], keep && step == 0, step);
+    o.rk(c, mode, A[step + 1], B[step], keep && step == 0, step, make_src && step == 0);
   }
   st.read_stage = st.odd_stage = false;
   if (!c.prm.viscous && (nRK & 1)) o.copy_ufe(c);

@@ -185,7 +185,10 @@ void fused_begin(Ctx& c, bool mixed, bool src = false);
 void fused_end(Ctx& c);                // export U, divF_spts[0] and wave speeds
 // (keep: write divF_spts[0] at the first stage; steps whose residual nothing
 // reads skip it)
-void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep = true);
+// (make_src, where fused_em_source_in_step: the source less this step's first
+// residual becomes the source, as fused_em_residual's 1 before the step)
+void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep = true, bool make_src = false);
+bool fused_em_source_in_step(const Ctx& c);
 // P-multigrid cycle on element-major levels: work arrays and the FAS source
 // allocated; the start of a cycle; the residual (no source)
 // and the wave speeds, the residual written (how) 0: into divF_spts[0],
