@@ -241,13 +241,26 @@ int fhip_create(const fhip_desc* d, fhip_ctx** out) {
       // lanes of a wave take one flux point of consecutive elements and their
       // rows of every array are neighbours.  In the faces' order each lane's 40
       // bytes lie E rows from the next lane's.
-      std::vector<int> at((size_t)F * E, -1), sl, sr, sb;
-      for (int t = 0; t < z.nFaceFpts; t++) at[c.h_ptL[t]] = t;
-      for (int t : at)
-        if (t >= 0) {
-          sl.push_back(c.h_ptL[t]);
-          sr.push_back(c.h_ptR[t]);
-          sb.push_back(bc[t]);
+      std::vector<int> left((size_t)2 * D * E, -1), sl(z.nFaceFpts), sr(z.nFaceFpts), sb(z.nFaceFpts);
+      std::vector<size_t> at(F, 0);  // where the next element of each flux point goes
+      for (int f = 0; f < z.nFaces; f++) {
+        left[(size_t)d->face_ele_l[f] * 2 * D + d->face_loc_l[f]] = f;
+        at[(size_t)d->face_loc_l[f] * Ff]++;
+      }
+      for (size_t fpt = 0, sum = 0; fpt < (size_t)F; fpt += Ff) {
+        const size_t n = at[fpt];
+        for (int i = 0; i < Ff; i++, sum += n) at[fpt + i] = sum;
+      }
+      for (int e = 0; e < E; e++)
+        for (int l = 0; l < 2 * D; l++) {
+          const int f = left[(size_t)e * 2 * D + l];
+          if (f < 0) continue;
+          for (int i = 0; i < Ff; i++) {
+            const size_t t = (size_t)f * Ff + i, o = at[(size_t)l * Ff + i]++;
+            sl[o] = c.h_ptL[t];
+            sr[o] = c.h_ptR[t];
+            sb[o] = bc[t];
+          }
         }
       c.ft.ptL = dcopy(sl.data(), sl.size(), c.stream);
       c.ft.ptR = dcopy(sr.data(), sr.size(), c.stream);

@@ -2298,6 +2298,17 @@ static void ensure_work(Ctx& c) {
 }
 
 #ifndef FHIP_FAMILY
+// The face's normal, its left element's, at every element flux point (on the host
+// it was the longest part of setting up a 23^3 P4 mesh: 30 of 230 ms).
+static __global__ void k_face_normals(long long n, int F, int D, const int* __restrict__ fpart,
+                                      const double* __restrict__ norme, double* __restrict__ nfe) {
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const int code = fpart[q];
+  const long long l = (code & 3) == 1 ? code >> 2 : q, e = q / F, f = q - e * F, eL = l / F, fL = l - eL * F;
+  for (int x = 0; x < D; x++) nfe[(e * D + x) * F + f] = norme[(eL * D + x) * F + fL];
+}
+
 bool fused_setup(Ctx& c, const fhip_desc* d) {
   const Sizes& z = c.z;
   if (z.P < 0 || z.P > 5) return false;
@@ -2406,18 +2417,11 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
       // the face's normal
       if (E * F >= (1LL << 29)) throw std::invalid_argument("fused path: more than 2^29 element flux points");
       std::vector<int> part((size_t)E * F, -1), bt, bb;
-      std::vector<double> nl((size_t)E * D * F);
-      // the left element's normal at flux point q (element-major q = e*F + f)
-      auto put_normal = [&](int q, int qL) {
-        const long long e = q / F, f = q - e * F, eL = qL / F, fL = qL - eL * F;
-        for (long long x = 0; x < D; x++) nl[(e * D + x) * F + f] = d->norm_fpts[(fL * E + eL) * D + x];
-      };
       for (int t = 0; t < z.nFaceFpts; t++) {
         if (part[pl[t]] != -1 || (pr[t] >= 0 && part[pr[t]] != -1)) {
           fused_release(c);
           return false;
         }
-        put_normal(pl[t], pl[t]);
         if (pr[t] < 0) {
           bt.push_back(t);
           bb.push_back(bc[t]);
@@ -2425,7 +2429,6 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
         } else {
           part[pl[t]] = 4 * pr[t];
           part[pr[t]] = 4 * pl[t] + 1;
-          put_normal(pr[t], pl[t]);
         }
       }
       for (int q : part)
@@ -2437,8 +2440,11 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
       FCHK(hipMemcpy(st->fpart, part.data(), part.size() * 4, hipMemcpyHostToDevice));
       st->nBnd = (int)bt.size();
       st->bndBc = dal<int>(bb.size());
-      st->nfe = dal<double>(nl.size());
-      FCHK(hipMemcpy(st->nfe, nl.data(), nl.size() * 8, hipMemcpyHostToDevice));
+      st->nfe = dal<double>(E * D * F);
+      hipLaunchKernelGGL(k_face_normals, dim3(nblk(E * F, 256)), dim3(256), 0, c.stream, E * F, (int)F, (int)D,
+                         st->fpart, st->norme, st->nfe);
+      FCHK(hipGetLastError());
+      FCHK(hipStreamSynchronize(c.stream));
       if (!bt.empty()) {
         FCHK(hipMemcpy(st->bndBc, bb.data(), bb.size() * 4, hipMemcpyHostToDevice));
       }
