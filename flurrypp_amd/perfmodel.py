@@ -95,10 +95,10 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     if not viscous:
         rd += E * F * (f4 * (2 * N + D + 1) + i4) + nFF * d8 / nRK
     if viscous:
-        # 1/detJ; U across, normal, dA, side code; the corrected divergence, the
-        # LDG side parts and the last stage's wave speeds out
+        # 1/detJ; U across, normal, dA, side code; divF, the flux jump, the LDG
+        # side parts and the last stage's wave speeds out
         rd += E * (f4 * (S + D * F + F) + i4 * F) + f4 * 2 * nFFi * N
-        wr = E * f4 * N * S + f4 * 2 * nFFi * N + nFF * d8 / nRK
+        wr = E * f4 * (N * S + N * F) + f4 * 2 * nFFi * N + nFF * d8 / nRK
         out["mixed_volume_viscous"] = Work(rd + wr, fp["fused_volume_viscous"].flops)
     # classical RK stages keep their residuals in FP32 (the form without a
     # multigrid source); the FP64 state, written at the last stage only, is
@@ -107,7 +107,8 @@ def mixed_work(D: int, P: int, E: int, nFF: int, nFFb: int, viscous: bool, nRK: 
     for st in range(nRK):
         rd_ = E * d8 * S                               # detJ
         if viscous:
-            rd_ += E * (f4 * N * S + f4 * F + i4 * F) + f4 * 2 * nFFi * N  # divF, dA, code; partner's LDG part
+            # divF, the flux jump, dA, code; the partner's LDG part
+            rd_ += E * (f4 * (N * S + N * F + F) + i4 * F) + f4 * 2 * nFFi * N
         wr_ = E * (f4 * N * F + f4 * N * S)            # U at the faces, stage copy of U
         if time_type >= 5:
             rd_ += E * d8 * N * S                      # U0

@@ -93,6 +93,7 @@ def footprint_bytes(nDims: int, order: int, nEles: int, viscous: bool = False, n
     d += 0.5 * (SN + 2 * FN + (nRK - 1) * SN + SN + D * D * S + S + 2 * D * F + F)
     if viscous:
         d += D * SN + D * FN + FN            # staged gradients and dUc
+        d += 0.5 * FN                        # FP32: the flux jump
     if pmg_source:
         d += SN                              # P-multigrid source, element-major
     return int(8 * d * nEles * 1.25) + (16 << 20)
