@@ -814,7 +814,7 @@ static void em_smooth(fhip_pmg* mg, fhip::Ctx& g, bool mixed, bool source) {
 // levels stay element-major from the fine level's import to the end (no
 // layout conversions around each residual and smoothing pass); the
 // transfers act on the element-major arrays.  The coarse levels' wave speeds
-// come in once (the face kernel rewrites only the left and boundary entries,
+// come in once (the stage kernel rewrites only the left and boundary entries,
 // the dt sums all of them).  At the end every level's U, and the fine level's
 // divF_spts[0] and wave speeds, are written back to FlurryPP's layouts (the
 // coarse levels' residual and the wave speeds the cycle computed stay

@@ -68,6 +68,8 @@ extern __shared__ __align__(16) unsigned char fhip_lds[];
 constexpr int kMaxBlock = 512;
 constexpr size_t kMaxLds = 64 * 1024;
 constexpr long long kStreamBytes = 64ll << 20;
+// (kVolume: the stage kernel on inviscid runs; kFaceBnd: no kernel, the place in
+// the block sizes' order remains)
 enum { kExtrap = 0, kFaceInv = 1, kVolume = 2, kFaceBnd = 3, kRk = 4 };
 
 // Sparse operator tables (device pointers into one allocation).  Indices of
@@ -615,7 +617,7 @@ __device__ __forceinline__ void st_s(T v, T* p) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
   else *p = v;
 }
-// A product rounded on its own (never contracted into a following add).
+// A product meant to be rounded on its own before a following add.
 __device__ __forceinline__ double mul_rn(double a, double b) { return __dmul_rn(a, b); }
 __device__ __forceinline__ float mul_rn(float a, float b) { return __fmul_rn(a, b); }
 
@@ -2540,7 +2542,7 @@ struct Runner {
   // 26.4 / 28.9, P2 28^3 (27783) 64.2 / 62.2.
   static constexpr long long kApartWaves = D == 3 && P >= 1 && P <= 3 && sizeof(R) == 8 ? 12288 : 4096;
   static bool apart(const Ctx& c) { return (long long)c.z.E * (S + F) <= kApartWaves * 64; }
-  // LDS bytes of an element kernel at block size nt (0 for the face kernels)
+  // LDS bytes of an element kernel at block size nt (0 for the face kernel)
   static size_t lds(int k, int nt, bool visc) {
     const size_t EB = nt / S;
     const size_t SF = (visc && F > D * S) ? F : D * S;
@@ -2788,7 +2790,7 @@ struct Runner {
   // keep the fastest.  The RK kernel (and the stage kernel of inviscid runs,
   // which includes the update) runs in its middle-stage mode, which rewrites
   // U and the RK accumulator: both are saved and restored, as are the wave
-  // speeds the face kernel writes; block shapes never change results.
+  // speeds; block shapes never change results.
   static void tune(Ctx& c) {
     FusedState& st = fs(c);
     const bool visc = c.prm.viscous != 0;
