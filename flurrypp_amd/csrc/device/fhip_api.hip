@@ -849,7 +849,7 @@ static void pmg_cycle_body_em(fhip_pmg* mg, bool mixed) {
     // (a coarse level smooths from there)
     fhip::pmg_prolong_em(up, mixed, g.z.S, mg->Pro[i], fhip::fused_em_array(g, 0), mg->sol[i], i + 2 < n);
   }
-  fhip::fused_em_end(coarse.data(), n - 1, &top, 1);
+  fhip::fused_em_end(coarse.data(), n - 1, &top, 1, mg->smooth > 0);
 }
 
 // The batched cycle: every mesh goes through the steps of
@@ -898,7 +898,7 @@ static void pmg_cycle_body_batch(fhip_pmg* mg, bool mixed) {
       fhip::pmg_prolong_em(up, mixed, g.z.S, mg->Pro[j], fhip::fused_em_array(g, 0) + offA, mg->sol[j] + offA, true);
     }
   }
-  fhip::fused_em_end(coarse.data(), nc, fine.data(), (int)fine.size());
+  fhip::fused_em_end(coarse.data(), nc, fine.data(), (int)fine.size(), mg->smooth > 0);
 }
 
 // The first cycle on a path runs launch by launch (it also allocates what the

@@ -489,6 +489,40 @@ template <>
 inline Work<float>& FusedState::work<float>() { return w32; }
 
 // ---------------------------------------------------------------------------
+// Minimum over the block (a multiple of 64 threads, at most 256), returned to
+// every thread: across each wave by lane exchanges, then across the waves
+// through red.  min is exact, so the order of the comparisons does not matter.
+__device__ __forceinline__ double block_min(double v, double* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
+  __syncthreads();  // red may still be read by an earlier call
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = red[0];
+  for (int w = 1; w < (int)(blockDim.x >> 6); w++) v = fmin(v, red[w]);
+  return v;
+}
+
+// The minimum of `blocks` blocks' minima (thread 0 of each calls this) at out, put
+// there by the block that finishes last, which also sets counter and accumulator
+// back (0, infinity) for the next launch; a single block's minimum is the result at
+// once.  Through atomics alone: a release here would write back what the kernel
+// before left in the L2, which took longer than all else.  The minimum's own result
+// is waited for, so it is in place before the block is counted, and the last
+// block's exchange comes after all of them.
+__device__ __forceinline__ void grid_min(double bmin, unsigned blocks, double* acc, unsigned* ticket, double* out) {
+  if (blocks == 1) {
+    *out = bmin;
+    return;
+  }
+  const double before = __hip_atomic_fetch_min(acc, bmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::"v"(before) : "memory");
+  const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t != blocks - 1) return;
+  *out = __hip_atomic_exchange(acc, double(INFINITY), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 #ifndef FHIP_FAMILY
 // Layout conversions between FlurryPP's [pt][ele][k] and element-major
 // [ele][k][pt]: both are the transpose of a matrix with one row per point,
@@ -497,19 +531,43 @@ inline Work<float>& FusedState::work<float>() { return w32; }
 // a call converts at one place (Layouts): on a small mesh each launch is some 4
 // us.  One each -> together: a step of the 8x8 P3 vortex 55 -> 49 us, update and
 // cycle of the P4 channel 67x29 690 -> 652 us.
-constexpr int kTile = 32, kMaxLayouts = 16;
+//
+// The same launch puts the minimum of an array at one place (Least), in blocks after
+// the tiles: the solver's dt after local time steps, whose elements' the stage
+// kernel forms (a launch of its own per level would be some 4 us of a call's 600).
+constexpr int kTile = 32, kMaxLayouts = 16, kMaxLeast = 8;
+constexpr long long kLeastPerBlock = 4096;
 struct LayoutJobs {
-  int n = 0;
-  unsigned tiles = 0;
+  int n = 0, nLeast = 0;
+  unsigned tiles = 0, blocks = 0;  // blocks: tiles and the minima's blocks
   struct Job {
     long long R, C;  // in [R][C] -> out [C][R]
     const double* in;
     double* out;
     unsigned first;  // its first tile
   } job[kMaxLayouts];
+  struct Least {
+    long long n;
+    const double* in;
+    double *acc, *out;
+    unsigned* ticket;
+    unsigned first, blocks;  // its first block after the tiles, their number
+  } least[kMaxLeast];
 };
 static __global__ __launch_bounds__(256) void k_transpose(LayoutJobs jobs) {
   __shared__ double t[kTile][kTile + 1];
+  if (blockIdx.x >= jobs.tiles) {
+    const unsigned b = blockIdx.x - jobs.tiles;
+    int n = 0;
+    while (n + 1 < jobs.nLeast && b >= jobs.least[n + 1].first) n++;
+    const LayoutJobs::Least& lb = jobs.least[n];
+    double v = INFINITY;
+    for (long long i = (long long)(b - lb.first) * blockDim.x + threadIdx.x; i < lb.n; i += (long long)lb.blocks * blockDim.x)
+      v = fmin(v, lb.in[i]);
+    v = block_min(v, &t[0][0]);
+    if (threadIdx.x == 0) grid_min(v, lb.blocks, lb.acc, lb.ticket, lb.out);
+    return;
+  }
   int n = 0;
   while (n + 1 < jobs.n && blockIdx.x >= jobs.job[n + 1].first) n++;
   const LayoutJobs::Job& jb = jobs.job[n];
@@ -538,20 +596,27 @@ struct Layouts {
   hipStream_t st;
   LayoutJobs jobs;
   explicit Layouts(hipStream_t s) : st(s) {}
+  void least(long long n, const double* in, double* acc, unsigned* ticket, double* out) {
+    if (jobs.nLeast == kMaxLeast) go();
+    const unsigned blocks = (unsigned)((n + kLeastPerBlock - 1) / kLeastPerBlock);
+    jobs.least[jobs.nLeast++] = LayoutJobs::Least{n, in, acc, out, ticket, jobs.blocks - jobs.tiles, blocks};
+    jobs.blocks += blocks;
+  }
   void add(long long R, long long C, const double* in, double* out) {
     if (R == 0 || C == 0) return;
     const long long tiles = ((R + kTile - 1) / kTile) * ((C + kTile - 1) / kTile);
-    if (jobs.n == kMaxLayouts || jobs.tiles + tiles > 0x7fffffffll) go();
+    if (jobs.n == kMaxLayouts || jobs.blocks + tiles > 0x7fffffffll) go();
     jobs.job[jobs.n++] = LayoutJobs::Job{R, C, in, out, jobs.tiles};
     jobs.tiles += (unsigned)tiles;
+    jobs.blocks += (unsigned)tiles;
   }
   // in [P][E][K] -> out [E][K][P]
   void to_em(int P, long long E, int K, const double* in, double* out) { add(P, E * K, in, out); }
   // in [E][K][P] -> out [P][E][K]
   void from_em(int P, long long E, int K, const double* in, double* out) { add(E * K, P, in, out); }
   void go() {
-    if (jobs.n) {
-      hipLaunchKernelGGL(k_transpose, dim3(jobs.tiles), dim3(256), 0, st, jobs);
+    if (jobs.blocks) {
+      hipLaunchKernelGGL(k_transpose, dim3(jobs.blocks), dim3(256), 0, st, jobs);
       FCHK(hipGetLastError());
     }
     jobs = LayoutJobs();
@@ -1880,20 +1945,6 @@ __global__ void k_wave_em(int E, const R* __restrict__ Ufe, const double* __rest
   waveSpe[i] = (fabs(vN - 0.) + sqrt(csq));
 }
 
-// Minimum over the block (a multiple of 64 threads, at most 256), returned to
-// every thread: across each wave by lane exchanges, then across the waves
-// through red.  min is exact, so the order of the comparisons does not matter.
-__device__ __forceinline__ double block_min(double v, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-  __syncthreads();  // red may still be read by an earlier call
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  v = red[0];
-  for (int w = 1; w < (int)(blockDim.x >> 6); w++) v = fmin(v, red[w]);
-  return v;
-}
-
 // The element volumes calcDt divides by, once per context (the geometry is
 // fixed): the same sum as the reference's per call.
 template <int D, int P>
@@ -1920,10 +1971,8 @@ template <int D>
 constexpr int kDtEles = D == 2 ? 2 : 4;
 constexpr unsigned kDtBlocks = 256;
 
-// ele::calcDt per element (element-major inputs).  With a ticket counter, the
-// block that finishes last also puts the minimum of all at out, the global dt
-// (solver::calcDt, src/solver.cpp:447-468), and sets counter and accumulator back
-// for the next launch (a single block's minimum is the global dt at once).
+// ele::calcDt per element (element-major inputs) and, with a ticket counter, the
+// minimum of all at out, the global dt (solver::calcDt, src/solver.cpp:447-468).
 template <int D, int P>
 __global__ __launch_bounds__(256) void k_ele_dt_em(int E, const double* __restrict__ vole, const double* __restrict__ wf,
                                                     const double* __restrict__ waveSpe, const double* __restrict__ dAe,
@@ -1962,21 +2011,7 @@ __global__ __launch_bounds__(256) void k_ele_dt_em(int E, const double* __restri
   }
   const double bmin = block_min(dt, red);
   if (!ticket) return;  // merged meshes: per-mesh minima of eleDt follow
-  if (gridDim.x == 1) {  // one block: its minimum is the global one
-    if (threadIdx.x == 0) *out = bmin;
-    return;
-  }
-  if (threadIdx.x != 0) return;
-  // through atomics alone: a release here would write back what the stage before
-  // left in the L2, which took longer than all else.  The minimum's own result
-  // is waited for, so it is in place before the block is counted, and the last
-  // block's exchange comes after all of them.
-  const double before = __hip_atomic_fetch_min(acc, bmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  asm volatile("s_waitcnt vmcnt(0)" ::"v"(before) : "memory");
-  const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (t != gridDim.x - 1) return;
-  *out = __hip_atomic_exchange(acc, double(INFINITY), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) grid_min(bmin, gridDim.x, acc, ticket, out);
 }
 
 // Per-mesh minimum of the element time steps (batched contexts, dt_type 1).
@@ -2278,6 +2313,10 @@ static void set_geometry(Ctx& c, Work<float>& w) {
 // A single-stage step with a CFL time step takes its dt from the wave speeds of
 // the residual it is about to apply (solver::update), so they are formed in a
 // launch of their own before it.
+static bool folds_dt(const Ctx& c) {
+  // whether a step's first stage forms the elements' time steps itself
+  return c.z.D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1;
+}
 static bool face_first(const Ctx& c) { return !c.prm.viscous && c.z.nRK == 1 && c.prm.dt_type != 0; }
 
 template <class R>
@@ -2662,8 +2701,6 @@ struct Runner {
     else if (bnd) launch_stage_t<false, true, true, false, MK>(c, nt, ra, fold);
     else launch_stage_t<false, false, true, false, MK>(c, nt, ra, fold);
   }
-  // whether a step's first stage forms the elements' time steps itself
-  static bool folds_dt(const Ctx& c) { return D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1; }
   static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src = false) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
@@ -2881,7 +2918,6 @@ struct Ops {
   void (*face)(Ctx&);
   void (*residual)(Ctx&, bool);
   void (*copy_ufe)(Ctx&);
-  bool (*folds_dt)(const Ctx&);
   void (*rk)(Ctx&, int, double, double, bool, int, bool);
   void (*ensure)(Ctx&);
   void (*tune)(Ctx&);
@@ -2894,7 +2930,7 @@ struct Ops {
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::folds_dt, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
+  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
 }
 
 // The kernels of one dimension, precision and range of orders.  This file is
@@ -3061,6 +3097,13 @@ double* fused_em_array(Ctx& c, int which) {
   return which == 0 ? st.Ue : (which == 1 ? st.divF0e : st.srce);
 }
 
+// The solver's dt of a call whose steps formed the elements' in their stages: their
+// minimum (solver::calcDt, src/solver.cpp:447-468).  Merged meshes have none.
+static void add_dt(Ctx& c, Layouts& lay) {
+  FusedState& st = fs(c);
+  if (folds_dt(c) && st.nMesh == 1) lay.least(c.z.E, c.eleDt, st.dtAcc, st.dtTicket, c.d_dt);
+}
+
 static void add_end(Ctx& c, Layouts& lay) {
   FusedState& st = fs(c);
   st.use_src = false;
@@ -3070,14 +3113,15 @@ static void add_end(Ctx& c, Layouts& lay) {
   lay.from_em(z.F, z.E, 1, st.waveSpe, c.waveSp);
 }
 
-// The end of a cycle on the element-major levels: U of the coarse levels cs, and
-// what fused_end writes back of the fine ones.
-void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf) {
+// The end of a cycle on the element-major levels: U of the coarse levels (stepped:
+// and their dt), U, divF_spts[0] and wave speeds of the fine ones, which took no step.
+void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool stepped) {
   Layouts lay(fine[0]->stream);
   for (int i = 0; i < nc; i++) {
     Ctx& c = *coarse[i];
     fs(c).use_src = false;
     lay.from_em(c.z.S, c.z.E, c.z.N, fs(c).Ue, c.U);
+    if (stepped) add_dt(c, lay);
   }
   for (int i = 0; i < nf; i++) add_end(*fine[i], lay);
   lay.go();
@@ -3121,6 +3165,7 @@ void pmg_prolong_em(Ctx& up, bool mixed, int Sc, const double* Pm, const double*
 void fused_end(Ctx& c) {
   Layouts lay(c.stream);
   add_end(c, lay);
+  add_dt(c, lay);
   lay.go();
 }
 
@@ -3163,7 +3208,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   }
   if (cfl) {
     if (refresh) o.wave(c);
-    if (!o.folds_dt(c)) o.dt(c, cflfac);
+    if (!folds_dt(c)) o.dt(c, cflfac);
   }
   for (int step = 0; step < nRK; step++) {
     st.read_stage = step > 0;

@@ -182,7 +182,7 @@ bool fused_setup(Ctx& c, const fhip_desc* d);  // false: configuration not cover
 void fused_release(Ctx& c);
 // import U, wave speeds [and the P-multigrid source], extrapolate U to the faces
 void fused_begin(Ctx& c, bool mixed, bool src = false);
-void fused_end(Ctx& c);                // export U, divF_spts[0] and wave speeds
+void fused_end(Ctx& c);                // after steps: export U, divF_spts[0], wave speeds and dt
 // (keep: write divF_spts[0] at the first stage; steps whose residual nothing
 // reads skip it)
 // (make_src, where fused_em_source_in_step: the source less this step's first
@@ -203,7 +203,7 @@ void fused_em_begin(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool m
 void fused_em_residual(Ctx& c, bool mixed, int how = 0);
 void fused_em_set_src(Ctx& c, bool on);
 double* fused_em_array(Ctx& c, int which);
-void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf);
+void fused_em_end(Ctx* const* coarse, int nc, Ctx* const* fine, int nf, bool stepped);
 // (restriction into the coarse elements [e0, e0 + ne) from the fine rows Uf,
 // divFf of those elements)
 void pmg_restrict_em(Ctx& c, bool mixed, long long e0, long long ne, int Sf, const double* R, const double* Uf,
