@@ -2311,13 +2311,14 @@ static void set_geometry(Ctx& c, Work<float>& w) {
 }
 
 // A single-stage step with a CFL time step takes its dt from the wave speeds of
-// the residual it is about to apply (solver::update), so they are formed in a
-// launch of their own before it.
+// the residual it is about to apply (solver::update), so they are formed, and on
+// the refresh step replaced by the points' own, in launches of their own before it.
+// Its stage kernel then leaves them.
+static bool face_first(const Ctx& c) { return !c.prm.viscous && c.z.nRK == 1 && c.prm.dt_type != 0; }
+// Whether a step's first stage forms the elements' time steps itself.
 static bool folds_dt(const Ctx& c) {
-  // whether a step's first stage forms the elements' time steps itself
   return c.z.D == 2 && !c.prm.viscous && c.prm.dt_type == 2 && c.z.nRK > 1;
 }
-static bool face_first(const Ctx& c) { return !c.prm.viscous && c.z.nRK == 1 && c.prm.dt_type != 0; }
 
 template <class R>
 static void ensure_work(Ctx& c) {
@@ -2645,7 +2646,7 @@ struct Runner {
     Work<R>& w = st.work<R>();
     // wave speeds are read by the next step's dt and after the call: stages
     // that another stage follows leave them
-    const bool wave = ra.fin || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
+    const bool wave = (ra.fin && !face_first(c)) || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
     const StageFace<R> fc{st.fpart, st.odd_stage ? w.Ufe2 : w.Ufe, w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
                           st.bst, fold ? c.wf : nullptr, st.waveSpe, st.dAe, st.vole,
                           fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
@@ -3197,7 +3198,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   st.odd_stage = false;
   if (nRK == 1) {
     if (c.prm.viscous) o.residual(c, true);
-    else if (cfl) o.face(c);
+    else if (face_first(c)) o.face(c);
     if (cfl) {
       if (refresh) o.wave(c);
       o.dt(c, cflfac);
