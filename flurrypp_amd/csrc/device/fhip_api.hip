@@ -77,10 +77,8 @@ void destroy_ctx(fhip::Ctx& c) {
   if (c.device >= 0) (void)hipSetDevice(c.device);
   fhip::fused_release(c);
   fhip::staged_release(c);
-  for (auto& plane : c.graph)
-    for (auto& row : plane)
-      for (auto& g : row)
-        if (g) (void)hipGraphExecDestroy(g);
+  for (auto& g : c.graph)
+    if (g) (void)hipGraphExecDestroy(g);
   void* ptrs[] = {c.sf, c.grad, c.efn, c.corr, c.corru, c.ws, c.wf, c.tp, c.jginv, c.detj, c.norm, c.da,
                   c.ft.ptL, c.ft.ptR, c.ft.bc, c.U, c.U0, c.Uf, c.Fs, c.dU, c.dUf, c.dUc, c.disFn, c.Fn,
                   c.divF, c.waveSp, c.eleDt, c.faceFn, c.src, c.Uacc, c.d_dt, c.partial, c.flag};
@@ -494,9 +492,12 @@ static void update_step(fhip::Ctx& c, bool fused, bool mixed, bool src = false, 
     // Steady-state steps replay one captured graph; the wave-speed refresh
     // step and timed runs launch kernel by kernel.
     if (!refresh && !c.timing && c.use_graphs && !t_capturing_cycle) {
-      hipGraphExec_t& ge = c.graph[src ? 1 : 0][keep ? 1 : 0][mixed ? 1 + (c.bf16 ? c.bf16 - 1 : 0) : 0];
+      const bool flipped = fhip::fused_flipped(c);
+      hipGraphExec_t& ge =
+          c.graph[fhip::Ctx::graph_slot(src, keep, mixed ? 1 + (c.bf16 ? c.bf16 - 1 : 0) : 0, flipped)];
       if (!ge) ge = capture(c.stream, [&] { fhip::fused_rk_step(c, false, mixed, keep); });
       HCHK(hipGraphLaunch(ge, c.stream));
+      fhip::fused_set_flipped(c, flipped != fhip::fused_step_flips(c));
     } else {
       fhip::fused_rk_step(c, refresh, mixed, keep);
     }

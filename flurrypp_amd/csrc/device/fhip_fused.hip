@@ -409,7 +409,7 @@ template <class R>
 struct Work {
   R *divFe = nullptr, *Ufe = nullptr;
   // inviscid runs: U at the flux points of every second stage (a stage reads
-  // one of Ufe, Ufe2 and writes the other; a step starts and ends in Ufe)
+  // one of Ufe, Ufe2 and writes the other; a call starts in Ufe)
   R* Ufe2 = nullptr;
   // viscous runs: each flux point's side of the LDG flux [ele][N][F] (divFe then
   // holds the divergence corrected with all but the other sides' parts)
@@ -461,8 +461,10 @@ struct FusedState {
   // stages after the first of an RK step); otherwise from the state itself.
   // FP32 kernels always read the FP32 copy.
   bool read_stage = false;
-  // inviscid runs: the stage being formed reads U at the flux points from Ufe2
-  bool odd_stage = false;
+  // inviscid runs: U at the flux points of the current state is in Ufe2.  A step of
+  // an odd number of stages ends there (a copy back to Ufe took 2.4 of the 28.5 us
+  // of a single-stage step of a channel 113x41 P3).
+  bool flipped = false;
   // stream once-touched arrays past the caches: set when U alone (FP64,
   // element-major) exceeds kStreamBytes, i.e. a stage's arrays are many times
   // the 256 MiB infinity cache
@@ -1748,11 +1750,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
   }
 }
 
-template <class R>
-__global__ void k_copy_em(long long n, R* __restrict__ dst, const R* __restrict__ src) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
 
 // P-multigrid transfers in element-major layout ([ele][field][point] rows of
 // S values), the products the staged operator GEMM forms in FlurryPP's layout
@@ -2603,15 +2600,18 @@ struct Runner {
     // written by a step's first stage (which reads the state itself)
     auto* kern = st.tb.w1 ? k_extrap<D, P, R, true> : k_extrap<D, P, R, false>;
     hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kExtrap, nt, false), c.stream, c.z.E, st.Ue, w.Ufe, sizeof(R) == 4 ? w.Us : nullptr, st.tb);
+    st.flipped = false;
     FCHK(hipGetLastError());
   }
+  // U at the flux points of the current state
+  static R* cur_ufe(Ctx& c) { return fs(c).flipped ? fs(c).work<R>().Ufe2 : fs(c).work<R>().Ufe; }
   static void launch_face_inv(Ctx& c, int nt) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     const int nFF = c.z.nFaceFpts;
     if (nFF == 0) return;
     hipLaunchKernelGGL((k_face_inv<D, P, R>), dim3(nblk(nFF, nt)), dim3(nt), 0, c.stream, nFF, st.pL, st.pR, st.bc,
-                       w.Ufe, w.nrm, st.waveSpe, c.ph, st.bst);
+                       cur_ufe(c), w.nrm, st.waveSpe, c.ph, st.bst);
     FCHK(hipGetLastError());
   }
   // viscous runs: the volume kernel.  Quads and FP32 are held to 4 waves per
@@ -2647,10 +2647,10 @@ struct Runner {
     // wave speeds are read by the next step's dt and after the call: stages
     // that another stage follows leave them
     const bool wave = (ra.fin && !face_first(c)) || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
-    const StageFace<R> fc{st.fpart, st.odd_stage ? w.Ufe2 : w.Ufe, w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
+    const StageFace<R> fc{st.fpart, cur_ufe(c), w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
                           st.bst, fold ? c.wf : nullptr, st.waveSpe, st.dAe, st.vole,
                           fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
-    ra.Ufe = st.odd_stage ? w.Ufe : w.Ufe2;
+    ra.Ufe = st.flipped ? w.Ufe : w.Ufe2;
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
     int EB = APART ? stage_eles(nt) : nt / S;
     auto bytes = [&] { return stage_lds(EB) + (MK ? EB * F * sizeof(double) : 0); };
@@ -2731,15 +2731,6 @@ struct Runner {
                        rk_args(c, mode, a, b, write0, stage), st.tb, st.fpart, w.dA, w.Bve, w.Jne);
     FCHK(hipGetLastError());
   }
-  // after a step with an odd number of stages: U at the flux points back
-  // where every step starts
-  static void copy_ufe(Ctx& c) {
-    Work<R>& w = fs(c).work<R>();
-    const long long n = (long long)c.z.E * N * F;
-    Launch L(c, nm("fused_copy", "mixed_copy"));
-    hipLaunchKernelGGL(k_copy_em<R>, dim3(nblk(n, 256)), dim3(256), 0, c.stream, n, w.Ufe, w.Ufe2);
-    FCHK(hipGetLastError());
-  }
   static void extrap(Ctx& c) {
     Launch L(c, nm("fused_extrapolate", "mixed_extrapolate"));
     launch_extrap(c, blk(c, kExtrap));
@@ -2760,6 +2751,7 @@ struct Runner {
     hipLaunchKernelGGL(kern, dim3(nblk(ne, EB)), dim3(nr * S), bytes, c.stream, (int)ne, EB, Sf, kc, A, Uf, divFf,
                        st.Ue + off, st.srce + off, solc + off, w.Ufe + e0 * N * F,
                        sizeof(R) == 4 ? w.Us + off : nullptr, st.tb);
+    st.flipped = false;
     FCHK(hipGetLastError());
     return true;
   }
@@ -2772,6 +2764,7 @@ struct Runner {
     auto* kern = st.tb.w1 ? k_prolong_lds<D, P, R, true> : k_prolong_lds<D, P, R, false>;
     hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(nr * S), bytes, c.stream, c.z.E, EB, Sc, kc, A, Uc, solc,
                        st.Ue, extrap ? w.Ufe : nullptr, sizeof(R) == 4 ? w.Us : nullptr, st.tb);
+    if (extrap) st.flipped = false;
     FCHK(hipGetLastError());
     return true;
   }
@@ -2779,7 +2772,7 @@ struct Runner {
     FusedState& st = fs(c);
     long long n = (long long)c.z.E * Sh::F;
     Launch L(c, nm("fused_wave_speed", "mixed_wave_speed"));
-    hipLaunchKernelGGL((k_wave_em<D, P, R>), dim3(nblk(n, 256)), dim3(256), 0, c.stream, c.z.E, st.work<R>().Ufe, st.norme,
+    hipLaunchKernelGGL((k_wave_em<D, P, R>), dim3(nblk(n, 256)), dim3(256), 0, c.stream, c.z.E, cur_ufe(c), st.norme,
                        st.waveSpe, c.ph.gamma);
     FCHK(hipGetLastError());
   }
@@ -2819,6 +2812,8 @@ struct Runner {
       Launch L(c, nm("fused_stage", "mixed_stage"));
       launch_stage(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage, make_src),
                    folds_dt(c) && (mode == 0 || mode == 6));
+      // (the residual alone leaves U)
+      if (mode != 5 && mode != 7 && mode != 8) fs(c).flipped = !fs(c).flipped;
       return;
     }
     Launch L(c, nm("fused_rk_update", "mixed_rk_update"));
@@ -2918,7 +2913,6 @@ struct Ops {
   void (*dt)(Ctx&, double);
   void (*face)(Ctx&);
   void (*residual)(Ctx&, bool);
-  void (*copy_ufe)(Ctx&);
   void (*rk)(Ctx&, int, double, double, bool, int, bool);
   void (*ensure)(Ctx&);
   void (*tune)(Ctx&);
@@ -2931,7 +2925,7 @@ struct Ops {
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::copy_ufe, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
+  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
 }
 
 // The kernels of one dimension, precision and range of orders.  This file is
@@ -3019,7 +3013,7 @@ void fused_get_blocks(Ctx& c, bool mixed, int* out) {
 // What a call on the fused paths starts from, element-major.
 static void add_begin(Ctx& c, bool mixed, bool src, Layouts& lay) {
   FusedState& st = fs(c);
-  st.read_stage = st.odd_stage = false;
+  st.read_stage = st.flipped = false;
   const Sizes& z = c.z;
   get_ops(c, mixed).ensure(c);
   long long nS = (long long)z.E * z.N * z.S;
@@ -3050,7 +3044,7 @@ static int opgemm_chunk(int k) { return k <= 16 ? 16 : (k <= 32 ? 32 : 64); }
 
 void fused_em_prepare(Ctx& c, bool mixed) {
   FusedState& st = fs(c);
-  st.read_stage = st.odd_stage = false;
+  st.read_stage = st.flipped = false;
   get_ops(c, mixed).ensure(c);
   if (!st.srce) {
     c.drop_graphs();
@@ -3195,7 +3189,6 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   const bool cfl = c.prm.dt_type != 0;
   const double cflfac = cfl ? c.prm.cfl * cfl_limit_f(c.z.P) : 0.;
   const bool jameson = c.prm.time_type >= 5;
-  st.odd_stage = false;
   if (nRK == 1) {
     if (c.prm.viscous) o.residual(c, true);
     else if (face_first(c)) o.face(c);
@@ -3204,7 +3197,6 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
       o.dt(c, cflfac);
     }
     o.rk(c, jameson ? 4 : 3, A[1], B[0], keep, 0, false);
-    if (!c.prm.viscous) o.copy_ufe(c);
     return;
   }
   if (cfl) {
@@ -3213,7 +3205,6 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   }
   for (int step = 0; step < nRK; step++) {
     st.read_stage = step > 0;
-    st.odd_stage = !c.prm.viscous && (step & 1);
     o.residual(c, step == nRK - 1);
     // the Jameson form's first stage reads the state itself (the step's U0)
     int mode;
@@ -3221,9 +3212,12 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
     else mode = (step == 0) ? 0 : (step == nRK - 1 ? 2 : 1);
     o.rk(c, mode, A[step + 1], B[step], keep && step == 0, step, make_src && step == 0);
   }
-  st.read_stage = st.odd_stage = false;
-  if (!c.prm.viscous && (nRK & 1)) o.copy_ufe(c);
+  st.read_stage = false;
 }
+
+bool fused_flipped(const Ctx& c) { return ((const FusedState*)c.fused)->flipped; }
+void fused_set_flipped(Ctx& c, bool flipped) { fs(c).flipped = flipped; }
+bool fused_step_flips(const Ctx& c) { return !c.prm.viscous && (c.z.nRK & 1); }
 
 #endif  // FHIP_FAMILY
 

@@ -97,27 +97,27 @@ struct Ctx {
   bool timing = false;
   Timer timer;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // captured RK steps (fused path): [with P-multigrid source][keeping
-  // divF_spts[0]][FP64, mixed, mixed with BF16 hi+lo, mixed with BF16
-  // hi+mid+lo].  A graph holds the device pointers of the moment it was
-  // captured: drop them whenever an array they use is (re)allocated.
-  hipGraphExec_t graph[2][2][4] = {};
+  // captured RK steps (fused path), by graph_slot: with P-multigrid source,
+  // keeping divF_spts[0], FP64, mixed, mixed with BF16 hi+lo, mixed with BF16
+  // hi+mid+lo, U at the flux points in the second copy (fused_flipped).  A graph
+  // holds the device pointers of the moment it was captured: drop them
+  // whenever an array they use is (re)allocated.
+  hipGraphExec_t graph[32] = {};
+  static int graph_slot(bool src, bool keep, int precision, bool flipped) {
+    return ((flipped * 4 + precision) * 2 + keep) * 2 + src;
+  }
   // mixed path: BF16 pieces of the matrix-core z contractions (0: none)
   int bf16 = 0;
   unsigned long long graph_gen = 0;  // bumped by drop_graphs: graphs over several contexts check it
   void drop_graphs() {
     graph_gen++;
     bool any = false;
-    for (auto& plane : graph)
-      for (auto& row : plane)
-        for (auto& g : row) any = any || g != nullptr;
+    for (auto& g : graph) any = any || g != nullptr;
     if (any) (void)hipStreamSynchronize(stream);  // no replay still in flight
-    for (auto& plane : graph)
-      for (auto& row : plane)
-        for (auto& g : row) {
-          if (g) (void)hipGraphExecDestroy(g);
-          g = nullptr;
-        }
+    for (auto& g : graph) {
+      if (g) (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
   }
   bool fused_ok = false;
   bool use_graphs = true;
@@ -189,6 +189,11 @@ void fused_end(Ctx& c);                // after steps: export U, divF_spts[0], w
 // residual becomes the source, as fused_em_residual's 1 before the step)
 void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep = true, bool make_src = false);
 bool fused_em_source_in_step(const Ctx& c);
+// Inviscid runs: whether U at the flux points lies in the second of its two copies
+// (after an odd number of stages since the call's start); a replayed step's flip.
+bool fused_flipped(const Ctx& c);
+void fused_set_flipped(Ctx& c, bool flipped);
+bool fused_step_flips(const Ctx& c);
 // P-multigrid cycle on element-major levels: work arrays and the FAS source
 // allocated; the start of a cycle; the residual (no source)
 // and the wave speeds, the residual written (how) 0: into divF_spts[0],
