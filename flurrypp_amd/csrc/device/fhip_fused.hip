@@ -491,9 +491,9 @@ template <>
 inline Work<float>& FusedState::work<float>() { return w32; }
 
 // ---------------------------------------------------------------------------
-// Minimum over the block (a multiple of 64 threads, at most 256), returned to
-// every thread: across each wave by lane exchanges, then across the waves
-// through red.  min is exact, so the order of the comparisons does not matter.
+// Minimum over the block (a multiple of 64 threads), returned to every thread:
+// across each wave by lane exchanges, then across the waves through red, one
+// entry each.  min is exact, so the order of the comparisons does not matter.
 __device__ __forceinline__ double block_min(double v, double* red) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
@@ -1961,7 +1961,11 @@ __global__ __launch_bounds__(256) void k_ele_vol(int E, const double* __restrict
 // thread per element walked its points one after the other, each read 8 F bytes
 // from its neighbour's, on E/256 blocks, and each block's release wrote back the
 // L2.  Runs of 20, 10 and 4 steps on 32^2 P3, 17^3 P2 and 23^3 P4 mixed: 580 -> 547,
-// 886 -> 850, 1690 -> 1523 us.
+// 886 -> 850, 1690 -> 1523 us.  Meshes that need more than kDtBlocks blocks of 256
+// threads take blocks of 1024, a wave's loads being what a block waits for: 30^3 P3 with
+// 256 / 1024 threads 42 / 22 us (the thread per element: 24), 48^3 P1 51 / 26 (34),
+// 400^2 P3 37 / 21 (34); 256 threads in more blocks take longer (30^3 P3, 1024
+// blocks: 26), and on small meshes 1024 threads do (8^3 P2 8.2 / 10.4).
 template <int F>
 constexpr int kDtLanes = F <= 16 ? 16 : (F <= 32 ? 32 : 64);
 template <int D>
@@ -1970,17 +1974,17 @@ constexpr unsigned kDtBlocks = 256;
 
 // ele::calcDt per element (element-major inputs) and, with a ticket counter, the
 // minimum of all at out, the global dt (solver::calcDt, src/solver.cpp:447-468).
-template <int D, int P>
-__global__ __launch_bounds__(256) void k_ele_dt_em(int E, const double* __restrict__ vole, const double* __restrict__ wf,
+template <int D, int P, int NT>
+__global__ __launch_bounds__(NT) void k_ele_dt_em(int E, const double* __restrict__ vole, const double* __restrict__ wf,
                                                     const double* __restrict__ waveSpe, const double* __restrict__ dAe,
                                                     double cflfac, double* __restrict__ eleDt, double* acc,
                                                     unsigned* ticket, double* __restrict__ out) {
   using Sh = Shape<D, P>;
   constexpr int F = Sh::F, Ff = Sh::Ff, G = kDtLanes<F>;
-  __shared__ double red[4];
+  __shared__ double red[NT / 64];
   const int l = threadIdx.x % G;
   double dt = INFINITY;
-  constexpr int EB = 256 / G, M = kDtEles<D>;
+  constexpr int EB = NT / G, M = kDtEles<D>;
   for (int e0 = blockIdx.x * (EB * M); e0 < E; e0 += gridDim.x * (EB * M)) {  // uniform over the block
     double iw[M], vol[M];
 #pragma unroll
@@ -2778,12 +2782,17 @@ struct Runner {
   }
   static void dt(Ctx& c, double cflfac) {
     FusedState& st = fs(c);
-    const unsigned nb = std::min(nblk(c.z.E, 256 / kDtLanes<F> * kDtEles<D>), kDtBlocks);
+    const bool one = st.nMesh == 1;
+    // (blocks of merged meshes take no turns)
+    const unsigned small = nblk(c.z.E, 256 / kDtLanes<F> * kDtEles<D>);
+    const bool big = one && small > kDtBlocks;
+    const int nt = big ? 1024 : 256;
+    const unsigned nb = big ? std::min(nblk(c.z.E, nt / kDtLanes<F> * kDtEles<D>), kDtBlocks) : small;
+    auto* kern = big ? k_ele_dt_em<D, P, 1024> : k_ele_dt_em<D, P, 256>;
     {
       // one mesh: the element kernel's last block forms the global minimum
       Launch L(c, nm("fused_ele_dt", "mixed_ele_dt"));
-      const bool one = st.nMesh == 1;
-      hipLaunchKernelGGL((k_ele_dt_em<D, P>), dim3(nb), dim3(256), 0, c.stream, c.z.E, st.vole, c.wf, st.waveSpe,
+      hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.vole, c.wf, st.waveSpe,
                          st.dAe, cflfac, c.eleDt, st.dtAcc, one ? st.dtTicket : nullptr, c.d_dt);
       FCHK(hipGetLastError());
     }

@@ -1,0 +1,50 @@
+"""The CFL time step's kernel on meshes that take its large blocks (more than 256
+blocks of 256 threads): just past the limit, ragged, with one block's worth over,
+and merged meshes, which never do.  Against the oracle; twice, since a launch
+leaves the counters for the next."""
+import numpy as np
+import pytest
+
+from flurrypp_amd import cases
+from flurrypp_amd._native import PATH_FUSED, PATH_MIXED
+from flurrypp_amd.batch import BatchedSolver, Member
+from flurrypp_amd.solver import Solver
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+# elements that 256 blocks of 256 threads have in flight: quads 8192 (P0 to P3), 4096 (P4);
+# hexes 8192 (P1), 4096 (P2)
+@pytest.mark.parametrize("kind,n,order,limit", [("vortex2d", 91, 0, 8192), ("vortex2d", 90, 3, 8192),
+                                                ("vortex2d", 91, 3, 8192), ("vortex2d", 65, 4, 4096),
+                                                ("vortex3d", 20, 1, 8192), ("vortex3d", 21, 1, 8192),
+                                                ("vortex3d", 17, 2, 4096)])
+def test_dt(kind, n, order, limit):
+    setup, U = getattr(cases, kind)(n=n, order=order)
+    print(f"{kind} {n} P{order}: {setup.nEles} elements, limit {limit}", flush=True)
+    s, o = Solver(setup.params, setup=setup), Oracle.from_setup(setup)
+    s.initializeSolution(U)
+    o.initializeSolution(U, 1)
+    for path in (PATH_FUSED, PATH_FUSED, PATH_MIXED):
+        s.update(2, path=path)
+        o.update(2)
+        # the bars of the parity tests for the FP64 and the mixed path
+        rtol = 1e-12 if path == PATH_FUSED else 1e-6
+        np.testing.assert_allclose(s.dt, o.dt, rtol=rtol)
+        np.testing.assert_allclose(s.get("ele_dt"), o.get("ele_dt"), rtol=rtol)
+    s.close()
+
+
+def test_merged():
+    """Three copies of a mesh in one context step as the mesh alone."""
+    setup, U = cases.vortex2d(n=61, order=2)
+    states = []
+    for m in (1, 3):
+        b = BatchedSolver([Member(setup, U) for _ in range(m)], path=PATH_FUSED)
+        b.step(3)
+        states += b.states()
+        b.close()
+    for st in states[1:]:
+        # both forms of the stage kernel, whose sums are contracted differently at most
+        np.testing.assert_allclose(st, states[0], rtol=1e-13, atol=1e-13)
