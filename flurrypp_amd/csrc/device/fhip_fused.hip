@@ -422,7 +422,7 @@ struct Work {
   R* Us = nullptr;
   // geometry in the kernels' arithmetic type: the FP64 arrays themselves, or
   // FP32 copies rounded once (the values the FP32 kernels would convert to)
-  const R *JG = nullptr, *iJ = nullptr, *nrm = nullptr, *dA = nullptr, *nf = nullptr;
+  const R *JG = nullptr, *iJ = nullptr, *dA = nullptr, *nf = nullptr;
   void* geo_mem = nullptr;
   bool ready = false;
   void release() {
@@ -439,7 +439,6 @@ struct FusedState {
   // FP64 element-major state, metrics and wave speeds (both paths)
   double *Ue = nullptr, *Uacc = nullptr, *divF0e = nullptr, *JGe = nullptr, *detJe = nullptr,
          *iJe = nullptr, *norme = nullptr, *dAe = nullptr, *waveSpe = nullptr;
-  int *pL = nullptr, *pR = nullptr, *bc = nullptr;
   // per element flux point, 4 * (partner flux point e*F + f) + side (0 left,
   // 1 right) or 4 * boundary slot + 2; the face's normal (the left element's)
   // at every element flux point; boundary codes by slot
@@ -476,9 +475,9 @@ struct FusedState {
   ~FusedState() {
     w64.release();
     w32.release();
-    void* ps[] = {tab_mem, Ue,           Uacc,    divF0e,    JGe,    detJe,  iJe,   norme, dAe, waveSpe, pL,
-                  pR,      bc,  fpart,   nfe,       bst,    meshDt, meshRes, eleMesh, meshStart, active, srce,
-                  dtTicket, dtAcc, vole, bndBc};
+    void* ps[] = {tab_mem, Ue,  Uacc,   divF0e,  JGe,     detJe,     iJe,    norme, dAe,      waveSpe, fpart,
+                  nfe,     bst, meshDt, meshRes, eleMesh, meshStart, active, srce,  dtTicket, dtAcc,   vole,
+                  bndBc};
     for (void* p : ps)
       if (p) (void)hipFree(p);
   }
@@ -722,36 +721,6 @@ __device__ __forceinline__ bool pair_flux(bool bnd, const R* UL, const R* UR, co
   }
   lam = double(rusanov<D, R>(UL, UR, n, fn, R(ph.gamma)));
   return true;
-}
-
-// The wave speeds of the common inviscid flux, one thread per point pair, for
-// the inviscid runs that need them ahead of their stage kernel (face_first).
-template <int D, int P, class R>
-__global__ __launch_bounds__(kMaxBlock) void k_face_inv(int nFF, const int* __restrict__ pLa, const int* __restrict__ pRa,
-                                                   const int* __restrict__ bca, const R* __restrict__ Ufe,
-                                                   const R* __restrict__ norme, double* __restrict__ waveSpe, Phys ph,
-                                                   const double* __restrict__ bst) {
-  using Sh = Shape<D, P>;
-  constexpr int F = Sh::F, N = Sh::N;
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nFF) return;
-  const int pl = pLa[t], pr = pRa[t], bc = bca[t];
-  const long long eL = pl / F, fL = pl - eL * F;
-  const long long bL = eL * N * F + fL;
-  R UL[N], UR[N], n[D], fn[N];
-#pragma unroll
-  for (int k = 0; k < N; k++) UL[k] = Ufe[bL + k * F];
-#pragma unroll
-  for (int d = 0; d < D; d++) n[d] = norme[(eL * D + d) * F + fL];
-  if (pr < 0) {
-    bc_state<D, R>(bc, UL, n, UR, ph, bst);
-  } else {
-    const long long eR = pr / F, fR = pr - eR * F, bR = eR * N * F + fR;
-#pragma unroll
-    for (int k = 0; k < N; k++) UR[k] = Ufe[bR + k * F];
-  }
-  double lam;
-  if (pair_flux<D, R>(pr < 0, UL, UR, n, fn, ph, lam)) waveSpe[pl] = lam;
 }
 
 // ---------------------------------------------------------------------------
@@ -2015,6 +1984,95 @@ __global__ __launch_bounds__(NT) void k_ele_dt_em(int E, const double* __restric
   if (threadIdx.x == 0) grid_min(bmin, gridDim.x, acc, ticket, out);
 }
 
+// The wave speeds of the common inviscid flux at the left and boundary points, for
+// the steps that need them ahead of their stage kernel (face_first); right points
+// keep theirs (and, with Roe's flux, all but the boundary's).
+template <int D, int P, class R>
+__global__ __launch_bounds__(kMaxBlock) void k_pair_wave(int n, const int* __restrict__ fpart, const R* __restrict__ Ufe,
+                                                    const R* __restrict__ nfe, const int* __restrict__ bndBc,
+                                                    double* __restrict__ waveSpe, Phys ph,
+                                                    const double* __restrict__ bst) {
+  using Sh = Shape<D, P>;
+  constexpr int F = Sh::F, N = Sh::N;
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const int code = fpart[q], side = code & 3;
+  if (side == 1) return;
+  const int e = q / F, f = q - e * F;
+  R UL[N], UR[N], nv[D], fn[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) UL[k] = Ufe[((long long)e * N + k) * F + f];
+#pragma unroll
+  for (int d = 0; d < D; d++) nv[d] = nfe[((long long)e * D + d) * F + f];
+  if (side == 2) {
+    bc_state<D, R>(bndBc[code >> 2], UL, nv, UR, ph, bst);
+  } else {
+    const int p = code >> 2, ep = p / F, fp = p - ep * F;
+#pragma unroll
+    for (int k = 0; k < N; k++) UR[k] = Ufe[((long long)ep * N + k) * F + fp];
+  }
+  double lam;
+  if (pair_flux<D, R>(side == 2, UL, UR, nv, fn, ph, lam)) waveSpe[q] = lam;
+}
+
+// The same and the elements' time steps from them in one pass, up to kWaveDtPoints
+// flux points: one launch less, but in the dt kernel's blocks, which are too few for
+// the gathers of a large mesh.  Together / apart: channel 113x41 P3 (74 k points) 10.0 /
+// 14.7 us, quads 200^2 P2 (480 k) 17.0 / 21.9; 30^3 P3 (2.6 M) 64 / 56.
+constexpr long long kWaveDtPoints = 1 << 20;
+template <int D, int P, class R, int NT>
+__global__ __launch_bounds__(NT) void k_wave_dt(int E, const int* __restrict__ fpart, const R* __restrict__ Ufe,
+                                                const R* __restrict__ nfe, const int* __restrict__ bndBc,
+                                                const double* __restrict__ bst, Phys ph,
+                                                const double* __restrict__ vole, const double* __restrict__ wf,
+                                                double* waveSpe, const double* __restrict__ dAe, double cflfac,
+                                                double* __restrict__ eleDt, double* acc, unsigned* ticket,
+                                                double* __restrict__ out) {
+  using Sh = Shape<D, P>;
+  constexpr int F = Sh::F, Ff = Sh::Ff, N = Sh::N, G = kDtLanes<F>, EB = NT / G;
+  __shared__ double red[NT / 64];
+  const int l = threadIdx.x % G;
+  double dt = INFINITY;
+  for (int e0 = blockIdx.x * EB; e0 < E; e0 += gridDim.x * EB) {  // uniform over the block
+    const int e = e0 + threadIdx.x / G;
+    double iw = 0;
+#pragma unroll
+    for (int f0 = 0; f0 < F; f0 += G) {
+      const int f = f0 + l;
+      if (f >= F || e >= E) continue;
+      const long long q = (long long)e * F + f;
+      const int code = fpart[q], side = code & 3;
+      double lam = waveSpe[q];
+      if (side != 1) {
+        R UL[N], UR[N], n[D], fn[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) UL[k] = Ufe[((long long)e * N + k) * F + f];
+#pragma unroll
+        for (int d = 0; d < D; d++) n[d] = nfe[((long long)e * D + d) * F + f];
+        if (side == 2) {
+          bc_state<D, R>(bndBc[code >> 2], UL, n, UR, ph, bst);
+        } else {
+          const int p = code >> 2, ep = p / F;
+#pragma unroll
+          for (int k = 0; k < N; k++) UR[k] = Ufe[((long long)ep * N + k) * F + (p - ep * F)];
+        }
+        if (pair_flux<D, R>(side == 2, UL, UR, n, fn, ph, lam)) waveSpe[q] = lam;
+      }
+      iw += lam * wf[f % Ff] * dAe[q];
+    }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) iw += __shfl_xor(iw, o);
+    if (e < E) {
+      const double v = cflfac * 2 * vole[e] / iw;
+      if (l == 0) eleDt[e] = v;
+      dt = fmin(dt, v);
+    }
+  }
+  const double bmin = block_min(dt, red);
+  if (!ticket) return;
+  if (threadIdx.x == 0) grid_min(bmin, gridDim.x, acc, ticket, out);
+}
+
 // Per-mesh minimum of the element time steps (batched contexts, dt_type 1).
 static __global__ void k_mesh_dt_min(const int* __restrict__ start, const double* __restrict__ eleDt,
                               double* __restrict__ meshDt) {
@@ -2287,26 +2345,23 @@ static void set_geometry(Ctx& c, Work<double>& w) {
   FusedState& st = fs(c);
   w.JG = st.JGe;
   w.iJ = st.iJe;
-  w.nrm = st.norme;
   w.dA = st.dAe;
   w.nf = st.nfe;
 }
 static void set_geometry(Ctx& c, Work<float>& w) {
   FusedState& st = fs(c);
   const long long E = c.z.E, S = c.z.S, F = c.z.F, D = c.z.D;
-  const long long n[5] = {E * D * D * S, E * S, E * D * F, E * F, st.nfe ? E * D * F : 0};
-  const double* src[5] = {st.JGe, st.iJe, st.norme, st.dAe, st.nfe};
+  const long long n[4] = {E * D * D * S, E * S, E * F, E * D * F};
+  const double* src[4] = {st.JGe, st.iJe, st.dAe, st.nfe};
   long long tot = 0;
   for (long long v : n) tot += (v + 63) / 64 * 64;
   float* m = dal<float>(tot);
   w.geo_mem = m;
-  const float** dst[5] = {&w.JG, &w.iJ, &w.nrm, &w.dA, &w.nf};
-  for (int i = 0; i < 5; i++) {
-    *dst[i] = n[i] ? m : nullptr;
-    if (n[i]) {
-      hipLaunchKernelGGL(k_round_f32, dim3(1024), dim3(256), 0, c.stream, n[i], src[i], m);
-      FCHK(hipGetLastError());
-    }
+  const float** dst[4] = {&w.JG, &w.iJ, &w.dA, &w.nf};
+  for (int i = 0; i < 4; i++) {
+    *dst[i] = m;
+    hipLaunchKernelGGL(k_round_f32, dim3(1024), dim3(256), 0, c.stream, n[i], src[i], m);
+    FCHK(hipGetLastError());
     m += (n[i] + 63) / 64 * 64;
   }
 }
@@ -2448,12 +2503,6 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
       }
       bc[t] = (r < 0) ? (d->face_bc[t / z.Ff] | ((row + 1) << 4)) : -1;
     }
-    st->pL = dal<int>(pl.size());
-    st->pR = dal<int>(pr.size());
-    st->bc = dal<int>(bc.size());
-    FCHK(hipMemcpy(st->pL, pl.data(), pl.size() * 4, hipMemcpyHostToDevice));
-    FCHK(hipMemcpy(st->pR, pr.data(), pr.size() * 4, hipMemcpyHostToDevice));
-    FCHK(hipMemcpy(st->bc, bc.data(), bc.size() * 4, hipMemcpyHostToDevice));
     {
       // every element flux point must lie on exactly one face point pair;
       // its code: 4 * partner flux point + side, or 4 * boundary slot + 2, and
@@ -2609,15 +2658,6 @@ struct Runner {
   }
   // U at the flux points of the current state
   static R* cur_ufe(Ctx& c) { return fs(c).flipped ? fs(c).work<R>().Ufe2 : fs(c).work<R>().Ufe; }
-  static void launch_face_inv(Ctx& c, int nt) {
-    FusedState& st = fs(c);
-    Work<R>& w = st.work<R>();
-    const int nFF = c.z.nFaceFpts;
-    if (nFF == 0) return;
-    hipLaunchKernelGGL((k_face_inv<D, P, R>), dim3(nblk(nFF, nt)), dim3(nt), 0, c.stream, nFF, st.pL, st.pR, st.bc,
-                       cur_ufe(c), w.nrm, st.waveSpe, c.ph, st.bst);
-    FCHK(hipGetLastError());
-  }
   // viscous runs: the volume kernel.  Quads and FP32 are held to 4 waves per
   // SIMD (128 VGPRs); FP64 hexes, which spill under that hold, to 3 (168 VGPRs:
   // P3 without spills, where the unheld compiler would take 211 and leave 2
@@ -2780,33 +2820,60 @@ struct Runner {
                        st.waveSpe, c.ph.gamma);
     FCHK(hipGetLastError());
   }
+  // Threads and blocks of the dt kernels, which have `eles` elements in flight in a
+  // block of 256 (blocks of merged meshes take no turns, so they are not limited).
+  static std::pair<int, unsigned> dt_grid(Ctx& c, int eles, unsigned limit) {
+    const unsigned small = nblk(c.z.E, eles);
+    if (small <= limit || fs(c).nMesh > 1) return {256, small};
+    return {1024, std::min(nblk(c.z.E, 4 * eles), kDtBlocks)};
+  }
   static void dt(Ctx& c, double cflfac) {
     FusedState& st = fs(c);
-    const bool one = st.nMesh == 1;
-    // (blocks of merged meshes take no turns)
-    const unsigned small = nblk(c.z.E, 256 / kDtLanes<F> * kDtEles<D>);
-    const bool big = one && small > kDtBlocks;
-    const int nt = big ? 1024 : 256;
-    const unsigned nb = big ? std::min(nblk(c.z.E, nt / kDtLanes<F> * kDtEles<D>), kDtBlocks) : small;
-    auto* kern = big ? k_ele_dt_em<D, P, 1024> : k_ele_dt_em<D, P, 256>;
     {
       // one mesh: the element kernel's last block forms the global minimum
       Launch L(c, nm("fused_ele_dt", "mixed_ele_dt"));
-      hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.vole, c.wf, st.waveSpe,
-                         st.dAe, cflfac, c.eleDt, st.dtAcc, one ? st.dtTicket : nullptr, c.d_dt);
+      const auto [nt, nb] = dt_grid(c, 256 / kDtLanes<F> * kDtEles<D>, kDtBlocks);
+      auto* kern = nt == 1024 ? k_ele_dt_em<D, P, 1024> : k_ele_dt_em<D, P, 256>;
+      hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.vole, c.wf, st.waveSpe, st.dAe, cflfac,
+                         c.eleDt, st.dtAcc, st.nMesh == 1 ? st.dtTicket : nullptr, c.d_dt);
       FCHK(hipGetLastError());
     }
-    // merged meshes: per-mesh minima for a global CFL dt per mesh (a local
-    // CFL dt uses the element values alone)
-    if (st.nMesh > 1 && c.prm.dt_type == 1) {
-      Launch L(c, nm("fused_dt_min", "mixed_dt_min"));
-      hipLaunchKernelGGL(k_mesh_dt_min, dim3(st.nMesh), dim3(256), 0, c.stream, st.meshStart, c.eleDt, st.meshDt);
-      FCHK(hipGetLastError());
-    }
+    mesh_dt(c);
   }
-  static void face(Ctx& c) {
-    Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
-    launch_face_inv(c, blk(c, kFaceInv));
+  // wave speeds of the common flux, and the time steps from them
+  static void wave_dt(Ctx& c, double cflfac) {
+    FusedState& st = fs(c);
+    Work<R>& w = st.work<R>();
+    const int n = c.z.E * F;
+    if (n > kWaveDtPoints) {
+      {
+        Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
+        const int nt = blk(c, kFaceInv);
+        hipLaunchKernelGGL((k_pair_wave<D, P, R>), dim3(nblk(n, nt)), dim3(nt), 0, c.stream, n, st.fpart, cur_ufe(c),
+                           w.nf, st.bndBc, st.waveSpe, c.ph, st.bst);
+        FCHK(hipGetLastError());
+      }
+      return dt(c, cflfac);
+    }
+    {
+      Launch L(c, nm("fused_wave_dt", "mixed_wave_dt"));
+      const auto [nt, nb] = dt_grid(c, 256 / kDtLanes<F>, 2 * kDtBlocks);
+      auto* kern = nt == 1024 ? k_wave_dt<D, P, R, 1024> : k_wave_dt<D, P, R, 256>;
+      hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.fpart, cur_ufe(c), w.nf, st.bndBc, st.bst,
+                         c.ph, st.vole, c.wf, st.waveSpe, st.dAe, cflfac, c.eleDt, st.dtAcc,
+                         st.nMesh == 1 ? st.dtTicket : nullptr, c.d_dt);
+      FCHK(hipGetLastError());
+    }
+    mesh_dt(c);
+  }
+  // merged meshes: per-mesh minima for a global CFL dt per mesh (a local CFL dt
+  // uses the element values alone)
+  static void mesh_dt(Ctx& c) {
+    FusedState& st = fs(c);
+    if (st.nMesh == 1 || c.prm.dt_type != 1) return;
+    Launch L(c, nm("fused_dt_min", "mixed_dt_min"));
+    hipLaunchKernelGGL(k_mesh_dt_min, dim3(st.nMesh), dim3(256), 0, c.stream, st.meshStart, c.eleDt, st.meshDt);
+    FCHK(hipGetLastError());
   }
   // calcResidual up to what the RK update needs: the volume kernel of viscous
   // runs (wave: with the wave speeds, which stages that another stage follows
@@ -2920,7 +2987,7 @@ struct Ops {
   void (*extrap)(Ctx&);
   void (*wave)(Ctx&);
   void (*dt)(Ctx&, double);
-  void (*face)(Ctx&);
+  void (*wave_dt)(Ctx&, double);
   void (*residual)(Ctx&, bool);
   void (*rk)(Ctx&, int, double, double, bool, int, bool);
   void (*ensure)(Ctx&);
@@ -2934,7 +3001,7 @@ struct Ops {
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::face, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
+  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::wave_dt, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
 }
 
 // The kernels of one dimension, precision and range of orders.  This file is
@@ -3200,8 +3267,9 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   const bool jameson = c.prm.time_type >= 5;
   if (nRK == 1) {
     if (c.prm.viscous) o.residual(c, true);
-    else if (face_first(c)) o.face(c);
-    if (cfl) {
+    if (cfl && !refresh && face_first(c)) {
+      o.wave_dt(c, cflfac);
+    } else if (cfl) {
       if (refresh) o.wave(c);
       o.dt(c, cflfac);
     }

@@ -81,16 +81,16 @@ def footprint_bytes(nDims: int, order: int, nEles: int, viscous: bool = False, n
     SN, FN = S * N, F * N
     # staged: U, U0, F_spts, divF[nRK]; U_fpts, disFn, Fn, face Fn; wave speeds, metrics, face tables
     d = SN * (2 + D + nRK) + 4 * FN + F * (3.5 + D) + D * D * S + S + 1
-    # fused FP64: U, its stage copy, RK accumulator, divF0; wave speeds, metrics (+1/detJ), face
-    # tables, the points' side codes, element volumes
-    d += 4 * SN + F * (2 + D) + D * D * S + 2 * S + 1.5 * F + 0.5 * F + 1
+    # fused FP64: U, its stage copy, RK accumulator, divF0; wave speeds, metrics (+1/detJ), the
+    # points' side and boundary codes, element volumes
+    d += 4 * SN + F * (2 + D) + D * D * S + 2 * S + 0.5 * F + 0.5 * F + 1
     # the faces' normals at every flux point
     d += D * F
     # FP64 work: stage copy or divF, two arrays at the flux points (U, and its second copy on inviscid
     # runs or the LDG side parts)
     d += SN + 2 * FN
     # FP32 work (half a double each): the same, stage residuals, FP32 U, FP32 geometry
-    d += 0.5 * (SN + 2 * FN + (nRK - 1) * SN + SN + D * D * S + S + 2 * D * F + F)
+    d += 0.5 * (SN + 2 * FN + (nRK - 1) * SN + SN + D * D * S + S + D * F + F)
     if viscous:
         d += D * SN + D * FN + FN            # staged gradients and dUc
         d += 0.5 * FN                        # FP32: the flux jump

@@ -58,7 +58,7 @@ def _stages(setup, n):
 
 @pytest.mark.parametrize("path", [PATH_FUSED, PATH_MIXED])
 def test_launches_of_a_step(path):
-    """A single-stage step is the wave speeds, the time step and the stage."""
+    """A single-stage step is the wave speeds with the time step, and the stage."""
     setup, U = CASES["bump2d"](2)
     s = Solver(setup.params, setup=setup)
     s.initializeSolution(U)
@@ -67,7 +67,7 @@ def test_launches_of_a_step(path):
     s.update(4, path=path)
     n = {k.split("_", 1)[1]: v[1] for k, v in s.kernel_times().items()}
     s.close()
-    assert n == {"extrapolate": 1, "face_inviscid": 4, "ele_dt": 4, "stage": 4}
+    assert n == {"extrapolate": 1, "wave_dt": 4, "stage": 4}
 
 
 @pytest.mark.parametrize("path", [PATH_FUSED, PATH_MIXED])
@@ -121,3 +121,32 @@ def test_multigrid(stages, smooth, dt_type, path, tol):
         assert np.linalg.norm(s.get_U() - o.get_U()) <= tol * np.linalg.norm(o.get_U()), s.order
     mg.close()
     fine.close()
+
+
+def _euler_step(setup):
+    setup.params.timeType = setup.fp.time_type = 0
+    _stages(setup, 1)
+
+
+@pytest.mark.parametrize("path", [PATH_FUSED, PATH_MIXED])
+@pytest.mark.parametrize("make", [
+    lambda: cases.bump2d(nx=131, ny=67, order=3, dt_type=2, cfl=0.3),   # 8777 of 16 points: blocks of 1024
+    lambda: cases.bump2d(nx=128, ny=64, order=3, dt_type=1, cfl=0.3),   # 8192: the last of 256
+    lambda: cases.vortex2d(n=257, order=3, cfl=0.3),                    # 1.06 million points: in two launches
+    lambda: cases.vortex3d(n=4, order=3), lambda: cases.vortex3d(n=13, order=4)],
+    ids=["quads_1024", "quads_256", "quads_apart", "hexes_256", "hexes_1024"])
+def test_wave_speeds_and_time_steps(make, path):
+    """The pass that forms both, at the edges of its block sizes and past its limit."""
+    setup, U = make()
+    _euler_step(setup)
+    s, o = Solver(setup.params, setup=setup), Oracle.from_setup(setup)
+    s.initializeSolution(U)
+    o.initializeSolution(U, setup.params.dtType)
+    for n in (1, 2):
+        s.update(n, path=path)
+        o.update(n)
+        np.testing.assert_allclose(s.get("waveSp"), o.get("waveSp"), rtol=RTOL[path])
+        # sums of the wave speeds: their bar
+        np.testing.assert_allclose(s.get("ele_dt"), o.get("ele_dt"), rtol=RTOL[path])
+        assert s.dt == s.get("ele_dt").min()
+    s.close()
