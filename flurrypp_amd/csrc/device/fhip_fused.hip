@@ -441,7 +441,7 @@ struct FusedState {
          *iJe = nullptr, *norme = nullptr, *dAe = nullptr, *waveSpe = nullptr;
   // per element flux point, 4 * (partner flux point e*F + f) + side (0 left,
   // 1 right) or 4 * boundary slot + 2; the face's normal (the left element's)
-  // at every element flux point; boundary codes by slot
+  // at every element flux point; boundary codes by slot (behind fpart)
   int *fpart = nullptr, *bndBc = nullptr;
   double* nfe = nullptr;
   int nBnd = 0;
@@ -449,8 +449,8 @@ struct FusedState {
   int nMesh = 1;
   std::vector<int> h_meshStart;
   double *bst = nullptr, *meshDt = nullptr, *meshRes = nullptr;
-  unsigned* dtTicket = nullptr;  // blocks of the dt kernel that have finished (zero between launches)
-  double* dtAcc = nullptr;       // their minimum so far (infinity between launches)
+  double* dtAcc = nullptr;       // minimum of the blocks of the dt kernel that have finished (infinity between launches)
+  unsigned* dtTicket = nullptr;  // their number (zero between launches), behind it
   double* vole = nullptr;        // element volumes, sum_s detJ w_s (calcDt's numerator)
   int *eleMesh = nullptr, *meshStart = nullptr, *active = nullptr;
   // P-multigrid source term (element-major copy of src_spts), used while use_src
@@ -476,8 +476,7 @@ struct FusedState {
     w64.release();
     w32.release();
     void* ps[] = {tab_mem, Ue,  Uacc,   divF0e,  JGe,     detJe,     iJe,    norme, dAe,      waveSpe, fpart,
-                  nfe,     bst, meshDt, meshRes, eleMesh, meshStart, active, srce,  dtTicket, dtAcc,   vole,
-                  bndBc};
+                  nfe,     bst, meshDt, meshRes, eleMesh, meshStart, active, srce,  dtAcc,    vole};
     for (void* p : ps)
       if (p) (void)hipFree(p);
   }
@@ -2140,20 +2139,21 @@ static T* dal(size_t n) {
 // in the other directions are exactly 0 or 1).
 static bool build_d1(const Ctx& c, const fhip_desc* dsc, std::vector<double>& d1) {
   const int D = c.z.D, S = c.z.S, P1 = c.z.P + 1;
-  auto coord = [&](int q, int dd) { return dd == 0 ? q % P1 : (dd == 1 ? (q / P1) % P1 : q / (P1 * P1)); };
-  auto tangent = [&](int q, int dd) {  // the point's coordinates in the other directions
-    return dd == 0 ? q / P1 : (dd == 1 ? q % P1 + P1 * (q / (P1 * P1)) : q % (P1 * P1));
-  };
   d1.assign(P1 * P1, 0.);
   for (int i = 0; i < P1; i++)
     for (int m = 0; m < P1; m++) d1[i * P1 + m] = dsc->opp_grad_spts[(size_t)i * S + m];  // d = 0, line 0
-  for (int dd = 0; dd < D; dd++)
-    for (int q = 0; q < S; q++)
-      for (int r = 0; r < S; r++) {
-        const double v = dsc->opp_grad_spts[((size_t)dd * S + q) * S + r];
-        const bool on = tangent(r, dd) == tangent(q, dd);
-        if (!(v == (on ? d1[coord(q, dd) * P1 + coord(r, dd)] : 0.))) return false;  // +0 == -0
+  for (int dd = 0, step = 1; dd < D; dd++, step *= P1)
+    for (int q = 0; q < S; q++) {
+      const double* const row = dsc->opp_grad_spts + ((size_t)dd * S + q) * S;
+      const int at = (q / step) % P1, line = q - at * step;  // the point's place on its line, the line's first point
+      int on = 0;
+      for (int m = 0; m < P1; m++) {
+        const double v = row[line + m * step];
+        if (!(v == d1[at * P1 + m])) return false;  // +0 == -0
+        on += v != 0.;
       }
+      if (count_nonzeros(row, S) != on) return false;
+    }
   return true;
 }
 
@@ -2180,25 +2180,34 @@ static bool build_ten(const Ctx& c, const fhip_desc* d, const std::vector<double
       w[T::C + hi * P1 + m] = d->opp_correction[(size_t)q * F + T::face_fpt(j, cc)];
     }
   }
+  // every entry on a flux point's line as the factors give it, and no others
+  long long nc = 0;  // of the corrections
   for (int f = 0; f < F; f++) {
     const typename T::Face face(f);
     const int j = f / Sh::Ff;
     if (face.dn != T::face_dir(j) || face.hi != T::face_hi(j)) return false;
-    for (int m = 0; m < P1; m++) at[(size_t)f * P1 + m] = face.at(m);
-    for (int q = 0; q < S; q++) {
-      const typename T::Point p(q);
-      bool on = true;
-      for (int x = 0; x < D; x++) on = on && (x == face.dn || p.c[x] == face.c[x]);
-      if (on != (T::face_fpt(j, p.c) == f)) return false;
-      const double l = on ? w[T::L + face.hi * P1 + p.c[face.dn]] : 0., cr = on ? w[T::C + face.hi * P1 + p.c[face.dn]] : 0.;
-      if (!(d->opp_spts_to_fpts[(size_t)f * S + q] == l && d->opp_correction[(size_t)q * F + f] == cr)) return false;
-      for (int x = 0; x < D; x++) {
-        const double sg = x == face.dn ? (face.hi ? 1. : -1.) : 0.;
-        if (!(d->opp_extrapolate_fn[((size_t)x * F + f) * S + q] == l * sg)) return false;
-        if (c.prm.viscous && !(d->opp_correct_u[((size_t)x * S + q) * F + f] == cr * sg)) return false;
-      }
+    const double sg = face.hi ? 1. : -1.;
+    int nl = 0;
+    for (int m = 0; m < P1; m++) {
+      at[(size_t)f * P1 + m] = face.at(m);
+      int cc[3] = {face.c[0], face.c[1], face.c[2]};
+      cc[face.dn] = m;
+      if (T::face_fpt(j, cc) != f) return false;
+      const size_t q = cc[0] + P1 * (cc[1] + P1 * cc[2]);
+      const double l = w[T::L + face.hi * P1 + m], cr = w[T::C + face.hi * P1 + m];
+      if (!(d->opp_spts_to_fpts[(size_t)f * S + q] == l && d->opp_correction[q * F + f] == cr &&
+            d->opp_extrapolate_fn[((size_t)face.dn * F + f) * S + q] == l * sg))
+        return false;
+      if (c.prm.viscous && !(d->opp_correct_u[((size_t)face.dn * S + q) * F + f] == cr * sg)) return false;
+      nl += l != 0.;
+      nc += cr != 0.;
     }
+    if (count_nonzeros(d->opp_spts_to_fpts + (size_t)f * S, S) != nl) return false;
+    for (int x = 0; x < D; x++)
+      if (count_nonzeros(d->opp_extrapolate_fn + ((size_t)x * F + f) * S, S) != (x == face.dn ? nl : 0)) return false;
   }
+  if (count_nonzeros(d->opp_correction, (long long)S * F) != nc) return false;
+  if (c.prm.viscous && count_nonzeros(d->opp_correct_u, (long long)D * S * F) != nc) return false;
   line = at;
   return true;
 }
@@ -2231,11 +2240,10 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
     // the face's normal direction: the only d with non-zero extrapolate_fn entries
     int dn = -1;
     for (int dd = 0; dd < D; dd++)
-      for (int q = 0; q < S; q++)
-        if (d->opp_extrapolate_fn[((size_t)dd * F + f) * S + q] != 0.) {
-          if (dn >= 0 && dn != dd) return false;
-          dn = dd;
-        }
+      if (count_nonzeros(d->opp_extrapolate_fn + ((size_t)dd * F + f) * S, S)) {
+        if (dn >= 0) return false;
+        dn = dd;
+      }
     efn_dir[f] = dn < 0 ? 0 : dn;
     int n = 0;
     for (int q = 0; q < S; q++) {
@@ -2253,37 +2261,37 @@ static bool build_tables(const Ctx& c, const fhip_desc* d, std::vector<char>& bl
   for (int dd = 0; dd < D; dd++)
     for (int q0 = 0; q0 < S; q0++) {
       int n = 0;
-      for (int q = 0; q < S; q++) {
-        double v = d->opp_grad_spts[((size_t)dd * S + q0) * S + q];
-        if (v == 0.) continue;
-        if (n >= P1) return false;
-        grd_idx[((size_t)dd * S + q0) * P1 + n] = spt_lds(D, P1, q);
-        grd_w[((size_t)dd * S + q0) * P1 + n] = v;
-        n++;
-      }
+      const double* const row = d->opp_grad_spts + ((size_t)dd * S + q0) * S;
+      if (!each_nonzero(row, S, [&](int q) {
+            if (n >= P1) return false;
+            grd_idx[((size_t)dd * S + q0) * P1 + n] = spt_lds(D, P1, q);
+            grd_w[((size_t)dd * S + q0) * P1 + n++] = row[q];
+            return true;
+          }))
+        return false;
       for (int m = n; m < P1; m++) grd_idx[((size_t)dd * S + q0) * P1 + m] = spt_lds(D, P1, q0);
     }
   for (int q = 0; q < S; q++) {
     int n = 0;
-    for (int f = 0; f < F; f++) {
-      double v = d->opp_correction[(size_t)q * F + f];
-      if (v == 0.) continue;
-      if (n >= NC) return false;
-      cor_idx[(size_t)q * NC + n] = f;
-      cor_w[(size_t)q * NC + n] = v;
-      n++;
-    }
+    const double* const row = d->opp_correction + (size_t)q * F;
+    if (!each_nonzero(row, F, [&](int f) {
+          if (n >= NC) return false;
+          cor_idx[(size_t)q * NC + n] = f;
+          cor_w[(size_t)q * NC + n++] = row[f];
+          return true;
+        }))
+      return false;
     if (c.prm.viscous)
       for (int dd = 0; dd < D; dd++) {
         int m = 0;
-        for (int f = 0; f < F; f++) {
-          double v = d->opp_correct_u[((size_t)dd * S + q) * F + f];
-          if (v == 0.) continue;
-          if (m >= 2) return false;
-          cu_idx[((size_t)dd * S + q) * 2 + m] = f;
-          cu_w[((size_t)dd * S + q) * 2 + m] = v;
-          m++;
-        }
+        const double* const ru = d->opp_correct_u + ((size_t)dd * S + q) * F;
+        if (!each_nonzero(ru, F, [&](int f) {
+              if (m >= 2) return false;
+              cu_idx[((size_t)dd * S + q) * 2 + m] = f;
+              cu_w[((size_t)dd * S + q) * 2 + m++] = ru[f];
+              return true;
+            }))
+          return false;
       }
   }
   auto put = [&](const void* p, size_t bytes, size_t& o) {
@@ -2432,11 +2440,10 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
   st->Uacc = dal<double>(E * N * S);
   st->divF0e = dal<double>(E * N * S);
   st->waveSpe = dal<double>(E * F);
-  st->dtTicket = dal<unsigned>(1);
-  FCHK(hipMemset(st->dtTicket, 0, sizeof(unsigned)));
-  st->dtAcc = dal<double>(1);
-  const double inf = INFINITY;
-  FCHK(hipMemcpy(st->dtAcc, &inf, sizeof(double), hipMemcpyHostToDevice));
+  const double none[2] = {INFINITY, 0.0};  // no minimum yet, no block finished
+  st->dtAcc = dal<double>(2);
+  st->dtTicket = reinterpret_cast<unsigned*>(st->dtAcc + 1);
+  FCHK(hipMemcpy(st->dtAcc, none, sizeof(none), hipMemcpyHostToDevice));
   st->JGe = dal<double>(E * D * D * S);
   st->detJe = dal<double>(E * S);
   st->iJe = dal<double>(E * S);
@@ -2508,16 +2515,15 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
       // its code: 4 * partner flux point + side, or 4 * boundary slot + 2, and
       // the face's normal
       if (E * F >= (1LL << 29)) throw std::invalid_argument("fused path: more than 2^29 element flux points");
-      std::vector<int> part((size_t)E * F, -1), bt, bb;
+      std::vector<int> part((size_t)E * F, -1), bb;
       for (int t = 0; t < z.nFaceFpts; t++) {
         if (part[pl[t]] != -1 || (pr[t] >= 0 && part[pr[t]] != -1)) {
           fused_release(c);
           return false;
         }
         if (pr[t] < 0) {
-          bt.push_back(t);
+          part[pl[t]] = 4 * (int)bb.size() + 2;
           bb.push_back(bc[t]);
-          part[pl[t]] = 4 * (int)(bt.size() - 1) + 2;
         } else {
           part[pl[t]] = 4 * pr[t];
           part[pr[t]] = 4 * pl[t] + 1;
@@ -2528,18 +2534,15 @@ bool fused_setup(Ctx& c, const fhip_desc* d) {
           fused_release(c);
           return false;
         }
+      st->nBnd = (int)bb.size();
+      part.insert(part.end(), bb.begin(), bb.end());
       st->fpart = dal<int>(part.size());
+      st->bndBc = st->fpart + E * F;
       FCHK(hipMemcpy(st->fpart, part.data(), part.size() * 4, hipMemcpyHostToDevice));
-      st->nBnd = (int)bt.size();
-      st->bndBc = dal<int>(bb.size());
       st->nfe = dal<double>(E * D * F);
       hipLaunchKernelGGL(k_face_normals, dim3(nblk(E * F, 256)), dim3(256), 0, c.stream, E * F, (int)F, (int)D,
                          st->fpart, st->norme, st->nfe);
       FCHK(hipGetLastError());
-      FCHK(hipStreamSynchronize(c.stream));
-      if (!bt.empty()) {
-        FCHK(hipMemcpy(st->bndBc, bb.data(), bb.size() * 4, hipMemcpyHostToDevice));
-      }
     }
   }
   return true;

@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include <map>
 #include <string>
@@ -55,6 +57,28 @@ inline void poison_fill(void* p, size_t bytes) {
   (void)hipDeviceSynchronize();
 }
 
+// f(l) for the non-zeros a[l] of a dense operator's k entries, ascending, until one
+// returns false; false then.  Mostly zeros: eight at a time (the sign bit out of the
+// way), since set-up of a small mesh is largely these scans.
+template <class F>
+inline bool each_nonzero(const double* a, int k, F&& f) {
+  for (int l0 = 0; l0 < k; l0 += 8) {
+    const int m8 = std::min(8, k - l0);
+    unsigned long long v[8] = {}, any = 0;
+    std::memcpy(v, a + l0, m8 * sizeof(double));
+    for (unsigned long long x : v) any |= x << 1;
+    if (!any) continue;
+    for (int l = l0; l < l0 + m8; l++)
+      if (a[l] != 0.0 && !f(l)) return false;
+  }
+  return true;
+}
+inline long long count_nonzeros(const double* a, long long k) {
+  long long n = 0;
+  for (long long l = 0; l < k; l++) n += a[l] != 0.0;
+  return n;
+}
+
 // A dense operator kept as its non-zero entries, row by row: q entries (padded
 // with zero weights) in each of `groups` partial sums, idx the row of the
 // operand.  q == 0: too many non-zeros per row, applied dense.
@@ -78,6 +102,7 @@ struct Ctx {
   // directions, gradient correction, normal-flux extrapolation and divergence
   // over the stacked directions, divergence correction (staged path)
   RowOp r_sf, r_grad, r_corru, r_efn, r_div, r_corr;
+  void* row_mem = nullptr;  // their tables
   // 1-D tensor-product factors for the fused path (see fhip_fused.hip)
   double* tp = nullptr;
   // metrics
