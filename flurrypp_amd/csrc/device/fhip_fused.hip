@@ -2987,6 +2987,7 @@ struct Runner {
 };
 
 struct Ops {
+  bool (*apart)(const Ctx&);
   void (*extrap)(Ctx&);
   void (*wave)(Ctx&);
   void (*dt)(Ctx&, double);
@@ -3004,7 +3005,7 @@ struct Ops {
 template <int D, int P, class R>
 static Ops ops_for() {
   using Rn = Runner<D, P, R>;
-  return Ops{Rn::extrap, Rn::wave, Rn::dt, Rn::wave_dt, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
+  return Ops{Rn::apart, Rn::extrap, Rn::wave, Rn::dt, Rn::wave_dt, Rn::residual, Rn::rk, Rn::ensure, Rn::tune, Rn::check, Rn::fit, Rn::restrict_lds, Rn::prolong_lds};
 }
 
 // The kernels of one dimension, precision and range of orders.  This file is
@@ -3043,9 +3044,11 @@ static Ops get_ops(const Ctx& c, bool mixed) {
 }
 
 // Tuned block sizes, shared by the contexts of one process: keyed by
-// (nDims, order, precision, viscous, log2 of the element count).
+// (nDims, order, precision, viscous, log2 of the element count) and by what else
+// decides which kernels run: the form of the stage kernel (inviscid runs; it
+// changes within one log2 of the element count), operators from factors or tables.
 static std::mutex g_tune_mu;
-static std::map<std::array<int, 5>, std::array<int, 5>> g_tuned;
+static std::map<std::array<int, 7>, std::array<int, 5>> g_tuned;
 
 void fused_autotune(Ctx& c, bool mixed, int* out) {
   FusedState& st = fs(c);
@@ -3053,7 +3056,8 @@ void fused_autotune(Ctx& c, bool mixed, int* out) {
   const int m = mixed ? 1 : 0;
   int lg = 0;
   for (long long e = c.z.E; e > 1; e >>= 1) lg++;
-  const std::array<int, 5> key{c.z.D, c.z.P, m, c.prm.viscous ? 1 : 0, lg};
+  const bool visc = c.prm.viscous != 0;
+  const std::array<int, 7> key{c.z.D, c.z.P, m, visc, lg, !visc && o.apart(c), st.tb.w1 != nullptr};
   bool hit = false;
   {
     std::lock_guard<std::mutex> g(g_tune_mu);
