@@ -1255,6 +1255,17 @@ constexpr bool kJumpOut = sizeof(R) == 4;
 template <int D, int P>
 constexpr bool jump_over_u = P > 0;
 
+// Threads that an element takes in the volume kernel.  One per solution point, which
+// then take ceil(F/S) flux points each; at low orders, where that is 2 to 6, one per
+// flux point instead, the solution points in the first of them: a round over flux
+// points is most of the kernel's instructions, a mesh of this order fills few
+// waves, and the rounds' values kept in registers spilled (P0 quads 243 of them).
+// us a step with walls, in the three kernels before / one per solution point / now:
+// quads 64^2 P0 116 / 194 / 80, 16^2 P1 92 / 106 / 78, 200^2 P2 320 / 331 / 232; hexes
+// 24^3 P0 195 / 295 / 132, 12^3 P1 139 / 159 / 96, 48^3 P1 1690 / 1368 / 1078.
+template <int D, int P>
+constexpr int kVolThreads = P <= 1 || (D == 2 && P == 2) ? Shape<D, P>::F : Shape<D, P>::S;
+
 // Volume kernel of viscous runs: all of a stage's residual but the other sides'
 // parts of the LDG flux.  Solution points and then flux points in the same
 // threads, EB elements per block, element data staged in LDS.
@@ -1276,7 +1287,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
                                             R* __restrict__ divFe, const VFace<R>& vf, const Tabs& tb, const Phys& ph) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
-  const int EB = blockDim.x / S;
+  const int EB = blockDim.x / kVolThreads<D, P>;
   // sU holds U until the flux has been formed, then the flux jump; sF holds, in
   // turn: dUc at the flux points, the physical gradient until it has been
   // extrapolated to the faces, then the transformed flux at the same indices as
@@ -1295,7 +1306,7 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
   const bool act = b < nb;
   const long long e = e0 + b;
   // the thread's flux points: fi(u) < nP
-  constexpr int KF = (F + S - 1) / S;
+  constexpr int KF = (F + kVolThreads<D, P> - 1) / kVolThreads<D, P>;
   const int nP = nb * F;
   auto fi = [&](int u) { return (int)threadIdx.x + u * (int)blockDim.x; };
   // matrix-core contractions: this lane's operator entry d1[s % 4][s / 16]
@@ -2638,11 +2649,14 @@ struct Runner {
   // LDS bytes of an element kernel at block size nt (0 for the face kernel)
   static size_t lds(int k, int nt, bool visc) {
     const size_t EB = nt / S;
-    const size_t SF = (visc && F > D * S) ? F : D * S;
     if (k == kExtrap) return EB * N * S * sizeof(R);
-    if (k == kVolume) return visc ? EB * N * ((!kJumpOut<R> && jump_over_u<D, P> && F > S ? F : S) + SF) * sizeof(R) : EB * N * (S + SF + F) * sizeof(R);
+    if (k == kVolume) return visc ? volume_lds(EB) : EB * N * (S + D * S + F) * sizeof(R);
     if (k == kRk) return EB * N * (S + F) * sizeof(R);
     return 0;
+  }
+  // (a viscous volume block holds nt / kVolThreads elements, which is never more)
+  static constexpr size_t volume_lds(size_t EB) {
+    return EB * N * ((!kJumpOut<R> && jump_over_u<D, P> && F > S ? F : S) + (F > D * S ? F : D * S)) * sizeof(R);
   }
   static bool valid(int k, int nt, bool visc) {
     if (nt < 64 || nt > kMaxBlock) return false;
@@ -2671,8 +2685,9 @@ struct Runner {
     Work<R>& w = st.work<R>();
     const VFace<R> vf{st.fpart, w.Ufe, w.nf, w.dA, w.Bve, w.Jne, wave ? st.waveSpe : nullptr, st.bndBc, st.bst};
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
+    const int EB = nt / kVolThreads<D, P>;
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, nt / S)), dim3(nt), lds(kVolume, nt, true), c.stream, c.z.E, st.Ue, us,
+      hipLaunchKernelGGL(kern, dim3(nblk(c.z.E, EB)), dim3(nt), volume_lds(EB), c.stream, c.z.E, st.Ue, us,
                          w.JG, w.iJ, w.divFe, vf, st.tb, c.ph);
     };
     if constexpr (kBf16<D, P, R>) {
