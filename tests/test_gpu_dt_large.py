@@ -14,10 +14,11 @@ from oracle.oracle import Oracle
 pytestmark = pytest.mark.gpu
 
 
-# elements that 256 blocks of 256 threads have in flight: quads 8192 (P0 to P3), 4096 (P4);
-# hexes 8192 (P1), 4096 (P2)
-@pytest.mark.parametrize("kind,n,order,limit", [("vortex2d", 91, 0, 8192), ("vortex2d", 90, 3, 8192),
-                                                ("vortex2d", 91, 3, 8192), ("vortex2d", 65, 4, 4096),
+# elements that 256 blocks of 256 threads have in flight: quads 32768 (P0), 16384 (P1), 8192 (P3),
+# 4096 (P4); hexes 32768 (P0), 8192 (P1), 4096 (P2)
+@pytest.mark.parametrize("kind,n,order,limit", [("vortex2d", 182, 0, 32768), ("vortex2d", 129, 1, 16384),
+                                                ("vortex2d", 90, 3, 8192), ("vortex2d", 91, 3, 8192),
+                                                ("vortex2d", 65, 4, 4096), ("vortex3d", 33, 0, 32768),
                                                 ("vortex3d", 20, 1, 8192), ("vortex3d", 21, 1, 8192),
                                                 ("vortex3d", 17, 2, 4096)])
 def test_dt(kind, n, order, limit):
