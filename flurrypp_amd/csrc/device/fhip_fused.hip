@@ -2644,8 +2644,11 @@ struct Runner {
   // 13.3, 16^3 (10240) 23.2 / 19.5.  FP64 hexes of orders 1 to 3, whose
   // registers hold the other form to 3 waves per SIMD and whose blocks fill
   // their waves, gain further up: P2 20^3 (10125) 27.7 / 30.3, P3 16^3 (10240)
-  // 26.4 / 28.9, P2 28^3 (27783) 64.2 / 62.2.
-  static constexpr long long kApartWaves = D == 3 && P >= 1 && P <= 3 && sizeof(R) == 8 ? 12288 : 4096;
+  // 26.4 / 28.9, P2 28^3 (27783) 64.2 / 62.2.  P0, whose solution points would take 4
+  // or 6 rounds over flux points, stays apart at every size: quads 300x200 (4688)
+  // 15.1 / 22.7, 600x500 (23438) 42 / 49, hexes 60^3 (23625) 57 / 70, with walls 60 / 84.
+  static constexpr long long kApartWaves =
+      P == 0 ? 1ll << 40 : (D == 3 && P <= 3 && sizeof(R) == 8 ? 12288 : 4096);
   static bool apart(const Ctx& c) { return (long long)c.z.E * (S + F) <= kApartWaves * 64; }
   // LDS bytes of an element kernel at block size nt (0 for the face kernel)
   static size_t lds(int k, int nt, bool visc) {
@@ -2760,10 +2763,8 @@ struct Runner {
     const bool bnd = fs(c).nBnd > 0;
     // operators read from their tables: one instance for every mesh
     if (!fs(c).tb.w1) launch_stage_t<false, true, false, false, MK>(c, nt, ra, fold);
-    else if (apart(c) && bnd) launch_stage_t<false, true, true, true, MK>(c, nt, ra, fold);
-    else if (apart(c)) launch_stage_t<false, false, true, true, MK>(c, nt, ra, fold);
-    else if (bnd) launch_stage_t<false, true, true, false, MK>(c, nt, ra, fold);
-    else launch_stage_t<false, false, true, false, MK>(c, nt, ra, fold);
+    else if (apart(c)) bnd ? launch_stage_t<false, true, true, true, MK>(c, nt, ra, fold) : launch_stage_t<false, false, true, true, MK>(c, nt, ra, fold);
+    else if constexpr (P > 0) bnd ? launch_stage_t<false, true, true, false, MK>(c, nt, ra, fold) : launch_stage_t<false, false, true, false, MK>(c, nt, ra, fold);
   }
   static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src = false) {
     FusedState& st = fs(c);

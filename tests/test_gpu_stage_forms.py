@@ -1,6 +1,6 @@
 """Both forms of the inviscid stage kernel (solution and flux points in threads
 of their own, and in the same threads), on either side of the size where one
-takes over: E * (S + F) of 64 lanes * 4096 waves for quads.  Copies of one mesh
+takes over: E * (S + F) of 64 lanes * 4096 waves for quads (P0 has but one form).  Copies of one mesh
 merged into a context reach it; the element counts say which side each is on."""
 import numpy as np
 import pytest
@@ -23,7 +23,7 @@ def _apart(setup, copies=1):
 
 @pytest.mark.parametrize("path,rtol", [(PATH_FUSED, 1e-13), (PATH_MIXED, 1e-6)])
 @pytest.mark.parametrize("dt_type", [1, 2])
-@pytest.mark.parametrize("nx,ny,order,copies", [(201, 131, 0, 3), (160, 101, 1, 2), (101, 83, 2, 2), (67, 33, 3, 5),
+@pytest.mark.parametrize("nx,ny,order,copies", [(160, 101, 1, 2), (101, 83, 2, 2), (67, 33, 3, 5),
                                                 (60, 61, 4, 2), (45, 53, 5, 2)])
 def test_both_forms_agree(nx, ny, order, copies, dt_type, path, rtol):
     setup, U = cases.bump2d(nx=nx, ny=ny, order=order, cfl=0.3, dt_type=dt_type)
@@ -69,14 +69,16 @@ def test_multigrid_beyond_the_limit(time_type, dt_type):
     fine.close()
 
 
-@pytest.mark.parametrize("nt", [64, 192, 256])
-def test_block_sizes_of_p0(nt):
-    """P0 quads at block sizes other than the default, against the oracle."""
-    setup, U = cases.bump2d(nx=29, ny=13, order=0, cfl=0.3)
+@pytest.mark.parametrize("nx,ny,nt", [(29, 13, 64), (29, 13, 192), (29, 13, 256), (241, 223, 0)])
+def test_p0(nx, ny, nt):
+    """P0 quads at block sizes other than the default, and more of them than other
+    orders keep apart, against the oracle."""
+    setup, U = cases.bump2d(nx=nx, ny=ny, order=0, cfl=0.3)
     s, o = Solver(setup.params, setup=setup), Oracle.from_setup(setup)
     s.initializeSolution(U)
     o.initializeSolution(U, setup.params.dtType)
-    s.set_block_sizes([256, 64, nt, 64, 256], PATH_FUSED)
+    if nt:
+        s.set_block_sizes([256, 64, nt, 64, 256], PATH_FUSED)
     s.update(10, path=PATH_FUSED)
     o.update(10)
     assert np.linalg.norm(s.get_U() - o.get_U()) < 1e-12 * np.linalg.norm(o.get_U())
