@@ -1009,6 +1009,7 @@ template <class R>
 struct StageFace {
   const int* fpart;    // [E*F] 4 * partner flux point + side, or 4 * boundary slot + 2
   const R* Ufe;        // [E][N][F] U at the flux points, this stage's
+  const R* Fne;        // [E][N][F] kGiven: the common flux, at left and boundary points
   const R* nfe;        // [E][D][F] the face's normal (its left element's)
   const R* dA;         // [E][F] face area factor
   double* wave;        // wave speeds of the left and boundary points, or null: not read before they change again
@@ -1032,12 +1033,20 @@ struct StageFace {
 // (kApartWaves below).
 __host__ __device__ constexpr int up64(int n) { return (n + 63) / 64 * 64; }
 
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, bool MK = false>
+//
+// FORM: the usual one; kMakeSrc, a multigrid level's first smoothing stage (rk_point's
+// MK); kGiven, a single-stage step whose common flux was formed with the wave speeds
+// that its time step needs (k_wave_dt): it is read, once per pair, and U at the flux
+// points is not, so the new one takes its place.  Formed again here a step of
+// channels 200x150 P2 took 46.8 us (in two kernels 42.1), now 43.0; mixed 41.5 (34.6), 36.2.
+enum { kUsual = 0, kMakeSrc = 1, kGiven = 2 };
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, int FORM>
 __device__ __forceinline__ void stage_body(int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us,
                                            const R* __restrict__ JGe, const StageFace<R>& fc, const Tabs& tb,
                                            const Phys& ph, const RkArgs<R>& ra) {
   using Sh = Shape<D, P>;
   constexpr int S = Sh::S, F = Sh::F, N = Sh::N, P1 = Sh::P1;
+  constexpr bool MK = FORM == kMakeSrc, GV = FORM == kGiven;
   // U, the transformed flux and the flux jump of the block's elements:
   // [EB*N*S] [EB*D*N*S] [EB*N*F]
   R* const sU = reinterpret_cast<R*>(fhip_lds);
@@ -1094,6 +1103,18 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   auto load_face = [&](int u) {
     const int i = fi(u), bb = i / F, f = i - bb * F;
     const long long ob = (long long)(e0 + bb) * N * F + f;
+    if constexpr (GV) {
+      // the common flux, at the pair's left point
+      dA = ld_s<NT>(&fc.dA[(long long)e0 * F + i]);
+      long long pb = ob;
+      if ((cd[u] & 3) == 1) {
+        const int p = cd[u] >> 2, ep = p / F;
+        pb = (long long)ep * N * F + (p - ep * F);
+      }
+#pragma unroll
+      for (int k = 0; k < N; k++) fo[u][k] = fc.Fne[pb + k * F];
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < N; k++) own[k] = fc.Ufe[ob + k * F];
 #pragma unroll
@@ -1112,6 +1133,14 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
   // the common flux times this side's dA, negated on the right side
   auto common = [&](int u) {
     const int side = cd[u] & 3;
+    if constexpr (GV) {
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const R v = mul_rn(fo[u][k], dA);
+        fo[u][k] = side == 1 ? -v : v;
+      }
+      return;
+    }
     if constexpr (BND) {
       if (side == 2) bc_state<D, R>(fc.bndBc[cd[u] >> 2], own, n, oth, ph, fc.bst);
     }
@@ -1214,17 +1243,17 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
 
 // Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
 // for FP64 hexes.
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int FORM>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_w3(
     int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, APART, 0>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, 0, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF = 0, bool MK = false>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, int FORM>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
     int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, APART, BF, MK>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, BF, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
 
 // ---------------------------------------------------------------------------
@@ -1934,23 +1963,27 @@ __global__ __launch_bounds__(256) void k_ele_vol(int E, const double* __restrict
   vole[e] = vol;
 }
 
-// The dt kernel: lanes that sum one element's flux points (16 for the 4 of P0 quads
-// cost 300x200 of them 3 of 105 us a step), elements that a group
-// of lanes has in flight (2 for quads, 4 for hexes; 2 for both measured 10.6 and 4.9
-// us below), and blocks at most, each of which takes its turn at two atomics.  A
-// thread per element walked its points one after the other, each read 8 F bytes
-// from its neighbour's, on E/256 blocks, and each block's release wrote back the
-// L2.  Runs of 20, 10 and 4 steps on 32^2 P3, 17^3 P2 and 23^3 P4 mixed: 580 -> 547,
-// 886 -> 850, 1690 -> 1523 us.  Meshes that need more than kDtBlocks blocks of 256
-// threads take blocks of 1024, a wave's loads being what a block waits for: 30^3 P3 with
-// 256 / 1024 threads 42 / 22 us (the thread per element: 24), 48^3 P1 51 / 26 (34),
-// 400^2 P3 37 / 21 (34); 256 threads in more blocks take longer (30^3 P3, 1024
-// blocks: 26), and on small meshes 1024 threads do (8^3 P2 8.2 / 10.4).
+// The dt kernel: lanes that sum one element's flux points, elements that a group of
+// lanes has in flight, and blocks at most, each of which takes its turn at two atomics,
+// some 20 ns.  (A thread per element, each read 8 F bytes from its neighbour's, on E/256
+// blocks whose release wrote back the L2, took 8 to 52 us below.)  More lanes per
+// element than these are more blocks; fewer, longer chains: as many as flux points up
+// to 64, 16 for all, these, 8 for all: quads 86^2 P2 11.0, -, 8.6, 8.6 us, 64^2 P5 11.7,
+// -, 7.2, 7.2; hexes 17^3 P2 11.4, 9.5, 9.5, 9.6, 20^3 P3 13.4, 10.3, 10.3, 10.0, 23^3 P4
+// 20.2, 15.6, 15.6, 24.1, 48^3 P1 24.5, -, 16.3, 16.3.
+//
+// Meshes that need more than kDtSmall blocks of 256 threads take blocks of 1024:
+// fewer turns, and on more than kDtBlocks more loads in flight.  256 / 1024 threads:
+// quads 120^2 P2 (225 blocks) 11.0 / 8.9 us, 100^2 P3 (157) 9.1 / 8.5, 64^2 P5 (64) 7.3 /
+// 8.8; hexes 23^3 P4 (191) 15.8 / 26, 20^3 P3 (125) 10.3 / 13.3.  30^3 P3 with lanes for 64
+// flux points 42 / 22, in 1024 blocks of 256 threads 26; 400^2 P3 37 / 21.
 template <int F>
-constexpr int kDtLanes = F <= 4 ? 4 : (F <= 8 ? 8 : (F <= 16 ? 16 : (F <= 32 ? 32 : 64)));
+constexpr int kDtLanes = F <= 4 ? 4 : (F <= 24 ? 8 : 16);
 template <int D>
 constexpr int kDtEles = D == 2 ? 2 : 4;
 constexpr unsigned kDtBlocks = 256;
+template <int D>
+constexpr unsigned kDtSmall = D == 2 ? 128 : 256;
 
 // ele::calcDt per element (element-major inputs) and, with a ticket counter, the
 // minimum of all at out, the global dt (solver::calcDt, src/solver.cpp:447-468).
@@ -1995,13 +2028,13 @@ __global__ __launch_bounds__(NT) void k_ele_dt_em(int E, const double* __restric
   if (threadIdx.x == 0) grid_min(bmin, gridDim.x, acc, ticket, out);
 }
 
-// The wave speeds of the common inviscid flux at the left and boundary points, for
-// the steps that need them ahead of their stage kernel (face_first); right points
-// keep theirs (and, with Roe's flux, all but the boundary's).
+// The common inviscid flux and its wave speeds at the left and boundary points, for
+// the steps that need the speeds ahead of their stage kernel (face_first); right points
+// keep their speeds (and, with Roe's flux, all but the boundary's).
 template <int D, int P, class R>
 __global__ __launch_bounds__(kMaxBlock) void k_pair_wave(int n, const int* __restrict__ fpart, const R* __restrict__ Ufe,
                                                     const R* __restrict__ nfe, const int* __restrict__ bndBc,
-                                                    double* __restrict__ waveSpe, Phys ph,
+                                                    double* __restrict__ waveSpe, R* __restrict__ Fne, Phys ph,
                                                     const double* __restrict__ bst) {
   using Sh = Shape<D, P>;
   constexpr int F = Sh::F, N = Sh::N;
@@ -2024,23 +2057,29 @@ __global__ __launch_bounds__(kMaxBlock) void k_pair_wave(int n, const int* __res
   }
   double lam;
   if (pair_flux<D, R>(side == 2, UL, UR, nv, fn, ph, lam)) waveSpe[q] = lam;
+#pragma unroll
+  for (int k = 0; k < N; k++) Fne[((long long)e * N + k) * F + f] = fn[k];
 }
 
 // The same and the elements' time steps from them in one pass, up to kWaveDtPoints
 // flux points: one launch less, but in the dt kernel's blocks, which are too few for
-// the gathers of a large mesh.  Together / apart: channel 113x41 P3 (74 k points) 10.0 /
-// 14.7 us, quads 200^2 P2 (480 k) 17.0 / 21.9; 30^3 P3 (2.6 M) 64 / 56.
-constexpr long long kWaveDtPoints = 1 << 20;
+// the gathers of a large mesh.  A step of quads in one / two launches: 64^2 P4 (82 k
+// points) 23.7 / 26.5 us, 64^2 P5 (98 k) 28.4 / 29, 200^2 P3 (640 k) 62 / 57; hexes 6^3 P3 (21 k)
+// 18.3 / 22.
+constexpr long long kWaveDtPoints = 1 << 17;
+template <int D>
+constexpr int kWaveDtLanes = D == 2 ? 8 : 32;
 template <int D, int P, class R, int NT>
 __global__ __launch_bounds__(NT) void k_wave_dt(int E, const int* __restrict__ fpart, const R* __restrict__ Ufe,
                                                 const R* __restrict__ nfe, const int* __restrict__ bndBc,
                                                 const double* __restrict__ bst, Phys ph,
                                                 const double* __restrict__ vole, const double* __restrict__ wf,
-                                                double* waveSpe, const double* __restrict__ dAe, double cflfac,
+                                                double* waveSpe, R* __restrict__ Fne,
+                                                const double* __restrict__ dAe, double cflfac,
                                                 double* __restrict__ eleDt, double* acc, unsigned* ticket,
                                                 double* __restrict__ out) {
   using Sh = Shape<D, P>;
-  constexpr int F = Sh::F, Ff = Sh::Ff, N = Sh::N, G = kDtLanes<F>, EB = NT / G;
+  constexpr int F = Sh::F, Ff = Sh::Ff, N = Sh::N, G = kWaveDtLanes<D>, EB = NT / G;
   __shared__ double red[NT / 64];
   const int l = threadIdx.x % G;
   double dt = INFINITY;
@@ -2068,6 +2107,8 @@ __global__ __launch_bounds__(NT) void k_wave_dt(int E, const int* __restrict__ f
           for (int k = 0; k < N; k++) UR[k] = Ufe[((long long)ep * N + k) * F + (p - ep * F)];
         }
         if (pair_flux<D, R>(side == 2, UL, UR, n, fn, ph, lam)) waveSpe[q] = lam;
+#pragma unroll
+        for (int k = 0; k < N; k++) Fne[((long long)e * N + k) * F + f] = fn[k];
       }
       iw += lam * wf[f % Ff] * dAe[q];
     }
@@ -2388,8 +2429,8 @@ static void set_geometry(Ctx& c, Work<float>& w) {
 
 // A single-stage step with a CFL time step takes its dt from the wave speeds of
 // the residual it is about to apply (solver::update), so they are formed, and on
-// the refresh step replaced by the points' own, in launches of their own before it.
-// Its stage kernel then leaves them.
+// the refresh step replaced by the points' own, in launches of their own before it,
+// with the common flux, which its stage kernel then reads (kGiven).
 static bool face_first(const Ctx& c) { return !c.prm.viscous && c.z.nRK == 1 && c.prm.dt_type != 0; }
 // Whether a step's first stage forms the elements' time steps itself.
 static bool folds_dt(const Ctx& c) {
@@ -2706,20 +2747,20 @@ struct Runner {
     FCHK(hipGetLastError());
   }
   // inviscid runs: the stage kernel with the RK update ra
-  template <bool NT, bool BND, bool TEN, bool APART, bool MK = false>
+  template <bool NT, bool BND, bool TEN, bool APART, int FORM>
   static void launch_stage_t(Ctx& c, int nt, RkArgs<R> ra, bool fold) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     // wave speeds are read by the next step's dt and after the call: stages
     // that another stage follows leave them
-    const bool wave = (ra.fin && !face_first(c)) || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
-    const StageFace<R> fc{st.fpart, cur_ufe(c), w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
+    const bool wave = (ra.fin && FORM != kGiven) || ra.mode == 5 || ra.mode == 7 || ra.mode == 8;
+    const StageFace<R> fc{st.fpart, cur_ufe(c), w.Ufe2, w.nf, w.dA, wave ? st.waveSpe : nullptr, st.bndBc,
                           st.bst, fold ? c.wf : nullptr, st.waveSpe, st.dAe, st.vole,
                           fold ? c.prm.cfl * cfl_limit_f(P) : 0., c.eleDt};
-    ra.Ufe = st.flipped ? w.Ufe : w.Ufe2;
+    ra.Ufe = FORM == kGiven || st.flipped ? w.Ufe : w.Ufe2;
     const R* us = (sizeof(R) == 4 || st.read_stage) ? w.Us : nullptr;
     int EB = APART ? stage_eles(nt) : nt / S;
-    auto bytes = [&] { return stage_lds(EB) + (MK ? EB * F * sizeof(double) : 0); };
+    auto bytes = [&] { return stage_lds(EB) + (FORM == kMakeSrc ? EB * F * sizeof(double) : 0); };
     while (EB > 1 && bytes() > kMaxLds) EB--;
     const int threads = APART ? stage_threads(EB) : (EB == nt / S ? nt : EB * S);
     auto go = [&](auto kern) {
@@ -2727,13 +2768,13 @@ struct Runner {
                          w.JG, fc, st.tb, c.ph, ra);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 2>);
-      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 3>);
-      else go(k_stage_w4<D, P, R, NT, BND, TEN, APART>);
+      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 2, FORM>);
+      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 3, FORM>);
+      else go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, FORM>);
     } else if constexpr (kHold<D, R>) {
-      go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, MK>);
+      go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, FORM>);
     } else {
-      go(k_stage_w3<D, P, R, NT, BND, TEN, APART>);
+      go(k_stage_w3<D, P, R, NT, BND, TEN, APART, FORM>);
     }
     FCHK(hipGetLastError());
   }
@@ -2747,24 +2788,25 @@ struct Runner {
     if (bnd) launch_volume_t<false, true, true>(c, nt, wave);
     else launch_volume_t<false, false, true>(c, nt, wave);
   }
-  static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false) {
-    if constexpr (D == 2) {
-      if (ra.makeSrc) return launch_stage_i<true>(c, nt, ra, fold);
-    }
-    if constexpr (kEleRowsWhole) {
-      if (fs(c).tb.w1 && fs(c).stream)
-        return fs(c).nBnd > 0 ? launch_stage_t<true, true, true, false>(c, nt, ra, fold)
-                              : launch_stage_t<true, false, true, false>(c, nt, ra, fold);
-    }
-    launch_stage_i<false>(c, nt, ra, fold);
-  }
-  template <bool MK>
-  static void launch_stage_i(Ctx& c, int nt, const RkArgs<R>& ra, bool fold) {
+  static void launch_stage(Ctx& c, int nt, const RkArgs<R>& ra, bool fold = false, bool given = false) {
     const bool bnd = fs(c).nBnd > 0;
+    if (given) return launch_stage_f<kGiven, false>(c, nt, ra, fold);
+    if constexpr (D == 2) {
+      if (ra.makeSrc)
+        return bnd ? launch_stage_f<kMakeSrc, true>(c, nt, ra, fold) : launch_stage_f<kMakeSrc, false>(c, nt, ra, fold);
+    }
+    bnd ? launch_stage_f<kUsual, true>(c, nt, ra, fold) : launch_stage_f<kUsual, false>(c, nt, ra, fold);
+  }
+  // (with the flux given there is no boundary state to form)
+  template <int FORM, bool BND>
+  static void launch_stage_f(Ctx& c, int nt, const RkArgs<R>& ra, bool fold) {
     // operators read from their tables: one instance for every mesh
-    if (!fs(c).tb.w1) launch_stage_t<false, true, false, false, MK>(c, nt, ra, fold);
-    else if (apart(c)) bnd ? launch_stage_t<false, true, true, true, MK>(c, nt, ra, fold) : launch_stage_t<false, false, true, true, MK>(c, nt, ra, fold);
-    else if constexpr (P > 0) bnd ? launch_stage_t<false, true, true, false, MK>(c, nt, ra, fold) : launch_stage_t<false, false, true, false, MK>(c, nt, ra, fold);
+    if (!fs(c).tb.w1) return launch_stage_t<false, FORM != kGiven, false, false, FORM>(c, nt, ra, fold);
+    if constexpr (kEleRowsWhole && FORM != kMakeSrc) {
+      if (fs(c).stream) return launch_stage_t<true, BND, true, false, FORM>(c, nt, ra, fold);
+    }
+    if (apart(c)) return launch_stage_t<false, BND, true, true, FORM>(c, nt, ra, fold);
+    if constexpr (P > 0) launch_stage_t<false, BND, true, false, FORM>(c, nt, ra, fold);
   }
   static RkArgs<R> rk_args(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src = false) {
     FusedState& st = fs(c);
@@ -2852,7 +2894,7 @@ struct Runner {
     {
       // one mesh: the element kernel's last block forms the global minimum
       Launch L(c, nm("fused_ele_dt", "mixed_ele_dt"));
-      const auto [nt, nb] = dt_grid(c, 256 / kDtLanes<F> * kDtEles<D>, kDtBlocks);
+      const auto [nt, nb] = dt_grid(c, 256 / kDtLanes<F> * kDtEles<D>, kDtSmall<D>);
       auto* kern = nt == 1024 ? k_ele_dt_em<D, P, 1024> : k_ele_dt_em<D, P, 256>;
       hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.vole, c.wf, st.waveSpe, st.dAe, cflfac,
                          c.eleDt, st.dtAcc, st.nMesh == 1 ? st.dtTicket : nullptr, c.d_dt);
@@ -2860,27 +2902,29 @@ struct Runner {
     }
     mesh_dt(c);
   }
-  // wave speeds of the common flux, and the time steps from them
-  static void wave_dt(Ctx& c, double cflfac) {
+  // The common flux (into Ufe2), its wave speeds and the time steps from them; refresh:
+  // from the points' own speeds, which replace these.
+  static void wave_dt(Ctx& c, double cflfac, bool refresh) {
     FusedState& st = fs(c);
     Work<R>& w = st.work<R>();
     const int n = c.z.E * F;
-    if (n > kWaveDtPoints) {
+    if (n > kWaveDtPoints || refresh) {
       {
         Launch L(c, nm("fused_face_inviscid", "mixed_face_inviscid"));
         const int nt = blk(c, kFaceInv);
         hipLaunchKernelGGL((k_pair_wave<D, P, R>), dim3(nblk(n, nt)), dim3(nt), 0, c.stream, n, st.fpart, cur_ufe(c),
-                           w.nf, st.bndBc, st.waveSpe, c.ph, st.bst);
+                           w.nf, st.bndBc, st.waveSpe, w.Ufe2, c.ph, st.bst);
         FCHK(hipGetLastError());
       }
+      if (refresh) wave(c);
       return dt(c, cflfac);
     }
     {
       Launch L(c, nm("fused_wave_dt", "mixed_wave_dt"));
-      const auto [nt, nb] = dt_grid(c, 256 / kDtLanes<F>, 2 * kDtBlocks);
+      const auto [nt, nb] = dt_grid(c, 256 / kWaveDtLanes<D>, kDtSmall<D>);
       auto* kern = nt == 1024 ? k_wave_dt<D, P, R, 1024> : k_wave_dt<D, P, R, 256>;
       hipLaunchKernelGGL(kern, dim3(nb), dim3(nt), 0, c.stream, c.z.E, st.fpart, cur_ufe(c), w.nf, st.bndBc, st.bst,
-                         c.ph, st.vole, c.wf, st.waveSpe, st.dAe, cflfac, c.eleDt, st.dtAcc,
+                         c.ph, st.vole, c.wf, st.waveSpe, w.Ufe2, st.dAe, cflfac, c.eleDt, st.dtAcc,
                          st.nMesh == 1 ? st.dtTicket : nullptr, c.d_dt);
       FCHK(hipGetLastError());
     }
@@ -2906,10 +2950,10 @@ struct Runner {
   static void rk(Ctx& c, int mode, double a, double b, bool write0, int stage, bool make_src) {
     if (!c.prm.viscous) {
       Launch L(c, nm("fused_stage", "mixed_stage"));
+      const bool update = mode != 5 && mode != 7 && mode != 8, given = update && face_first(c);
       launch_stage(c, blk(c, kVolume), rk_args(c, mode, a, b, write0, stage, make_src),
-                   folds_dt(c) && (mode == 0 || mode == 6));
-      // (the residual alone leaves U)
-      if (mode != 5 && mode != 7 && mode != 8) fs(c).flipped = !fs(c).flipped;
+                   folds_dt(c) && (mode == 0 || mode == 6), given);
+      if (update && !given) fs(c).flipped = !fs(c).flipped;
       return;
     }
     Launch L(c, nm("fused_rk_update", "mixed_rk_update"));
@@ -3008,7 +3052,7 @@ struct Ops {
   void (*extrap)(Ctx&);
   void (*wave)(Ctx&);
   void (*dt)(Ctx&, double);
-  void (*wave_dt)(Ctx&, double);
+  void (*wave_dt)(Ctx&, double, bool);
   void (*residual)(Ctx&, bool);
   void (*rk)(Ctx&, int, double, double, bool, int, bool);
   void (*ensure)(Ctx&);
@@ -3291,8 +3335,8 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
   const bool jameson = c.prm.time_type >= 5;
   if (nRK == 1) {
     if (c.prm.viscous) o.residual(c, true);
-    if (cfl && !refresh && face_first(c)) {
-      o.wave_dt(c, cflfac);
+    if (face_first(c)) {
+      o.wave_dt(c, cflfac, refresh);
     } else if (cfl) {
       if (refresh) o.wave(c);
       o.dt(c, cflfac);
@@ -3318,7 +3362,7 @@ void fused_rk_step(Ctx& c, bool refresh, bool mixed, bool keep, bool make_src) {
 
 bool fused_flipped(const Ctx& c) { return ((const FusedState*)c.fused)->flipped; }
 void fused_set_flipped(Ctx& c, bool flipped) { fs(c).flipped = flipped; }
-bool fused_step_flips(const Ctx& c) { return !c.prm.viscous && (c.z.nRK & 1); }
+bool fused_step_flips(const Ctx& c) { return !c.prm.viscous && (c.z.nRK & 1) && !face_first(c); }
 
 #endif  // FHIP_FAMILY
 

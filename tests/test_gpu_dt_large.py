@@ -1,5 +1,5 @@
-"""The CFL time step's kernel on meshes that take its large blocks (more than 256
-blocks of 256 threads): just past the limit, ragged, with one block's worth over,
+"""The CFL time step's kernel on meshes that take its large blocks (more than 128
+or 256 blocks of 256 threads): just past the limit, ragged, with one block's worth over,
 and merged meshes, which never do.  Against the oracle; twice, since a launch
 leaves the counters for the next."""
 import numpy as np
@@ -14,13 +14,13 @@ from oracle.oracle import Oracle
 pytestmark = pytest.mark.gpu
 
 
-# elements that 256 blocks of 256 threads have in flight: quads 32768 (P0), 16384 (P1), 8192 (P3),
-# 4096 (P4); hexes 32768 (P0), 8192 (P1), 4096 (P2)
-@pytest.mark.parametrize("kind,n,order,limit", [("vortex2d", 182, 0, 32768), ("vortex2d", 129, 1, 16384),
-                                                ("vortex2d", 90, 3, 8192), ("vortex2d", 91, 3, 8192),
-                                                ("vortex2d", 65, 4, 4096), ("vortex3d", 33, 0, 32768),
-                                                ("vortex3d", 20, 1, 8192), ("vortex3d", 21, 1, 8192),
-                                                ("vortex3d", 17, 2, 4096)])
+# elements in flight in 128 blocks (quads) or 256 (hexes): quads 16384 (P0), 8192 (P1 to P5); hexes
+# 32768 (P0, P1), 16384 (P2)
+@pytest.mark.parametrize("kind,n,order,limit", [("vortex2d", 129, 0, 16384), ("vortex2d", 90, 1, 8192),
+                                                ("vortex2d", 91, 1, 8192), ("vortex2d", 91, 3, 8192),
+                                                ("vortex2d", 91, 5, 8192), ("vortex3d", 33, 0, 32768),
+                                                ("vortex3d", 32, 1, 32768), ("vortex3d", 33, 1, 32768),
+                                                ("vortex3d", 26, 2, 16384)])
 def test_dt(kind, n, order, limit):
     setup, U = getattr(cases, kind)(n=n, order=order)
     print(f"{kind} {n} P{order}: {setup.nEles} elements, limit {limit}", flush=True)

@@ -130,11 +130,12 @@ def _euler_step(setup):
 
 @pytest.mark.parametrize("path", [PATH_FUSED, PATH_MIXED])
 @pytest.mark.parametrize("make", [
-    lambda: cases.bump2d(nx=131, ny=67, order=3, dt_type=2, cfl=0.3),   # 8777 of 16 points: blocks of 1024
-    lambda: cases.bump2d(nx=128, ny=64, order=3, dt_type=1, cfl=0.3),   # 8192: the last of 256
-    lambda: cases.vortex2d(n=257, order=3, cfl=0.3),                    # 1.06 million points: in two launches
-    lambda: cases.vortex3d(n=4, order=3), lambda: cases.vortex3d(n=13, order=4)],
-    ids=["quads_1024", "quads_256", "quads_apart", "hexes_256", "hexes_1024"])
+    lambda: cases.bump2d(nx=67, ny=61, order=3, dt_type=2, cfl=0.3),    # 4087 of 8 lanes: the last in 256 threads
+    lambda: cases.bump2d(nx=69, ny=61, order=3, dt_type=1, cfl=0.3),    # 4209: blocks of 1024
+    lambda: cases.vortex2d(n=91, order=3, cfl=0.3),                     # 132 k points: in two launches
+    lambda: cases.vortex3d(n=4, order=3), lambda: cases.vortex3d(n=16, order=1),  # 4096 of 24 points, 2048 a turn
+    lambda: cases.vortex3d(n=11, order=4)],
+    ids=["quads_256", "quads_1024", "quads_apart", "hexes_256", "hexes_1024", "hexes_apart"])
 def test_wave_speeds_and_time_steps(make, path):
     """The pass that forms both, at the edges of its block sizes and past its limit."""
     setup, U = make()
