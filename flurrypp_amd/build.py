@@ -12,6 +12,7 @@ import hashlib
 import os
 import subprocess
 import sys
+import tempfile
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -71,28 +72,32 @@ def build_host() -> Path:
 
 def build_hip() -> Path:
     """Each source to an object (in parallel: each holds its own kernels and
-    their launches), then one shared library."""
+    their launches), then one shared library.  The objects lie in a folder of this
+    build's own: linked with those of another build, also a killed one's, every
+    kernel would be there twice."""
     LIB.mkdir(exist_ok=True)
     out = LIB / "libflurry_hip.so"
     dev = CSRC / "device"
-    obj = LIB / "obj"
-    obj.mkdir(exist_ok=True)
     # the fused kernels' file is compiled per family of shapes, too
     units = [(n, n, []) for n in ("fhip_api", "fhip_staged", "fhip_fused")]
     units += [(f"fhip_fused_{k}", "fhip_fused", [f"-DFHIP_FAMILY={k}"]) for k in range(6)]
     names = [u[0] for u in units]
     digest = source_hash("hip")
-    procs = []
-    for n, src, defs in units:
-        cmd = [HIPCC, *HIP_FLAGS, *defs, f"-I{INC}", f"-I{dev}", "-c", str(dev / f"{src}.hip"), "-o", str(obj / f"{n}.o")]
-        print("+", " ".join(cmd), flush=True)
-        procs.append(subprocess.Popen(cmd))
-    bad = [n for n, p in zip(names, procs) if p.wait() != 0]
-    if bad:
-        raise subprocess.CalledProcessError(1, f"hipcc {' '.join(bad)}")
-    tmp = out.with_suffix(".so.tmp")
-    _run([HIPCC, *HIP_FLAGS, "-shared", *(str(obj / f"{n}.o") for n in names), "-o", str(tmp)])
-    os.replace(tmp, out)
+    (LIB / "obj").mkdir(exist_ok=True)
+    with tempfile.TemporaryDirectory(dir=LIB / "obj") as own:
+        obj = Path(own)
+        procs = []
+        for n, src, defs in units:
+            cmd = [HIPCC, *HIP_FLAGS, *defs, f"-I{INC}", f"-I{dev}", "-c", str(dev / f"{src}.hip"),
+                   "-o", str(obj / f"{n}.o")]
+            print("+", " ".join(cmd), flush=True)
+            procs.append(subprocess.Popen(cmd))
+        bad = [n for n, p in zip(names, procs) if p.wait() != 0]
+        if bad:
+            raise subprocess.CalledProcessError(1, f"hipcc {' '.join(bad)}")
+        so = obj / out.name
+        _run([HIPCC, *HIP_FLAGS, "-shared", *(str(obj / f"{n}.o") for n in names), "-o", str(so)])
+        os.replace(so, out)
     _stamp(out).write_text(digest + "\n")
     return out
 
