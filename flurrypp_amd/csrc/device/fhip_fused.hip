@@ -66,6 +66,8 @@ struct Shape {
 // each kernel is chosen per context (default 256, or by fused_autotune).
 extern __shared__ __align__(16) unsigned char fhip_lds[];
 constexpr int kMaxBlock = 512;
+// Dynamic LDS that a block may take.  (The factors of the operators are up to 480
+// bytes of static LDS more; a workgroup may have 160 KiB.)
 constexpr size_t kMaxLds = 64 * 1024;
 constexpr long long kStreamBytes = 64ll << 20;
 // (kVolume: the stage kernel on inviscid runs; kFaceBnd: no kernel, the place in
@@ -1297,7 +1299,7 @@ constexpr int kVolThreads = P <= 1 || (D == 2 && P == 2) ? Shape<D, P>::F : Shap
 
 // Volume kernel of viscous runs: all of a stage's residual but the other sides'
 // parts of the LDG flux.  Solution points and then flux points in the same
-// threads, EB elements per block, element data staged in LDS.
+// threads (kVolThreads an element), EB elements per block, element data in LDS.
 //
 // What a stage costs is its traffic, and most of that was intermediates: the
 // common inviscid flux and the common U, written by a face kernel and read here
@@ -1305,8 +1307,9 @@ constexpr int kVolThreads = P <= 1 || (D == 2 && P == 2) ? Shape<D, P>::F : Shap
 // sides of a pair now form the common flux from U there and across (one read of
 // U at the flux points; the own side is extrapolated again from the slab), and
 // FP64 corrects the divergence with this side's part of the jump before it is
-// written: 7.3 -> 4.6 GB per stage at 48^3 P3.  Sums that form a value are pinned before what uses them: otherwise
-// both are live at once and the FP64 P3 kernel spills 136 registers.
+// written: 7.3 -> 4.6 GB per stage at 48^3 P3.  Sums that form a value are pinned
+// before what uses them: otherwise both are live at once and the FP64 P3 kernel
+// spills 136 registers.
 // Measured, three kernels -> two: Navier-Stokes Taylor-Green 4 steps, 48^3 P3
 // 20.07 -> 16.8 ms; 37^3 P2 6.89 -> 4.30 ms; 40^3 P3 mixed 7.93 -> 6.86 ms; 21^3
 // P4 with monitor 1.43 -> 1.22 ms.
@@ -1692,9 +1695,9 @@ __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) 
 }
 
 // After the viscous volume kernel: correction of the divergence with the other
-// sides' LDG parts (FP32: with the whole flux jump), RK update and U at the flux points.  With NT, the arrays
-// this kernel reads or writes exactly once per launch go through nontemporal
-// loads and stores (they stream past the caches).
+// sides' LDG parts (FP32: with the whole flux jump), RK update and U at the flux
+// points.  With NT, the arrays this kernel reads or writes exactly once per launch
+// go through nontemporal loads and stores (they stream past the caches).
 template <int D, int P, class R, bool NT, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ divFe, RkArgs<R> ra, Tabs tb,
                                              const int* __restrict__ fpart, const R* __restrict__ dAe,
@@ -1759,6 +1762,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_rk(int E, const R* __restrict__ d
 }
 
 
+#ifndef FHIP_FAMILY
 // P-multigrid transfers in element-major layout ([ele][field][point] rows of
 // S values), the products the staged operator GEMM forms in FlurryPP's layout
 // with the same sums (chunks of kc columns of the operator, added in turn).
@@ -1815,6 +1819,8 @@ static __global__ void k_prolong_em(long long rows, int Su, int Sc, int kc, cons
   }
   Uu[t] = c;
 }
+
+#endif  // FHIP_FAMILY
 
 // The same transfers with the operator (transposed, so that the lanes of a
 // wave read consecutive entries) and the rows of the block's EB elements staged in
@@ -2141,6 +2147,7 @@ static __global__ void k_mesh_dt_min(const int* __restrict__ start, const double
   if (threadIdx.x == 0) meshDt[m] = red[0];
 }
 
+#ifndef FHIP_FAMILY
 // Per-mesh residual norm over divF_spts[0] (element-major), as
 // ele::getNormResidual summed over the mesh's elements (src/ele.cpp:1922-1945).
 static __global__ void k_mesh_res(int S, int N, int type, const int* __restrict__ start, const double* __restrict__ divF0e,
@@ -2168,6 +2175,8 @@ static __global__ void k_mesh_res(int S, int N, int type, const int* __restrict_
     __syncthreads();
   }
 }
+
+#endif  // FHIP_FAMILY
 
 // ---------------------------------------------------------------------------
 // Host side.

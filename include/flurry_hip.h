@@ -193,17 +193,22 @@ int fhip_path_supported(fhip_ctx* ctx, int path);
 enum { FHIP_OPT_GRAPHS = 1 };
 int fhip_set_option(fhip_ctx* ctx, int option, int value);
 
-/* Block sizes (threads per block, 64..512) of the fused kernels, in the order
- * extrapolate, face_inviscid (wave speeds of single-stage inviscid steps),
- * volume (inviscid runs: the whole stage), face_boundary (unused: boundary
- * points are the volume kernel's), rk_update (viscous runs), for path
- * FHIP_PATH_FUSED or FHIP_PATH_MIXED (no counterpart in the reference, which
- * has no kernels).  fhip_autotune times every valid size of every kernel on
- * the context's current data, keeps the fastest and returns them in
- * block_sizes (may be NULL); the state is left unchanged.  Results are cached
- * for the process per (nDims, order, precision, viscous, log2 nEles).  Block
- * shapes never change results.  Default 256 each, or the largest multiple
- * of 64 below it whose LDS slabs fit 64 KiB (P0 hexes). */
+/* Block sizes (64..512) of the fused kernels, in the order extrapolate,
+ * face_inviscid (wave speeds of large single-stage inviscid steps), volume
+ * (inviscid runs: the whole stage), face_boundary (unused: boundary points are
+ * the volume kernel's), rk_update (viscous runs), for path FHIP_PATH_FUSED or
+ * FHIP_PATH_MIXED (no counterpart in the reference, which has no kernels).  A
+ * size is the threads of a block; where the stage kernel gives solution and
+ * flux points waves of their own (small inviscid meshes, P0), it bounds the
+ * elements of a block, whose threads are those waves' (one element at least,
+ * also where that is more threads).  fhip_autotune times every valid size of
+ * the kernels that take part in most of a run (extrapolate, volume, and
+ * rk_update on viscous runs) on the context's current data, keeps the fastest
+ * and returns all five in block_sizes (may be NULL), the others as they were;
+ * the state is left unchanged.  Results are cached for the process per (nDims,
+ * order, precision, viscous, log2 nEles, form of the kernels).  Block shapes
+ * never change results.  Default 256 each, or the largest multiple of 64 below
+ * it whose LDS slabs fit 64 KiB (P0 hexes). */
 int fhip_autotune(fhip_ctx* ctx, int path, int* block_sizes);
 int fhip_set_block_sizes(fhip_ctx* ctx, int path, const int* block_sizes);
 int fhip_get_block_sizes(fhip_ctx* ctx, int path, int* block_sizes);
