@@ -925,7 +925,7 @@ __device__ __forceinline__ void face_point(int i, int e0, const Packed<P + 1>& l
 }
 
 // Shapes whose volume kernel is held to 4 waves per SIMD (128 VGPRs): quads
-// and the FP32 path.  FP64 hexes need more registers and are held to 3.
+// and the FP32 path (but its BF16 forms).  FP64 hexes need more registers and are held to 3.
 template <int D, class R>
 constexpr bool kHold = D == 2 || sizeof(R) == 4;
 
@@ -1244,18 +1244,19 @@ __device__ __forceinline__ void stage_body(int E, int EB, const double* __restri
 }
 
 // Held as the viscous volume kernels: 4 waves per SIMD for quads and FP32, 3
-// for FP64 hexes.
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int FORM>
+// for FP64 hexes and the BF16 forms (which spill 41-78 VGPRs under 4: Taylor-Green
+// 30^3 142.9 us, under 3 107.6).
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, int FORM>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_stage_w3(
     int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, APART, 0, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, BF, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
-template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int BF, int FORM>
+template <int D, int P, class R, bool NT, bool BND, bool TEN, bool APART, int FORM>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_stage_w4(
     int E, int EB, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, StageFace<R> fc, Tabs tb,
     Phys ph, RkArgs<R> ra) {
-  stage_body<D, P, R, NT, BND, TEN, APART, BF, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
+  stage_body<D, P, R, NT, BND, TEN, APART, 0, FORM>(E, EB, Ue, Us, JGe, fc, tb, ph, ra);
 }
 
 // ---------------------------------------------------------------------------
@@ -1680,18 +1681,20 @@ __device__ __forceinline__ void volume_body(int E, const double* __restrict__ Ue
 // The volume kernel held to 4 waves per SIMD (at most 128 VGPRs) for quads
 // and the FP32 path, which fit there without spilling (holding the FP32
 // viscous hex kernel to 5 or 6 waves spills 26 or 41 VGPRs and was measured
-// 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes.
-template <int D, int P, class R, bool NT, bool BND, bool TEN>
+// 13-16% slower), and to 3 waves (168 VGPRs) for FP64 hexes and for the BF16 forms,
+// whose pieces of a whole column and its accumulators are live at once: 153 VGPRs, under
+// the 4-wave hold 21-29 spilled (Navier-Stokes Taylor-Green 24^3 84.1 us, under 3 67.8).
+template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_volume_w3(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, const R* __restrict__ iJe,
     R* __restrict__ divFe, VFace<R> vf, Tabs tb, Phys ph) {
-  volume_body<D, P, R, NT, BND, TEN>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
+  volume_body<D, P, R, NT, BND, TEN, BF>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
 }
-template <int D, int P, class R, bool NT, bool BND, bool TEN, int BF = 0>
+template <int D, int P, class R, bool NT, bool BND, bool TEN>
 __global__ __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_volume_w4(
     int E, const double* __restrict__ Ue, const R* __restrict__ Us, const R* __restrict__ JGe, const R* __restrict__ iJe,
     R* __restrict__ divFe, VFace<R> vf, Tabs tb, Phys ph) {
-  volume_body<D, P, R, NT, BND, TEN, BF>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
+  volume_body<D, P, R, NT, BND, TEN>(E, Ue, Us, JGe, iJe, divFe, vf, tb, ph);
 }
 
 // After the viscous volume kernel: correction of the divergence with the other
@@ -2730,7 +2733,7 @@ struct Runner {
   // U at the flux points of the current state
   static R* cur_ufe(Ctx& c) { return fs(c).flipped ? fs(c).work<R>().Ufe2 : fs(c).work<R>().Ufe; }
   // viscous runs: the volume kernel.  Quads and FP32 are held to 4 waves per
-  // SIMD (128 VGPRs); FP64 hexes, which spill under that hold, to 3 (168 VGPRs:
+  // SIMD (128 VGPRs); FP64 hexes and the BF16 forms, which spill under that hold, to 3 (168 VGPRs:
   // P3 without spills, where the unheld compiler would take 211 and leave 2
   // waves)
   template <bool NT, bool BND, bool TEN>
@@ -2745,8 +2748,8 @@ struct Runner {
                          w.JG, w.iJ, w.divFe, vf, st.tb, c.ph);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_volume_w4<D, P, R, NT, BND, TEN, 2>);
-      else if (c.bf16 == 3) go(k_volume_w4<D, P, R, NT, BND, TEN, 3>);
+      if (c.bf16 == 2) go(k_volume_w3<D, P, R, NT, BND, TEN, 2>);
+      else if (c.bf16 == 3) go(k_volume_w3<D, P, R, NT, BND, TEN, 3>);
       else go(k_volume_w4<D, P, R, NT, BND, TEN>);
     } else if constexpr (kHold<D, R>) {
       go(k_volume_w4<D, P, R, NT, BND, TEN>);
@@ -2777,13 +2780,13 @@ struct Runner {
                          w.JG, fc, st.tb, c.ph, ra);
     };
     if constexpr (kBf16<D, P, R>) {
-      if (c.bf16 == 2) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 2, FORM>);
-      else if (c.bf16 == 3) go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 3, FORM>);
-      else go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, FORM>);
+      if (c.bf16 == 2) go(k_stage_w3<D, P, R, NT, BND, TEN, APART, 2, FORM>);
+      else if (c.bf16 == 3) go(k_stage_w3<D, P, R, NT, BND, TEN, APART, 3, FORM>);
+      else go(k_stage_w4<D, P, R, NT, BND, TEN, APART, FORM>);
     } else if constexpr (kHold<D, R>) {
-      go(k_stage_w4<D, P, R, NT, BND, TEN, APART, 0, FORM>);
+      go(k_stage_w4<D, P, R, NT, BND, TEN, APART, FORM>);
     } else {
-      go(k_stage_w3<D, P, R, NT, BND, TEN, APART, FORM>);
+      go(k_stage_w3<D, P, R, NT, BND, TEN, APART, 0, FORM>);
     }
     FCHK(hipGetLastError());
   }
