@@ -435,6 +435,10 @@ struct Work {
   }
 };
 
+// The kernels whose block sizes a run uses: FP64 0, mixed 1, mixed with 2 or 3 BF16
+// pieces 2 or 3.
+static int tune_form(const Ctx& c, bool mixed) { return mixed ? std::max(c.bf16, 1) : 0; }
+
 struct FusedState {
   Tabs tb{};
   void* tab_mem = nullptr;
@@ -470,8 +474,11 @@ struct FusedState {
   // element-major) exceeds kStreamBytes, i.e. a stage's arrays are many times
   // the 256 MiB infinity cache
   bool stream = false;
-  // block size of each kernel (kExtrap..kRk) for FP64 [0] and mixed [1]
-  int nt[2][5] = {{256, 256, 256, 256, 256}, {256, 256, 256, 256, 256}};
+  // block size of each kernel (kExtrap..kRk), by tune_form()
+  int nt[4][5] = {{256, 256, 256, 256, 256},
+                  {256, 256, 256, 256, 256},
+                  {256, 256, 256, 256, 256},
+                  {256, 256, 256, 256, 256}};
   Work<double> w64;
   Work<float> w32;
   ~FusedState() {
@@ -2677,7 +2684,7 @@ struct Runner {
   // The element kernels store rows of S or F values per field; a wave's
   // streamed store covers whole blocks only when those rows are whole blocks.
   static constexpr bool kEleRowsWhole = (S * sizeof(R)) % 64 == 0 && (F * sizeof(R)) % 64 == 0;
-  static int& blk(Ctx& c, int k) { return fs(c).nt[sizeof(R) == 4 ? 1 : 0][k]; }
+  static int& blk(Ctx& c, int k) { return fs(c).nt[tune_form(c, sizeof(R) == 4)][k]; }
   // Elements of a block of the stage kernel's form with solution and flux points
   // apart, within nt threads (one at least), and its threads: whole waves of
   // solution points, then whole waves of flux points
@@ -3116,17 +3123,21 @@ static Ops get_ops(const Ctx& c, bool mixed) {
   return mixed ? ops_3d_f32_high(P) : ops_3d_f64_high(P);
 }
 
-// Tuned block sizes, shared by the contexts of one process: keyed by
-// (nDims, order, precision, viscous, log2 of the element count) and by what else
-// decides which kernels run: the form of the stage kernel (inviscid runs; it
-// changes within one log2 of the element count), operators from factors or tables.
+// Tuned block sizes, shared by the contexts of one process: keyed by (nDims, order,
+// tune_form, viscous, log2 of the element count) and by what else decides which
+// kernels run: the form of the stage kernel (inviscid runs; it changes within one
+// log2 of the element count), operators from factors or tables.  The BF16 kernels
+// are held to 3 waves per SIMD, under which a CU takes one block of 512 threads and
+// no two: on Taylor-Green 48^3 512 threads are the mixed path's best size or close
+// to it, and the BF16 forms' worst but ragged ones (stage 567 us, 410 with 128;
+// Navier-Stokes volume 703 us, 505).
 static std::mutex g_tune_mu;
 static std::map<std::array<int, 7>, std::array<int, 5>> g_tuned;
 
 void fused_autotune(Ctx& c, bool mixed, int* out) {
   FusedState& st = fs(c);
   Ops o = get_ops(c, mixed);
-  const int m = mixed ? 1 : 0;
+  const int m = tune_form(c, mixed);
   int lg = 0;
   for (long long e = c.z.E; e > 1; e >>= 1) lg++;
   const bool visc = c.prm.viscous != 0;
@@ -3157,12 +3168,12 @@ void fused_set_blocks(Ctx& c, bool mixed, const int* nt) {
   Ops o = get_ops(c, mixed);
   if (!o.check(c, nt)) throw std::invalid_argument("block size not valid for this kernel and order");
   c.drop_graphs();
-  std::copy(nt, nt + 5, fs(c).nt[mixed ? 1 : 0]);
+  std::copy(nt, nt + 5, fs(c).nt[tune_form(c, mixed)]);
 }
 
 void fused_get_blocks(Ctx& c, bool mixed, int* out) {
   get_ops(c, mixed).fit(c);
-  const int* nt = fs(c).nt[mixed ? 1 : 0];
+  const int* nt = fs(c).nt[tune_form(c, mixed)];
   std::copy(nt, nt + 5, out);
 }
 

@@ -197,7 +197,7 @@ int fhip_set_option(fhip_ctx* ctx, int option, int value);
  * face_inviscid (wave speeds of large single-stage inviscid steps), volume
  * (inviscid runs: the whole stage), face_boundary (unused: boundary points are
  * the volume kernel's), rk_update (viscous runs), for path FHIP_PATH_FUSED or
- * FHIP_PATH_MIXED (no counterpart in the reference, which has no kernels).  A
+ * a mixed one (no counterpart in the reference, which has no kernels).  A
  * size is the threads of a block; where the stage kernel gives solution and
  * flux points waves of their own (small inviscid meshes, P0), it bounds the
  * elements of a block, whose threads are those waves' (one element at least,
@@ -206,9 +206,9 @@ int fhip_set_option(fhip_ctx* ctx, int option, int value);
  * rk_update on viscous runs) on the context's current data, keeps the fastest
  * and returns all five in block_sizes (may be NULL), the others as they were;
  * the state is left unchanged.  Results are cached for the process per (nDims,
- * order, precision, viscous, log2 nEles, form of the kernels).  Block shapes
- * never change results.  Default 256 each, or the largest multiple of 64 below
- * it whose LDS slabs fit 64 KiB (P0 hexes). */
+ * order, path, viscous, log2 nEles, form of the kernels).  Each fused path has
+ * sizes of its own.  Block shapes never change results.  Default 256 each, or
+ * the largest multiple of 64 below it whose LDS slabs fit 64 KiB (P0 hexes). */
 int fhip_autotune(fhip_ctx* ctx, int path, int* block_sizes);
 int fhip_set_block_sizes(fhip_ctx* ctx, int path, const int* block_sizes);
 int fhip_get_block_sizes(fhip_ctx* ctx, int path, int* block_sizes);
