@@ -327,7 +327,7 @@ class Solver:
         return out
 
     def desc_arrays(self) -> dict:
-        """The host arrays handed to fhip_create (for checkers)."""
+        """The host arrays handed to fhip_create (for tests)."""
         o, g, f = self.opers, self.geo, self.faces
         return dict(opers=o, geo=g, faces=f, params=self._fp)
 

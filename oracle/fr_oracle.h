@@ -2,7 +2,7 @@
  * fr_oracle.h -- CPU restatement of FlurryPP's FR residual and RK update.
  *
  * TEST INFRASTRUCTURE ONLY.  Only tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py may load this library, and only as the checker
+ * cpu_baseline leg of bench.py may load this library, and only as the oracle
  * or the CPU baseline; nothing in flurrypp_amd/ may call it.
  *
  * The restatement follows src/solver.cpp:319-1158, src/face.cpp:119-615,

@@ -1,7 +1,7 @@
 """ctypes wrapper of the CPU restatement (liboracle_fr.so, fr_oracle.h).
 
 TEST INFRASTRUCTURE ONLY: used by tests/, __graft_entry__.smoke() and the
-cpu_baseline leg of bench.py as the checker or the CPU baseline.
+cpu_baseline leg of bench.py as the oracle or the CPU baseline.
 """
 from __future__ import annotations
 

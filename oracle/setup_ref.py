@@ -1,6 +1,6 @@
 """Literal restatement of FlurryPP's face construction, for small meshes.
 
-TEST INFRASTRUCTURE ONLY (the checker of libflurry_host's O(n) set-up).
+TEST INFRASTRUCTURE ONLY (what the tests hold libflurry_host's O(n) set-up to).
 
 It follows the reference step by step, including its quadratic searches:
   processConn2D / processConn3D   src/geo.cpp:221-570 (matrix::unique, src/matrix.cpp:668-695)
